@@ -95,6 +95,31 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch():
         assert torch.equal(one[0], full[r])
 
 
+@pytest.mark.parametrize("N,K,shift", [(37, 64, 0), (48, 4096, 0), (130, 288, 0), (130, 292, 0), (65, 1027, 0), (96, 320, 1),
+                                       (6144, 96, 0), (6150, 260, 0)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_f32_kernels_give_one_row_the_same_bits(N, K, shift, accumulate):
+    """Every number of rows at which the kernel changes (8 / 9, 16 / 17, 32 / 33 rows, tiles of 32 and 64), output widths and
+    K that fill no tile, K that 16-byte loads do not take, rows that do not start on 16 bytes (`shift`): within the bound of
+    the sums' order (a chain of at most K / 8 + 32 roundings of half an ulp a segment, eight segments, the addition), and
+    the same bits for every number of rows."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(N + K)
+    most = 200
+    x = torch.randn(most, K + shift, generator=g).to(DEV)[:, shift:]
+    w = torch.randn(N, K + shift, generator=g).to(DEV)[:, shift:]
+    c0 = torch.randn(most, N, generator=g).to(DEV)
+    full = c0.clone()
+    ops.linear(full, x, w, accumulate=accumulate)
+    ref = x.double() @ w.double().t() + (c0.double() if accumulate else 0)
+    mag = x.abs().double() @ w.abs().double().t() + c0.abs().double()
+    assert ((full.double() - ref).abs() <= (K / 8 + 48) * 2.0 ** -24 * mag).all()
+    for m in (1, 2, 8, 9, 16, 17, 31, 32, 33, 63, 64, 65, 128, 129):
+        out = c0[:m].clone()
+        ops.linear(out, x[:m], w, accumulate=accumulate)
+        assert torch.equal(out, full[:m]), f"{m} rows"
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (1, 4096, 4096), (8, 100, 256), (16, 33, 1000), (17, 64, 128),
                                    (64, 172, 96), (5, 96, 172), (33, 320, 96), (3, 50, 20)])
 @pytest.mark.parametrize("kernel", [1, 2])

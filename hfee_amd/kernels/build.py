@@ -35,7 +35,7 @@ FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-fvisibility=h
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument"]
 
-CORE_SOURCES = ["elementwise.hip", "gemm_f32.hip", "attention_ref.hip", "gemm_bf16.hip", "gemm_skinny.hip",
+CORE_SOURCES = ["elementwise.hip", "gemm_f32.hip", "attention_ref.hip", "attention_f32.hip", "gemm_bf16.hip", "gemm_skinny.hip",
                 "sampling.hip", "random_fill.hip", "yardstick.hip", "attention_kv.hip", "rowwise.hip", "attention_mix.hip",
                 "recurrent.hip", "moe.hip", "gated_rows.hip", "post_norm.hip", "linear_chunks.hip",
                 "grouped_rows.hip", "delta_chunks.hip"]

@@ -393,10 +393,11 @@ def rope_cache_write(q, k, v, positions, token_segment, block_tables, cos, sin, 
 
 
 def attention_plain(out, q, cache_layer, positions, token_segment, block_tables, num_heads: int,
-                    kv_heads: int, head_dim: int, page_size: int, scale: float, window: int = 0):
-    """One wave per (token, head): the 32-bit path's attention and the slow twin of
-    the matrix-core kernels.  Token t reads keys max(0, pos-window+1)..pos of its
-    segment's pages."""
+                    kv_heads: int, head_dim: int, page_size: int, scale: float, window: int = 0, singles: bool = False):
+    """The 32-bit path's attention, and in bfloat16 the slow twin of the matrix-core kernels.  Token t reads keys
+    max(0, pos-window+1)..pos of its segment's pages.  In float32, heads that are multiples of 16 go through the
+    float32 matrix instruction, up to 16 query rows a workgroup; everything else is one wave per (token, head).
+    singles: every token is the only one of its segment (no result changes with it)."""
     _gpu(out, q, cache_layer, positions, token_segment, block_tables)
     n, w, ldq = _rows2d(q, "attention q")
     no, wo, ldo = _rows2d(out, "attention out")
@@ -408,6 +409,11 @@ def attention_plain(out, q, cache_layer, positions, token_segment, block_tables,
     _i32(token_segment, "attention token_segment", n)
     _check(block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.stride(1) == 1,
            "attention: block tables")
+    if q.dtype == torch.float32 and head_dim % 16 == 0 and head_dim <= 256 and cache_layer.data_ptr() % 16 == 0:
+        lib.core().call("hfee_attention_f32", _ptr(out), ldo, _ptr(q), ldq, _ptr(cache_layer), _ptr(positions),
+                        _ptr(token_segment), _ptr(block_tables), block_tables.stride(0), num_heads, kv_heads, head_dim,
+                        page_size, float(scale), int(window), int(singles), n, _stream())
+        return
     lib.core().call("hfee_attention_ref", _ptr(out), ldo, _ptr(q), ldq, _ptr(cache_layer), _dt(q),
                     _ptr(positions), _ptr(token_segment), _ptr(block_tables), block_tables.stride(0),
                     num_heads, kv_heads, head_dim, page_size, float(scale), int(window), n, _stream())

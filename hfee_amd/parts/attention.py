@@ -214,7 +214,7 @@ class Attention(Mixer):
         att = ctx.rows("attention.out", self.q_width)
         if self.dtype == torch.float32:
             ops.attention_plain(att, q, cache, ctx.positions, ctx.token_segment, tables, H, K, hd,
-                                ctx.page_size, self.scale, self.window)
+                                ctx.page_size, self.scale, self.window, singles=n == len(ctx.segments))
         else:
             tiles = ctx.extra["attention.tiles"]
             if tiles.shape[0]:

@@ -675,6 +675,57 @@ def test_attention_kernels(H, K, hd, T, window, dtype):
     _check_attention(H, K, hd, T, window, dtype, 16)
 
 
+@pytest.mark.parametrize("H,K,hd,window,ps", [(8, 2, 64, 0, 16), (5, 5, 80, 0, 32), (3, 1, 16, 21, 16), (40, 2, 48, 0, 16),
+                                              (4, 1, 256, 40, 64), (16, 1, 128, 0, 16), (14, 2, 144, 0, 16)])
+def test_attention_f32_does_not_depend_on_the_company(H, K, hd, window, ps):
+    """The 32-bit attention on the matrix instruction: groups of 1, 3, 4, 14, 16 and 20 heads a key head, both ways of keeping
+    a tile in registers, windows, requests of 1 to 200 tokens whose rows share workgroups, pages in any order that hold
+    NaN wherever nothing was written.  Within 2e-5 of the reference formula, and a token has the same bits in one call with
+    all, request by request, and alone (`singles`)."""
+    from plain_llama import plain_attention
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(H + hd)
+    lengths = [1, 200, 33, 2, 64, 31]
+    blocks = [(n + ps - 1) // ps for n in lengths]
+    order = torch.randperm(sum(blocks) + 3, generator=g).tolist()
+    layer = torch.full((len(order), 2, K, ps * hd), float("nan"))
+    tables = torch.zeros(len(lengths), max(blocks), dtype=torch.int32)
+    qs, refs, at = [], [], 0
+    scale = hd ** -0.5
+    for i, n in enumerate(lengths):
+        q, k, v = torch.randn(n, H, hd, generator=g), torch.randn(n, K, hd, generator=g), torch.randn(n, K, hd, generator=g)
+        refs.append(plain_attention(q, k, v, scale, window=window).reshape(n, H * hd))
+        qs.append(q.reshape(n, H * hd))
+        pages = order[at:at + blocks[i]]
+        at += blocks[i]
+        tables[i, :blocks[i]] = torch.tensor(pages)
+        for t in range(n):
+            page, slot = pages[t // ps], t % ps
+            for h in range(K):
+                kslot(layer[page, 0, h], ps, hd, slot)[:] = k[t, h].view(-1, 16)
+                layer[page, 1, h].view(hd, ps)[:, vslot(slot)] = v[t, h]
+    layer, tables = layer.to(DEV), tables.to(DEV)
+    q, ref = torch.cat(qs).to(DEV), torch.cat(refs)
+    positions = torch.cat([torch.arange(n, dtype=torch.int32) for n in lengths]).to(DEV)
+    seg = torch.cat([torch.full((n,), i, dtype=torch.int32) for i, n in enumerate(lengths)]).to(DEV)
+
+    def run(rows, **kw):
+        out = torch.zeros(len(rows), H * hd, device=DEV)
+        ops.attention_plain(out, q[rows].contiguous(), layer, positions[rows].contiguous(), seg[rows].contiguous(), tables, H, K,
+                            hd, ps, scale, window, **kw)
+        return out
+    everything = torch.arange(q.shape[0], device=DEV)
+    full = run(everything)
+    close(full, ref, 2e-5)
+    assert torch.equal(run(everything, singles=True), full)
+    begin = 0
+    for n in lengths:
+        rows = everything[begin:begin + n]
+        assert torch.equal(run(rows), full[rows])
+        assert torch.equal(run(rows[n // 2:]), full[rows[n // 2:]])
+        begin += n
+
+
 @pytest.mark.parametrize("H,K,hd,T,window,ps", [(4, 1, 128, 130, 0, 32), (8, 2, 64, 150, 40, 64), (4, 1, 48, 300, 0, 128),
                                                 (16, 2, 32, 97, 50, 32)])
 def test_attention_kernels_with_larger_pages(H, K, hd, T, window, ps):

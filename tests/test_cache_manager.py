@@ -231,6 +231,30 @@ def test_the_same_prefix_is_kept_once():
     m.check()
 
 
+@pytest.mark.parametrize("as_array", [False, True])
+def test_a_release_may_know_other_tokens_than_the_admission(as_array):
+    """What stays behind lies under the tokens that the release names: more than the prompt's, fewer, or others from some
+    place on, which must not be found under the prompt's digests."""
+    import numpy as np
+    give = (lambda t: np.asarray(t)) if as_array else (lambda t: t)
+    m = keeping(pages=12)
+    prompt = list(range(40, 120))                       # five pages, of which an admission looks at four
+    run_whole(m, "a", give(prompt))
+    m.release("a", give(prompt))
+    rc = m.admit("b", give(prompt))
+    assert rc.length == 64
+    m.reserve("b", 48), m.commit("b", 48)               # 112 tokens: seven pages
+    other = prompt[:40] + list(range(500, 572))         # (another third page)
+    m.release("b", give(other))
+    m.check()
+    assert m.admit("c", give(prompt)).length == 32      # two pages are the prompt's still
+    m.release("c", give(prompt[:16]))                   # fewer tokens than it holds: one page stays
+    m.check()
+    assert m.admit("d", give(other)).length == 16
+    m.check()
+    m.release("d")
+
+
 def test_prefixes_are_not_kept_where_a_window_has_given_pages_back():
     with pytest.raises(CacheError, match="every cache group keeps every token"):
         CacheManager([CacheGroupSpec("window", (2, 1, 16), (0,), window=32)], 16, 8, 2, keep_prefixes=True)

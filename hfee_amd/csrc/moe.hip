@@ -29,11 +29,13 @@
 // the experts' bytes, and for float32.
 //
 // Grouped (moe_group, moe_group_tiled, moe_combine; bfloat16): the (token, expert) pairs of a step are put
-// in the order of their experts on the device, cut into tiles of 64 pairs of one expert, and a workgroup
-// multiplies a tile by 256 rows of that expert's matrix on the matrix cores (both operands staged through
-// LDS in steps of 32 columns, a wave 64 x 64 of v_mfma_f32_32x32x16_bf16): an expert's matrices are read
-// once a 64 pairs and not once a pair.  A pair's numbers do not depend on which pairs share its tile.
+// in the order of their experts on the device, cut into tiles of up to 128 pairs of one expert, and a workgroup
+// multiplies a tile by 256 rows of that expert's matrix on the matrix cores, both operands straight into LDS
+// (moe_direct; sizes that are no multiples of 64: tiles of 64 pairs by way of registers): an expert's matrices are
+// read once for its pairs and not once a pair.  A pair's numbers do not depend on which pairs share its tile.
 #include "common.h"
+
+#include <type_traits>
 
 using namespace hfee;
 
@@ -163,7 +165,8 @@ constexpr int kTilePairs = 64, kTileRows = 256;
 // left to chance; nothing that is computed depends on it.
 __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order, int* __restrict__ tiles, int most_tiles,
                                                          const int* __restrict__ chosen, const int* __restrict__ table,
-                                                         const int* __restrict__ token_ids, int n, int top, int experts) {
+                                                         const int* __restrict__ token_ids, int n, int top, int experts,
+                                                         int tile_pairs) {
   extern __shared__ int lds[];
   int* counts = lds;                  // [experts]
   int* starts = lds + experts;        // [experts]
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
       starts[e] = at;
       first_tile[e] = tile;
       at += counts[e];
-      tile += (counts[e] + kTilePairs - 1) / kTilePairs;
+      tile += (counts[e] + tile_pairs - 1) / tile_pairs;
     }
     tiles[3 * most_tiles] = tile;
   }
@@ -193,11 +196,11 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
     if (e >= 0 && e < experts) order[starts[e] + atomicAdd(&cursor[e], 1)] = p;
   }
   for (int e = threadIdx.x; e < experts; e += blockDim.x)
-    for (int i = 0; i * kTilePairs < counts[e]; ++i) {
+    for (int i = 0; i * tile_pairs < counts[e]; ++i) {
       int* tl = tiles + 3 * (first_tile[e] + i);
       tl[0] = e;
-      tl[1] = starts[e] + i * kTilePairs;
-      tl[2] = min(kTilePairs, counts[e] - i * kTilePairs);
+      tl[1] = starts[e] + i * tile_pairs;
+      tl[2] = min(tile_pairs, counts[e] - i * tile_pairs);
     }
 }
 
@@ -210,7 +213,15 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
 // four neighbouring rows of the matrix for one pair and stores them at once.  A sum runs over K in the same
 // order whichever pairs share the tile.
 //   KIND 0: act = silu(gate) * up, or the clipped gate's product      KIND 1: act = relu(weight * up)^2      KIND 2: out (+)= scale * down
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ void barrier_no_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 constexpr int kStageK = 32, kStagePitch = 40;
 
 template <int KIND>
@@ -337,6 +348,208 @@ __global__ __launch_bounds__(256) void moe_group_tiled_kernel(
         }
     }
   }
+}
+
+// What becomes of four neighbouring rows' sums of one pair.
+template <int KIND>
+__device__ __forceinline__ void store_pair_rows(void* dst, int64_t ldo, int pair, int f, const f32x4& v, const f32x4& up, int add,
+                                                float scale, int gate_act, GateNumbers numbers) {
+  if constexpr (KIND == 2) {
+    float* o = (float*)dst + (int64_t)pair * ldo + f;
+    if (add || ldo % 4 != 0 || (uintptr_t)dst % 16 != 0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = add ? fmaf(v[r], scale, o[r]) : v[r];
+    } else {
+      *reinterpret_cast<f32x4*>(o) = v;
+    }
+  } else {
+    bf16_t four[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (KIND == 0) {
+        four[r] = float_to_bf16(gate_act == GATE_CLIPPED ? clipped_gate(v[r], up[r], numbers) : v[r] / (1.0f + expf(-v[r])) * up[r]);
+      } else {
+        const float u = fmaxf(v[r] * scale, 0.f);
+        four[r] = float_to_bf16(u * u);
+      }
+    }
+    *reinterpret_cast<u32x2*>((bf16_t*)dst + (int64_t)pair * ldo + f) = *reinterpret_cast<const u32x2*>(four);
+  }
+}
+
+// The same products for K in multiples of 64: tiles of up to 128 pairs and 256 rows of weights, four waves with all the
+// pairs and 64 rows each (KIND 0: 32 of each matrix), `16x16x32` instructions with the weights as the row operand.  A
+// step of 64 columns is 128 bytes a row; rows go from memory straight into one of three buffers in LDS, asked for two
+// steps before they are read, and a row's eight 16-byte chunks lie at chunk ^ (row % 8), so that the rows that a read
+// asks the same chunk of spread over the banks.  A tile of at most 64 pairs brings and multiplies only those.
+//
+// Why 128 pairs: with 64 pairs a step's 20 KB fed 256 cycles of the matrix cores, more than the 64 bytes a cycle that a CU
+// gets from L2, and the loads came by way of registers one step ahead.  2,048 tokens on two of 16 experts of 2,048, width
+// 4,096 (137 and 69 GFLOP, 537 and 268 MB of weights): gate and up 488 -> 215 us, down 254 -> 147; the whole feed-forward at 9 /
+// 128 / 800 / 2,048 tokens 216 / 242 / 416 / 801 -> 128 / 168 / 202 / 401 us.  What bounds it now is the wait for weight rows
+// from memory: LDS holds two steps ahead.
+constexpr int kWidePairs = 128;
+
+template <int KIND>
+__global__ __launch_bounds__(256) void moe_direct_kernel(
+    void* __restrict__ dst, int64_t ldo, const bf16_t* __restrict__ src, int64_t ld_src, const bf16_t* __restrict__ w0,
+    const bf16_t* __restrict__ w1, const int* __restrict__ order, const int* __restrict__ tiles, int most_tiles, int top,
+    int n_rows, int K, int add, const float* __restrict__ pair_weights, float weight, int gate_act, GateNumbers numbers,
+    uint32_t src_bytes) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the host pass has no buffer resources; it only needs the stub
+  constexpr int BUFFERS = 3, ROW = 128, BUFFER = (kWidePairs + kTileRows) * ROW;
+  constexpr int kRowsOut = KIND == 0 ? kTileRows / 2 : kTileRows;      // rows of the result a workgroup makes
+  extern __shared__ __attribute__((aligned(1024))) char lds_bytes[];
+  const int n_tiles = tiles[3 * most_tiles], row_blocks = (n_rows + kRowsOut - 1) / kRowsOut, items = n_tiles * row_blocks;
+  if ((int)blockIdx.x >= items) return;
+  // An XCD gets a run of items; an expert's items follow one another, its tiles of pairs within its blocks of rows, so that
+  // weight rows are read from memory once and the pairs' rows by the one or two XCDs that have the expert.
+  const int xcd = blockIdx.x % 8, item = xcd * (items / 8) + min(xcd, items % 8) + (int)blockIdx.x / 8;
+  const int lane = threadIdx.x & 63, some_tile = item / row_blocks, e = tiles[3 * some_tile];       // (a tile of the item's expert)
+  int tile0 = some_tile, tile1 = some_tile + 1;                                                     // the expert's tiles
+  for (bool more = true; more;) {
+    const int at = tile0 - 1 - lane;
+    const uint64_t other = __ballot(at < 0 || tiles[3 * max(at, 0)] != e);
+    tile0 -= other ? __builtin_ctzll(other) : 64;
+    more = other == 0;
+  }
+  for (bool more = true; more;) {
+    const int at = tile1 + lane;
+    const uint64_t other = __ballot(at >= n_tiles || tiles[3 * min(at, n_tiles - 1)] != e);
+    tile1 += other ? __builtin_ctzll(other) : 64;
+    more = other == 0;
+  }
+  const int within = item - tile0 * row_blocks, row0 = within / (tile1 - tile0) * kRowsOut;
+  const int* tl = tiles + 3 * (tile0 + within % (tile1 - tile0));
+  const int first = tl[1], count = tl[2];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  // (a block of rows begins its walk over K at a place of its own: rows are a power of two apart, and with all
+  // workgroups at the same column their lines lie in few of the memory's channels)
+  const int steps = K / 64, begin = (row0 / kRowsOut * 13 + e * 5) % steps;
+
+  typedef __attribute__((address_space(3))) void* lds_ptr;
+  const int lrow = 8 * wave + (lane >> 3), chunk = (lane & 7) ^ (lrow & 7);      // of the rows that a wave's request t brings: + 32 t
+  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, (int)src_bytes, 0x00020000);
+  const int64_t expert = (int64_t)e * n_rows * K;
+  const int matrix_bytes = (int)((uint32_t)n_rows * (uint32_t)K * 2u);
+  const __amdgpu_buffer_rsrc_t w0_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(w0 + expert), 0, matrix_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w1_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)((KIND == 0 ? w1 : w0) + expert), 0, matrix_bytes, 0x00020000);
+  uint32_t a_off[kWidePairs / 32], w_off[kTileRows / 32];
+#pragma unroll
+  for (int t = 0; t < kWidePairs / 32; ++t) {
+    const int pair = order[first + min(lrow + 32 * t, count - 1)];
+    a_off[t] = (uint32_t)((KIND == 2 ? pair : pair / top) * ld_src + 8 * chunk) * 2;
+  }
+#pragma unroll
+  for (int t = 0; t < kTileRows / 32; ++t) {
+    const int s = lrow + 32 * t;                                     // the row's place in the staged tile
+    w_off[t] = ((uint32_t)min(row0 + (KIND == 0 && s >= kRowsOut ? s - kRowsOut : s), n_rows - 1) * (uint32_t)K + 8 * chunk) * 2;
+  }
+
+  const auto work = [&](auto subtiles) {
+    constexpr int PS = decltype(subtiles)::value;                    // groups of 16 pairs
+    constexpr int A_LOADS = PS / 2, LOADS = A_LOADS + kTileRows / 32, READS = PS + 4, PRODUCTS = 4 * PS;
+    const auto load_one = [&](int step, int buffer, int t) {
+      const int turned = min(step, steps - 1) + begin;               // (past the end: a repeat that nobody uses)
+      const int at = (turned < steps ? turned : turned - steps) * ROW;
+      char* to = lds_bytes + buffer * BUFFER + wave * 1024;
+      if (t < A_LOADS) __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr)(to + t * 4096), 16, a_off[t], at, 0, 0);
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(t - A_LOADS < kTileRows / 64 ? w0_rsrc : w1_rsrc,
+                                                    (lds_ptr)(to + kWidePairs * ROW + (t - A_LOADS) * 4096), 16, w_off[t - A_LOADS], at, 0, 0);
+    };
+    struct Operands {
+      bf16x8 w[4], a[PS];
+    };
+    const auto read_one = [&](int buffer, int half, Operands& o, int i) {      // in the order in which the products need them
+      const char* tile = lds_bytes + buffer * BUFFER + r * ROW + (((4 * half + g) ^ (r & 7)) << 4);
+      if (i < 4) {
+        const int row = KIND == 0 ? (i >> 1) * kRowsOut + wave * 32 + (i & 1) * 16 : wave * 64 + i * 16;
+        o.w[i] = *reinterpret_cast<const bf16x8*>(tile + (kWidePairs + row) * ROW);
+      } else {
+        o.a[i - 4] = *reinterpret_cast<const bf16x8*>(tile + (i - 4) * 16 * ROW);
+      }
+    };
+    f32x4 acc[4][PS];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int m = 0; m < PS; ++m) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+#pragma unroll
+    for (int s = 0; s < BUFFERS; ++s)
+#pragma unroll
+      for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+    barrier_no_fence();
+    Operands o[2];
+#pragma unroll
+    for (int i = 0; i < READS; ++i) read_one(0, 0, o[0], i);
+    int now = 0;                                                     // the step's buffer
+    for (int s = 0; s < steps; ++s) {
+      const int next = now == BUFFERS - 1 ? 0 : now + 1;
+      // the first 32 columns, with the reads of the others
+#pragma unroll
+      for (int p = 0; p < PRODUCTS; ++p) {
+        acc[p & 3][p >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[0].w[p & 3], o[0].a[p >> 2], acc[p & 3][p >> 2], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < READS; ++i)
+          if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(now, 1, o[1], i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // this wave's part of step s + 1 has landed and its reads of step s are done; behind the barrier everybody's
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
+      barrier_no_fence();
+#pragma unroll
+      for (int p = 0; p < PRODUCTS; ++p) {
+        acc[p & 3][p >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[1].w[p & 3], o[1].a[p >> 2], acc[p & 3][p >> 2], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < READS; ++i)
+          if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(next, 0, o[0], i);
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l)
+          if (l >= LOADS * p / PRODUCTS && l < LOADS * (p + 1) / PRODUCTS) load_one(s + BUFFERS, now, l);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      now = next;
+    }
+    // the repeats asked for past the end still write into this workgroup's LDS: they land before the wave ends
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+#pragma unroll
+    for (int m = 0; m < PS; ++m) {
+      if (16 * m + r >= count) continue;
+      const int pair = order[first + 16 * m + r];
+      const float scale = KIND == 0 ? 1.0f : KIND == 1 ? (pair_weights != nullptr ? pair_weights[pair] : 1.0f)
+                                          : add ? (pair_weights != nullptr ? pair_weights[pair] : weight) : 1.0f;
+#pragma unroll
+      for (int i = 0; i < (KIND == 0 ? 2 : 4); ++i) {
+        const int f = row0 + (KIND == 0 ? wave * 32 : wave * 64) + 16 * i + 4 * g;
+        if (f < n_rows) store_pair_rows<KIND>(dst, ldo, pair, f, acc[i][m], acc[KIND == 0 ? i + 2 : i][m], add, scale, gate_act, numbers);
+      }
+    }
+  };
+  if (count > 64) work(std::integral_constant<int, 8>{});
+  else work(std::integral_constant<int, 4>{});
+#endif
+}
+
+template <int KIND>
+int launch_direct(int most, void* dst, int64_t ldo, const bf16_t* src, int64_t ld_src, int64_t src_rows, const bf16_t* w0,
+                  const bf16_t* w1, const int* order, const int* tiles, int top, int n_rows, int K, int add,
+                  const float* pair_weights, float weight, int gate_act, GateNumbers numbers, hipStream_t stream) {
+  constexpr int rows_out = KIND == 0 ? kTileRows / 2 : kTileRows;
+  constexpr int lds = 3 * (kWidePairs + kTileRows) * 128;
+  static const hipError_t raised =
+      hipFuncSetAttribute((const void*)moe_direct_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  HFEE_REQUIRE(raised == hipSuccess, "moe_grouped: %s", hipGetErrorString(raised));
+  const int64_t grid = (int64_t)most * ((n_rows + rows_out - 1) / rows_out);
+  HFEE_REQUIRE(grid < (int64_t)1 << 31, "moe_grouped: too many tiles");
+  moe_direct_kernel<KIND><<<(unsigned)grid, 256, lds, stream>>>(dst, ldo, src, ld_src, w0, w1, order, tiles, most, top, n_rows, K, add,
+                                                              pair_weights, weight, gate_act, numbers,
+                                                              (uint32_t)(((src_rows - 1) * ld_src + K) * 2));
+  HFEE_CHECK_LAUNCH("moe_grouped");
+  return 0;
 }
 
 // x[t] += sum_j weight_tj y[t * top + j], j ascending.
@@ -560,24 +773,41 @@ HFEE_API int hfee_moe_grouped(float* x, int64_t ldx, const void* h, int64_t ldh,
   HFEE_REQUIRE(order != nullptr && tiles != nullptr && act != nullptr && ((top == 1 && x != nullptr) || y != nullptr), "moe_grouped: scratch missing");
   HFEE_REQUIRE((int64_t)n * top < (1 << 30), "moe_grouped: too many pairs");
   if (n == 0) return 0;
-  const int most = hfee_moe_group_tiles(n, top, experts);
-  moe_group_kernel<<<1, 1024, 4 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts);
+  // (tiles through LDS loads: steps of 64 columns, and offsets of 32 bits from the first row of an operand)
+  const int64_t limit32 = (int64_t)1 << 31;
+  const bool direct = width % 64 == 0 && ff % 64 == 0 && ((int64_t)n * ldh) * 2 < limit32 && (int64_t)n * top * ff * 2 < limit32 &&
+                      (int64_t)ff * width * 2 < limit32;
+  const int tile_pairs = direct ? kWidePairs : kTilePairs, most = (int)(((int64_t)n * top + tile_pairs - 1) / tile_pairs) + experts;
+  moe_group_kernel<<<1, 1024, 4 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts, tile_pairs);
   HFEE_CHECK_LAUNCH("moe_group");
-  // (rows in whole groups of four: ff and width are multiples of 32)
-  if (w_gate != nullptr)
-    moe_group_tiled_kernel<0><<<dim3(most, (ff + kTileRows / 2 - 1) / (kTileRows / 2)), 256, 0, stream>>>(
-        act, ff, (const bf16_t*)h, ldh, (const bf16_t*)w_gate, (const bf16_t*)w_up, order, tiles, most, top, ff, width, 0,
-        nullptr, 1.0f, gate_act, numbers);
-  else
-    moe_group_tiled_kernel<1><<<dim3(most, (ff + kTileRows - 1) / kTileRows), 256, 0, stream>>>(
-        act, ff, (const bf16_t*)h, ldh, (const bf16_t*)w_up, nullptr, order, tiles, most, top, ff, width, 0, in_weights, 1.0f,
-        GATE_SILU, numbers);
-  HFEE_CHECK_LAUNCH("moe_group_up");
   const bool straight = top == 1 && x != nullptr;
-  moe_group_tiled_kernel<2><<<dim3(most, (width + kTileRows - 1) / kTileRows), 256, 0, stream>>>(
-      straight ? (void*)x : (void*)y, straight ? ldx : (int64_t)width, (const bf16_t*)act, ff, (const bf16_t*)w_down, nullptr,
-      order, tiles, most, top, width, ff, straight ? 1 : 0, pair_weights, weight, GATE_SILU, numbers);
-  HFEE_CHECK_LAUNCH("moe_group_down");
+  void* down = straight ? (void*)x : (void*)y;
+  const int64_t ld_down = straight ? ldx : (int64_t)width;
+  if (direct) {
+    if (w_gate != nullptr ? launch_direct<0>(most, act, ff, (const bf16_t*)h, ldh, n, (const bf16_t*)w_gate, (const bf16_t*)w_up, order,
+                                             tiles, top, ff, width, 0, nullptr, 1.0f, gate_act, numbers, stream)
+                          : launch_direct<1>(most, act, ff, (const bf16_t*)h, ldh, n, (const bf16_t*)w_up, nullptr, order, tiles, top, ff,
+                                             width, 0, in_weights, 1.0f, GATE_SILU, numbers, stream))
+      return 1;
+    if (launch_direct<2>(most, down, ld_down, (const bf16_t*)act, ff, (int64_t)n * top, (const bf16_t*)w_down, nullptr, order, tiles, top,
+                         width, ff, straight ? 1 : 0, pair_weights, weight, GATE_SILU, numbers, stream))
+      return 1;
+  } else {
+    // (rows in whole groups of four: ff and width are multiples of 32)
+    if (w_gate != nullptr)
+      moe_group_tiled_kernel<0><<<dim3(most, (ff + kTileRows / 2 - 1) / (kTileRows / 2)), 256, 0, stream>>>(
+          act, ff, (const bf16_t*)h, ldh, (const bf16_t*)w_gate, (const bf16_t*)w_up, order, tiles, most, top, ff, width, 0,
+          nullptr, 1.0f, gate_act, numbers);
+    else
+      moe_group_tiled_kernel<1><<<dim3(most, (ff + kTileRows - 1) / kTileRows), 256, 0, stream>>>(
+          act, ff, (const bf16_t*)h, ldh, (const bf16_t*)w_up, nullptr, order, tiles, most, top, ff, width, 0, in_weights, 1.0f,
+          GATE_SILU, numbers);
+    HFEE_CHECK_LAUNCH("moe_group_up");
+    moe_group_tiled_kernel<2><<<dim3(most, (width + kTileRows - 1) / kTileRows), 256, 0, stream>>>(
+        down, ld_down, (const bf16_t*)act, ff, (const bf16_t*)w_down, nullptr, order, tiles, most, top, width, ff, straight ? 1 : 0,
+        pair_weights, weight, GATE_SILU, numbers);
+    HFEE_CHECK_LAUNCH("moe_group_down");
+  }
   if (top > 1 && x != nullptr) {
     int parts = (width + 255) / 256;
     if (parts > 64) parts = 64;

@@ -290,6 +290,50 @@ def test_short_convolution_carries_its_inputs(dtype, K):
     assert float(state[:2].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("counts,width,ff", [((1, 0, 64, 65, 128, 129, 300), 128, 192), ((16, 17, 0, 2), 64, 64),
+                                             ((200, 3), 576, 320), ((70, 129, 31), 96, 160)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_grouped_experts_at_the_edges_of_their_tiles(counts, width, ff, gated):
+    """Tiles of up to 128 pairs and 256 weight rows (sizes in multiples of 64; the last sizes go through the tiles of 64
+    pairs): experts with none, one, a tile's and a tile's and one more pairs, rows that fill no block, a single step of
+    K.  Against the sums in float64 over the bfloat16 operands and activations: a float32 sum of K products is off by at
+    most K roundings of its terms' sizes, an activation by half a bfloat16 ulp more.  A pair's numbers stay the same,
+    bit for bit, among fewer pairs."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(sum(counts) + width)
+    E, n = len(counts), sum(counts)
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(n, generator=g)].to(torch.int32).view(n, 1)
+    rand = lambda *shape: (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(torch.bfloat16).cuda()      # noqa: E731
+    h, wg, wu, wd = rand(n, width) * width ** 0.5, rand(E, ff, width), rand(E, ff, width), rand(E, width, ff)
+    h = h.to(torch.bfloat16)
+
+    def run(rows):
+        m = len(rows)
+        order = torch.zeros(m, dtype=torch.int32, device="cuda")
+        tiles = torch.zeros(3 * ops.moe_group_tiles(m, 1, E) + 1, dtype=torch.int32, device="cuda")
+        act = torch.zeros(m, ff, dtype=torch.bfloat16, device="cuda")
+        y = torch.full((m, width), 7.0, dtype=torch.float32, device="cuda")
+        ops.moe_grouped(None, h[rows].contiguous(), wg if gated else None, wu, wd, 1, order, tiles, act, y, chosen=chosen[rows.cpu()].cuda())
+        return act, y
+    everything = torch.arange(n, device="cuda")
+    act, y = run(everything)
+    e = chosen.view(-1).long().cuda()
+    up = torch.einsum("nfw,nw->nf", wu[e].double(), h.double())
+    if gated:
+        gate = torch.einsum("nfw,nw->nf", wg[e].double(), h.double())
+        want = gate / (1 + torch.exp(-gate)) * up
+    else:
+        want = torch.relu(up) ** 2
+    assert ((act.double() - want).abs() <= 2.0 ** -8 * want.abs() + width * 2.0 ** -24 * 30).all()
+    down = torch.einsum("nwf,nf->nw", wd[e].double(), act.double())
+    size = torch.einsum("nwf,nf->nw", wd[e].double().abs(), act.double().abs())
+    assert ((y.double() - down).abs() <= (ff + 2) * 2.0 ** -24 * size).all()
+    some = everything[::3]
+    act2, y2 = run(some)
+    assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
+
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_experts_by_table(dtype):
     from hfee_amd.kernels import ops

@@ -81,6 +81,36 @@ __device__ __forceinline__ void two_dots(const T* a, const T* a2, const T* b, in
   }
 }
 
+// The same for R rows and P vectors at once (bfloat16, wide): a wave has two turns of R loads in flight, and a row's bytes
+// serve every vector.
+template <int R, int P>
+__device__ __forceinline__ void many_dots(const bf16_t* const (&rows)[R], const bf16_t* const (&b)[P], int count, int lane, float (&s)[P][R]) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int q = 0; q < P; ++q)
+#pragma unroll
+    for (int k = 0; k < R; ++k) s[q][k] = 0.f;
+#pragma unroll 2
+  for (int c = lane * 8; c < count; c += 64 * 8) {
+    u32x4_t v[R], vb[P];
+#pragma unroll
+    for (int k = 0; k < R; ++k) v[k] = load_streamed(reinterpret_cast<const u32x4_t*>(rows[k] + c));
+#pragma unroll
+    for (int q = 0; q < P; ++q) vb[q] = *reinterpret_cast<const u32x4_t*>(b[q] + c);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const float b0 = __uint_as_float(vb[q][i] << 16), b1 = __uint_as_float(vb[q][i] & 0xffff0000u);
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          s[q][k] = fmaf(__uint_as_float(v[k][i] << 16), b0, s[q][k]);
+          s[q][k] = fmaf(__uint_as_float(v[k][i] & 0xffff0000u), b1, s[q][k]);
+        }
+      }
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ bool rows_aligned(const T* a, const T* b, int count, int64_t row_stride_b) {
   return sizeof(T) == 2 && count % 8 == 0 && row_stride_b % 8 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
@@ -123,6 +153,69 @@ __global__ __launch_bounds__(256) void moe_up_kernel(T* __restrict__ act, const 
   }
 }
 
+// moe_up for gated experts in bfloat16 and at most 64 pairs, expert by expert: grid (blocks of 16 rows, experts), so that an expert's rows come
+// through every XCD.  Every wave
+// finds the pairs that use the workgroup's expert and takes up to four of them at a time over its four rows of both
+// matrices, so that an expert's rows come once however many tokens chose it.  16 experts of 2,048, width 4,096, the
+// matrices from memory (events around the call, some 8 us of it): 8 tokens on two experts each, 9 different ones, 93 -> 64
+// us; 2 tokens 48 -> 33; one 45 -> 30.  (With the experts as the faster index all of an expert's blocks went to one XCD: 94.)
+template <int P>
+__device__ __forceinline__ void up_for_pairs(bf16_t* act, const bf16_t* h, int64_t ldh, const bf16_t* const (&rows)[2 * kRowsPerWave],
+                                             const int (&pairs)[P], int top, int f0, int F, int width, int lane, int gate_act,
+                                             GateNumbers numbers) {
+  const bf16_t* b[P];
+  float s[P][2 * kRowsPerWave];
+#pragma unroll
+  for (int q = 0; q < P; ++q) b[q] = h + (int64_t)(pairs[q] / top) * ldh;
+  many_dots<2 * kRowsPerWave, P>(rows, b, width, lane, s);
+#pragma unroll
+  for (int q = 0; q < P; ++q)
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const float sg = wave_sum(s[q][r]), su = wave_sum(s[q][kRowsPerWave + r]);
+      if (lane == r && f0 + r < F)
+        act[(int64_t)pairs[q] * F + f0 + r] =
+            float_to_bf16(gate_act == GATE_CLIPPED ? clipped_gate_exact(sg, su, numbers) : sg / (1.0f + expf(-sg)) * su);
+    }
+}
+
+__global__ __launch_bounds__(256) void moe_up_by_expert_kernel(bf16_t* __restrict__ act, const bf16_t* __restrict__ h, int64_t ldh,
+                                                               const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_up,
+                                                               const int* __restrict__ chosen, const int* __restrict__ table,
+                                                               const int* __restrict__ token_ids, int n_pairs, int top, int F, int width,
+                                                               int gate_act, GateNumbers numbers) {
+  const int e = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, f0 = (blockIdx.x * 4 + wave) * kRowsPerWave;
+  uint64_t users = __ballot(lane < n_pairs && expert_of(chosen, table, token_ids, min(lane, n_pairs - 1) / top, min(lane, n_pairs - 1) % top, top) == e);
+  if (users == 0 || f0 >= F) return;
+  const bf16_t* rows[2 * kRowsPerWave];
+#pragma unroll
+  for (int r = 0; r < kRowsPerWave; ++r) {
+    const int64_t row = (int64_t)e * F + min(f0 + r, F - 1);
+    rows[r] = w_gate + row * width;
+    rows[kRowsPerWave + r] = w_up + row * width;
+  }
+  const auto next = [&]() {
+    const int p = __builtin_ctzll(users);
+    users &= users - 1;
+    return p;
+  };
+  while (users != 0) {
+    const int left = __popcll(users);
+    if (left >= 3) {                       // (three: the third twice)
+      const int a = next(), b = next(), c = next(), d = left >= 4 ? next() : c;
+      const int pairs[4] = {a, b, c, d};
+      up_for_pairs<4>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
+    } else if (left == 2) {
+      const int a = next(), b = next();
+      const int pairs[2] = {a, b};
+      up_for_pairs<2>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
+    } else {
+      const int pairs[1] = {next()};
+      up_for_pairs<1>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
+    }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, int64_t ldx, const T* __restrict__ act,
                                                        const T* __restrict__ w_down, const int* __restrict__ chosen,
@@ -132,6 +225,32 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
   const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c0 = (blockIdx.y * 4 + wave) * kRowsPerWave;
   const bool wide = rows_aligned<T>(w_down, act, F, F);
+  if constexpr (sizeof(T) == 2) {
+    if (wide) {                             // a wave's four rows side by side
+      if (c0 >= width) return;
+      float total[kRowsPerWave] = {};
+      for (int j = 0; j < top; ++j) {
+        const int e = expert_of(chosen, table, token_ids, t, j, top);
+        if (e < 0 || e >= experts) continue;
+        const bf16_t* rows[kRowsPerWave];
+        float s[1][kRowsPerWave];
+#pragma unroll
+        for (int r = 0; r < kRowsPerWave; ++r) rows[r] = w_down + ((int64_t)e * width + min(c0 + r, width - 1)) * F;
+        const bf16_t* const one[1] = {act + ((int64_t)t * top + j) * F};
+        many_dots<kRowsPerWave, 1>(rows, one, F, lane, s);
+        const float w = pair_weights != nullptr ? pair_weights[(int64_t)t * top + j] : weight;
+#pragma unroll
+        for (int r = 0; r < kRowsPerWave; ++r) total[r] = fmaf(wave_sum(s[0][r]), w, total[r]);
+      }
+#pragma unroll
+      for (int r = 0; r < kRowsPerWave; ++r)
+        if (lane == r && c0 + r < width) {
+          float* o = x + (int64_t)t * ldx + c0 + r;
+          *o = accumulate ? *o + total[r] : total[r];
+        }
+      return;
+    }
+  }
 #pragma unroll
   for (int r = 0; r < kRowsPerWave; ++r) {
     const int c = c0 + r;
@@ -833,6 +952,12 @@ HFEE_API int hfee_moe_up(void* act, const void* h, int64_t ldh, const void* w_ga
     moe_up_kernel<float><<<grid, 256, 0, stream>>>((float*)act, (const float*)h, ldh, (const float*)w_gate, (const float*)w_up,
                                                    chosen, table, token_ids, top, experts, ff, width, in_weights,
                                                     gate_act, numbers);
+  // (expert by expert where the pairs fit a wave's lanes and there are not so many experts that most workgroups leave at once)
+  else if (dtype == 1 && w_gate != nullptr && (int64_t)n * top <= 64 && experts <= 256 && width % 8 == 0 && ldh % 8 == 0 &&
+           (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_up) & 15) == 0)
+    moe_up_by_expert_kernel<<<dim3(grid.y, experts), 256, 0, stream>>>((bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate,
+                                                                     (const bf16_t*)w_up, chosen, table, token_ids, n * top, top, ff,
+                                                                     width, gate_act, numbers);
   else if (dtype == 1)
     moe_up_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate,
                                                     (const bf16_t*)w_up, chosen, table, token_ids, top, experts, ff, width, in_weights,

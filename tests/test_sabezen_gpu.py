@@ -290,6 +290,37 @@ def test_short_convolution_carries_its_inputs(dtype, K):
     assert float(state[:2].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("users,width,ff", [((1, 2, 3, 4, 5, 9), 64, 50), ((64,), 520, 16), ((0, 7, 0, 1), 1032, 33)])
+@pytest.mark.parametrize("numbers", [None, (7.0, 1.702)])
+def test_few_tokens_expert_by_expert(users, width, ff, numbers):
+    """The first product of up to 64 (token, expert) pairs, an expert's rows once for all its tokens: every number of
+    tokens that are taken together, rows that fill no block, and pairs whose expert number stands for no matrix, whose
+    rows stay as they were.  Against float64: an activation is off by half a bfloat16 ulp and its sums' roundings."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + ff)
+    E = len(users)
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(users)] + ([] if sum(users) == 64 else [torch.full((2,), E + 1)]))
+    n = len(chosen)
+    chosen = chosen[torch.randperm(n, generator=g)].to(torch.int32).view(n, 1)
+    rand = lambda *shape: (torch.randn(*shape, generator=g) * 0.3).to(torch.bfloat16).cuda()      # noqa: E731
+    h, wg, wu = rand(n, width), rand(E, ff, width), rand(E, ff, width)
+    act = torch.full((n, ff), 5.0, dtype=torch.bfloat16, device="cuda")
+    ops.moe_up(act, h, wg, wu, 1, chosen=chosen.cuda(), **(dict(activation="clipped", numbers=numbers) if numbers else {}))
+    for t in range(n):
+        e = int(chosen[t, 0])
+        if e >= E:
+            assert (act[t] == 5.0).all()
+            continue
+        gate, up = wg[e].double() @ h[t].double(), wu[e].double() @ h[t].double()
+        if numbers:
+            gate, up = gate.clamp(max=numbers[0]), up.clamp(-numbers[0], numbers[0])
+            want = gate * torch.sigmoid(numbers[1] * gate) * (up + 1)
+        else:
+            want = gate * torch.sigmoid(gate) * up
+        size = (wg[e].double().abs() @ h[t].double().abs() + 1) * (wu[e].double().abs() @ h[t].double().abs() + 1)
+        assert ((act[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + width * 2.0 ** -23 * size).all(), t
+
+
 @pytest.mark.parametrize("H,G,D,V", [(3, 3, 128, 40), (4, 2, 32, 16), (2, 1, 64, 33), (2, 2, 100, 8), (1, 1, 4, 5), (2, 1, 20, 50)])
 @pytest.mark.parametrize("rule", ["delta", "decay_add"])
 @pytest.mark.parametrize("kind", ["plain", "all forgotten", "no decay", "alike"])

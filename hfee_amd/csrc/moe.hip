@@ -272,6 +272,80 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
   }
 }
 
+// moe_down in bfloat16 for at most 64 pairs, expert by expert: a workgroup has four rows of the result, its four waves take
+// the step's different experts in turn, up to four of an expert's pairs at a time on the same bytes; the pairs' sums
+// meet in LDS, where a token's are added up in the order of its experts, as above.  16 experts of 2,048, width 4,096, 8 tokens
+// on two each: 43 -> 32 us in a step.
+template <int P>
+__device__ __forceinline__ void down_for_pairs(float (*sums)[kRowsPerWave], const bf16_t* act, const bf16_t* const (&rows)[kRowsPerWave],
+                                               const int (&pairs)[P], int F, int lane) {
+  const bf16_t* b[P];
+  float s[P][kRowsPerWave];
+#pragma unroll
+  for (int q = 0; q < P; ++q) b[q] = act + (int64_t)pairs[q] * F;
+  many_dots<kRowsPerWave, P>(rows, b, F, lane, s);
+#pragma unroll
+  for (int q = 0; q < P; ++q)
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) {
+      const float sum = wave_sum(s[q][r]);
+      if (lane == r) sums[pairs[q]][r] = sum;
+    }
+}
+
+__global__ __launch_bounds__(256) void moe_down_by_expert_kernel(float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ act,
+                                                                 const bf16_t* __restrict__ w_down, const int* __restrict__ chosen,
+                                                                 const int* __restrict__ table, const int* __restrict__ token_ids,
+                                                                 const float* __restrict__ pair_weights, float weight, int n_pairs, int top,
+                                                                 int experts, int F, int width, int accumulate) {
+  __shared__ float sums[64][kRowsPerWave];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c0 = blockIdx.x * kRowsPerWave;
+  int e = -1;
+  if (lane < n_pairs) e = expert_of(chosen, table, token_ids, lane / top, lane % top, top);
+  if (e >= experts) e = -1;
+  int turn = 0;
+  for (uint64_t left = __ballot(e >= 0); left != 0; ++turn) {
+    const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+    uint64_t users = __ballot(e == mine);
+    left &= ~users;
+    if ((turn & 3) != wave) continue;
+    const bf16_t* rows[kRowsPerWave];
+#pragma unroll
+    for (int r = 0; r < kRowsPerWave; ++r) rows[r] = w_down + ((int64_t)mine * width + min(c0 + r, width - 1)) * F;
+    const auto next = [&]() {
+      const int p = __builtin_ctzll(users);
+      users &= users - 1;
+      return p;
+    };
+    while (users != 0) {
+      const int many = __popcll(users);
+      if (many >= 3) {                     // (three: the third twice)
+        const int a = next(), b = next(), c = next(), d = many >= 4 ? next() : c;
+        const int pairs[4] = {a, b, c, d};
+        down_for_pairs<4>(sums, act, rows, pairs, F, lane);
+      } else if (many == 2) {
+        const int a = next(), b = next();
+        const int pairs[2] = {a, b};
+        down_for_pairs<2>(sums, act, rows, pairs, F, lane);
+      } else {
+        const int pairs[1] = {next()};
+        down_for_pairs<1>(sums, act, rows, pairs, F, lane);
+      }
+    }
+  }
+  __syncthreads();
+  const int t = threadIdx.x / kRowsPerWave, r = threadIdx.x % kRowsPerWave;
+  if (t >= n_pairs / top || c0 + r >= width) return;
+  float total = 0.f;
+  for (int j = 0; j < top; ++j) {
+    const int p = t * top + j, ep = expert_of(chosen, table, token_ids, t, j, top);
+    if (ep < 0 || ep >= experts) continue;
+    total = fmaf(sums[p][r], pair_weights != nullptr ? pair_weights[p] : weight, total);
+  }
+  float* o = x + (int64_t)t * ldx + c0 + r;
+  *o = accumulate ? *o + total : total;
+}
+
 // ---------------------------------------------------------------------------- grouped
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -980,6 +1054,11 @@ HFEE_API int hfee_moe_down(float* x, int64_t ldx, const void* act, const void* w
   if (dtype == 0)
     moe_down_kernel<float><<<grid, 256, 0, stream>>>(x, ldx, (const float*)act, (const float*)w_down, chosen, table,
                                                      token_ids, pair_weights, weight, top, experts, ff, width, accumulate);
+  // (expert by expert as in moe_up)
+  else if (dtype == 1 && (int64_t)n * top <= 64 && ff % 8 == 0 && (((uintptr_t)act | (uintptr_t)w_down) & 15) == 0)
+    moe_down_by_expert_kernel<<<(width + kRowsPerWave - 1) / kRowsPerWave, 256, 0, stream>>>(
+        x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table, token_ids, pair_weights, weight, n * top, top, experts, ff, width,
+        accumulate);
   else if (dtype == 1)
     moe_down_kernel<bf16_t><<<grid, 256, 0, stream>>>(x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table,
                                                       token_ids, pair_weights, weight, top, experts, ff, width, accumulate);

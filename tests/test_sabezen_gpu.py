@@ -40,6 +40,19 @@ def i32(a):
 
 # ------------------------------------------------------------------ kernels alone
 
+@pytest.mark.parametrize("d", [4, 60, 260, 4096, 4100, 8192, 8196])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_layernorm_in_fours(d, dt):
+    """Widths of whole fours: less than a wave's, one and two fours a thread, and the first that goes back to one value at a
+    time; rows far from zero, gathered.  A float32 mean and variance of d numbers are off by some roundings each."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(d)
+    x, w = torch.randn(5, d, generator=g) * 2 + 9, (1 + torch.randn(d, generator=g) * 0.3).to(dt)
+    out = torch.zeros(3, d, dtype=dt, device="cuda")
+    ops.layernorm(out, x.cuda(), w.cuda(), 1e-5, i32([4, 0, 4]))
+    assert su.rel(out.double().cpu(), ps.layer_norm(x.double(), w.double(), 1e-5)[[4, 0, 4]]) < (2e-6 if dt == torch.float32 else 6e-3)
+
+
 def test_layernorm_and_scaled_embedding():
     from hfee_amd.kernels import ops
     g = torch.Generator().manual_seed(0)
@@ -319,6 +332,36 @@ def test_few_tokens_expert_by_expert(users, width, ff, numbers):
             want = gate * torch.sigmoid(gate) * up
         size = (wg[e].double().abs() @ h[t].double().abs() + 1) * (wu[e].double().abs() @ h[t].double().abs() + 1)
         assert ((act[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + width * 2.0 ** -23 * size).all(), t
+
+
+@pytest.mark.parametrize("n,top,E,width,ff", [(1, 2, 5, 64, 40), (8, 2, 3, 70, 520), (16, 4, 9, 33, 16), (64, 1, 2, 6, 1032), (21, 3, 4, 4, 8)])
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_few_tokens_second_product(n, top, E, width, ff, accumulate):
+    """The second product of up to 64 pairs, expert by expert: tokens that share experts and ones that name one beyond the
+    last (left out), widths that fill no four.  Against float64 over the same bfloat16 numbers: a float32 sum of ff products
+    a pair, added up over the pairs; and a token's numbers stay the same, bit for bit, alone."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(n * width + ff)
+    chosen = torch.rand(n, E + 2, generator=g).topk(top, dim=1).indices.to(torch.int32).cuda()
+    act, wd = torch.randn(n * top, ff, generator=g).bfloat16().cuda(), torch.randn(E, width, ff, generator=g).bfloat16().cuda()
+    weights = torch.rand(n, top, generator=g).cuda()
+    x0 = torch.randn(n, width, generator=g).cuda()
+
+    def run(rows):
+        x = x0[rows].clone()
+        a = act.view(n, top, ff)[rows].reshape(-1, ff).contiguous()
+        ops.moe_down(x, a, wd, top, pair_weights=weights[rows].contiguous(), chosen=chosen[rows].contiguous(), accumulate=accumulate)
+        return x
+    out = run(list(range(n)))
+    for t in range(n):
+        want, size = (x0[t].double() if accumulate else torch.zeros(width, dtype=torch.float64, device="cuda")), x0[t].double().abs()
+        for j in range(top):
+            e = int(chosen[t, j])
+            if e < E:
+                want = want + weights[t, j].double() * (wd[e].double() @ act[t * top + j].double())
+                size = size + wd[e].double().abs() @ act[t * top + j].double().abs()
+        assert ((out[t].double() - want).abs() <= (ff / 32 + 24) * 2.0 ** -24 * size).all(), t
+    assert torch.equal(run([n - 1])[0], out[n - 1])
 
 
 @pytest.mark.parametrize("H,G,D,V", [(3, 3, 128, 40), (4, 2, 32, 16), (2, 1, 64, 33), (2, 2, 100, 8), (1, 1, 4, 5), (2, 1, 20, 50)])

@@ -328,8 +328,9 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaArgs p) {
 // k_j R(t, j) in registers: every product of decays is again a product of its own factors, however strong they are.  For
 // the walk it leaves q_t G(t), k_j R(L - 1, j) and G(L - 1); without DELTA u_t = v_t and there is nothing to solve.
 // A lane has DT channels; eight waves, each with two groups of four tokens, a short and a long one.
-// 2,048 tokens, 16 heads of 128 and 256: token by token 806 us (delta rule) and 686 us (linear attention); in chunks 159 + 171 and 119 + 119 us, this
-// kernel and the walk.
+// 2,048 tokens, 16 heads of 128 and 256: token by token 806 us (delta rule) and 686 us (linear attention); in chunks
+// 86 + 171 and 59 + 120 us, this kernel and the walk (159 and 119 us here while a token's read waited for the sums of the
+// one before).
 template <int DT, bool DELTA>
 __global__ __launch_bounds__(512) void channel_solve_kernel(DeltaArgs p) {
   constexpr int DP = 16 * DT, ROW = DP + 4;
@@ -367,22 +368,48 @@ __global__ __launch_bounds__(512) void channel_solve_kernel(DeltaArgs p) {
     float kj[DT], m[DT];
 #pragma unroll
     for (int i = 0; i < DT; ++i) kj[i] = m[i] = ka[j * ROW + d0 + i];
-    for (int t = 4 * group; t < L; ++t) {
-      const float *kt = &ka[t * ROW + d0], *qt = &qa[t * ROW + d0], *dt = &da[t * ROW + d0];
+    struct Token {
+      float k[DT], q[DT], d[DT];
+    };
+    const auto read = [&](Token& x, int t) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        x.q[i] = qa[t * ROW + d0 + i];
+        x.d[i] = da[t * ROW + d0 + i];
+        x.k[i] = DELTA ? ka[t * ROW + d0 + i] : 0.f;
+      }
+    };
+    const auto use = [&](const Token& x, int t, bool behind) {                  // behind: t lies behind j
       float sq = 0.f, sk = 0.f;
 #pragma unroll
       for (int i = 0; i < DT; ++i) {
-        m[i] = t > j ? m[i] * dt[i] : kj[i];
-        sq = fmaf(qt[i], m[i], sq);
-        if (DELTA) sk = fmaf(kt[i], m[i], sk);
+        m[i] = behind ? m[i] * x.d[i] : kj[i];
+        sq = fmaf(x.q[i], m[i], sq);
+        if (DELTA) sk = fmaf(x.k[i], m[i], sk);
       }
       sq = column_sum(sq);
       if (DELTA) sk = column_sum(sk);
       if (part == 0 && t >= j) {
         P[t * kPitch + j] = sq;
-        if (DELTA && t > j) A[t * kPitch + j] = -beta[t] * sk;                  // (-A)
+        if (DELTA && behind) A[t * kPitch + j] = -beta[t] * sk;                 // (-A)
       }
+    };
+    // (the group's own four tokens, some of them in front of j, then those behind; a token is read in front of the sums of
+    // the one before, whose stores the compiler would not move a read across)
+    Token even, odd;
+    for (int t = 4 * group; t < min(4 * group + 4, L); ++t) {
+      read(even, t);
+      use(even, t, t > j);
     }
+    int t = 4 * group + 4;
+    if (t < L) read(even, t);
+    for (; t + 1 < L; t += 2) {
+      read(odd, t + 1);
+      use(even, t, true);
+      read(even, min(t + 2, L - 1));
+      use(odd, t + 1, true);
+    }
+    if (t < L) use(even, t, true);
     if (j < L) {
 #pragma unroll
       for (int i = 0; i < DT; ++i)

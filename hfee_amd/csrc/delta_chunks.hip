@@ -156,9 +156,6 @@ struct DeltaArgs {
   float* Y;                  // [heads][rows][V]
   float* upto;               // [heads][rows]: G(t)
   float* behind;             // [heads][rows]: R(L - 1, t)
-  float* Q;                  // (decays a channel) [heads][rows][D]: q_t G(t)
-  float* K;                  // [heads][rows][D]: k_t R(L - 1, t)
-  float* all;                // [heads][rows][D]: G(L - 1), in the row of a chunk's first token
   const int* segment_rows;
   const int* segment_lengths;
   const int* segment_slots;
@@ -173,67 +170,6 @@ __device__ __forceinline__ f32x4 block_product(f32x4 rows, f32x4 columns, f32x4 
 #pragma unroll
   for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rows[i], columns[i], acc, 0, 0, 0);
   return acc;
-}
-
-// The diagonal blocks of (I + A)^-1, a lane a column (the four g alike); A holds -A, waves 0 to 3 do a block each.
-__device__ __forceinline__ void invert_diagonal_block(const float* A, float* T, int wave, int r, int g) {
-  float x[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    float sum = i == r ? 1.0f : 0.f;
-    const float* row = &A[(wave * 16 + i) * kPitch + wave * 16];
-#pragma unroll
-    for (int j = 0; j < i; ++j) sum = fmaf(row[j], x[j], sum);
-    x[i] = sum;
-    if (g == 0) T[(wave * 16 + i) * 20 + r] = sum;
-  }
-}
-
-// W and Y, (I + A)^-1 times sixteen columns a tile, tiles in turn over the workgroup's waves.  key(t, d): what stands in the
-// row of token t (up to the last) and column d of C / b_t.
-template <typename Key>
-__device__ __forceinline__ void solve_columns(const DeltaArgs& p, const float* A, const float* T, const float* beta, int64_t at, int row0, int h,
-                                              int L, int wave, int waves, int r, int g, Key key) {
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 inverse[4], below[6];
-#pragma unroll
-  for (int I = 0; I < 4; ++I) {
-    inverse[I] = *reinterpret_cast<const f32x4*>(&T[(I * 16 + r) * 20 + 4 * g]);
-#pragma unroll
-    for (int J = 0; J < I; ++J)
-      below[I * (I - 1) / 2 + J] = *reinterpret_cast<const f32x4*>(&A[(I * 16 + r) * kPitch + J * 16 + 4 * g]);
-  }
-  const int key_tiles = (p.D + 15) / 16, value_tiles = (p.V + 15) / 16;
-  const float* vb = p.v + (int64_t)row0 * p.ldv + (int64_t)h * p.V;
-  for (int tile = wave; tile < key_tiles + value_tiles; tile += waves) {
-    const bool keys = tile < key_tiles;
-    const int col = (keys ? tile : tile - key_tiles) * 16 + r, width = keys ? p.D : p.V;
-    const bool live = col < width;
-    f32x4 x[4];
-#pragma unroll
-    for (int I = 0; I < 4; ++I)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = min(I * 16 + 4 * g + e, L - 1), c = live ? col : 0;
-        x[I][e] = keys ? key(t, c) : vb[(int64_t)t * p.ldv + c];
-      }
-#pragma unroll
-    for (int I = 0; I < 4; ++I) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) x[I][e] *= beta[I * 16 + 4 * g + e];
-#pragma unroll
-      for (int J = 0; J < I; ++J) x[I] = block_product(below[I * (I - 1) / 2 + J], x[J], x[I]);
-      x[I] = block_product(inverse[I], x[I], zero);
-    }
-    float* to = (keys ? p.W : p.Y) + at * width + col;
-#pragma unroll
-    for (int I = 0; I < 4; ++I)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int t = I * 16 + 4 * g + e;
-        if (live && t < L) to[(int64_t)t * width] = x[I][e];
-      }
-  }
 }
 
 template <int DT>
@@ -317,122 +253,59 @@ __global__ __launch_bounds__(256) void delta_solve_kernel(DeltaArgs p) {
     }
   }
   __syncthreads();
-  invert_diagonal_block(A, T, wave, r, g);
-  __syncthreads();
-  solve_columns(p, A, T, beta, at, row0, h, L, wave, 4, r, g, [&](int t, int d) { return kb[(int64_t)t * p.ldk + d] * upto[t]; });
-}
-
-// The same for decays a key channel, with the products of decays R(t, j) and G(t) a number a channel: they stand inside the
-// sums over the channels, A(t, j) = b_t sum_d k_t k_j R(t, j), P(t, j) = sum_d q_t k_j R(t, j), so those are not matrix
-// products.  Sixteen lanes have a token j, each its share of the channels, and walk over the tokens behind it with
-// k_j R(t, j) in registers: every product of decays is again a product of its own factors, however strong they are.  For
-// the walk it leaves q_t G(t), k_j R(L - 1, j) and G(L - 1); without DELTA u_t = v_t and there is nothing to solve.
-// A lane has DT channels; eight waves, each with two groups of four tokens, a short and a long one.
-// 2,048 tokens, 16 heads of 128 and 256: token by token 806 us (delta rule) and 686 us (linear attention); in chunks
-// 86 + 171 and 59 + 120 us, this kernel and the walk (159 and 119 us here while a token's read waited for the sums of the
-// one before).
-template <int DT, bool DELTA>
-__global__ __launch_bounds__(512) void channel_solve_kernel(DeltaArgs p) {
-  constexpr int DP = 16 * DT, ROW = DP + 4;
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  float *ka = lds, *qa = ka + kChunk * ROW, *da = qa + kChunk * ROW;           // keys, queries, decays
-  float *A = da + kChunk * ROW, *P = A + kChunk * kPitch, *T = P + kChunk * kPitch, *beta = T + kChunk * 20;
-  const int seg = blockIdx.z, h = blockIdx.y, len = p.segment_lengths[seg], first = blockIdx.x * kChunk;
-  if (len < kLeastTokens || first >= len) return;
-  const int row0 = p.segment_rows[seg] + first, L = min(kChunk, len - first), tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, part = lane & 15;
-  const int kg = h / (p.heads / p.qk_heads);
-  const int64_t at = (int64_t)h * p.rows + row0;
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
-
-  for (int e = tid; e < kChunk * DP / 4; e += 512) {          // (tokens behind the last: keys of zero, decays of one)
-    const int t = e / (DP / 4), d = e % (DP / 4) * 4;
-    const bool in = t < L && d < p.D;
-    const int64_t row = row0 + min(t, L - 1);
-    const int dd = d < p.D ? d : 0;
-    const f32x4 kv = *reinterpret_cast<const f32x4*>(p.k + row * p.ldk + (int64_t)kg * p.D + dd);
-    const f32x4 qv = *reinterpret_cast<const f32x4*>(p.q + row * p.ldq + (int64_t)kg * p.D + dd);
-    const f32x4 dv = *reinterpret_cast<const f32x4*>(p.decay + row * p.ldd + (int64_t)h * p.D + dd);
-    *reinterpret_cast<f32x4*>(&ka[t * ROW + d]) = in ? kv : zero;
-    *reinterpret_cast<f32x4*>(&qa[t * ROW + d]) = in ? qv : zero;
-    *reinterpret_cast<f32x4*>(&da[t * ROW + d]) = in ? dv : one;
-  }
-  for (int e = tid; e < 2 * kChunk * kPitch; e += 512) A[e] = 0.f;             // (and P behind it)
-  if (DELTA && tid < kChunk) beta[tid] = tid < L ? p.beta[(int64_t)(row0 + tid) * p.ldb + h] : 0.f;
-  __syncthreads();
-
-  const int d0 = part * DT;
+  {                          // (I + A)^-1 of a diagonal block, a lane a column (the four g alike)
+    float x[16];
 #pragma unroll
-  for (int turn = 0; turn < 2; ++turn) {
-    const int group = turn ? 15 - wave : wave, j = 4 * group + (lane >> 4);
-    float kj[DT], m[DT];
+    for (int i = 0; i < 16; ++i) {
+      float sum = i == r ? 1.0f : 0.f;
+      const float* row = &A[(wave * 16 + i) * kPitch + wave * 16];
 #pragma unroll
-    for (int i = 0; i < DT; ++i) kj[i] = m[i] = ka[j * ROW + d0 + i];
-    struct Token {
-      float k[DT], q[DT], d[DT];
-    };
-    const auto read = [&](Token& x, int t) {
-#pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        x.q[i] = qa[t * ROW + d0 + i];
-        x.d[i] = da[t * ROW + d0 + i];
-        x.k[i] = DELTA ? ka[t * ROW + d0 + i] : 0.f;
-      }
-    };
-    const auto use = [&](const Token& x, int t, bool behind) {                  // behind: t lies behind j
-      float sq = 0.f, sk = 0.f;
-#pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        m[i] = behind ? m[i] * x.d[i] : kj[i];
-        sq = fmaf(x.q[i], m[i], sq);
-        if (DELTA) sk = fmaf(x.k[i], m[i], sk);
-      }
-      sq = column_sum(sq);
-      if (DELTA) sk = column_sum(sk);
-      if (part == 0 && t >= j) {
-        P[t * kPitch + j] = sq;
-        if (DELTA && behind) A[t * kPitch + j] = -beta[t] * sk;                 // (-A)
-      }
-    };
-    // (the group's own four tokens, some of them in front of j, then those behind; a token is read in front of the sums of
-    // the one before, whose stores the compiler would not move a read across)
-    Token even, odd;
-    for (int t = 4 * group; t < min(4 * group + 4, L); ++t) {
-      read(even, t);
-      use(even, t, t > j);
-    }
-    int t = 4 * group + 4;
-    if (t < L) read(even, t);
-    for (; t + 1 < L; t += 2) {
-      read(odd, t + 1);
-      use(even, t, true);
-      read(even, min(t + 2, L - 1));
-      use(odd, t + 1, true);
-    }
-    if (t < L) use(even, t, true);
-    if (j < L) {
-#pragma unroll
-      for (int i = 0; i < DT; ++i)
-        if (d0 + i < p.D) p.K[(at + j) * p.D + d0 + i] = m[i];
+      for (int j = 0; j < i; ++j) sum = fmaf(row[j], x[j], sum);
+      x[i] = sum;
+      if (g == 0) T[(wave * 16 + i) * 20 + r] = sum;
     }
   }
   __syncthreads();
-  for (int e = tid; e < L * kChunk; e += 512) p.P[at * kChunk + e] = P[e / kChunk * kPitch + e % kChunk];
-  if (tid < DP) {                                              // G, channel by channel; k_t G(t) in the decays' place
-    float product = 1.0f;
-#pragma unroll 4
-    for (int t = 0; t < L; ++t) {
-      product *= da[t * ROW + tid];
-      if (DELTA) da[t * ROW + tid] = ka[t * ROW + tid] * product;
-      if (tid < p.D) p.Q[(at + t) * p.D + tid] = qa[t * ROW + tid] * product;
-    }
-    if (tid < p.D) p.all[at * p.D + tid] = product;
+  f32x4 inverse[4], below[6];
+#pragma unroll
+  for (int I = 0; I < 4; ++I) {
+    inverse[I] = *reinterpret_cast<const f32x4*>(&T[(I * 16 + r) * 20 + 4 * g]);
+#pragma unroll
+    for (int J = 0; J < I; ++J)
+      below[I * (I - 1) / 2 + J] = *reinterpret_cast<const f32x4*>(&A[(I * 16 + r) * kPitch + J * 16 + 4 * g]);
   }
-  if constexpr (DELTA) {
-    const int r = lane & 15, g = lane >> 4;
-    if (wave >= 4) invert_diagonal_block(A, T, wave - 4, r, g);
-    __syncthreads();
-    solve_columns(p, A, T, beta, at, row0, h, L, wave, 8, r, g, [&](int t, int d) { return da[t * ROW + d]; });
+  const int key_tiles = (p.D + 15) / 16, value_tiles = (p.V + 15) / 16;
+  const float* vb = p.v + (int64_t)row0 * p.ldv + (int64_t)h * p.V;
+  for (int tile = wave; tile < key_tiles + value_tiles; tile += 4) {
+    const bool keys = tile < key_tiles;
+    const int col = (keys ? tile : tile - key_tiles) * 16 + r, width = keys ? p.D : p.V;
+    const bool live = col < width;
+    const float* base = (keys ? kb : vb) + (live ? col : 0);
+    const int64_t ld = keys ? p.ldk : p.ldv;
+    f32x4 x[4];
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[I][e] = base[(int64_t)min(I * 16 + 4 * g + e, L - 1) * ld];
+#pragma unroll
+    for (int I = 0; I < 4; ++I) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = I * 16 + 4 * g + e;
+        x[I][e] *= keys ? beta[t] * upto[t] : beta[t];
+      }
+#pragma unroll
+      for (int J = 0; J < I; ++J) x[I] = block_product(below[I * (I - 1) / 2 + J], x[J], x[I]);
+      x[I] = block_product(inverse[I], x[I], zero);
+    }
+    float* to = (keys ? p.W : p.Y) + at * width + col;
+#pragma unroll
+    for (int I = 0; I < 4; ++I)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = I * 16 + 4 * g + e;
+        if (live && t < L) to[(int64_t)t * width] = x[I][e];
+      }
   }
 }
 
@@ -445,21 +318,16 @@ struct WalkOperands {
   float y[4], upto[4], behind[4];                 // of tokens 4 g + i of the wave's 16, in its column
   float k[TILES][16];                             // the chunk's keys in its rows of S
   float all;                                      // G(L - 1)
-  f32x4 alls[TILES];                              // the same for decays a channel
 };
 
-// What the walk is for.  HEAD: the delta rule with a decay a head; CHANNEL_DELTA, CHANNEL_ADD: decays a channel, where
-// queries and keys come with their products of decays, with and without the delta rule.
-enum { HEAD = 0, CHANNEL_DELTA = 1, CHANNEL_ADD = 2 };
-
 // DT: the key size in groups of 16, filled up (dims at and beyond D count as zeros).
-template <int DT, int MODE>
+template <int DT>
 __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs p) {
   typedef WalkOperands<DT> Operands;
   constexpr int TILES = Operands::TILES, PITCH = DT * 16 + 4;
   __shared__ __attribute__((aligned(16))) float St[kColumns * PITCH];      // S transposed: [column][row]
   __shared__ __attribute__((aligned(16))) float Ut[kColumns * kPitch];     // u: [column][token]
-  __shared__ __attribute__((aligned(16))) float Ub[MODE == HEAD ? kColumns * kPitch : 4];      // u times R(L - 1, token)
+  __shared__ __attribute__((aligned(16))) float Ub[kColumns * kPitch];     // u times R(L - 1, token)
   const int seg = blockIdx.z, h = blockIdx.x, len = p.segment_lengths[seg];
   if (len < kLeastTokens) return;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
@@ -485,14 +353,14 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs p) {
   auto load = [&](int first, Operands& o) {
     const int L = min(kChunk, len - first);
     const int64_t row0 = row_first + first, at = (int64_t)h * p.rows + row0;
-    const float* qb = MODE == HEAD ? p.q + row0 * p.ldq + (int64_t)kg * p.D : p.Q + at * p.D;
-    const float* kb = MODE == HEAD ? p.k + row0 * p.ldk + (int64_t)kg * p.D : p.K + at * p.D;
+    const float* qb = p.q + row0 * p.ldq + (int64_t)kg * p.D;
+    const float* kb = p.k + row0 * p.ldk + (int64_t)kg * p.D;
     const float* wb = p.W + at * p.D;
-    const int t = min(wave * 16 + r, L - 1), ldq = MODE == HEAD ? (int)p.ldq : p.D, ldk = MODE == HEAD ? (int)p.ldk : p.D;
+    const int t = min(wave * 16 + r, L - 1), ldq = (int)p.ldq, ldk = (int)p.ldk;
 #pragma unroll
     for (int s = 0; s < DT; ++s) {
       const int d = s * 16 + 4 * g < p.D ? s * 16 + 4 * g : first_four;
-      if (MODE != CHANNEL_ADD) o.w[s] = *reinterpret_cast<const f32x4*>(wb + t * p.D + d);
+      o.w[s] = *reinterpret_cast<const f32x4*>(wb + t * p.D + d);
       o.q[s] = *reinterpret_cast<const f32x4*>(qb + t * ldq + d);
     }
 #pragma unroll
@@ -500,20 +368,11 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = min(wave * 16 + 4 * g + i, L - 1);
-      o.y[i] = MODE == CHANNEL_ADD ? p.v[(row0 + row) * p.ldv + (int64_t)h * p.V + (live ? col : 0)] : p.Y[(at + row) * p.V + (live ? col : 0)];
-      if (MODE == HEAD) {
-        o.upto[i] = p.upto[at + row];
-        o.behind[i] = p.behind[at + row];
-      }
+      o.y[i] = p.Y[(at + row) * p.V + (live ? col : 0)];
+      o.upto[i] = p.upto[at + row];
+      o.behind[i] = p.behind[at + row];
     }
-    if (MODE == HEAD) o.all = p.upto[at + L - 1];
-    else {
-#pragma unroll
-      for (int tile = 0; tile < TILES; ++tile) {
-        const int d = (wave + 4 * tile) * 16 + 4 * g;
-        o.alls[tile] = *reinterpret_cast<const f32x4*>(p.all + at * p.D + (d < p.D ? d : 0));
-      }
-    }
+    o.all = p.upto[at + L - 1];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int row = min((e >> 2) * 16 + 4 * g + (e & 3), L - 1);
@@ -541,10 +400,10 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs p) {
     for (int s = 0; s < DT; ++s) {
       const f32x4 st = *reinterpret_cast<const f32x4*>(&St[r * PITCH + s * 16 + 4 * g]);
       if (s & 1) {
-        if (MODE != CHANNEL_ADD) u1 = block_product(now.w[s], st, u1);
+        u1 = block_product(now.w[s], st, u1);
         o1 = block_product(now.q[s], st, o1);
       } else {
-        if (MODE != CHANNEL_ADD) u0 = block_product(now.w[s], st, u0);
+        u0 = block_product(now.w[s], st, u0);
         o0 = block_product(now.q[s], st, o0);
       }
     }
@@ -553,17 +412,17 @@ __global__ __launch_bounds__(256) void delta_walk_kernel(DeltaArgs p) {
     for (int i = 0; i < 4; ++i) {
       const bool in = wave * 16 + 4 * g + i < L;
       u[i] = in ? now.y[i] - (u0[i] + u1[i]) : 0.f;
-      if (MODE == HEAD) ub[i] = u[i] * now.behind[i];
-      o0[i] = (o0[i] + o1[i]) * (MODE == HEAD ? now.upto[i] : 1.0f);
+      ub[i] = u[i] * now.behind[i];
+      o0[i] = (o0[i] + o1[i]) * now.upto[i];
     }
     *reinterpret_cast<f32x4*>(&Ut[r * kPitch + wave * 16 + 4 * g]) = u;
-    if (MODE == HEAD) *reinterpret_cast<f32x4*>(&Ub[r * kPitch + wave * 16 + 4 * g]) = ub;
+    *reinterpret_cast<f32x4*>(&Ub[r * kPitch + wave * 16 + 4 * g]) = ub;
     __syncthreads();             // every wave has read the copy of the old S, and all u are there
 #pragma unroll
-    for (int tile = 0; tile < TILES; ++tile) S[tile] = MODE == HEAD ? S[tile] * now.all : S[tile] * now.alls[tile];
+    for (int tile = 0; tile < TILES; ++tile) S[tile] = S[tile] * now.all;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const f32x4 ubs = *reinterpret_cast<const f32x4*>(&(MODE == HEAD ? Ub : Ut)[r * kPitch + s * 16 + 4 * g]);
+      const f32x4 ubs = *reinterpret_cast<const f32x4*>(&Ub[r * kPitch + s * 16 + 4 * g]);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -673,67 +532,17 @@ HFEE_API int hfee_delta_chunks(float* out, int64_t ldo, float* state, const floa
   float* upto = W + places * dim;
   float* behind = upto + places;
   float* Y = behind + places;
-  const DeltaArgs p{out, ldo, state, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, P, W, Y, upto, behind, nullptr, nullptr, nullptr, segment_rows,
+  const DeltaArgs p{out, ldo, state, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, P, W, Y, upto, behind, segment_rows,
                     segment_lengths, segment_slots, rows, heads, qk_heads, dim, vdim, rows_a_lane};
   const dim3 solve((longest + kChunk - 1) / kChunk, heads, segments), walk(heads, (vdim + kColumns - 1) / kColumns, segments);
 #define LAUNCH(DT)                                                                                                   \
   do {                                                                                                               \
     delta_solve_kernel<DT><<<solve, 256, 0, stream>>>(p);                                                            \
     HFEE_CHECK_LAUNCH("delta_chunks (solve)");                                                                       \
-    delta_walk_kernel<DT, HEAD><<<walk, 256, 0, stream>>>(p);                                                              \
+    delta_walk_kernel<DT><<<walk, 256, 0, stream>>>(p);                                                              \
   } while (0)
   if (dim <= 32) LAUNCH(2); else if (dim <= 64) LAUNCH(4); else if (dim <= 128) LAUNCH(8); else LAUNCH(16);
 #undef LAUNCH
   HFEE_CHECK_LAUNCH("delta_chunks (walk)");
   return 0;
-}
-
-namespace {
-
-template <int DT, bool DELTA>
-int launch_channel(const DeltaArgs& p, dim3 solve, dim3 walk, hipStream_t stream) {
-  constexpr size_t lds = (size_t)(3 * kChunk * (16 * DT + 4) + 2 * kChunk * kPitch + kChunk * 20 + kChunk) * sizeof(float);
-  static const hipError_t raised =
-      hipFuncSetAttribute((const void*)channel_solve_kernel<DT, DELTA>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  HFEE_REQUIRE(raised == hipSuccess, "channel_chunks: %s", hipGetErrorString(raised));
-  channel_solve_kernel<DT, DELTA><<<solve, 512, lds, stream>>>(p);
-  HFEE_CHECK_LAUNCH("channel_chunks (solve)");
-  delta_walk_kernel<DT, DELTA ? CHANNEL_DELTA : CHANNEL_ADD><<<walk, 256, 0, stream>>>(p);
-  HFEE_CHECK_LAUNCH("channel_chunks (walk)");
-  return 0;
-}
-
-}  // namespace
-
-// Decays a key channel, [rows][heads * dim]; beta null: gated linear attention, S <- diag(a) S + k v^T.  As
-// hfee_delta_chunks, with decay rows aligned like the keys', dim at most 128 and scratch float32
-// [heads * rows * (64 + 3 dim)], with beta [heads * rows * (64 + 4 dim + vdim)].
-HFEE_API int hfee_channel_chunks(float* out, int64_t ldo, float* state, const float* q, int64_t ldq, const float* k, int64_t ldk,
-                                 const float* v, int64_t ldv, const float* decay, int64_t ldd, const float* beta, int64_t ldb,
-                                 const int* segment_rows, const int* segment_lengths, const int* segment_slots, int segments,
-                                 int longest, int rows, int heads, int qk_heads, int dim, int vdim, int rows_a_lane, float* scratch,
-                                 int64_t scratch_floats, hipStream_t stream) {
-  HFEE_REQUIRE(segments >= 0 && segments <= 65535 && rows >= 0, "channel_chunks: bad segment count");
-  if (segments == 0 || longest < kLeastTokens) return 0;
-  HFEE_REQUIRE(heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && heads <= 65535,
-               "channel_chunks: %d heads are not a multiple of %d query/key heads", heads, qk_heads);
-  HFEE_REQUIRE(dim >= 4 && dim <= 128 && dim % 4 == 0 && vdim >= 1 && rows_a_lane >= 1 && 16 * rows_a_lane >= dim,
-               "channel_chunks: key sizes of 4 to 128 in fours");
-  HFEE_REQUIRE(ldq % 4 == 0 && ldk % 4 == 0 && ldd % 4 == 0 &&
-               (((uintptr_t)q | (uintptr_t)k | (uintptr_t)decay | (uintptr_t)scratch) & 15) == 0,
-               "channel_chunks: query, key and decay rows must be 16-byte aligned");
-  HFEE_REQUIRE(ldq >= (int64_t)qk_heads * dim && ldk >= (int64_t)qk_heads * dim && ldv >= (int64_t)heads * vdim &&
-               ldo >= (int64_t)heads * vdim && ldd >= (int64_t)heads * dim && (beta == nullptr || ldb >= heads), "channel_chunks: rows too short");
-  const int64_t places = (int64_t)heads * rows, floats = places * (kChunk + 3 * dim + (beta != nullptr ? dim + vdim : 0));
-  HFEE_REQUIRE(longest <= rows && scratch != nullptr && scratch_floats >= floats, "channel_chunks: the scratch needs room for every row of every head");
-  HFEE_REQUIRE((vdim + kColumns - 1) / kColumns <= 65535, "channel_chunks: values too wide");
-  float *P = scratch, *Q = P + places * kChunk, *K = Q + places * dim, *all = K + places * dim, *W = all + places * dim, *Y = W + places * dim;
-  const DeltaArgs p{out, ldo, state, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, P, W, Y, nullptr, nullptr, Q, K, all, segment_rows,
-                    segment_lengths, segment_slots, rows, heads, qk_heads, dim, vdim, rows_a_lane};
-  const dim3 solve((longest + kChunk - 1) / kChunk, heads, segments), walk(heads, (vdim + kColumns - 1) / kColumns, segments);
-  if (beta != nullptr)
-    return dim <= 32 ? launch_channel<2, true>(p, solve, walk, stream) : dim <= 64 ? launch_channel<4, true>(p, solve, walk, stream)
-                                                                                   : launch_channel<8, true>(p, solve, walk, stream);
-  return dim <= 32 ? launch_channel<2, false>(p, solve, walk, stream) : dim <= 64 ? launch_channel<4, false>(p, solve, walk, stream)
-                                                                                  : launch_channel<8, false>(p, solve, walk, stream);
 }

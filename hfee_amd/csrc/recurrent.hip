@@ -178,6 +178,22 @@ struct ScanToken {
   }
 };
 
+// Over the sixteen lanes of a column, which are one row of the data-parallel primitives: neighbours in a
+// quad, the quads of a half, the halves.  Every step adds two numbers that both lanes of a pair hold the
+// other way round, so all sixteen lanes end with the same bits.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+
+__device__ __forceinline__ float column_sum(float x) {
+  x += dpp_move<0xB1>(x);      // quad_perm [1, 0, 3, 2]
+  x += dpp_move<0x4E>(x);      // quad_perm [2, 3, 0, 1]
+  x += dpp_move<0x141>(x);     // row_half_mirror: lane i of eight reads lane 7 - i
+  x += dpp_move<0x140>(x);     // row_mirror: lane i of sixteen reads lane 15 - i
+  return x;
+}
+
 template <int DPT, int RULE>
 __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
     float* __restrict__ out, int64_t ldo, float* __restrict__ state, const float* __restrict__ q, int64_t ldq,

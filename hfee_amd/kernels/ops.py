@@ -1666,16 +1666,6 @@ def delta_chunks_scratch(longest: int, rows: int, heads: int, dim: int, vdim: in
     return heads * rows * (LINEAR_CHUNK + dim + vdim + 2)
 
 
-def channel_chunks_scratch(longest: int, rows: int, heads: int, dim: int, vdim: int, delta: bool) -> int:
-    """float32 words with which `linear_scan` walks the long portions of a step with decays a key channel in chunks (rule
-    "delta", or "decay_add"); 0 where it has none: few tokens, key sizes that the kernels do not take, or a step so large
-    that the scratch would pass a gigabyte."""
-    if dim % 4 or not 4 <= dim <= 128 or longest < int(lib.core().raw("hfee_delta_chunks_least")()):
-        return 0
-    words = heads * rows * (LINEAR_CHUNK + 3 * dim + (dim + vdim if delta else 0))
-    return words if words <= 1 << 28 else 0
-
-
 def delta_inputs_fit(channels: int, dim: int, taps: int) -> bool:
     """Whether `delta_inputs` takes these sizes (else: the short convolution, `unit_heads` and `scan_gate`)."""
     return bool(lib.core().raw("hfee_delta_inputs_fit")(int(channels), int(dim), int(taps)))
@@ -1712,7 +1702,7 @@ def delta_inputs(y, decay, beta, x, a, b, state, taps, dt_bias, a_log, token_seg
 
 def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths, segment_slots, heads: int,
                 qk_heads: int, dim: int, vdim: int, rule: str, decay_per_head: bool = False, longest: int = 0,
-                shortest: int = 0, scratch=None, channel_scratch=None):
+                shortest: int = 0, scratch=None):
     """Walks each segment's rows in order from state[slot] (float32 [slots, heads, `scan_state_shape`],
     updated in place: a head's matrix in blocks of four columns).  rule "decay_add": S <- diag(decay) S + k v^T; "delta": S <- diag(decay) S,
     S <- S + k (beta (v - S^T k))^T; "scaled_add": S <- diag(decay) S + k (beta v)^T; out = S^T q.
@@ -1721,8 +1711,7 @@ def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths,
     of a head's rows (or [heads]: the same decays for every token); beta [n, heads].
     With rule "decay_add" and the same decays for every token, `scratch` (float32, `linear_chunks_scratch` words) and
     the lengths of the step's longest and shortest portion: long portions go in chunks through the matrix cores,
-    in float32 as well; likewise with rule "delta" and one decay a head and token (`delta_chunks_scratch` words).  With
-    decays a key channel and rule "delta" or "decay_add", `channel_scratch` (`channel_chunks_scratch` words) does that."""
+    in float32 as well; likewise with rule "delta" and one decay a head and token (`delta_chunks_scratch` words)."""
     _gpu(out, state, q, k, v, decay, beta, segment_rows, segment_lengths, segment_slots)
     n, wq, ldq = _f32rows(q, "linear_scan q")
     nk, wk, ldk = _f32rows(k, "linear_scan k")
@@ -1748,19 +1737,6 @@ def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths,
     _i32(segment_lengths, "linear_scan segment_lengths", segments)
     _i32(segment_slots, "linear_scan segment_slots", segments)
     skip_from = 0
-    if channel_scratch is not None:
-        _gpu(channel_scratch)
-        _check(rule != "scaled_add" and not decay_per_head, 'linear_scan: channel_scratch is for decays a channel and the rules "delta" and "decay_add"')
-        _check(channel_scratch.dtype == torch.float32 and channel_scratch.is_contiguous() and 0 < shortest <= longest <= n,
-               "linear_scan: scratch and lengths")
-        if all(t.data_ptr() % 16 == 0 and ld % 4 == 0 for t, ld in ((q, ldq), (k, ldk), (decay, ldd))):
-            skip_from = int(lib.core().raw("hfee_delta_chunks_least")())
-            lib.core().call("hfee_channel_chunks", _ptr(out), ldo, _ptr(state), _ptr(q), ldq, _ptr(k), ldk, _ptr(v), ldv, _ptr(decay),
-                            ldd, _ptr(beta if rule == "delta" else None), ldb, _ptr(segment_rows), _ptr(segment_lengths),
-                            _ptr(segment_slots), segments, int(longest), n, heads, qk_heads, dim, vdim, _scan_rows_a_lane(dim),
-                            _ptr(channel_scratch), channel_scratch.numel(), _stream())
-            if shortest >= skip_from:
-                return
     if scratch is not None:
         _gpu(scratch)
         chunked_delta = rule == "delta" and decay_per_head and decay.dim() == 2

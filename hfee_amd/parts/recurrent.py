@@ -86,16 +86,6 @@ class _StateMixer(Mixer):
             return {}
         return dict(scratch=ctx.workspace.flat("recurrent.chunks", words, torch.float32), longest=max(lengths), shortest=min(lengths))
 
-    @staticmethod
-    def _channel_chunks(ctx, heads: int, dim: int, vdim: int, delta: bool) -> dict:
-        """The same for decays a key channel.  Not in the 32-bit path: chunks count from a portion's first token, and there a
-        token has the same bits however its prompt was cut."""
-        lengths = [s.length for s in ctx.segments]
-        words = 0 if ctx.dtype == torch.float32 else ops.channel_chunks_scratch(max(lengths), ctx.n, heads, dim, vdim, delta)
-        if not words:
-            return {}
-        return dict(channel_scratch=ctx.workspace.flat("recurrent.chunks", words, torch.float32), longest=max(lengths), shortest=min(lengths))
-
 
 @register_mixer("gated_delta")
 class GatedDelta(_StateMixer):
@@ -222,9 +212,9 @@ class GatedDelta(_StateMixer):
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)
 
     def _delta_chunks(self, ctx) -> dict:
-        """The arguments with which `ops.linear_scan` walks a step's long portions in chunks."""
+        """The arguments with which `ops.linear_scan` walks a step's long portions in chunks (one decay a head only)."""
         if not self.decay_per_head:
-            return self._channel_chunks(ctx, self.heads, self.dim, self.vdim, True)
+            return {}
         lengths = [s.length for s in ctx.segments]
         words = ops.delta_chunks_scratch(max(lengths), ctx.n, self.heads, self.dim, self.vdim)
         if not words:
@@ -310,8 +300,7 @@ class GatedLinearAttention(_StateMixer):
         decay = ctx.rows("gla.decay", self.qk_width, torch.float32)
         ops.scan_gate(decay, z, "root_sigmoid", bias=self.a_bias, number=self.tau)
         o = ctx.rows("gla.read", self.v_width, torch.float32)
-        ops.linear_scan(o, self.state, q, k, v, decay, None, rows, lengths, slots, H, H, D, V, "decay_add",
-                        **self._channel_chunks(ctx, H, D, V, False))
+        ops.linear_scan(o, self.state, q, k, v, decay, None, rows, lengths, slots, H, H, D, V, "decay_add")
         gated = ctx.rows("gla.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:self.at_a], self.norm_weight, H, V, self.norm_eps, "silu")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=True)

@@ -364,71 +364,6 @@ def test_few_tokens_second_product(n, top, E, width, ff, accumulate):
     assert torch.equal(run([n - 1])[0], out[n - 1])
 
 
-@pytest.mark.parametrize("H,G,D,V", [(3, 3, 128, 40), (4, 2, 32, 16), (2, 1, 64, 33), (2, 2, 100, 8), (1, 1, 4, 5), (2, 1, 20, 50)])
-@pytest.mark.parametrize("rule", ["delta", "decay_add"])
-@pytest.mark.parametrize("kind", ["plain", "all forgotten", "no decay", "alike"])
-def test_recurrences_with_decays_a_channel_in_chunks(H, G, D, V, rule, kind):
-    """Long portions through the chunks of 64 tokens (portions of 1, 15, 16, 63 to 65, 128 and 150 tokens side by side, on scratch
-    full of NaN, another request's state left alone), key sizes that fill no tile, against the recurrence token by token in
-    float64: decays down to 1e-30 and to zero, whose quotients do not exist, decays of one, keys nearly alike.  Off by at
-    most 2e-5 of the largest read, as the kernel that walks token by token is allowed elsewhere."""
-    from hfee_amd.kernels import ops
-    g = torch.Generator().manual_seed(H + D + V)
-    if rule == "decay_add":
-        G = H
-    lengths, slots, data, want, last = [300, 100], [2, 0], [], [], []
-    for n in lengths:
-        q, k, v = torch.randn(n, G, D, generator=g), torch.randn(n, G, D, generator=g), torch.randn(n, H, V, generator=g)
-        if kind == "alike":
-            k = torch.randn(1, G, D, generator=g) + 0.05 * k
-        q, k = q / q.norm(dim=-1, keepdim=True), k / k.norm(dim=-1, keepdim=True)
-        decay, beta = 0.7 + 0.3 * torch.rand(n, H, D, generator=g), torch.rand(n, H, generator=g)
-        decay[::7] *= 0.02
-        if kind == "no decay":
-            decay.fill_(1.0)
-        if kind == "all forgotten":
-            decay[::5] = 0.0
-            decay[3::11] = 1e-30
-        data.append((q, k, v, beta, decay))
-        S, reads = torch.zeros(H, D, V, dtype=torch.float64), []
-        qq, kk = q.double().repeat_interleave(H // G, 1), k.double().repeat_interleave(H // G, 1)
-        for t in range(n):
-            S = decay[t].double()[..., None] * S
-            u = v[t].double()
-            if rule == "delta":
-                u = beta[t].double()[:, None] * (u - torch.einsum("hdv,hd->hv", S, kk[t]))
-            S = S + kk[t][..., None] * u[:, None]
-            reads.append(torch.einsum("hdv,hd->hv", S, qq[t]))
-        want.append(torch.stack(reads))
-        last.append(S)
-    state = torch.zeros(4, H, *ops.scan_state_shape(D, V), device="cuda")
-    state[1].fill_(float("nan"))
-    fed, chunked = [0, 0], 0
-    for sizes in ([5, 2], [1, 1], [63, 0], [16, 15], [150, 16], [65, 64], [0, 2]):
-        segs = [(s, n) for s, n in enumerate(sizes) if n]
-        cat = lambda i: torch.cat([data[s][i][fed[s]:fed[s] + n].reshape(n, -1) for s, n in segs]).cuda()      # noqa: E731
-        q, k, v, beta, decay = (cat(i) for i in range(5))
-        rows = [sum(n for _, n in segs[:i]) for i in range(len(segs))]
-        out = torch.zeros(q.shape[0], H * V, device="cuda")
-        words, more = ops.channel_chunks_scratch(max(n for _, n in segs), q.shape[0], H, D, V, rule == "delta"), {}
-        if words:
-            more = dict(channel_scratch=torch.full((words,), float("nan"), device="cuda"), longest=max(n for _, n in segs),
-                        shortest=min(n for _, n in segs))
-            chunked += 1
-        ops.linear_scan(out, state, q, k, v, decay, beta if rule == "delta" else None, i32(rows), i32([n for _, n in segs]),
-                        i32([slots[s] for s, _ in segs]), H, G, D, V, rule, **more)
-        row = 0
-        for s, n in segs:
-            w = want[s][fed[s]:fed[s] + n].reshape(n, -1)
-            assert (out[row:row + n].double().cpu() - w).abs().max() < 2e-5 * want[s].abs().max(), (sizes, s)
-            fed[s] += n
-            row += n
-    assert fed == lengths and chunked == 4 and torch.isnan(state[1]).all() and torch.isfinite(state[[0, 2, 3]]).all()
-    for s in (0, 1):
-        got = ops.scan_state_matrix(state[slots[s]], D, V).double().cpu()
-        assert (got - last[s]).abs().max() < 2e-5 * last[s].abs().max()
-
-
 @pytest.mark.parametrize("counts,width,ff", [((1, 0, 64, 65, 128, 129, 300), 128, 192), ((16, 17, 0, 2), 64, 64),
                                              ((200, 3), 576, 320), ((70, 129, 31), 96, 160)])
 @pytest.mark.parametrize("gated", [True, False])
@@ -665,6 +600,36 @@ def test_grouped_experts_inside_replayed_decode_steps(tmp_path):
         if len(toks) > 44:
             want[(rid, len(toks) - 1)] = logits[len(toks) - 1]
     compare(got, want, TOL["bfloat16"], "grouped experts in graphs")
+
+
+@pytest.mark.parametrize("name", ["A", "D"])
+def test_a_prompts_recurrences_have_the_bits_of_single_tokens(folders, name, monkeypatch):
+    """What the recurrences of a bfloat16 step make of whole prompts, outputs and states, is what the same tokens give one
+    at a time: ids chosen among close candidates do not depend on how long a portion is."""
+    from hfee_amd.kernels import ops
+    from hfee_amd.trace_replay import Replayer
+    scan, seen = ops.linear_scan, []
+
+    def record(out, state, q, k, v, decay, beta, rows, lengths, slots, *sizes, **more):
+        before = state.clone()
+        scan(out, state, q, k, v, decay, beta, rows, lengths, slots, *sizes, **more)
+        seen.append((out.clone(), before, state.clone(), q.clone(), k.clone(), v.clone(), decay.clone(),
+                     None if beta is None else beta.clone(), lengths.tolist(), slots.clone(), sizes))
+
+    monkeypatch.setattr(ops, "linear_scan", record)
+    reqs = tu.make_requests(60, [100, 17, 70, 1], seed=3)
+    tu.run(Replayer(folders[(name, "bfloat16")], "bfloat16", 192, max_requests=4), tu.whole(reqs))
+    assert any(max(s[8]) == 100 for s in seen) and len(seen) >= 2
+    for out, state, after, q, k, v, decay, beta, lengths, slots, sizes in seen:
+        row0 = 0
+        for i, n in enumerate(lengths):
+            for t in range(row0, row0 + n):
+                one = torch.zeros_like(out[t:t + 1])
+                scan(one, state, *(x[t:t + 1].contiguous() for x in (q, k, v, decay)),
+                     None if beta is None else beta[t:t + 1].contiguous(), i32([0]), i32([1]), slots[i:i + 1].contiguous(), *sizes)
+                assert torch.equal(one, out[t:t + 1]), f"request {i}, token {t - row0}"
+            row0 += n
+        assert torch.equal(state, after)
 
 
 def test_a_far_token_shows_through_the_states(folders):

@@ -571,17 +571,21 @@ __device__ __forceinline__ void store_pair_rows(void* dst, int64_t ldo, int pair
 }
 
 // The same products for K in multiples of 64: tiles of up to 128 pairs and 256 rows of weights, four waves with all the
-// pairs and 64 rows each (KIND 0: 32 of each matrix), `16x16x32` instructions with the weights as the row operand.  A
-// step of 64 columns is 128 bytes a row; rows go from memory straight into one of three buffers in LDS, asked for two
-// steps before they are read, and a row's eight 16-byte chunks lie at chunk ^ (row % 8), so that the rows that a read
-// asks the same chunk of spread over the banks.  A tile of at most 64 pairs brings and multiplies only those.
+// pairs and 64 rows each (KIND 0: 32 of each matrix).  The instruction and the order of a sum over K are those of
+// moe_group_tiled, so a pair has the same bits in both.  A step of 64 columns is 128 bytes a row; rows go from memory
+// straight into one of three buffers in LDS, asked for two steps before they are read, and a row's eight 16-byte chunks lie
+// at chunk ^ (row % 8), so that the rows that a read asks the same chunk of spread over the banks.  A tile of at most 64
+// pairs brings and multiplies only those, and has room for a fourth buffer.
 //
 // Why 128 pairs: with 64 pairs a step's 20 KB fed 256 cycles of the matrix cores, more than the 64 bytes a cycle that a CU
-// gets from L2, and the loads came by way of registers one step ahead.  2,048 tokens on two of 16 experts of 2,048, width
-// 4,096 (137 and 69 GFLOP, 537 and 268 MB of weights): gate and up 488 -> 215 us, down 254 -> 147; the whole feed-forward at 9 /
-// 128 / 800 / 2,048 tokens 216 / 242 / 416 / 801 -> 128 / 168 / 202 / 401 us.  What bounds it now is the wait for weight rows
-// from memory: LDS holds two steps ahead.
-constexpr int kWidePairs = 128;
+// gets from L2, and the loads came by way of registers one step ahead.  The whole feed-forward, 9 / 128 / 800 / 2,048 tokens
+// on two of 16 experts of 2,048, width 4,096 (206 GFLOP at 2,048; 805 MB of weights): moe_group_tiled 225 / 252 / 428 / 804
+// us, this 128 / 178 / 213 / 374 (with three buffers at 64 pairs too 160 / 208 / 246 / 388).  What bounds it now is the wait
+// for weight rows from memory: LDS holds two or three steps ahead.  (Blocks of rows that begin their walk over K at places of
+// their own spread their lines over more of the memory's channels, 123 / 168 / 200 / 400 us with instructions of 16 x 16 and
+// three buffers, but then a pair's sums have another order of additions, and bits, than in moe_group_tiled.)
+constexpr int kWidePairs = 128, kDirectLds = 4 * (kWidePairs / 2 + kTileRows) * 128;      // (three buffers with all the pairs are less)
+static_assert(kDirectLds >= 3 * (kWidePairs + kTileRows) * 128 && kDirectLds <= 160 * 1024);
 
 template <int KIND>
 __global__ __launch_bounds__(256) void moe_direct_kernel(
@@ -590,7 +594,7 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
     int n_rows, int K, int add, const float* __restrict__ pair_weights, float weight, int gate_act, GateNumbers numbers,
     uint32_t src_bytes) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass has no buffer resources; it only needs the stub
-  constexpr int BUFFERS = 3, ROW = 128, BUFFER = (kWidePairs + kTileRows) * ROW;
+  constexpr int ROW = 128;
   constexpr int kRowsOut = KIND == 0 ? kTileRows / 2 : kTileRows;      // rows of the result a workgroup makes
   extern __shared__ __attribute__((aligned(1024))) char lds_bytes[];
   const int n_tiles = tiles[3 * most_tiles], row_blocks = (n_rows + kRowsOut - 1) / kRowsOut, items = n_tiles * row_blocks;
@@ -615,10 +619,8 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
   const int within = item - tile0 * row_blocks, row0 = within / (tile1 - tile0) * kRowsOut;
   const int* tl = tiles + 3 * (tile0 + within % (tile1 - tile0));
   const int first = tl[1], count = tl[2];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
-  // (a block of rows begins its walk over K at a place of its own: rows are a power of two apart, and with all
-  // workgroups at the same column their lines lie in few of the memory's channels)
-  const int steps = K / 64, begin = (row0 / kRowsOut * 13 + e * 5) % steps;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, g = lane >> 5;
+  const int steps = K / 64;
 
   typedef __attribute__((address_space(3))) void* lds_ptr;
   const int lrow = 8 * wave + (lane >> 3), chunk = (lane & 7) ^ (lrow & 7);      // of the rows that a wave's request t brings: + 32 t
@@ -641,39 +643,43 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
   }
 
   const auto work = [&](auto subtiles) {
-    constexpr int PS = decltype(subtiles)::value;                    // groups of 16 pairs
-    constexpr int A_LOADS = PS / 2, LOADS = A_LOADS + kTileRows / 32, READS = PS + 4, PRODUCTS = 4 * PS;
+    constexpr int PT = decltype(subtiles)::value;                    // groups of 32 pairs
+    // (a request a 32 rows; what a wave reads and multiplies of 32 columns, which are two instructions' 16 each)
+    constexpr int BUFFERS = PT == 4 ? 3 : 4, BUFFER = (32 * PT + kTileRows) * ROW;       // (kDirectLds bytes in all)
+    constexpr int A_LOADS = PT, LOADS = A_LOADS + kTileRows / 32, READS = 2 * (2 + PT), PRODUCTS = 2 * 2 * PT;
     const auto load_one = [&](int step, int buffer, int t) {
-      const int turned = min(step, steps - 1) + begin;               // (past the end: a repeat that nobody uses)
-      const int at = (turned < steps ? turned : turned - steps) * ROW;
+      const int at = min(step, steps - 1) * ROW;                     // (past the end: a repeat that nobody uses)
       char* to = lds_bytes + buffer * BUFFER + wave * 1024;
       if (t < A_LOADS) __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr)(to + t * 4096), 16, a_off[t], at, 0, 0);
       else __builtin_amdgcn_raw_ptr_buffer_load_lds(t - A_LOADS < kTileRows / 64 ? w0_rsrc : w1_rsrc,
-                                                    (lds_ptr)(to + kWidePairs * ROW + (t - A_LOADS) * 4096), 16, w_off[t - A_LOADS], at, 0, 0);
+                                                    (lds_ptr)(to + t * 4096), 16, w_off[t - A_LOADS], at, 0, 0);
     };
     struct Operands {
-      bf16x8 w[4], a[PS];
+      bf16x8 w[2][2], a[2][PT];
     };
     const auto read_one = [&](int buffer, int half, Operands& o, int i) {      // in the order in which the products need them
-      const char* tile = lds_bytes + buffer * BUFFER + r * ROW + (((4 * half + g) ^ (r & 7)) << 4);
-      if (i < 4) {
-        const int row = KIND == 0 ? (i >> 1) * kRowsOut + wave * 32 + (i & 1) * 16 : wave * 64 + i * 16;
-        o.w[i] = *reinterpret_cast<const bf16x8*>(tile + (kWidePairs + row) * ROW);
-      } else {
-        o.a[i - 4] = *reinterpret_cast<const bf16x8*>(tile + (i - 4) * 16 * ROW);
-      }
+      const int sixteen = i / (2 + PT), t = i % (2 + PT);
+      const char* tile = lds_bytes + buffer * BUFFER + r * ROW + (((4 * half + 2 * sixteen + g) ^ (r & 7)) << 4);
+      if (t < 2) o.w[sixteen][t] = *reinterpret_cast<const bf16x8*>(tile + (32 * PT + (KIND == 0 ? t * kRowsOut + wave * 32 : wave * 64 + t * 32)) * ROW);
+      else o.a[sixteen][t - 2] = *reinterpret_cast<const bf16x8*>(tile + (t - 2) * 32 * ROW);
     };
-    f32x4 acc[4][PS];
+    f32x16 acc[2][PT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int m = 0; m < PS; ++m) acc[i][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int m = 0; m < PT; ++m)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) acc[i][m][q] = 0.f;
+    const auto multiply_one = [&](const Operands& o, int p) {
+      const int sixteen = p / (2 * PT), i = p & 1, m = p / 2 % PT;
+      acc[i][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.w[sixteen][i], o.a[sixteen][m], acc[i][m], 0, 0, 0);
+    };
 
 #pragma unroll
     for (int s = 0; s < BUFFERS; ++s)
 #pragma unroll
       for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFFERS - 1) * LOADS) : "memory");
     barrier_no_fence();
     Operands o[2];
 #pragma unroll
@@ -684,18 +690,18 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
       // the first 32 columns, with the reads of the others
 #pragma unroll
       for (int p = 0; p < PRODUCTS; ++p) {
-        acc[p & 3][p >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[0].w[p & 3], o[0].a[p >> 2], acc[p & 3][p >> 2], 0, 0, 0);
+        multiply_one(o[0], p);
 #pragma unroll
         for (int i = 0; i < READS; ++i)
           if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(now, 1, o[1], i);
         __builtin_amdgcn_sched_barrier(0);
       }
       // this wave's part of step s + 1 has landed and its reads of step s are done; behind the barrier everybody's
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((BUFFERS - 2) * LOADS) : "memory");
       barrier_no_fence();
 #pragma unroll
       for (int p = 0; p < PRODUCTS; ++p) {
-        acc[p & 3][p >> 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[1].w[p & 3], o[1].a[p >> 2], acc[p & 3][p >> 2], 0, 0, 0);
+        multiply_one(o[1], p);
 #pragma unroll
         for (int i = 0; i < READS; ++i)
           if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(next, 0, o[0], i);
@@ -709,21 +715,26 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
     // the repeats asked for past the end still write into this workgroup's LDS: they land before the wave ends
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
+    // register q of lane l in (i, m): row 8 (q / 4) + 4 (l / 32) + q % 4 of the wave's group i, pair 32 m + l % 32
 #pragma unroll
-    for (int m = 0; m < PS; ++m) {
-      if (16 * m + r >= count) continue;
-      const int pair = order[first + 16 * m + r];
+    for (int m = 0; m < PT; ++m) {
+      if (32 * m + r >= count) continue;
+      const int pair = order[first + 32 * m + r];
       const float scale = KIND == 0 ? 1.0f : KIND == 1 ? (pair_weights != nullptr ? pair_weights[pair] : 1.0f)
                                           : add ? (pair_weights != nullptr ? pair_weights[pair] : weight) : 1.0f;
 #pragma unroll
-      for (int i = 0; i < (KIND == 0 ? 2 : 4); ++i) {
-        const int f = row0 + (KIND == 0 ? wave * 32 : wave * 64) + 16 * i + 4 * g;
-        if (f < n_rows) store_pair_rows<KIND>(dst, ldo, pair, f, acc[i][m], acc[KIND == 0 ? i + 2 : i][m], add, scale, gate_act, numbers);
-      }
+      for (int i = 0; i < (KIND == 0 ? 1 : 2); ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int f = row0 + (KIND == 0 ? wave * 32 : wave * 64 + 32 * i) + 8 * q + 4 * g;
+          const f32x4 v = {acc[i][m][4 * q], acc[i][m][4 * q + 1], acc[i][m][4 * q + 2], acc[i][m][4 * q + 3]};
+          const f32x4 up = {acc[1][m][4 * q], acc[1][m][4 * q + 1], acc[1][m][4 * q + 2], acc[1][m][4 * q + 3]};      // (KIND 0)
+          if (f < n_rows) store_pair_rows<KIND>(dst, ldo, pair, f, v, up, add, scale, gate_act, numbers);
+        }
     }
   };
-  if (count > 64) work(std::integral_constant<int, 8>{});
-  else work(std::integral_constant<int, 4>{});
+  if (count > 64) work(std::integral_constant<int, 4>{});
+  else work(std::integral_constant<int, 2>{});
 #endif
 }
 
@@ -732,13 +743,12 @@ int launch_direct(int most, void* dst, int64_t ldo, const bf16_t* src, int64_t l
                   const bf16_t* w1, const int* order, const int* tiles, int top, int n_rows, int K, int add,
                   const float* pair_weights, float weight, int gate_act, GateNumbers numbers, hipStream_t stream) {
   constexpr int rows_out = KIND == 0 ? kTileRows / 2 : kTileRows;
-  constexpr int lds = 3 * (kWidePairs + kTileRows) * 128;
   static const hipError_t raised =
-      hipFuncSetAttribute((const void*)moe_direct_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      hipFuncSetAttribute((const void*)moe_direct_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, kDirectLds);
   HFEE_REQUIRE(raised == hipSuccess, "moe_grouped: %s", hipGetErrorString(raised));
   const int64_t grid = (int64_t)most * ((n_rows + rows_out - 1) / rows_out);
   HFEE_REQUIRE(grid < (int64_t)1 << 31, "moe_grouped: too many tiles");
-  moe_direct_kernel<KIND><<<(unsigned)grid, 256, lds, stream>>>(dst, ldo, src, ld_src, w0, w1, order, tiles, most, top, n_rows, K, add,
+  moe_direct_kernel<KIND><<<(unsigned)grid, 256, kDirectLds, stream>>>(dst, ldo, src, ld_src, w0, w1, order, tiles, most, top, n_rows, K, add,
                                                               pair_weights, weight, gate_act, numbers,
                                                               (uint32_t)(((src_rows - 1) * ld_src + K) * 2));
   HFEE_CHECK_LAUNCH("moe_grouped");

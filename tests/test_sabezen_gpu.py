@@ -407,6 +407,37 @@ def test_grouped_experts_at_the_edges_of_their_tiles(counts, width, ff, gated):
     assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
 
 
+@pytest.mark.parametrize("form", ["gated", "clipped", "not gated"])
+@pytest.mark.parametrize("top", [1, 2])
+def test_grouped_experts_have_one_order_of_additions(form, top):
+    """Rows so far apart that an offset of 32 bits does not reach them all go through tiles of 64 pairs by way of registers,
+    rows side by side through tiles of 128 pairs straight into LDS: the same bits, in activations, pairs' outputs and the
+    stream that they are added to."""
+    from hfee_amd.kernels import ops
+    E, width, ff, n = 3, 320, 448, 259
+    g = torch.Generator().manual_seed(top)
+    rand = lambda *shape: (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(torch.bfloat16).cuda()      # noqa: E731
+    near, wg, wu, wd = rand(n, width) * 16, rand(E, ff, width), rand(E, ff, width), rand(E, width, ff)
+    apart = -(-(1 << 30) // n // 8) * 8 + 8
+    far = torch.empty(n, apart, dtype=torch.bfloat16, device="cuda")[:, :width]
+    far.copy_(near)
+    chosen = torch.rand(n, E, generator=g).topk(top).indices.to(torch.int32).cuda()
+    weights = torch.rand(n, top, generator=g).cuda()
+    more = dict(activation="clipped", numbers=(7.0, 1.702)) if form == "clipped" else {}
+    results = []
+    for h in (near, far):
+        order = torch.zeros(n * top, dtype=torch.int32, device="cuda")
+        tiles = torch.zeros(3 * ops.moe_group_tiles(n, top, E) + 1, dtype=torch.int32, device="cuda")
+        act = torch.zeros(n * top, ff, dtype=torch.bfloat16, device="cuda")
+        y = torch.zeros(n * top, width, device="cuda")
+        x = torch.ones(n, width, device="cuda")
+        which = dict(in_weights=weights) if form == "not gated" else dict(pair_weights=weights)
+        ops.moe_grouped(x, h, None if form == "not gated" else wg, wu, wd, top, order, tiles, act, y, chosen=chosen, **which, **more)
+        results.append((act, y, x))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    assert results[0][2].std() > 0
+
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_experts_by_table(dtype):

@@ -223,45 +223,63 @@ __global__ __launch_bounds__(256) void layernorm_kernel(TO* __restrict__ out, co
   for (int j = threadIdx.x; j < d; j += blockDim.x) o[j] = from_float<TO>((xr[j] - mean) * inv * to_float<TW>(w[j]));
 }
 
-// The same for rows of whole fours on 16 bytes (8 for bfloat16): a thread has NV fours, neighbours side by side, so that a
-// row of 4,096 is one load a thread.  What bounds it is the way from memory and through two sums over the workgroup: 8 rows of
-// 4,096 in a step 9.1 -> 5.0 us.
+// The same for rows of whole fours on 16 bytes (8 for bfloat16), with the same bits: a thread brings and writes NV fours, a
+// row of 4,096 is one load a thread, and between them the row lies in LDS, where the first 256 threads add up what they
+// add up in layernorm_kernel, in its order.  What bounds few rows is the way from memory and through two sums over the
+// workgroup: 8 rows of 4,096 in a row of launches 4.9 -> 3.3 us, of 8,192 13.5 -> 4.3.
 template <typename TO, typename TW, int NV>
 __global__ __launch_bounds__(1024) void layernorm_fours_kernel(TO* __restrict__ out, const float* __restrict__ x, const TW* __restrict__ w,
                                                                const int* __restrict__ rows, float eps, int d) {
-  __shared__ float scratch[16];
+  constexpr int OWN = 16 * NV;                     // values that one of the 256 adds up
+  __shared__ __attribute__((aligned(16))) float row[OWN * 256];
+  __shared__ float shares[2][4];
   const int64_t r = blockIdx.x;
   const float* xr = x + (int64_t)(rows ? rows[r] : r) * d;
-  float v[NV][4], wv[NV][4], sum = 0.f;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float v[NV][4], wv[NV][4];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int j = 4 * (threadIdx.x + i * blockDim.x);
-    const bool in = j < d;
-    hfee::load4<float>(v[i], xr + (in ? j : 0));
-    hfee::load4<TW>(wv[i], w + (in ? j : 0));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[i][e] = in ? v[i][e] : 0.f;
-      sum += v[i][e];
-    }
+    const int j = 4 * (tid + i * blockDim.x), at = j < d ? j : 0;
+    hfee::load4<float>(v[i], xr + at);
+    hfee::load4<TW>(wv[i], w + at);
   }
-  const float mean = block_sum(sum, scratch) / (float)d;
-  float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const bool in = 4 * (threadIdx.x + i * blockDim.x) < d;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[i][e] = in ? v[i][e] - mean : 0.f;
-      ss = fmaf(v[i][e], v[i][e], ss);
-    }
+    const int j = 4 * (tid + i * blockDim.x);
+    if (j < d) hfee::store4<float>(row + j, v[i]);
   }
-  const float inv = 1.0f / sqrtf(block_sum(ss, scratch) / (float)d + eps);
+  __syncthreads();
+  const auto total = [](const float* s) { return ((0.f + s[0]) + s[1]) + s[2] + s[3]; };
+  float own[OWN], sum = 0.f;
+  if (wave < 4) {
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int j = tid + 256 * i;
+      own[i] = j < d ? row[j] : 0.f;
+      sum += own[i];
+    }
+    sum = wave_sum(sum);
+    if (lane == 0) shares[0][wave] = sum;
+  }
+  __syncthreads();
+  const float mean = total(shares[0]) / (float)d;
+  if (wave < 4) {
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const float off = tid + 256 * i < d ? own[i] - mean : 0.f;
+      ss = fmaf(off, off, ss);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) shares[1][wave] = ss;
+  }
+  __syncthreads();
+  const float inv = 1.0f / sqrtf(total(shares[1]) / (float)d + eps);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int j = 4 * (threadIdx.x + i * blockDim.x);
+    const int j = 4 * (tid + i * blockDim.x);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[i][e] = v[i][e] * inv * wv[i][e];
+    for (int e = 0; e < 4; ++e) v[i][e] = (v[i][e] - mean) * inv * wv[i][e];
     if (j < d) hfee::store4<TO>(out + r * d + j, v[i]);
   }
 }
@@ -273,8 +291,13 @@ HFEE_API int hfee_layernorm(void* out, int out_dtype, const float* x, const void
   HFEE_REQUIRE(n >= 0 && d > 0, "layernorm: bad sizes n=%d d=%d", n, d);
   HFEE_REQUIRE(eps >= 0.f, "layernorm: eps must not be negative");
   if (n == 0) return 0;
-  const bool fours = d % 4 == 0 && d <= 8192 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
-  const int quads = d / 4, threads = d <= 4096 ? (quads + 63) / 64 * 64 : ((quads + 1) / 2 + 63) / 64 * 64;
+  // (A CU has room for eight rows of layernorm_kernel's 256 threads or two of a thousand: from 1,025 to 2,048 rows of more
+  // than 1,024 the former are one round over the chip and the latter three or four.  us layernorm_kernel / in fours: rows of
+  // 4,096, 1,024 of them 9.1 / 9.0, 1,200 9.8 / 10.3, 2,048 12.4 / 15.1, 2,304 17.1 / 16.8, 4,096 28.9 / 28.2; rows of 2,048,
+  // 1,200 of them 7.0 / 6.6, 2,048 8.6 / 9.0, 2,304 11.7 / 9.9; rows of 1,024, 2,048 of them 6.7 / 6.2.)
+  const bool one_round = d > 1024 && d <= 4096 && n > 1024 && n <= 2048;
+  const bool fours = !one_round && d % 4 == 0 && d <= 8192 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
+  const int each = d <= 4096 ? 4 : 8, needed = ((d + each - 1) / each + 63) / 64 * 64, threads = needed < 256 ? 256 : needed;
 #define LAUNCH(TO, TW)                                                                                                       \
   do {                                                                                                                       \
     if (!fours) layernorm_kernel<TO, TW><<<n, 256, 0, stream>>>((TO*)out, x, (const TW*)w, rows, eps, d);                    \

@@ -53,6 +53,55 @@ def test_layernorm_in_fours(d, dt):
     assert su.rel(out.double().cpu(), ps.layer_norm(x.double(), w.double(), 1e-5)[[4, 0, 4]]) < (2e-6 if dt == torch.float32 else 6e-3)
 
 
+@pytest.mark.parametrize("d", [4, 60, 90, 260, 1028, 4095, 4096, 4100, 8192, 8196])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_layernorm_has_one_order_of_additions(d, dt):
+    """Widths that go through fours and widths that do not: 256 shares, each its every 256th value in order, four waves of
+    them in a butterfly each, the waves in order.  The same sums in numpy give the same bits."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(d)
+    x, w = torch.randn(4, d, generator=g) * 2 + 9, (1 + torch.randn(d, generator=g) * 0.3).to(dt)
+    out = torch.zeros(4, d, dtype=dt, device="cuda")
+    ops.layernorm(out, x.cuda(), w.cuda(), 1e-5)
+
+    def workgroup(shares):                          # [rows, 256]
+        lanes = shares.reshape(-1, 4, 64)
+        for off in (32, 16, 8, 4, 2, 1):
+            lanes = lanes + lanes[:, :, np.arange(64) ^ off]
+        total = np.zeros(len(lanes), np.float32)
+        for wave in range(4):
+            total = total + lanes[:, wave, 0]
+        return total
+
+    f = np.float32
+    rows = np.zeros((4, -(-d // 256) * 256), f)
+    rows[:, :d] = x.numpy()
+    inside = np.arange(rows.shape[1]) < d
+    shares = np.zeros((4, 256), f)
+    for i in range(0, rows.shape[1], 256):
+        shares = shares + rows[:, i:i + 256]
+    off = np.where(inside, rows - (workgroup(shares) / f(d))[:, None], f(0))
+    squares = np.zeros((4, 256), f)
+    for i in range(0, rows.shape[1], 256):          # (one rounding a step: the product is exact in the wider type)
+        own = off[:, i:i + 256].astype(np.longdouble)
+        squares = (own * own + squares).astype(f)
+    inv = f(1) / np.sqrt(workgroup(squares) / f(d) + f(1e-5))
+    want = torch.from_numpy(off[:, :d] * inv[:, None] * w.float().numpy()).to(dt)
+    assert torch.equal(out.cpu(), want)
+
+
+@pytest.mark.parametrize("d", [1024, 1028, 2048, 4096, 4100])
+def test_layernorm_rows_have_the_same_bits_among_many(d):
+    """From 1,025 to 2,048 rows some widths go through another kernel."""
+    from hfee_amd.kernels import ops
+    x = torch.randn(2049, d, generator=torch.Generator().manual_seed(d)).cuda()
+    w, outs = torch.full((d,), 0.7, device="cuda"), []
+    for n in (3, 1024, 1025, 2048, 2049):
+        outs.append(torch.zeros(n, d, device="cuda"))
+        ops.layernorm(outs[-1], x[:n], w, 1e-5)
+    assert all(torch.equal(o, outs[-1][:len(o)]) for o in outs) and float(outs[-1].std()) > 0.5
+
+
 def test_layernorm_and_scaled_embedding():
     from hfee_amd.kernels import ops
     g = torch.Generator().manual_seed(0)

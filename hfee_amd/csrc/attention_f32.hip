@@ -9,7 +9,8 @@
 // maximum, sum and values (softmax as it goes), and the four are joined in their order at the end.  Which wave and which
 // place in it adds a key depends only on the key's position, and a tile of which a row sees nothing leaves the row's
 // numbers as they are: a token's result has the same bits however the work was cut into steps, whatever stands around it
-// in the batch, and wherever its pages lie.
+// in the batch, and wherever its pages lie.  (An infinity or NaN in a tile would not leave them: rows that share a workgroup
+// and come out with a NaN are done once more, one by one.)
 //
 // The operands need no rearrangement.  Keys lie in chunks of 16 dims by slot, so a lane's 16 bytes as the rows operand
 // stand in a kilobyte that the wave reads front to back; the scores come out with four keys of one query a lane, which is
@@ -60,6 +61,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
   constexpr bool BOTH = CHUNKS <= 8;        // keys and values of both halves of a tile in registers at once
   __shared__ f32x4 values[WAVES][CHUNKS][kWave];
   __shared__ float most[WAVES][ROWS], sums[WAVES][ROWS];
+  __shared__ bool no_number[WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int per = p.num_heads / lay.kv_heads, heads = min(per, ROWS), parts = (per + heads - 1) / heads;
   const int kvh = blockIdx.y / parts, head0 = (blockIdx.y % parts) * heads;
@@ -76,10 +78,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
     for (int i = 0; i < 4; ++i) q[c][i] = valid ? p.q[(int64_t)token * p.ldq + head * (16 * CHUNKS) + 16 * c + 4 * g + i] : 0.f;
 
   // one run of tokens of the same sequence after the other (nearly always there is one)
+  int longest_run = ROWS;
   for (int from = t0; from < t1;) {
     const int segment = p.token_segment[from];
     int to = from, last = -1, first = 0x7fffffff;
-    for (; to < t1 && p.token_segment[to] == segment; ++to) {
+    for (; to < t1 && to - from < longest_run && p.token_segment[to] == segment; ++to) {
       const int at = p.positions[to];
       last = max(last, at);
       first = min(first, p.window > 0 ? max(0, at - p.window + 1) : 0);
@@ -185,6 +188,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
       weight[w] = most[w][r] == -INFINITY ? 0.f : expf(most[w][r] - top);
       total += sums[w][r] * weight[w];
     }
+    bool nan = false;
     for (int c = wave; c < CHUNKS; c += WAVES) {
       f32x4 all = values[0][c][lane] * weight[0];
 #pragma unroll
@@ -192,7 +196,21 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
       if (mine) {
         float* to_row = p.out + (int64_t)token * p.ld_out + head * (16 * CHUNKS) + 16 * c + 4 * g;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) to_row[i] = all[i] / total;
+        for (int i = 0; i < 4; ++i) {
+          to_row[i] = all[i] / total;
+          nan = nan || isnan(all[i]);
+        }
+      }
+    }
+    // A key's values meet the weights of all rows, those that are zero because a row does not see the key as well, and zero
+    // times an infinity or NaN is NaN: a run with a NaN is done once more, token by token, where rows see the same keys.
+    if (to - from > 1) {
+      const bool some = __ballot(nan) != 0;
+      if (lane == 0) no_number[wave] = some;
+      __syncthreads();
+      if (no_number[0] || no_number[1] || no_number[2] || no_number[3]) {
+        longest_run = 1;
+        continue;
       }
     }
     from = to;

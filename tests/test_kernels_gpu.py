@@ -726,6 +726,42 @@ def test_attention_f32_does_not_depend_on_the_company(H, K, hd, window, ps):
         begin += n
 
 
+@pytest.mark.parametrize("H,K,hd,window", [(8, 2, 64, 0), (4, 4, 16, 0), (3, 1, 144, 0), (8, 2, 32, 9), (20, 1, 48, 30)])
+def test_attention_f32_keeps_what_a_token_does_not_see(H, K, hd, window):
+    """Infinities and NaN in the values and keys of some tokens, in the first, the middle and the last key tiles: tokens in
+    front of them, and behind a window that has passed them, have the bits that they have without, also where they share a
+    workgroup with tokens that do see them; every other token shows them."""
+    from hfee_amd.kernels import ops
+    ps, T = 16, 150
+    g = torch.Generator().manual_seed(H * hd)
+    q, k, v = torch.randn(T, H, hd, generator=g), torch.randn(T, K, hd, generator=g), torch.randn(T, K, hd, generator=g)
+    blocks = -(-T // ps)
+    pages = torch.randperm(blocks, generator=g).tolist()
+    inf = float("inf")
+    marks = {"value": [(37, 0, 1, inf), (110, K - 1, hd - 1, float("nan"))], "negative": [(5, 0, 0, -inf), (149, 0, 3, -inf)],
+             "key": [(70, K - 1, 2, float("nan"))]}
+    q, positions = q.reshape(T, H * hd).to(DEV), torch.arange(T, dtype=torch.int32, device=DEV)
+    seg, table = torch.zeros(T, dtype=torch.int32, device=DEV), torch.tensor([pages], dtype=torch.int32, device=DEV)
+
+    def run(k, v):
+        layer, _ = _paged((k, v), ps, pages)
+        out = torch.zeros(T, H * hd, device=DEV)
+        ops.attention_plain(out, q, layer.to(DEV), positions, seg, table, H, K, hd, ps, hd ** -0.5, window)
+        return out.view(T, H, hd)
+    clean = run(k, v)
+    for what, places in marks.items():
+        k2, v2 = k.clone(), v.clone()
+        for t, h, d, x in places:
+            (k2 if what == "key" else v2)[t, h, d] = x
+        got = run(k2, v2)
+        sees = torch.zeros(T, H, dtype=torch.bool)
+        for t, h, _, _ in places:
+            sees[t:min(T, t + window) if window else T, h * (H // K):(h + 1) * (H // K)] = True
+        sees = sees.to(DEV)
+        assert torch.equal(got[~sees], clean[~sees]), what
+        assert not torch.isfinite(got[sees]).all(-1).any(), what
+
+
 @pytest.mark.parametrize("H,K,hd,T,window,ps", [(4, 1, 128, 130, 0, 32), (8, 2, 64, 150, 40, 64), (4, 1, 48, 300, 0, 128),
                                                 (16, 2, 32, 97, 50, 32)])
 def test_attention_kernels_with_larger_pages(H, K, hd, T, window, ps):

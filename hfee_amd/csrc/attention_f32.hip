@@ -52,7 +52,8 @@ struct Args {
   const int* positions;
   const int* token_segment;
   const int* block_tables;
-  int bt_stride, num_heads, n, tokens, window;      // tokens: how many a workgroup takes
+  const int* items;                                 // (first token, how many) of each workgroup; null: `tokens` each
+  int bt_stride, num_heads, n, tokens, window;
   float scale;
 };
 
@@ -65,7 +66,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int per = p.num_heads / lay.kv_heads, heads = min(per, ROWS), parts = (per + heads - 1) / heads;
   const int kvh = blockIdx.y / parts, head0 = (blockIdx.y % parts) * heads;
-  const int t0 = blockIdx.x * p.tokens, t1 = min(t0 + p.tokens, p.n);
+  const int t0 = p.items != nullptr ? p.items[2 * blockIdx.x] : blockIdx.x * p.tokens;
+  const int t1 = min(t0 + (p.items != nullptr ? p.items[2 * blockIdx.x + 1] : p.tokens), p.n);
   const int token = t0 + r / heads, head = kvh * per + head0 + r % heads;
   const bool valid = token < t1 && head0 + r % heads < per;
   const int pos = valid ? p.positions[token] : -1;
@@ -77,7 +79,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[c][i] = valid ? p.q[(int64_t)token * p.ldq + head * (16 * CHUNKS) + 16 * c + 4 * g + i] : 0.f;
 
-  // one run of tokens of the same sequence after the other (nearly always there is one)
+  // one run of tokens of the same sequence after the other (with items there is one)
   int longest_run = ROWS;
   for (int from = t0; from < t1;) {
     const int segment = p.token_segment[from];
@@ -225,11 +227,15 @@ void launch(const Args& p, const CacheLayout& lay, dim3 grid, hipStream_t stream
 
 }  // namespace
 
-// singles != 0: every token is the only one of its sequence in this call (a workgroup then takes one).
+// A workgroup takes up to 16 rows, which are 16 / heads of a KV head (up to 16) tokens; tokens of different sequences in one
+// would be one after the other, each through its own keys.  items: int32 [item_count][2], the tokens of each workgroup
+// (first, how many); null: neighbours, whatever their sequences, or with singles != 0 one each.  16 requests that decode at
+// 4,000 tokens beside a portion of 64, 4 heads of 64 on as many key heads: 2,250 us neighbour by neighbour, 149 with items
+// (1,610 with a wave a token and head); at 1,000 tokens, 32 heads of 128 on 8 key heads, 213 and 61 (760).
 HFEE_API int hfee_attention_f32(float* out, int64_t ld_out, const float* q, int64_t ldq, const float* cache,
                                 const int* positions, const int* token_segment, const int* block_tables, int bt_stride,
-                                int num_heads, int kv_heads, int head_dim, int page_size, float scale, int window, int singles,
-                                int n, hipStream_t stream) {
+                                int num_heads, int kv_heads, int head_dim, int page_size, float scale, int window, const int* items,
+                                int item_count, int singles, int n, hipStream_t stream) {
   HFEE_REQUIRE(n >= 0, "attention_f32: bad token count");
   if (n == 0) return 0;
   HFEE_REQUIRE(num_heads > 0 && kv_heads > 0 && num_heads % kv_heads == 0,
@@ -237,13 +243,14 @@ HFEE_API int hfee_attention_f32(float* out, int64_t ld_out, const float* q, int6
   HFEE_REQUIRE(head_dim >= 16 && head_dim <= 256 && head_dim % 16 == 0, "attention_f32: head_dim %d is no multiple of 16 up to 256", head_dim);
   HFEE_REQUIRE(num_heads <= 65535, "attention_f32: too many heads");
   HFEE_REQUIRE(window >= 0, "attention_f32: negative window");
+  HFEE_REQUIRE(items == nullptr || item_count > 0, "attention_f32: no items");
   HFEE_REQUIRE(ldq >= (int64_t)num_heads * head_dim && ld_out >= (int64_t)num_heads * head_dim, "attention_f32: q/out row too short");
   HFEE_REQUIRE((uintptr_t)cache % 16 == 0, "attention_f32: the cache layer must start on 16 bytes");
   CacheLayout lay;
   if (make_cache_layout(&lay, kv_heads, head_dim, page_size)) return 1;
   const int per = num_heads / kv_heads, heads = per < ROWS ? per : ROWS, tokens = singles ? 1 : ROWS / heads;
-  const dim3 grid((n + tokens - 1) / tokens, kv_heads * ((per + heads - 1) / heads));
-  const Args p{out, ld_out, q, ldq, cache, positions, token_segment, block_tables, bt_stride, num_heads, n, tokens, window, scale};
+  const dim3 grid(items != nullptr ? item_count : (n + tokens - 1) / tokens, kv_heads * ((per + heads - 1) / heads));
+  const Args p{out, ld_out, q, ldq, cache, positions, token_segment, block_tables, items, bt_stride, num_heads, n, tokens, window, scale};
   switch (head_dim / 16) {
 #define HFEE_CHUNKS(C) case C: launch<C>(p, lay, grid, stream); break;
     HFEE_CHUNKS(1) HFEE_CHUNKS(2) HFEE_CHUNKS(3) HFEE_CHUNKS(4) HFEE_CHUNKS(5) HFEE_CHUNKS(6) HFEE_CHUNKS(7) HFEE_CHUNKS(8)

@@ -392,12 +392,21 @@ def rope_cache_write(q, k, v, positions, token_segment, block_tables, cos, sin, 
                     n, int(portions), _stream())
 
 
+def attention_items(portions, group: int) -> list:
+    """Which tokens share a workgroup of the 32-bit attention: for portions (first row, rows), (first row, rows) of each
+    workgroup.  It takes 16 query rows, those of `group` heads a token, and only tokens of one portion."""
+    most = 16 // min(group, 16)
+    return [(row + at, min(most, rows - at)) for row, rows in portions for at in range(0, rows, most)]
+
+
 def attention_plain(out, q, cache_layer, positions, token_segment, block_tables, num_heads: int,
-                    kv_heads: int, head_dim: int, page_size: int, scale: float, window: int = 0, singles: bool = False):
+                    kv_heads: int, head_dim: int, page_size: int, scale: float, window: int = 0, singles: bool = False,
+                    items=None):
     """The 32-bit path's attention, and in bfloat16 the slow twin of the matrix-core kernels.  Token t reads keys
     max(0, pos-window+1)..pos of its segment's pages.  In float32, heads that are multiples of 16 go through the
     float32 matrix instruction, up to 16 query rows a workgroup; everything else is one wave per (token, head).
-    singles: every token is the only one of its segment (no result changes with it)."""
+    singles: every token is the only one of its segment; items: `attention_items` of the call's portions as int32
+    (no result changes with either: they say which tokens share a workgroup)."""
     _gpu(out, q, cache_layer, positions, token_segment, block_tables)
     n, w, ldq = _rows2d(q, "attention q")
     no, wo, ldo = _rows2d(out, "attention out")
@@ -409,10 +418,15 @@ def attention_plain(out, q, cache_layer, positions, token_segment, block_tables,
     _i32(token_segment, "attention token_segment", n)
     _check(block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.stride(1) == 1,
            "attention: block tables")
+    if items is not None:
+        _gpu(items)
+        _check(items.dtype == torch.int32 and items.dim() == 2 and items.shape[1] == 2 and items.shape[0] > 0 and items.is_contiguous(),
+               "attention: items int32 [number, 2]")
     if q.dtype == torch.float32 and head_dim % 16 == 0 and head_dim <= 256 and cache_layer.data_ptr() % 16 == 0:
         lib.core().call("hfee_attention_f32", _ptr(out), ldo, _ptr(q), ldq, _ptr(cache_layer), _ptr(positions),
                         _ptr(token_segment), _ptr(block_tables), block_tables.stride(0), num_heads, kv_heads, head_dim,
-                        page_size, float(scale), int(window), int(singles), n, _stream())
+                        page_size, float(scale), int(window), _ptr(items), items.shape[0] if items is not None else 0,
+                        int(singles), n, _stream())
         return
     lib.core().call("hfee_attention_ref", _ptr(out), ldo, _ptr(q), ldq, _ptr(cache_layer), _dt(q),
                     _ptr(positions), _ptr(token_segment), _ptr(block_tables), block_tables.stride(0),

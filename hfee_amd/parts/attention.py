@@ -66,6 +66,7 @@ class Attention(Mixer):
             self.second_half_rows = 0      # (the product that would finish a norm's second half is the fused one)
         self.q_width = self.num_heads * self.head_dim
         self.kv_width = self.kv_heads * self.head_dim
+        self._items = f"attention.items of {self.num_heads // self.kv_heads} heads"
         self.w_qkv = self.w_o = None
 
     # ---- weights
@@ -134,6 +135,10 @@ class Attention(Mixer):
             self.position.prepare(info.num_positions, info.device)
 
     def plan(self, plan):
+        # (neighbours share workgroups anyway where there is one portion, and nobody does where each has one token)
+        portions = [(seg.row0, seg.length) for seg in plan.segments]
+        if self.dtype == torch.float32 and self._items not in plan.arrays and 1 < len(portions) < sum(n for _, n in portions):
+            plan.add(self._items, np.asarray(ops.attention_items(portions, self.num_heads // self.kv_heads), dtype=np.int32))
         if self.dtype != torch.bfloat16 or "attention.tiles" in plan.arrays:
             return
         tiles, runs, d_rows, d_pos, d_tab = [], [], [], [], []
@@ -214,7 +219,7 @@ class Attention(Mixer):
         att = ctx.rows("attention.out", self.q_width)
         if self.dtype == torch.float32:
             ops.attention_plain(att, q, cache, ctx.positions, ctx.token_segment, tables, H, K, hd,
-                                ctx.page_size, self.scale, self.window, singles=n == len(ctx.segments))
+                                ctx.page_size, self.scale, self.window, singles=n == len(ctx.segments), items=ctx.extra.get(self._items))
         else:
             tiles = ctx.extra["attention.tiles"]
             if tiles.shape[0]:

@@ -762,6 +762,36 @@ def test_attention_f32_keeps_what_a_token_does_not_see(H, K, hd, window):
         assert not torch.isfinite(got[sees]).all(-1).any(), what
 
 
+@pytest.mark.parametrize("H,K,hd", [(4, 4, 16), (3, 1, 64), (20, 1, 48), (32, 2, 32)])
+def test_attention_f32_by_portions(H, K, hd):
+    """Which tokens share a workgroup: every row once, sixteen query rows at most, one portion only; and no result changes
+    with it, among requests that decode, short portions and a prompt."""
+    from hfee_amd.kernels import ops
+    ps, portions, starts, row = 16, [], [37, 200, 5, 90, 0, 64, 1], 0
+    for n in (1, 1, 2, 3, 70, 1, 17):
+        portions.append((row, n))
+        row += n
+    items = ops.attention_items(portions, H // K)
+    assert [r for at, n in items for r in range(at, at + n)] == list(range(row))
+    for at, n in items:
+        assert 1 <= n and (n == 1 or n * (H // K) <= 16) and any(a <= at and at + n <= a + m for a, m in portions)
+    g = torch.Generator().manual_seed(H)
+    blocks = [-(-(s + n) // ps) for s, (_, n) in zip(starts, portions)]
+    layer = torch.randn(sum(blocks), 2, K, ps * hd, generator=g).to(DEV)
+    tables, at = torch.zeros(len(blocks), max(blocks), dtype=torch.int32), 0
+    for i, b in enumerate(blocks):
+        tables[i, :b] = torch.arange(at, at + b)
+        at += b
+    q = torch.randn(row, H * hd, generator=g).to(DEV)
+    positions = torch.cat([torch.arange(s, s + n, dtype=torch.int32) for s, (_, n) in zip(starts, portions)]).to(DEV)
+    seg = torch.cat([torch.full((n,), i, dtype=torch.int32) for i, (_, n) in enumerate(portions)]).to(DEV)
+    outs = []
+    for kw in ({}, dict(items=torch.tensor(items, dtype=torch.int32, device=DEV))):
+        outs.append(torch.full((row, H * hd), float("nan"), device=DEV))
+        ops.attention_plain(outs[-1], q, layer, positions, seg, tables.to(DEV), H, K, hd, ps, hd ** -0.5, 0, **kw)
+    assert torch.equal(*outs) and torch.isfinite(outs[0]).all()
+
+
 @pytest.mark.parametrize("H,K,hd,T,window,ps", [(4, 1, 128, 130, 0, 32), (8, 2, 64, 150, 40, 64), (4, 1, 48, 300, 0, 128),
                                                 (16, 2, 32, 97, 50, 32)])
 def test_attention_kernels_with_larger_pages(H, K, hd, T, window, ps):

@@ -116,6 +116,9 @@ class Model:
     def state_specs(self):
         return [s for p in self.parts() for s in p.state_specs()]
 
+    def scratch_bytes(self, rows: int) -> int:
+        return sum({p.scratch_bytes(rows) for p in self.parts()})
+
     def prepare(self, info: EngineInfo):
         for p in self.parts():
             p.prepare(info)

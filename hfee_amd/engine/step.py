@@ -121,7 +121,8 @@ class Engine:
     def _workspace_estimate(self) -> int:
         widest = max([s.shape[0] for s in self.model.tensor_specs() if len(s.shape) == 2 and s.shape[0] != self.vocab]
                      or [self.model.spec.hidden])
-        return capacity.workspace_bytes(self.max_batch_tokens, self.vocab, max(widest, self.model.spec.hidden))
+        return (capacity.workspace_bytes(self.max_batch_tokens, self.vocab, max(widest, self.model.spec.hidden))
+                + self.model.scratch_bytes(self.max_batch_tokens))
 
     def _state_bytes(self) -> int:
         total = 0

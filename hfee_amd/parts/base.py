@@ -122,6 +122,11 @@ class Part:
         by a request's slot) and clears a slot when a request is admitted."""
         return []
 
+    def scratch_bytes(self, rows: int) -> int:
+        """What this part asks of the workspace for a step of at most `rows` tokens beside rows of its products' widths;
+        parts that ask for as much share it."""
+        return 0
+
     def prepare(self, engine_info) -> None:
         """Called once before the first step (tables, state tensors...)."""
 

@@ -77,14 +77,24 @@ class _StateMixer(Mixer):
     def _segments(self, ctx):
         return ctx.segment_rows, ctx.segment_lengths, ctx.segment_slots
 
-    @staticmethod
-    def _in_chunks(ctx, heads: int, dim: int) -> dict:
-        """The arguments with which `ops.linear_scan` walks a step's long portions in chunks (fixed decays only)."""
+    def chunk_words(self, longest: int, rows: int) -> int:
+        """float32 words with which `ops.linear_scan` walks the long portions of a step (the longest of `longest` tokens,
+        `rows` in all) in chunks; 0 where it goes token by token."""
+        return 0
+
+    def scratch_bytes(self, rows: int) -> int:
+        return 4 * self.chunk_words(rows, rows)
+
+    def _chunks(self, ctx) -> dict:
+        """The arguments with which `ops.linear_scan` walks a step's long portions in chunks.  The scratch is asked for
+        once, for the most rows that a step can have: sized by the step, every step larger than those before would leave
+        an outgrown buffer behind, which the workspace keeps."""
         lengths = [s.length for s in ctx.segments]
-        words = ops.linear_chunks_scratch(max(lengths), ctx.n, heads, dim)
+        words = self.chunk_words(max(lengths), ctx.workspace.capacity)
         if not words:
             return {}
-        return dict(scratch=ctx.workspace.flat("recurrent.chunks", words, torch.float32), longest=max(lengths), shortest=min(lengths))
+        scratch = ctx.workspace.flat(f"recurrent.chunks of {words}", words, torch.float32)
+        return dict(scratch=scratch, longest=max(lengths), shortest=min(lengths))
 
 
 @register_mixer("gated_delta")
@@ -202,7 +212,7 @@ class GatedDelta(_StateMixer):
         q, k, v = y[:, :self.qk_width], y[:, self.qk_width:2 * self.qk_width], y[:, 2 * self.qk_width:]
         o = ctx.rows("gated_delta.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, decay, beta, rows, lengths, slots, H, G, D, V, "delta",
-                        decay_per_head=self.decay_per_head, **self._delta_chunks(ctx))
+                        decay_per_head=self.decay_per_head, **self._chunks(ctx))
         gate = proj[:, self.g_columns]
         if self.gate_rank is not None:
             gate = ctx.rows("gated_delta.gate", self.v_width)
@@ -211,15 +221,8 @@ class GatedDelta(_StateMixer):
         ops.head_norm_gate(gated, o, gate, self.norm_weight, H, V, self.norm_eps, self.gate_activation)
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)
 
-    def _delta_chunks(self, ctx) -> dict:
-        """The arguments with which `ops.linear_scan` walks a step's long portions in chunks (one decay a head only)."""
-        if not self.decay_per_head:
-            return {}
-        lengths = [s.length for s in ctx.segments]
-        words = ops.delta_chunks_scratch(max(lengths), ctx.n, self.heads, self.dim, self.vdim)
-        if not words:
-            return {}
-        return dict(scratch=ctx.workspace.flat("recurrent.chunks", words, torch.float32), longest=max(lengths), shortest=min(lengths))
+    def chunk_words(self, longest, rows):
+        return ops.delta_chunks_scratch(longest, rows, self.heads, self.dim, self.vdim) if self.decay_per_head else 0
 
     def _inputs(self, ctx, y, beta, proj):
         """What enters the recurrence, a launch a mechanism: fills y and beta, returns the decays."""
@@ -351,6 +354,9 @@ class Retention(_StateMixer):
         if self.position is not None:
             self.position.prepare(info.num_positions, info.device)
 
+    def chunk_words(self, longest, rows):
+        return ops.linear_chunks_scratch(longest, rows, self.heads, self.dim)
+
     def forward_add(self, ctx, x, h, cache_layer: int, writes_cache: bool):
         self._run(ctx, x, h, add=True)
 
@@ -374,7 +380,7 @@ class Retention(_StateMixer):
         q, k, v = qkv[:, :self.qk_width], qkv[:, self.qk_width:self.at_v], qkv[:, self.at_v:]
         o = ctx.rows("retention.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, self.decays, None, rows, lengths, slots, H, H, D, V, "decay_add",
-                        decay_per_head=True, **self._in_chunks(ctx, H, D))
+                        decay_per_head=True, **self._chunks(ctx))
         gated = ctx.rows("retention.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:], self.norm_weight, H, V, self.norm_eps, "silu")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)
@@ -421,6 +427,9 @@ class LightningAttention(_StateMixer):
     def prepare(self, info):
         self.state = info.storage.states[self.prefix + "state"]
 
+    def chunk_words(self, longest, rows):
+        return ops.linear_chunks_scratch(longest, rows, self.heads, self.dim)
+
     def forward_add(self, ctx, x, h, cache_layer: int, writes_cache: bool):
         self._run(ctx, x, h, add=True)
 
@@ -439,7 +448,7 @@ class LightningAttention(_StateMixer):
         q, k, v = qkv[:, :self.qk_width], qkv[:, self.qk_width:self.at_v], qkv[:, self.at_v:]
         o = ctx.rows("lightning.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, self.decays, None, rows, lengths, slots, H, H, D, V, "decay_add",
-                        decay_per_head=True, **self._in_chunks(ctx, H, D))
+                        decay_per_head=True, **self._chunks(ctx))
         gated = ctx.rows("lightning.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:], self.norm_weight, 1, self.v_width, self.norm_eps, "sigmoid")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)

@@ -537,6 +537,22 @@ def test_an_early_token_shows_much_later_through_the_recurrence_alone(folders, a
             assert np.abs(want).max() == 0.0 and np.array_equal(got[("a", 100)], got[("b", 100)])
 
 
+def test_portions_that_grow_ask_for_scratch_once(folders):
+    """Prompts each longer than the one before: what the recurrences' long portions are walked with is one buffer a size of
+    layer, counted beside the step's rows, and none is outgrown."""
+    from hfee_amd.trace_replay import Replayer
+    rep = Replayer(folders[("C", "bfloat16")], "bfloat16", 512, max_requests=2)
+    ws = rep.engine.workspace
+    seen = []
+    for n in (20, 33, 64, 100, 150, 300):
+        toks = np.random.default_rng(n).integers(0, 60, size=n).tolist()
+        tu.run(rep, [{"entries": [("a", toks, [n - 1])], "end": ["a"]}])
+        seen.append({key: buf.data_ptr() for key, buf in ws._buffers.items() if str(key[0]).startswith("recurrent.chunks")})
+    assert seen[0] and all(s == seen[0] for s in seen[1:])
+    sizes = [ws._buffers[key].numel() * 4 for key in seen[0]]
+    assert sum(sizes) <= rep.engine.model.scratch_bytes(ws.capacity)
+
+
 def greedy(folder, prompt, count):
     seq = list(prompt)
     for _ in range(count):

@@ -437,10 +437,9 @@ double tile_cost(const Product& p) {
 template <int TM, int TN>
 void launch_direct(const Product& p, hipStream_t stream) {
   const dim3 grid((unsigned)tile_count<TM, TN>(p)), block(256);
-  const size_t lds = (size_t)4 * 32 * (TM + TN) * 128;
+  constexpr size_t lds = (size_t)4 * 32 * (TM + TN) * 128;
+  static_assert(lds <= 64 * 1024, "a kernel gets more LDS only after hipFuncSetAttribute");
   const auto go = [&](auto kernel) {
-    static const hipError_t raised = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    (void)raised;
     kernel<<<grid, block, lds, stream>>>(p.C, p.ldc, p.A, p.lda, p.W, p.ldw, p.M, p.N, p.K, p.wide_stores);
   };
   p.accumulate ? go(direct_kernel<TM, TN, true>) : go(direct_kernel<TM, TN, false>);

@@ -153,12 +153,27 @@ __global__ __launch_bounds__(256) void moe_up_kernel(T* __restrict__ act, const 
   }
 }
 
-// moe_up for gated experts in bfloat16 and at most 64 pairs, expert by expert: grid (blocks of 16 rows, experts), so that an expert's rows come
-// through every XCD.  Every wave
-// finds the pairs that use the workgroup's expert and takes up to four of them at a time over its four rows of both
-// matrices, so that an expert's rows come once however many tokens chose it.  16 experts of 2,048, width 4,096, the
-// matrices from memory (events around the call, some 8 us of it): 8 tokens on two experts each, 9 different ones, 93 -> 64
-// us; 2 tokens 48 -> 33; one 45 -> 30.  (With the experts as the faster index all of an expert's blocks went to one XCD: 94.)
+// Of at most 64 pairs, lane p the expert of pair p (negative: none): the pairs of the `which`-th different expert, in the
+// order of their first pairs; none where there are not so many.
+__device__ __forceinline__ uint64_t users_of(int e, int which) {
+  uint64_t left = __ballot(e >= 0), users = 0;
+  for (int i = 0; left != 0; ++i) {
+    const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
+    users = __ballot(e == mine);
+    if (i == which) return users;
+    left &= ~users;
+  }
+  return 0;
+}
+
+// moe_up for gated experts in bfloat16 and at most 64 pairs, expert by expert: grid (blocks of 16 rows, pairs or experts,
+// whichever are fewer), a column of workgroups a different expert of the step, so that an expert's rows come through every
+// XCD (with the experts as the faster index all of an expert's blocks went to one: 94 us for 64).  Every wave finds the
+// pairs that use its expert and takes up to four of them at a time over its four rows of both matrices, so that an
+// expert's rows come once however many tokens chose it.  us pair by pair / expert by expert: 16 experts of 2,048, width 4,096,
+// one token on two 35.5 / 16.0, 8 tokens on two each 84 / 62, 64 on one 323 / 130; 256 experts of 2,048, width 2,048, one token on
+// two 19.9 / 10.1 (28 with a column of workgroups an expert of the model, most of which left at once), 16 tokens on one each
+// 43.5 / 47, 64 on one each 179 / 158; 256 experts of 512 and the same 48.5 / 46.
 template <int P>
 __device__ __forceinline__ void up_for_pairs(bf16_t* act, const bf16_t* h, int64_t ldh, const bf16_t* const (&rows)[2 * kRowsPerWave],
                                              const int (&pairs)[P], int top, int f0, int F, int width, int lane, int gate_act,
@@ -182,11 +197,15 @@ __device__ __forceinline__ void up_for_pairs(bf16_t* act, const bf16_t* h, int64
 __global__ __launch_bounds__(256) void moe_up_by_expert_kernel(bf16_t* __restrict__ act, const bf16_t* __restrict__ h, int64_t ldh,
                                                                const bf16_t* __restrict__ w_gate, const bf16_t* __restrict__ w_up,
                                                                const int* __restrict__ chosen, const int* __restrict__ table,
-                                                               const int* __restrict__ token_ids, int n_pairs, int top, int F, int width,
-                                                               int gate_act, GateNumbers numbers) {
-  const int e = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, f0 = (blockIdx.x * 4 + wave) * kRowsPerWave;
-  uint64_t users = __ballot(lane < n_pairs && expert_of(chosen, table, token_ids, min(lane, n_pairs - 1) / top, min(lane, n_pairs - 1) % top, top) == e);
+                                                               const int* __restrict__ token_ids, int n_pairs, int top, int experts, int F,
+                                                               int width, int gate_act, GateNumbers numbers) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, f0 = (blockIdx.x * 4 + wave) * kRowsPerWave;
+  int own = -1;
+  if (lane < n_pairs) own = expert_of(chosen, table, token_ids, lane / top, lane % top, top);
+  if (own >= experts) own = -1;
+  uint64_t users = users_of(own, blockIdx.y);
   if (users == 0 || f0 >= F) return;
+  const int e = __builtin_amdgcn_readlane(own, __builtin_ctzll(users));
   const bf16_t* rows[2 * kRowsPerWave];
 #pragma unroll
   for (int r = 0; r < kRowsPerWave; ++r) {
@@ -272,10 +291,13 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
   }
 }
 
-// moe_down in bfloat16 for at most 64 pairs, expert by expert: a workgroup has four rows of the result, its four waves take
-// the step's different experts in turn, up to four of an expert's pairs at a time on the same bytes; the pairs' sums
-// meet in LDS, where a token's are added up in the order of its experts, as above.  16 experts of 2,048, width 4,096, 8 tokens
-// on two each: 43 -> 32 us in a step.
+// moe_down in bfloat16 for at most 64 pairs, expert by expert: a workgroup has four rows of the result, its waves take the
+// step's different experts in turn, up to four of an expert's pairs at a time on the same bytes; the pairs' sums meet in
+// LDS, where a token's are added up in the order of its experts, as above.  What bounds it is loads in flight: rows of a
+// narrow result are few workgroups, which then have more waves.  us token by token row by row / four waves / as now: 16 experts of
+// 2,048, width 4,096, 8 tokens on two each 44 / 32 / 32; 128 experts of 768, width 2,048, 16 tokens on one each 14.5 / 19.8 /
+// 14.7, one token on eight 46 / 11.7 / 9.7; 256 experts of 64, width 1,024, 64 tokens on one each 16.6 / 34.5 / 16.1; 16 waves at
+// width 4,096 47 for the first.
 template <int P>
 __device__ __forceinline__ void down_for_pairs(float (*sums)[kRowsPerWave], const bf16_t* act, const bf16_t* const (&rows)[kRowsPerWave],
                                                const int (&pairs)[P], int F, int lane) {
@@ -293,7 +315,8 @@ __device__ __forceinline__ void down_for_pairs(float (*sums)[kRowsPerWave], cons
     }
 }
 
-__global__ __launch_bounds__(256) void moe_down_by_expert_kernel(float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ act,
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void moe_down_by_expert_kernel(float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ act,
                                                                  const bf16_t* __restrict__ w_down, const int* __restrict__ chosen,
                                                                  const int* __restrict__ table, const int* __restrict__ token_ids,
                                                                  const float* __restrict__ pair_weights, float weight, int n_pairs, int top,
@@ -308,7 +331,7 @@ __global__ __launch_bounds__(256) void moe_down_by_expert_kernel(float* __restri
     const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
     uint64_t users = __ballot(e == mine);
     left &= ~users;
-    if ((turn & 3) != wave) continue;
+    if ((turn & (WAVES - 1)) != wave) continue;
     const bf16_t* rows[kRowsPerWave];
 #pragma unroll
     for (int r = 0; r < kRowsPerWave; ++r) rows[r] = w_down + ((int64_t)mine * width + min(c0 + r, width - 1)) * F;
@@ -1036,12 +1059,12 @@ HFEE_API int hfee_moe_up(void* act, const void* h, int64_t ldh, const void* w_ga
     moe_up_kernel<float><<<grid, 256, 0, stream>>>((float*)act, (const float*)h, ldh, (const float*)w_gate, (const float*)w_up,
                                                    chosen, table, token_ids, top, experts, ff, width, in_weights,
                                                     gate_act, numbers);
-  // (expert by expert where the pairs fit a wave's lanes and there are not so many experts that most workgroups leave at once)
-  else if (dtype == 1 && w_gate != nullptr && (int64_t)n * top <= 64 && experts <= 256 && width % 8 == 0 && ldh % 8 == 0 &&
+  // (expert by expert where the pairs fit a wave's lanes)
+  else if (dtype == 1 && w_gate != nullptr && (int64_t)n * top <= 64 && width % 8 == 0 && ldh % 8 == 0 &&
            (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_up) & 15) == 0)
-    moe_up_by_expert_kernel<<<dim3(grid.y, experts), 256, 0, stream>>>((bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate,
-                                                                     (const bf16_t*)w_up, chosen, table, token_ids, n * top, top, ff,
-                                                                     width, gate_act, numbers);
+    moe_up_by_expert_kernel<<<dim3(grid.y, n * top < experts ? n * top : experts), 256, 0, stream>>>(
+        (bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate, (const bf16_t*)w_up, chosen, table, token_ids, n * top, top, experts,
+        ff, width, gate_act, numbers);
   else if (dtype == 1)
     moe_up_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate,
                                                     (const bf16_t*)w_up, chosen, table, token_ids, top, experts, ff, width, in_weights,
@@ -1064,11 +1087,23 @@ HFEE_API int hfee_moe_down(float* x, int64_t ldx, const void* act, const void* w
   if (dtype == 0)
     moe_down_kernel<float><<<grid, 256, 0, stream>>>(x, ldx, (const float*)act, (const float*)w_down, chosen, table,
                                                      token_ids, pair_weights, weight, top, experts, ff, width, accumulate);
-  // (expert by expert as in moe_up)
-  else if (dtype == 1 && (int64_t)n * top <= 64 && ff % 8 == 0 && (((uintptr_t)act | (uintptr_t)w_down) & 15) == 0)
-    moe_down_by_expert_kernel<<<(width + kRowsPerWave - 1) / kRowsPerWave, 256, 0, stream>>>(
-        x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table, token_ids, pair_weights, weight, n * top, top, experts, ff, width,
-        accumulate);
+  // Expert by expert as in moe_up, but for tokens of one expert each that hardly share any: they have nothing to read
+  // together, and all waves work.  us token by token / expert by expert: one token, 16 experts of 2,048, width 4,096,
+  // 6.8 / 8.0; 2 tokens 9.0 / 9.6, 4 of them 13.8 / 14.4, 8 of them 26 / 22; 8 tokens, 64 experts of 1,408, width 2,048,
+  // 10.6 / 12.1, 16 of them 19.4 / 17.8; 2 tokens, 8 experts of 4,096, width 4,096, 15.8 / 14.5.
+  else if (dtype == 1 && (int64_t)n * top <= 64 && !(top == 1 && (n == 1 || experts >= 8 * n)) && ff % 8 == 0 &&
+           (((uintptr_t)act | (uintptr_t)w_down) & 15) == 0) {
+    const int different = n * top < experts ? n * top : experts, blocks = (width + kRowsPerWave - 1) / kRowsPerWave;
+    const auto go = [&](auto kernel, int waves) {
+      kernel<<<blocks, 64 * waves, 0, stream>>>(x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table, token_ids, pair_weights,
+                                                weight, n * top, top, experts, ff, width, accumulate);
+    };
+    // (as many waves as there can be different experts, and as make sixteen a CU)
+    const int waves = different < 4096 / blocks ? different : 4096 / blocks;
+    if (waves <= 4) go(moe_down_by_expert_kernel<4>, 4);
+    else if (waves <= 8) go(moe_down_by_expert_kernel<8>, 8);
+    else go(moe_down_by_expert_kernel<16>, 16);
+  }
   else if (dtype == 1)
     moe_down_kernel<bf16_t><<<grid, 256, 0, stream>>>(x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table,
                                                       token_ids, pair_weights, weight, top, experts, ff, width, accumulate);

@@ -413,6 +413,32 @@ def test_few_tokens_second_product(n, top, E, width, ff, accumulate):
     assert torch.equal(run([n - 1])[0], out[n - 1])
 
 
+@pytest.mark.parametrize("n,top,E,width,ff", [(5, 1, 48, 96, 64), (6, 1, 47, 96, 64), (2, 1, 16, 4100, 16), (7, 1, 7, 2500, 24),
+                                              (8, 8, 300, 1100, 40), (3, 2, 300, 4096, 8), (64, 1, 300, 64, 64)])
+def test_few_tokens_have_the_same_bits_alone(n, top, E, width, ff):
+    """Four, eight and sixteen waves a workgroup, tokens of one expert each on both sides of the line from which they go token
+    by token, more experts than pairs, among them numbers that stand for none: what a token alone gives, bit for bit."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(n * E)
+    rand = lambda *shape: (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(torch.bfloat16).cuda()      # noqa: E731
+    h, wg, wu, wd = rand(n, width) * 16, rand(E, ff, width), rand(E, ff, width), rand(E, width, ff)
+    chosen = torch.stack([torch.randperm(E + 1, generator=g)[:top] for _ in range(n)]).to(torch.int32).cuda()     # (E: no expert)
+    weights = torch.rand(n, top, generator=g).cuda()
+
+    def run(rows):
+        act = torch.zeros(len(rows) * top, ff, dtype=torch.bfloat16, device="cuda")
+        x = torch.ones(len(rows), width, device="cuda")
+        some = chosen[rows].contiguous()
+        ops.moe_up(act, h[rows].contiguous(), wg, wu, top, chosen=some)
+        ops.moe_down(x, act, wd, top, pair_weights=weights[rows].contiguous(), chosen=some)
+        return act.view(len(rows), top, ff), x
+    act, x = run(list(range(n)))
+    assert float(act.float().std()) > 0 and float(x.std()) > 0
+    for t in range(n):
+        one_act, one_x = run([t])
+        assert torch.equal(one_act[0], act[t]) and torch.equal(one_x[0], x[t])
+
+
 @pytest.mark.parametrize("counts,width,ff", [((1, 0, 64, 65, 128, 129, 300), 128, 192), ((16, 17, 0, 2), 64, 64),
                                              ((200, 3), 576, 320), ((70, 129, 31), 96, 160)])
 @pytest.mark.parametrize("gated", [True, False])

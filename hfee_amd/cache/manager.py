@@ -247,8 +247,8 @@ class CacheManager:
                           tables=[[] for _ in self.groups], first_live_block=[0] * len(self.groups),
                           arrays=[np.zeros(16, dtype=np.int32) for _ in self.groups])
         self.requests[request_id] = rc
-        if self.keep_prefixes and tokens is not None and self._kept:
-            n_pages = (len(tokens) - 1) // self.page_size
+        n_pages = (len(tokens) - 1) // self.page_size if self.keep_prefixes and tokens is not None and self._kept else 0
+        if n_pages > 0:
             rc.digests = PageDigests(self.page_size)
             rc.digests.cover(tokens, n_pages)
             taken = rc.digests.take_from(self._kept)
@@ -276,6 +276,7 @@ class CacheManager:
         keep = 0
         if self.keep_prefixes and tokens is not None:
             keep = min(len(tokens), rc.length) // self.page_size
+        if keep:
             own = rc.digests
             if own is None or not own.cover(tokens, keep):
                 own = PageDigests(self.page_size)

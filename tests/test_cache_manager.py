@@ -255,6 +255,19 @@ def test_a_release_may_know_other_tokens_than_the_admission(as_array):
     m.release("d")
 
 
+def test_less_than_a_page_is_not_digested():
+    """A prompt that fills no page, or just one (its last token has to run), is admitted and released without digests."""
+    m = keeping(pages=12)
+    run_whole(m, "a", list(range(64)))
+    m.release("a", list(range(64)))
+    for n in (0, 1, 15, 16):
+        assert m.admit("b", list(range(n))).digests is None and m.get("b").length == 0
+        m.release("b", list(range(n)))
+    assert m.admit("c", list(range(17))).length == 16
+    m.release("c")
+    m.check()
+
+
 def test_prefixes_are_not_kept_where_a_window_has_given_pages_back():
     with pytest.raises(CacheError, match="every cache group keeps every token"):
         CacheManager([CacheGroupSpec("window", (2, 1, 16), (0,), window=32)], 16, 8, 2, keep_prefixes=True)

@@ -152,8 +152,8 @@ class PageDigests:
             return False
         if end > have:
             more = list(tokens[have:end])
+            self.data += np.asarray(more, dtype=np.int64).tobytes()      # (raises before anything is taken in)
             self.tokens += more
-            self.data += np.asarray(more, dtype=np.int64).tobytes()
         return True
 
     def page(self, b: int) -> bytes:

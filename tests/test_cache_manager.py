@@ -268,6 +268,20 @@ def test_less_than_a_page_is_not_digested():
     m.check()
 
 
+def test_tokens_that_are_no_numbers_leave_a_request_as_it_was():
+    m = keeping(pages=12)
+    run_whole(m, "a", list(range(64)))
+    m.release("a", list(range(64)))
+    rc = m.admit("b", list(range(40)))
+    m.reserve("b", 32), m.commit("b", 32)
+    for _ in range(2):
+        with pytest.raises(OverflowError):
+            m.release("b", list(range(40)) + [2 ** 70] * 24)
+    assert len(rc.digests.data) == 8 * len(rc.digests.tokens)
+    m.release("b", list(range(64)))
+    m.check()
+
+
 def test_prefixes_are_not_kept_where_a_window_has_given_pages_back():
     with pytest.raises(CacheError, match="every cache group keeps every token"):
         CacheManager([CacheGroupSpec("window", (2, 1, 16), (0,), window=32)], 16, 8, 2, keep_prefixes=True)

@@ -1,5 +1,6 @@
 // Plain paged attention: one wave per (token, head), any head size, any page size.
-// It is the 32-bit path's attention and the slow twin of the matrix-core kernels.
+// It is the 32-bit path's attention for head sizes that are no multiple of 16 (others: attention_f32.hip) and the slow twin
+// of the bfloat16 kernels.
 //
 // The reference's order (/root/reference/internal/llm/forward.go:144-178,
 // /root/reference/internal/ggml/ops.go:136-150): score_j = dot(q, k_j) * scale for

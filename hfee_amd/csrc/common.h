@@ -187,6 +187,15 @@ __device__ __forceinline__ float gate_other_exact(float g, int act) {
   return fmaxf(g, 0.0f);
 }
 
+// A workgroup barrier without a fence.  The barrier instruction does not count as a
+// memory access for the compiler, so the empty statements on both sides keep the LDS
+// reads and the loads into the LDS where they were written, relative to it.
+__device__ __forceinline__ void barrier_no_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // ---- reductions with a fixed order -------------------------------------------
 // Every lane ends with the same value; the tree's shape does not depend on data.
 __device__ __forceinline__ float wave_sum(float v) {

@@ -904,15 +904,6 @@ __device__ __forceinline__ void accumulators_settle() {
 // K must be a multiple of 32 and every row's byte offset must fit 31 bits.
 constexpr int DBK = 32, DROW = DBK * 2;      // bytes of a tile row in a buffer
 
-// A workgroup barrier without a fence.  The barrier instruction does not count as a
-// memory access for the compiler, so the empty statements on both sides keep the LDS
-// reads and the loads into the LDS where they were written, relative to it.
-__device__ __forceinline__ void barrier_no_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 __device__ __forceinline__ uint32_t swizzle(uint32_t row) { return ((row >> 3) & 1u) | ((row >> 1) & 2u); }
 
 template <int MODE, int TM, int TN>

@@ -205,12 +205,6 @@ __device__ __forceinline__ void store_tile(float* C, int64_t ldc, int M, int N, 
   }
 }
 
-__device__ __forceinline__ void barrier_no_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // Tiles of 32 TM rows of A and 32 TN rows of W, two by two waves with 16 TM x 16 TN each.  K in steps of 32 columns; a
 // step's rows, 128 bytes each, go from memory straight into one of four buffers in LDS, asked for three steps before they
 // are read and read one step before they are multiplied.  A row's eight 16-byte chunks lie at chunk ^ (row % 8), so that

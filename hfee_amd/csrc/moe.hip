@@ -432,12 +432,6 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ void barrier_no_fence() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 constexpr int kStageK = 32, kStagePitch = 40;
 
 template <int KIND>

@@ -80,7 +80,10 @@ class Engine:
                                   *self._memory(), self._workspace_estimate())
             num_pages = list(wanted)
         else:
-            num_pages = capacity.choose_pages(wanted, at_most, *self._memory(), self._workspace_estimate(),
+            # (the parts' own scratch comes off a pool that is sized here; a number of pages that its caller insists on is
+            # not refused over it, as it is asked for by the steps that need it and out of the reserve)
+            scratch = model.scratch_bytes(max_batch_tokens) if wanted is None else 0
+            num_pages = capacity.choose_pages(wanted, at_most, *self._memory(), self._workspace_estimate() + scratch,
                                               page_size * bytes_per_token(self.groups, self.dtype),
                                               self._state_bytes())
         if not isinstance(num_pages, (list, tuple)) and any(g.every > 1 for g in self.groups):
@@ -121,8 +124,7 @@ class Engine:
     def _workspace_estimate(self) -> int:
         widest = max([s.shape[0] for s in self.model.tensor_specs() if len(s.shape) == 2 and s.shape[0] != self.vocab]
                      or [self.model.spec.hidden])
-        return (capacity.workspace_bytes(self.max_batch_tokens, self.vocab, max(widest, self.model.spec.hidden))
-                + self.model.scratch_bytes(self.max_batch_tokens))
+        return capacity.workspace_bytes(self.max_batch_tokens, self.vocab, max(widest, self.model.spec.hidden))
 
     def _state_bytes(self) -> int:
         total = 0

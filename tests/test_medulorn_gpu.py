@@ -624,6 +624,23 @@ def test_portions_that_grow_ask_for_scratch_once(folders):
     assert sum(sizes) <= rep.engine.model.scratch_bytes(ws.capacity)
 
 
+def test_scratch_does_not_refuse_a_pool_that_was_asked_for(folders, monkeypatch):
+    """Free memory for the pages that are asked for and not for the recurrences' scratch as well: by number they are
+    accepted, and a pool that the engine sizes itself leaves room for the scratch."""
+    from hfee_amd.cache import bytes_per_token
+    from hfee_amd.engine import Engine, load_model
+    model, _ = load_model(folders[("C", "bfloat16")], "bfloat16")
+    sizes = dict(page_size=16, max_requests=2, max_batch_tokens=512)
+    eng = Engine(model, num_pages=8, **sizes)
+    scratch, page, total = model.scratch_bytes(512), 16 * bytes_per_token(eng.groups, torch.bfloat16), 1 << 30
+    n = scratch // page + 3
+    free = eng._workspace_estimate() + eng._state_bytes() + n * page + int(0.05 * total)
+    monkeypatch.setattr(Engine, "_memory", lambda self: (free, total))
+    first = lambda e: e.num_pages[0] if isinstance(e.num_pages, (list, tuple)) else e.num_pages      # noqa: E731
+    assert scratch > page and first(Engine(model, num_pages=n, **sizes)) == n
+    assert 1 <= first(Engine(model, **sizes)) <= 3
+
+
 def greedy(folder, prompt, count):
     seq = list(prompt)
     for _ in range(count):

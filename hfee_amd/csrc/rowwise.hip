@@ -291,13 +291,13 @@ HFEE_API int hfee_layernorm(void* out, int out_dtype, const float* x, const void
   HFEE_REQUIRE(n >= 0 && d > 0, "layernorm: bad sizes n=%d d=%d", n, d);
   HFEE_REQUIRE(eps >= 0.f, "layernorm: eps must not be negative");
   if (n == 0) return 0;
-  // (A CU has room for eight rows of layernorm_kernel's 256 threads or two of a thousand: from 1,025 to 2,048 rows of more
-  // than 1,024 the former are one round over the chip and the latter three or four.  us layernorm_kernel / in fours: rows of
-  // 4,096, 1,024 of them 9.1 / 9.0, 1,200 9.8 / 10.3, 2,048 12.4 / 15.1, 2,304 17.1 / 16.8, 4,096 28.9 / 28.2; rows of 2,048,
-  // 1,200 of them 7.0 / 6.6, 2,048 8.6 / 9.0, 2,304 11.7 / 9.9; rows of 1,024, 2,048 of them 6.7 / 6.2.)
-  const bool one_round = d > 1024 && d <= 4096 && n > 1024 && n <= 2048;
-  const bool fours = !one_round && d % 4 == 0 && d <= 8192 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
   const int each = d <= 4096 ? 4 : 8, needed = ((d + each - 1) / each + 63) / 64 * 64, threads = needed < 256 ? 256 : needed;
+  // Wide rows of up to 4,096 go through fours while all are on the chip at once, a CU having room for 2,048 threads; of rows that
+  // come out in 32 bits, which have as much to write as to read, half as many.  us layernorm_kernel / in fours: rows of 4,096 in
+  // bfloat16, 256 of them 5.6 / 4.1, 512 6.0 / 4.8, 1,024 7.0 / 8.2, 8,192 41 / 47; in 32 bits, 256 of them 4.3 / 4.4, 512 5.1 / 5.3,
+  // 1,024 7.3 / 8.4, 8,192 39 / 49; rows of 2,048 in bfloat16, 1,024 of them 5.5 / 5.0; rows of 512, 8,192 of them 16 / 13.
+  const bool few = n <= 256 * ((out_dtype == 0 ? 1024 : 2048) / threads);
+  const bool fours = (d <= 1024 || d > 4096 || few) && d % 4 == 0 && d <= 8192 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0;
 #define LAUNCH(TO, TW)                                                                                                       \
   do {                                                                                                                       \
     if (!fours) layernorm_kernel<TO, TW><<<n, 256, 0, stream>>>((TO*)out, x, (const TW*)w, rows, eps, d);                    \

@@ -91,15 +91,16 @@ def test_layernorm_has_one_order_of_additions(d, dt):
 
 
 @pytest.mark.parametrize("d", [1024, 1028, 2048, 4096, 4100])
-def test_layernorm_rows_have_the_same_bits_among_many(d):
-    """From 1,025 to 2,048 rows some widths go through another kernel."""
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_layernorm_rows_have_the_same_bits_among_many(d, dt):
+    """From some number of rows on, another one for either type, rows of 1,025 to 4,096 go through another kernel."""
     from hfee_amd.kernels import ops
     x = torch.randn(2049, d, generator=torch.Generator().manual_seed(d)).cuda()
     w, outs = torch.full((d,), 0.7, device="cuda"), []
-    for n in (3, 1024, 1025, 2048, 2049):
-        outs.append(torch.zeros(n, d, device="cuda"))
+    for n in (3, 256, 257, 512, 513, 1024, 1025, 2049):
+        outs.append(torch.zeros(n, d, dtype=dt, device="cuda"))
         ops.layernorm(outs[-1], x[:n], w, 1e-5)
-    assert all(torch.equal(o, outs[-1][:len(o)]) for o in outs) and float(outs[-1].std()) > 0.5
+    assert all(torch.equal(o, outs[-1][:len(o)]) for o in outs) and float(outs[-1].float().std()) > 0.5
 
 
 def test_layernorm_and_scaled_embedding():

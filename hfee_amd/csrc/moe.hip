@@ -692,45 +692,60 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
       acc[i][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.w[sixteen][i], o.a[sixteen][m], acc[i][m], 0, 0, 0);
     };
 
+    if (steps < BUFFERS) {                                           // a buffer for every step, and no repeats
+      for (int s = 0; s < steps; ++s)
 #pragma unroll
-    for (int s = 0; s < BUFFERS; ++s)
-#pragma unroll
-      for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFFERS - 1) * LOADS) : "memory");
-    barrier_no_fence();
-    Operands o[2];
-#pragma unroll
-    for (int i = 0; i < READS; ++i) read_one(0, 0, o[0], i);
-    int now = 0;                                                     // the step's buffer
-    for (int s = 0; s < steps; ++s) {
-      const int next = now == BUFFERS - 1 ? 0 : now + 1;
-      // the first 32 columns, with the reads of the others
-#pragma unroll
-      for (int p = 0; p < PRODUCTS; ++p) {
-        multiply_one(o[0], p);
-#pragma unroll
-        for (int i = 0; i < READS; ++i)
-          if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(now, 1, o[1], i);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      // this wave's part of step s + 1 has landed and its reads of step s are done; behind the barrier everybody's
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((BUFFERS - 2) * LOADS) : "memory");
+        for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       barrier_no_fence();
+      for (int half = 0; half < 2 * steps; ++half) {
+        Operands o;
 #pragma unroll
-      for (int p = 0; p < PRODUCTS; ++p) {
-        multiply_one(o[1], p);
+        for (int i = 0; i < READS; ++i) read_one(half / 2, half % 2, o, i);
 #pragma unroll
-        for (int i = 0; i < READS; ++i)
-          if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(next, 0, o[0], i);
-#pragma unroll
-        for (int l = 0; l < LOADS; ++l)
-          if (l >= LOADS * p / PRODUCTS && l < LOADS * (p + 1) / PRODUCTS) load_one(s + BUFFERS, now, l);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int p = 0; p < PRODUCTS; ++p) multiply_one(o, p);
       }
-      now = next;
+    } else {
+#pragma unroll
+      for (int s = 0; s < BUFFERS; ++s)
+#pragma unroll
+        for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFFERS - 1) * LOADS) : "memory");
+      barrier_no_fence();
+      Operands o[2];
+#pragma unroll
+      for (int i = 0; i < READS; ++i) read_one(0, 0, o[0], i);
+      int now = 0;                                                     // the step's buffer
+      for (int s = 0; s < steps; ++s) {
+        const int next = now == BUFFERS - 1 ? 0 : now + 1;
+        // the first 32 columns, with the reads of the others
+#pragma unroll
+        for (int p = 0; p < PRODUCTS; ++p) {
+          multiply_one(o[0], p);
+#pragma unroll
+          for (int i = 0; i < READS; ++i)
+            if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(now, 1, o[1], i);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        // this wave's part of step s + 1 has landed and its reads of step s are done; behind the barrier everybody's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((BUFFERS - 2) * LOADS) : "memory");
+        barrier_no_fence();
+#pragma unroll
+        for (int p = 0; p < PRODUCTS; ++p) {
+          multiply_one(o[1], p);
+#pragma unroll
+          for (int i = 0; i < READS; ++i)
+            if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(next, 0, o[0], i);
+#pragma unroll
+          for (int l = 0; l < LOADS; ++l)
+            if (l >= LOADS * p / PRODUCTS && l < LOADS * (p + 1) / PRODUCTS) load_one(s + BUFFERS, now, l);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        now = next;
+      }
+      // the repeats asked for past the end still write into this workgroup's LDS: they land before the wave ends
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    // the repeats asked for past the end still write into this workgroup's LDS: they land before the wave ends
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
     // register q of lane l in (i, m): row 8 (q / 4) + 4 (l / 32) + q % 4 of the wave's group i, pair 32 m + l % 32
 #pragma unroll
@@ -993,9 +1008,12 @@ HFEE_API int hfee_moe_grouped(float* x, int64_t ldx, const void* h, int64_t ldh,
   HFEE_REQUIRE(order != nullptr && tiles != nullptr && act != nullptr && ((top == 1 && x != nullptr) || y != nullptr), "moe_grouped: scratch missing");
   HFEE_REQUIRE((int64_t)n * top < (1 << 30), "moe_grouped: too many pairs");
   if (n == 0) return 0;
-  // (tiles through LDS loads: steps of 64 columns, and offsets of 32 bits from the first row of an operand)
+  // Tiles through LDS loads: steps of 64 columns, and offsets of 32 bits from the first row of an operand.  (Not for many pairs
+  // of a width of one such step, which is no work to have a whole CU's LDS for.  us by way of registers / straight into LDS, width
+  // 64: 8 experts of 64, 500 pairs 27 / 25, 1,000 18.2 / 25, 16,384 35 / 41; 8 of 4,096, 130 pairs 78 / 40, 2,048 105 / 94,
+  // 16,384 172 / 252.)
   const int64_t limit32 = (int64_t)1 << 31;
-  const bool direct = width % 64 == 0 && ff % 64 == 0 && ((int64_t)n * ldh) * 2 < limit32 && (int64_t)n * top * ff * 2 < limit32 &&
+  const bool direct = width % 64 == 0 && ff % 64 == 0 && (width > 64 || (int64_t)n * top < 960) && ((int64_t)n * ldh) * 2 < limit32 && (int64_t)n * top * ff * 2 < limit32 &&
                       (int64_t)ff * width * 2 < limit32;
   const int tile_pairs = direct ? kWidePairs : kTilePairs, most = (int)(((int64_t)n * top + tile_pairs - 1) / tile_pairs) + experts;
   moe_group_kernel<<<1, 1024, 4 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts, tile_pairs);

@@ -440,7 +440,8 @@ def test_few_tokens_have_the_same_bits_alone(n, top, E, width, ff):
         assert torch.equal(one_act[0], act[t]) and torch.equal(one_x[0], x[t])
 
 
-@pytest.mark.parametrize("counts,width,ff", [((1, 0, 64, 65, 128, 129, 300), 128, 192), ((16, 17, 0, 2), 64, 64),
+@pytest.mark.parametrize("counts,width,ff", [((1, 0, 64, 65, 128, 129, 300), 128, 192), ((16, 17, 0, 2), 64, 64), ((100, 30), 64, 128),
+                                             ((129, 63), 256, 64), ((700, 300), 64, 64),
                                              ((200, 3), 576, 320), ((70, 129, 31), 96, 160)])
 @pytest.mark.parametrize("gated", [True, False])
 def test_grouped_experts_at_the_edges_of_their_tiles(counts, width, ff, gated):

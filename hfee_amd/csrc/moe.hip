@@ -111,6 +111,27 @@ __device__ __forceinline__ void many_dots(const bf16_t* const (&rows)[R], const 
   }
 }
 
+// wave_sum of N values (a power of two), with its additions: in a step a lane hands the half of the values that it does not
+// keep to the lane that does, so that 2 N moves do what 6 N did.  Lane l ends with the sum of value l / (64 / N).
+template <int N, int OFF = 32>
+__device__ __forceinline__ float wave_sums(const float (&v)[N], int lane) {
+  if constexpr (OFF == 0) {
+    return v[0];
+  } else if constexpr (N == 1) {
+    const float one[1] = {v[0] + __shfl_xor(v[0], OFF, kWave)};
+    return wave_sums<1, OFF / 2>(one, lane);
+  } else {
+    const bool upper = (lane & OFF) != 0;
+    float half[N / 2];
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const float keep = upper ? v[i + N / 2] : v[i], give = upper ? v[i] : v[i + N / 2];
+      half[i] = keep + __shfl_xor(give, OFF, kWave);
+    }
+    return wave_sums<N / 2, OFF / 2>(half, lane);
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ bool rows_aligned(const T* a, const T* b, int count, int64_t row_stride_b) {
   return sizeof(T) == 2 && count % 8 == 0 && row_stride_b % 8 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
@@ -153,45 +174,87 @@ __global__ __launch_bounds__(256) void moe_up_kernel(T* __restrict__ act, const 
   }
 }
 
-// Of at most 64 pairs, lane p the expert of pair p (negative: none): the pairs of the `which`-th different expert, in the
-// order of their first pairs; none where there are not so many.
+// The next (up to) four of a set of pairs; the set loses them.
+__device__ __forceinline__ uint64_t take_four(uint64_t& users) {
+  const uint64_t all = users;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) users &= users - 1;
+  return all & ~users;
+}
+
+// Of at most 64 pairs, lane p the expert of pair p (negative: none): the `which`-th group of up to four pairs of one expert;
+// none where there are not so many.
 __device__ __forceinline__ uint64_t users_of(int e, int which) {
-  uint64_t left = __ballot(e >= 0), users = 0;
-  for (int i = 0; left != 0; ++i) {
+  for (uint64_t left = __ballot(e >= 0); left != 0;) {
     const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
-    users = __ballot(e == mine);
-    if (i == which) return users;
+    uint64_t users = __ballot(e == mine);
     left &= ~users;
+    const int groups = (__popcll(users) + 3) / 4;
+    if (which < groups) {
+      for (; which > 0; --which) take_four(users);
+      return take_four(users);
+    }
+    which -= groups;
   }
   return 0;
 }
 
-// moe_up for gated experts in bfloat16 and at most 64 pairs, expert by expert: grid (blocks of 16 rows, pairs or experts,
-// whichever are fewer), a column of workgroups a different expert of the step, so that an expert's rows come through every
-// XCD (with the experts as the faster index all of an expert's blocks went to one: 94 us for 64).  Every wave finds the
-// pairs that use its expert and takes up to four of them at a time over its four rows of both matrices, so that an
-// expert's rows come once however many tokens chose it.  us pair by pair / expert by expert: 16 experts of 2,048, width 4,096,
-// one token on two 35.5 / 16.0, 8 tokens on two each 84 / 62, 64 on one 323 / 130; 256 experts of 2,048, width 2,048, one token on
-// two 19.9 / 10.1 (28 with a column of workgroups an expert of the model, most of which left at once), 16 tokens on one each
-// 43.5 / 47, 64 on one each 179 / 158; 256 experts of 512 and the same 48.5 / 46.
+// A group of one to four pairs as the bytes of a word, in go<P> of one, two or four (of three the third is there twice).  (As an
+// array, of which a lane picks, they would lie in LDS, whose place comes from the launch's packet in host memory: 14 us.)
+template <typename GO>
+__device__ __forceinline__ void with_pairs(uint64_t users, const GO& go) {
+  const int many = __popcll(users);
+  const auto next = [&]() {
+    const uint32_t p = __builtin_ctzll(users);
+    users &= users - 1;
+    return p;
+  };
+  if (many >= 3) {
+    const uint32_t a = next(), b = next(), c = next(), d = many == 4 ? next() : c;
+    go(std::integral_constant<int, 4>{}, a | b << 8 | c << 16 | d << 24);
+  } else if (many == 2) {
+    const uint32_t a = next(), b = next();
+    go(std::integral_constant<int, 2>{}, a | b << 8);
+  } else if (many == 1) {
+    go(std::integral_constant<int, 1>{}, next());
+  }
+}
+
+__device__ __forceinline__ int pair_of(uint32_t pairs, int q) { return (pairs >> (8 * q)) & 0xff; }
+
+// The most groups of up to four pairs of one expert that so many pairs make.
+int most_groups(int pairs, int experts) {
+  const int different = pairs < experts ? pairs : experts;
+  return different + (pairs - different) / 4;
+}
+
+// moe_up for gated experts in bfloat16 and at most 64 pairs, expert by expert: grid (blocks of 16 rows, groups), a column of
+// workgroups up to four pairs of one expert, so that an expert's rows come through every XCD (with the experts as the faster
+// index all of an expert's blocks went to one: 94 us for 64) and once for four pairs; many pairs of one expert are many
+// columns, side by side.  What bounds small experts is the chain of loads, sums over the wave and the code's own way from L2.
+// us pair by pair / an expert's pairs four after four in one column, six moves a sum / as now: 16 experts of 2,048, width
+// 4,096, one token on two 35 / 17.6 / 14.1, 8 tokens on two each 78 / 64 / 60, 64 on two in all 233 / 132 / 62; 128 experts of
+// 768, width 2,048, 64 tokens on two in all 49 / 94 / 12.9; 16 of 256, width 512, 16 on two 8.8 / 15.8 / 4.5.
 template <int P>
 __device__ __forceinline__ void up_for_pairs(bf16_t* act, const bf16_t* h, int64_t ldh, const bf16_t* const (&rows)[2 * kRowsPerWave],
-                                             const int (&pairs)[P], int top, int f0, int F, int width, int lane, int gate_act,
+                                             uint32_t pairs, int top, int f0, int F, int width, int lane, int gate_act,
                                              GateNumbers numbers) {
   const bf16_t* b[P];
-  float s[P][2 * kRowsPerWave];
+  float s[P][2 * kRowsPerWave], gate[kRowsPerWave * P], up[kRowsPerWave * P];
 #pragma unroll
-  for (int q = 0; q < P; ++q) b[q] = h + (int64_t)(pairs[q] / top) * ldh;
+  for (int q = 0; q < P; ++q) b[q] = h + (int64_t)(pair_of(pairs, q) / top) * ldh;
   many_dots<2 * kRowsPerWave, P>(rows, b, width, lane, s);
 #pragma unroll
-  for (int q = 0; q < P; ++q)
-#pragma unroll
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const float sg = wave_sum(s[q][r]), su = wave_sum(s[q][kRowsPerWave + r]);
-      if (lane == r && f0 + r < F)
-        act[(int64_t)pairs[q] * F + f0 + r] =
-            float_to_bf16(gate_act == GATE_CLIPPED ? clipped_gate_exact(sg, su, numbers) : sg / (1.0f + expf(-sg)) * su);
-    }
+  for (int i = 0; i < kRowsPerWave * P; ++i) {
+    gate[i] = s[i / kRowsPerWave][i % kRowsPerWave];
+    up[i] = s[i / kRowsPerWave][kRowsPerWave + i % kRowsPerWave];
+  }
+  constexpr int LANES = 64 / (kRowsPerWave * P);       // that end with the same sum
+  const float sg = wave_sums(gate, lane), su = wave_sums(up, lane);
+  const int at = lane / LANES, r = at % kRowsPerWave;
+  if (lane % LANES == 0 && f0 + r < F)
+    act[(int64_t)pair_of(pairs, at / kRowsPerWave) * F + f0 + r] =
+        float_to_bf16(gate_act == GATE_CLIPPED ? clipped_gate_exact(sg, su, numbers) : sg / (1.0f + expf(-sg)) * su);
 }
 
 __global__ __launch_bounds__(256) void moe_up_by_expert_kernel(bf16_t* __restrict__ act, const bf16_t* __restrict__ h, int64_t ldh,
@@ -199,11 +262,11 @@ __global__ __launch_bounds__(256) void moe_up_by_expert_kernel(bf16_t* __restric
                                                                const int* __restrict__ chosen, const int* __restrict__ table,
                                                                const int* __restrict__ token_ids, int n_pairs, int top, int experts, int F,
                                                                int width, int gate_act, GateNumbers numbers) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, f0 = (blockIdx.x * 4 + wave) * kRowsPerWave;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), f0 = (blockIdx.x * 4 + wave) * kRowsPerWave;
   int own = -1;
   if (lane < n_pairs) own = expert_of(chosen, table, token_ids, lane / top, lane % top, top);
   if (own >= experts) own = -1;
-  uint64_t users = users_of(own, blockIdx.y);
+  const uint64_t users = users_of(own, blockIdx.y);
   if (users == 0 || f0 >= F) return;
   const int e = __builtin_amdgcn_readlane(own, __builtin_ctzll(users));
   const bf16_t* rows[2 * kRowsPerWave];
@@ -213,26 +276,9 @@ __global__ __launch_bounds__(256) void moe_up_by_expert_kernel(bf16_t* __restric
     rows[r] = w_gate + row * width;
     rows[kRowsPerWave + r] = w_up + row * width;
   }
-  const auto next = [&]() {
-    const int p = __builtin_ctzll(users);
-    users &= users - 1;
-    return p;
-  };
-  while (users != 0) {
-    const int left = __popcll(users);
-    if (left >= 3) {                       // (three: the third twice)
-      const int a = next(), b = next(), c = next(), d = left >= 4 ? next() : c;
-      const int pairs[4] = {a, b, c, d};
-      up_for_pairs<4>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
-    } else if (left == 2) {
-      const int a = next(), b = next();
-      const int pairs[2] = {a, b};
-      up_for_pairs<2>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
-    } else {
-      const int pairs[1] = {next()};
-      up_for_pairs<1>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
-    }
-  }
+  with_pairs(users, [&](auto many, uint32_t pairs) {
+    up_for_pairs<decltype(many)::value>(act, h, ldh, rows, pairs, top, f0, F, width, lane, gate_act, numbers);
+  });
 }
 
 template <typename T>
@@ -247,7 +293,7 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
   if constexpr (sizeof(T) == 2) {
     if (wide) {                             // a wave's four rows side by side
       if (c0 >= width) return;
-      float total[kRowsPerWave] = {};
+      float total = 0.f;
       for (int j = 0; j < top; ++j) {
         const int e = expert_of(chosen, table, token_ids, t, j, top);
         if (e < 0 || e >= experts) continue;
@@ -258,15 +304,13 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
         const bf16_t* const one[1] = {act + ((int64_t)t * top + j) * F};
         many_dots<kRowsPerWave, 1>(rows, one, F, lane, s);
         const float w = pair_weights != nullptr ? pair_weights[(int64_t)t * top + j] : weight;
-#pragma unroll
-        for (int r = 0; r < kRowsPerWave; ++r) total[r] = fmaf(wave_sum(s[0][r]), w, total[r]);
+        total = fmaf(wave_sums(s[0], lane), w, total);
       }
-#pragma unroll
-      for (int r = 0; r < kRowsPerWave; ++r)
-        if (lane == r && c0 + r < width) {
-          float* o = x + (int64_t)t * ldx + c0 + r;
-          *o = accumulate ? *o + total[r] : total[r];
-        }
+      const int r = lane / (64 / kRowsPerWave);
+      if (lane % (64 / kRowsPerWave) == 0 && c0 + r < width) {
+        float* o = x + (int64_t)t * ldx + c0 + r;
+        *o = accumulate ? *o + total : total;
+      }
       return;
     }
   }
@@ -291,28 +335,24 @@ __global__ __launch_bounds__(256) void moe_down_kernel(float* __restrict__ x, in
   }
 }
 
-// moe_down in bfloat16 for at most 64 pairs, expert by expert: a workgroup has four rows of the result, its waves take the
-// step's different experts in turn, up to four of an expert's pairs at a time on the same bytes; the pairs' sums meet in
-// LDS, where a token's are added up in the order of its experts, as above.  What bounds it is loads in flight: rows of a
-// narrow result are few workgroups, which then have more waves.  us token by token row by row / four waves / as now: 16 experts of
-// 2,048, width 4,096, 8 tokens on two each 44 / 32 / 32; 128 experts of 768, width 2,048, 16 tokens on one each 14.5 / 19.8 /
-// 14.7, one token on eight 46 / 11.7 / 9.7; 256 experts of 64, width 1,024, 64 tokens on one each 16.6 / 34.5 / 16.1; 16 waves at
-// width 4,096 47 for the first.
+// moe_down in bfloat16 for at most 64 pairs, expert by expert: a workgroup has four rows of the result, its waves take groups
+// of up to four pairs of one expert in turn, on the same bytes; the pairs' sums meet in LDS, where a token's are added up in the
+// order of its experts, as above.  What bounds it is loads in flight: rows of a narrow result are few workgroups, which then
+// have more waves (16 waves at width 4,096 took half as long again).
 template <int P>
 __device__ __forceinline__ void down_for_pairs(float (*sums)[kRowsPerWave], const bf16_t* act, const bf16_t* const (&rows)[kRowsPerWave],
-                                               const int (&pairs)[P], int F, int lane) {
+                                               uint32_t pairs, int F, int lane) {
   const bf16_t* b[P];
-  float s[P][kRowsPerWave];
+  float s[P][kRowsPerWave], all[kRowsPerWave * P];
 #pragma unroll
-  for (int q = 0; q < P; ++q) b[q] = act + (int64_t)pairs[q] * F;
+  for (int q = 0; q < P; ++q) b[q] = act + (int64_t)pair_of(pairs, q) * F;
   many_dots<kRowsPerWave, P>(rows, b, F, lane, s);
 #pragma unroll
-  for (int q = 0; q < P; ++q)
-#pragma unroll
-    for (int r = 0; r < kRowsPerWave; ++r) {
-      const float sum = wave_sum(s[q][r]);
-      if (lane == r) sums[pairs[q]][r] = sum;
-    }
+  for (int i = 0; i < kRowsPerWave * P; ++i) all[i] = s[i / kRowsPerWave][i % kRowsPerWave];
+  constexpr int LANES = 64 / (kRowsPerWave * P);       // that end with the same sum
+  const float sum = wave_sums(all, lane);
+  const int at = lane / LANES;
+  if (lane % LANES == 0) sums[pair_of(pairs, at / kRowsPerWave)][at % kRowsPerWave] = sum;
 }
 
 template <int WAVES>
@@ -322,38 +362,23 @@ __global__ __launch_bounds__(64 * WAVES) void moe_down_by_expert_kernel(float* _
                                                                  const float* __restrict__ pair_weights, float weight, int n_pairs, int top,
                                                                  int experts, int F, int width, int accumulate) {
   __shared__ float sums[64][kRowsPerWave];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c0 = blockIdx.x * kRowsPerWave;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c0 = blockIdx.x * kRowsPerWave;
   int e = -1;
   if (lane < n_pairs) e = expert_of(chosen, table, token_ids, lane / top, lane % top, top);
   if (e >= experts) e = -1;
   int turn = 0;
-  for (uint64_t left = __ballot(e >= 0); left != 0; ++turn) {
-    const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(left));
-    uint64_t users = __ballot(e == mine);
+  for (uint64_t left = __ballot(e >= 0); left != 0;) {
+    uint64_t users = __ballot(e == __builtin_amdgcn_readlane(e, __builtin_ctzll(left)));
     left &= ~users;
-    if ((turn & (WAVES - 1)) != wave) continue;
-    const bf16_t* rows[kRowsPerWave];
-#pragma unroll
-    for (int r = 0; r < kRowsPerWave; ++r) rows[r] = w_down + ((int64_t)mine * width + min(c0 + r, width - 1)) * F;
-    const auto next = [&]() {
-      const int p = __builtin_ctzll(users);
-      users &= users - 1;
-      return p;
-    };
     while (users != 0) {
-      const int many = __popcll(users);
-      if (many >= 3) {                     // (three: the third twice)
-        const int a = next(), b = next(), c = next(), d = many >= 4 ? next() : c;
-        const int pairs[4] = {a, b, c, d};
-        down_for_pairs<4>(sums, act, rows, pairs, F, lane);
-      } else if (many == 2) {
-        const int a = next(), b = next();
-        const int pairs[2] = {a, b};
-        down_for_pairs<2>(sums, act, rows, pairs, F, lane);
-      } else {
-        const int pairs[1] = {next()};
-        down_for_pairs<1>(sums, act, rows, pairs, F, lane);
-      }
+      const uint64_t some = take_four(users);
+      if ((turn++ & (WAVES - 1)) != wave) continue;
+      // (read from the group, or the rows' addresses are made in front of the turns of other waves as well)
+      const int mine = __builtin_amdgcn_readlane(e, __builtin_ctzll(some));
+      const bf16_t* rows[kRowsPerWave];
+#pragma unroll
+      for (int r = 0; r < kRowsPerWave; ++r) rows[r] = w_down + ((int64_t)mine * width + min(c0 + r, width - 1)) * F;
+      with_pairs(some, [&](auto many, uint32_t pairs) { down_for_pairs<decltype(many)::value>(sums, act, rows, pairs, F, lane); });
     }
   }
   __syncthreads();
@@ -1071,10 +1096,11 @@ HFEE_API int hfee_moe_up(void* act, const void* h, int64_t ldh, const void* w_ga
     moe_up_kernel<float><<<grid, 256, 0, stream>>>((float*)act, (const float*)h, ldh, (const float*)w_gate, (const float*)w_up,
                                                    chosen, table, token_ids, top, experts, ff, width, in_weights,
                                                     gate_act, numbers);
-  // (expert by expert where the pairs fit a wave's lanes)
+  // (expert by expert where the pairs fit a wave's lanes, but for many pairs of next to no work: 8 experts of 64, width 64, 32
+  // pairs 5.8 us pair by pair, 6.8 by expert; 8 pairs 6.4 / 4.9)
   else if (dtype == 1 && w_gate != nullptr && (int64_t)n * top <= 64 && width % 8 == 0 && ldh % 8 == 0 &&
-           (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_up) & 15) == 0)
-    moe_up_by_expert_kernel<<<dim3(grid.y, n * top < experts ? n * top : experts), 256, 0, stream>>>(
+           (n * top <= 16 || (int64_t)n * top * ff * width > 1 << 18) && (((uintptr_t)h | (uintptr_t)w_gate | (uintptr_t)w_up) & 15) == 0)
+    moe_up_by_expert_kernel<<<dim3(grid.y, most_groups(n * top, experts)), 256, 0, stream>>>(
         (bf16_t*)act, (const bf16_t*)h, ldh, (const bf16_t*)w_gate, (const bf16_t*)w_up, chosen, table, token_ids, n * top, top, experts,
         ff, width, gate_act, numbers);
   else if (dtype == 1)
@@ -1096,26 +1122,31 @@ HFEE_API int hfee_moe_down(float* x, int64_t ldx, const void* act, const void* w
   const int per_block = 4 * kRowsPerWave;
   HFEE_REQUIRE((width + per_block - 1) / per_block <= 65535, "moe_down: rows too wide");
   dim3 grid(n, (width + per_block - 1) / per_block);
-  if (dtype == 0)
-    moe_down_kernel<float><<<grid, 256, 0, stream>>>(x, ldx, (const float*)act, (const float*)w_down, chosen, table,
-                                                     token_ids, pair_weights, weight, top, experts, ff, width, accumulate);
-  // Expert by expert as in moe_up, but for tokens of one expert each that hardly share any: they have nothing to read
-  // together, and all waves work.  us token by token / expert by expert: one token, 16 experts of 2,048, width 4,096,
-  // 6.8 / 8.0; 2 tokens 9.0 / 9.6, 4 of them 13.8 / 14.4, 8 of them 26 / 22; 8 tokens, 64 experts of 1,408, width 2,048,
-  // 10.6 / 12.1, 16 of them 19.4 / 17.8; 2 tokens, 8 experts of 4,096, width 4,096, 15.8 / 14.5.
-  else if (dtype == 1 && (int64_t)n * top <= 64 && !(top == 1 && (n == 1 || experts >= 8 * n)) && ff % 8 == 0 &&
-           (((uintptr_t)act | (uintptr_t)w_down) & 15) == 0) {
-    const int different = n * top < experts ? n * top : experts, blocks = (width + kRowsPerWave - 1) / kRowsPerWave;
+  // Token by token reads an expert's rows for every pair and walks a token's experts one after the other; expert by expert
+  // has every wave look through all groups.  The latter for many bytes of pairs, unless they may lie on many experts, for
+  // several experts a token with few groups, and where the former makes thousands of workgroups.  us token by token / expert
+  // by expert: 16 experts of 2,048, width 4,096, 4 tokens on one each 12.6 / 10.8, 8 on two each 41 / 31; 128 of 768, width 2,048,
+  // one on eight 18.2 / 9.6; 32 of 320, width 1,536, 16 on two each 9.1 / 16.8; 256 of 64, width 1,024, 64 on one each 10.6 / 19.0;
+  // 8 of 64, width 4,096, 32 on one each 19.6 / 10.5.
+  const int64_t pairs = (int64_t)n * top;
+  const int groups = pairs <= 64 ? most_groups((int)pairs, experts) : 0, blocks = (width + kRowsPerWave - 1) / kRowsPerWave;
+  const int64_t work = pairs * ff * width;
+  const bool by_expert = dtype == 1 && pairs <= 64 && ff % 8 == 0 && (((uintptr_t)act | (uintptr_t)w_down) & 15) == 0 &&
+                         ((work >= (int64_t)1 << 24 && groups <= 32) || work >= (int64_t)1 << 26 ||
+                          (groups <= 16 && (top >= 3 || (int64_t)top * ff >= 8192)) || (groups <= 24 && (int64_t)n * blocks >= 8192));
+  if (by_expert) {
     const auto go = [&](auto kernel, int waves) {
       kernel<<<blocks, 64 * waves, 0, stream>>>(x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table, token_ids, pair_weights,
                                                 weight, n * top, top, experts, ff, width, accumulate);
     };
-    // (as many waves as there can be different experts, and as make sixteen a CU)
-    const int waves = different < 4096 / blocks ? different : 4096 / blocks;
+    // (as many waves as there can be groups, and as make sixteen a CU)
+    const int waves = groups < 4096 / blocks ? groups : 4096 / blocks;
     if (waves <= 4) go(moe_down_by_expert_kernel<4>, 4);
     else if (waves <= 8) go(moe_down_by_expert_kernel<8>, 8);
     else go(moe_down_by_expert_kernel<16>, 16);
-  }
+  } else if (dtype == 0)
+    moe_down_kernel<float><<<grid, 256, 0, stream>>>(x, ldx, (const float*)act, (const float*)w_down, chosen, table,
+                                                     token_ids, pair_weights, weight, top, experts, ff, width, accumulate);
   else if (dtype == 1)
     moe_down_kernel<bf16_t><<<grid, 256, 0, stream>>>(x, ldx, (const bf16_t*)act, (const bf16_t*)w_down, chosen, table,
                                                       token_ids, pair_weights, weight, top, experts, ff, width, accumulate);

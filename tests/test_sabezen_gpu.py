@@ -384,7 +384,8 @@ def test_few_tokens_expert_by_expert(users, width, ff, numbers):
         assert ((act[t].double() - want).abs() <= 2.0 ** -8 * want.abs() + width * 2.0 ** -23 * size).all(), t
 
 
-@pytest.mark.parametrize("n,top,E,width,ff", [(1, 2, 5, 64, 40), (8, 2, 3, 70, 520), (16, 4, 9, 33, 16), (64, 1, 2, 6, 1032), (21, 3, 4, 4, 8)])
+@pytest.mark.parametrize("n,top,E,width,ff", [(1, 2, 5, 64, 40), (8, 2, 3, 70, 520), (16, 4, 9, 33, 16), (64, 1, 2, 6, 1032), (21, 3, 4, 4, 8),
+                                              (1, 3, 9, 33, 16), (2, 4, 6, 70, 40), (5, 3, 20, 66, 64), (21, 3, 3, 1023, 264)])
 @pytest.mark.parametrize("accumulate", [True, False])
 def test_few_tokens_second_product(n, top, E, width, ff, accumulate):
     """The second product of up to 64 pairs, expert by expert: tokens that share experts and ones that name one beyond the
@@ -415,10 +416,13 @@ def test_few_tokens_second_product(n, top, E, width, ff, accumulate):
 
 
 @pytest.mark.parametrize("n,top,E,width,ff", [(5, 1, 48, 96, 64), (6, 1, 47, 96, 64), (2, 1, 16, 4100, 16), (7, 1, 7, 2500, 24),
-                                              (8, 8, 300, 1100, 40), (3, 2, 300, 4096, 8), (64, 1, 300, 64, 64)])
+                                              (8, 8, 300, 1100, 40), (3, 2, 300, 4096, 8), (64, 1, 300, 64, 64),
+                                              (2, 4, 6, 72, 40), (5, 3, 20, 64, 64), (40, 1, 2, 4096, 512), (64, 1, 64, 2048, 520),
+                                              (21, 3, 3, 1024, 264), (12, 1, 4, 8192, 16), (2, 2, 16, 64, 4096), (17, 1, 2, 64, 64)])
 def test_few_tokens_have_the_same_bits_alone(n, top, E, width, ff):
-    """Four, eight and sixteen waves a workgroup, tokens of one expert each on both sides of the line from which they go token
-    by token, more experts than pairs, among them numbers that stand for none: what a token alone gives, bit for bit."""
+    """Every reason for which a second product goes expert by expert, with four, eight and sixteen waves a workgroup, and sizes
+    for which it goes token by token; groups of one to four pairs of an expert and several groups of one; more experts than
+    pairs, among them numbers that stand for none; many pairs of next to no work: what a token alone gives, bit for bit."""
     from hfee_amd.kernels import ops
     g = torch.Generator().manual_seed(n * E)
     rand = lambda *shape: (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(torch.bfloat16).cuda()      # noqa: E731

@@ -26,13 +26,14 @@
 //
 // Token by token (moe_up, moe_down): a wave a dot product, lanes over the summed dimension, added up in a
 // fixed order; every token reads the rows of its own experts.  For steps of few tokens, whose time is
-// the experts' bytes, and for float32.
+// the experts' bytes, and for float32.  In bfloat16 up to 64 (token, expert) pairs also go expert by expert
+// (moe_up_by_expert, moe_down_by_expert), an expert's rows once for up to four of its pairs, with the same sums.
 //
 // Grouped (moe_group, moe_group_tiled, moe_combine; bfloat16): the (token, expert) pairs of a step are put
 // in the order of their experts on the device, cut into tiles of up to 128 pairs of one expert, and a workgroup
 // multiplies a tile by 256 rows of that expert's matrix on the matrix cores, both operands straight into LDS
-// (moe_direct; sizes that are no multiples of 64: tiles of 64 pairs by way of registers): an expert's matrices are
-// read once for its pairs and not once a pair.  A pair's numbers do not depend on which pairs share its tile.
+// (moe_direct; sizes that are no multiples of 64 and many pairs of a width of 64: tiles of 64 pairs by way of registers):
+// an expert's matrices are read once for its pairs and not once a pair.  A pair's numbers do not depend on which pairs share its tile.
 #include "common.h"
 
 #include <type_traits>

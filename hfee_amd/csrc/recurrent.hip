@@ -131,33 +131,53 @@ __global__ __launch_bounds__(256) void scan_gate_kernel(float* __restrict__ out,
 // up in a fixed tree.  The keys, queries, decays, values and writing strengths of the next TB tokens are
 // asked for by the whole workgroup while it works on the current TB, and wait in LDS: the walk over the
 // tokens, which nothing can shorten, reads only LDS and registers.
+//
+// What bounds it: one wave a SIMD and a chain of sums a token, so what counts is how many instructions a token
+// takes and how long LDS takes to hand its numbers out (four waves read 24 numbers a lane and token: 192 cycles
+// at best).  So the LDS holds a lane's rows in pieces of four with the sixteen lanes' pieces side by side (a read
+// of 16 bytes a lane is 256 bytes in a row; with a lane's eight rows in a row every second bank stood idle); a block's
+// tokens are one straight piece of code, in which the sum that a token's value waits for runs beside the sum of the
+// token before; a block's results leave in one store a wave instead of one a token, and its numbers come in loads of
+// sixteen bytes where the rows allow.  One request, 16 heads of 128 x 256, 2,048 tokens: rule 1 704 -> 309 us, rule 0 633 ->
+// 248; eight requests of 100 tokens 152 -> 92 and 137 -> 77 (81 ns a token and workgroup, what the LDS reads take alone).
 constexpr int kScanParts = 16, kScanColumns = 4, kScanWaves = 4;
+
+typedef float scan_f32x4 __attribute__((ext_vector_type(4)));
+
+// the operand of s_waitcnt for "no load or store outstanding" (gfx9: vmcnt in bits 3:0 and 15:14, the others at their most)
+constexpr int SCAN_NOTHING_OUTSTANDING = (7 << 4) | (15 << 8);
 
 template <int DPT>
 struct ScanShape {
   static constexpr int DP = kScanParts * DPT;                       // rows of S, filled up
   static constexpr int TB = DPT <= 8 ? 16 : DPT == 16 ? 8 : 4;      // tokens a block
   static constexpr int WIDE = 3 * TB * DP;                          // k, q, a of a block
-  static constexpr int BUFFER = WIDE + TB * kScanWaves * kScanColumns + TB;
+  static constexpr int COLUMNS = kScanWaves * kScanColumns;
+  static constexpr int BUFFER = WIDE + TB * COLUMNS + TB;           // ... its values [column][token] and strengths
   static constexpr int PER_THREAD = WIDE / (kScanWaves * 64);
+  // where row d of a token's k (or q, or a) lies in LDS
+  __device__ static __forceinline__ int place(int d) {
+    if constexpr (DPT % 4 == 0) return (d % DPT / 4) * (4 * kScanParts) + d / DPT * 4 + d % 4;
+    else return d;
+  }
 };
 
-// What a lane needs of one token, read from a block in LDS (sixteen bytes a read where a lane has four
-// rows or more).
+// What a lane needs of one token's k, q and a, read from a block in LDS (sixteen bytes a read where a lane has
+// four rows or more).
 template <int DPT>
 struct ScanToken {
-  float k[DPT], q[DPT], a[DPT], v, b;
-  __device__ __forceinline__ void read(const float* buffer, int t, int d0, int column) {
+  float k[DPT], q[DPT], a[DPT];
+  __device__ __forceinline__ void read(const float* buffer, int t, int part) {
     typedef ScanShape<DPT> Sh;
-    typedef float f32x4_t __attribute__((ext_vector_type(4)));
-    const float* kt = buffer + t * Sh::DP + d0;
+    const float* kt = buffer + t * Sh::DP + part * (DPT % 4 == 0 ? 4 : DPT);
     const float* qt = kt + Sh::TB * Sh::DP;
     const float* at = qt + Sh::TB * Sh::DP;
     if constexpr (DPT % 4 == 0) {
 #pragma unroll
       for (int i = 0; i < DPT; i += 4) {
-        const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(kt + i), qv = *reinterpret_cast<const f32x4_t*>(qt + i),
-                      av = *reinterpret_cast<const f32x4_t*>(at + i);
+        const int at4 = i * kScanParts;
+        const scan_f32x4 kv = *reinterpret_cast<const scan_f32x4*>(kt + at4), qv = *reinterpret_cast<const scan_f32x4*>(qt + at4),
+                         av = *reinterpret_cast<const scan_f32x4*>(at + at4);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           k[i + j] = kv[j];
@@ -173,8 +193,6 @@ struct ScanToken {
         a[i] = at[i];
       }
     }
-    v = buffer[Sh::WIDE + t * kScanWaves * kScanColumns + column];
-    b = buffer[Sh::WIDE + Sh::TB * kScanWaves * kScanColumns + t];
   }
 };
 
@@ -194,7 +212,118 @@ __device__ __forceinline__ float column_sum(float x) {
   return x;
 }
 
+// Two such sums side by side: an instruction that reads another lane's number has to wait for it to be written,
+// and the other sum's instruction fills that time.
+__device__ __forceinline__ void column_sums(float& x, float& y) {
+  x += dpp_move<0xB1>(x);
+  y += dpp_move<0xB1>(y);
+  x += dpp_move<0x4E>(x);
+  y += dpp_move<0x4E>(y);
+  x += dpp_move<0x141>(x);
+  y += dpp_move<0x141>(y);
+  x += dpp_move<0x140>(x);
+  y += dpp_move<0x140>(y);
+}
+
+// A wave's place in the step and in S.
+template <int DPT>
+struct ScanPlace {
+  int seg, h, g, part, c, col, d0;
+  bool live, mine;
+  float* S;
+  __device__ __forceinline__ ScanPlace(float* state, const int* segment_slots, int heads, int qk_heads, int V) {
+    seg = blockIdx.z;
+    h = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    part = lane & (kScanParts - 1);
+    c = lane >> 4;
+    const int block = blockIdx.x * kScanWaves + wave;                 // of four columns
+    col = block * kScanColumns + c;
+    live = col < V;
+    g = h / (heads / qk_heads);
+    d0 = part * DPT;
+    const int blocks = (V + kScanColumns - 1) / kScanColumns;
+    // (a wave whose four columns all lie beyond V works on the last block's numbers and stores nothing)
+    mine = block < blocks;
+    S = state + (((int64_t)segment_slots[seg] * heads + h) * blocks + (mine ? block : blocks - 1)) * (DPT * 64) + lane;
+  }
+};
+
+// A single token, straight from memory.
 template <int DPT, int RULE>
+__device__ __forceinline__ void scan_single(const ScanPlace<DPT>& w, int64_t row, float* __restrict__ out, int64_t ldo,
+                                            const float* __restrict__ q, int64_t ldq, const float* __restrict__ k, int64_t ldk,
+                                            const float* __restrict__ v, int64_t ldv, const float* __restrict__ decay, int64_t ldd,
+                                            const float* __restrict__ beta, int64_t ldb, int D, int V, int decay_per_head) {
+  float s[DPT];
+#pragma unroll
+  for (int i = 0; i < DPT; ++i) s[i] = w.S[i * 64];
+  float u = w.live ? v[row * ldv + (int64_t)w.h * V + w.col] : 0.f;
+  float kk[DPT], qq[DPT], aa[DPT];
+  const float* kp = k + row * ldk + (int64_t)w.g * D + w.d0;
+  const float* qp = q + row * ldq + (int64_t)w.g * D + w.d0;
+  const float* ap = decay + row * ldd + (decay_per_head ? (int64_t)w.h : (int64_t)w.h * D + w.d0);
+  const int astep = decay_per_head ? 0 : 1;
+  if (DPT % 4 == 0 && D == DPT * kScanParts &&
+      (((uintptr_t)kp | (uintptr_t)qp | (decay_per_head ? (uintptr_t)0 : (uintptr_t)ap)) & 15) == 0) {
+    const float one_decay = decay_per_head ? ap[0] : 0.f;          // (sixteen bytes a load where the rows allow)
+#pragma unroll
+    for (int i = 0; i + 3 < DPT; i += 4) {
+      const scan_f32x4 kv = *reinterpret_cast<const scan_f32x4*>(kp + i), qv = *reinterpret_cast<const scan_f32x4*>(qp + i);
+      scan_f32x4 av = {one_decay, one_decay, one_decay, one_decay};
+      if (!decay_per_head) av = *reinterpret_cast<const scan_f32x4*>(ap + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        kk[i + j] = kv[j];
+        qq[i + j] = qv[j];
+        aa[i + j] = av[j];
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) {
+      const bool in = w.d0 + i < D;
+      kk[i] = in ? kp[i] : 0.f;
+      qq[i] = in ? qp[i] : 0.f;
+      aa[i] = in ? ap[i * astep] : 0.f;
+    }
+  }
+  if constexpr (RULE == 1) {
+    float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) {
+      s[i] *= aa[i];
+      if (i & 1) p1 = fmaf(s[i], kk[i], p1); else p0 = fmaf(s[i], kk[i], p0);
+    }
+    u = beta[row * ldb + w.h] * (u - column_sum(p0 + p1));
+  }
+  if constexpr (RULE == 2) u *= beta[row * ldb + w.h];
+  float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+  for (int i = 0; i < DPT; ++i) {
+    if constexpr (RULE == 1) s[i] = fmaf(kk[i], u, s[i]);
+    else s[i] = fmaf(s[i], aa[i], kk[i] * u);
+    if (i & 1) o1 = fmaf(s[i], qq[i], o1); else o0 = fmaf(s[i], qq[i], o0);
+    if (w.mine) w.S[i * 64] = s[i];
+  }
+  const float o = column_sum(o0 + o1);
+  if (w.live && w.part == 0) out[row * ldo + (int64_t)w.h * V + w.col] = o;
+}
+
+// A step of single tokens only: no LDS, so that as many workgroups as registers allow share a CU and keep its loads
+// of S in flight (the kernel below holds 50 KB, three a CU): 64 requests of 16 heads of 128 x 256, 54.4 -> 43.9 us, 6.1 TB/s.
+template <int DPT, int RULE>
+__global__ __launch_bounds__(kScanWaves * 64) void linear_scan_singles_kernel(
+    float* __restrict__ out, int64_t ldo, float* __restrict__ state, const float* __restrict__ q, int64_t ldq,
+    const float* __restrict__ k, int64_t ldk, const float* __restrict__ v, int64_t ldv, const float* __restrict__ decay,
+    int64_t ldd, const float* __restrict__ beta, int64_t ldb, const int* __restrict__ segment_rows,
+    const int* __restrict__ segment_slots, int heads, int qk_heads, int D, int V, int decay_per_head) {
+  const ScanPlace<DPT> w(state, segment_slots, heads, qk_heads, V);
+  scan_single<DPT, RULE>(w, segment_rows[w.seg], out, ldo, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, D, V, decay_per_head);
+}
+
+// WHOLE: D fills DP, a decay a channel, and every row of k, q and decay begins on 16 bytes.
+template <int DPT, int RULE, bool WHOLE>
 __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
     float* __restrict__ out, int64_t ldo, float* __restrict__ state, const float* __restrict__ q, int64_t ldq,
     const float* __restrict__ k, int64_t ldk, const float* __restrict__ v, int64_t ldv, const float* __restrict__ decay,
@@ -202,150 +331,172 @@ __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
     const int* __restrict__ segment_lengths, const int* __restrict__ segment_slots, int heads, int qk_heads, int D, int V,
     int decay_per_head, int skip_from) {
   typedef ScanShape<DPT> Sh;
+  constexpr int TB = Sh::TB, THREADS = kScanWaves * 64;
   extern __shared__ __attribute__((aligned(16))) float lds[];
-  const int seg = blockIdx.z, h = blockIdx.y, tid = threadIdx.x;
-  if (skip_from > 0 && segment_lengths[seg] >= skip_from) return;       // (linear_chunks.hip or delta_chunks.hip has this portion)
-  const int lane = tid & 63, wave = tid >> 6;
-  const int part = lane & (kScanParts - 1), c = lane >> 4;
-  const int block = blockIdx.x * kScanWaves + wave;                 // of four columns
-  const int col = block * kScanColumns + c;
-  const bool live = col < V;
-  const int g = h / (heads / qk_heads);
-  const int blocks = (V + kScanColumns - 1) / kScanColumns;
-  const int d0 = part * DPT;
-  // (a wave whose four columns all lie beyond V works on the last block's numbers and stores nothing)
-  const bool mine = block < blocks;
-  float* S = state + (((int64_t)segment_slots[seg] * heads + h) * blocks + (mine ? block : blocks - 1)) * (DPT * 64) + lane;
+  const ScanPlace<DPT> w(state, segment_slots, heads, qk_heads, V);
+  const int tid = threadIdx.x, part = w.part, h = w.h, g = w.g;
+  if (skip_from > 0 && segment_lengths[w.seg] >= skip_from) return;       // (linear_chunks.hip or delta_chunks.hip has this portion)
+  const int row0 = segment_rows[w.seg], len = segment_lengths[w.seg];
+  if (len < 1) return;                  // (every thread of the workgroup sees the same len)
+  if (len == 1) {
+    scan_single<DPT, RULE>(w, row0, out, ldo, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, D, V, decay_per_head);
+    return;
+  }
   float s[DPT];
 #pragma unroll
-  for (int i = 0; i < DPT; ++i) s[i] = S[i * 64];
-  const int row0 = segment_rows[seg], len = segment_lengths[seg];
+  for (int i = 0; i < DPT; ++i) s[i] = w.S[i * 64];
 
-  if (len == 1) {      // a single token (every thread of the workgroup sees the same len): straight from memory
-    const int64_t row = row0;
-    float u = live ? v[row * ldv + (int64_t)h * V + col] : 0.f;
-    float kk[DPT], qq[DPT], aa[DPT];
-    const float* kp = k + row * ldk + (int64_t)g * D + d0;
-    const float* qp = q + row * ldq + (int64_t)g * D + d0;
-    const float* ap = decay + row * ldd + (decay_per_head ? (int64_t)h : (int64_t)h * D + d0);
-    const int astep = decay_per_head ? 0 : 1;
-    if (DPT % 4 == 0 && D == DPT * kScanParts &&
-        (((uintptr_t)kp | (uintptr_t)qp | (decay_per_head ? (uintptr_t)0 : (uintptr_t)ap)) & 15) == 0) {
-      typedef float f32x4_t __attribute__((ext_vector_type(4)));      // (sixteen bytes a load where the rows allow)
-      const float one_decay = decay_per_head ? ap[0] : 0.f;
+  constexpr int FOURS = Sh::PER_THREAD / 4;                          // WHOLE: loads of sixteen bytes a thread and block
+  scan_f32x4 fours[WHOLE ? FOURS : 1];
+  float wide[WHOLE ? 1 : Sh::PER_THREAD], narrow = 0.f, strength = 0.f;
+  // The block of tokens that begins at `first`, into registers.  No load stands under a condition (past the portion's end
+  // it brings the last token again, past a row's end its last number), and what must not be used is left out by `put`:
+  // under a branch the compiler waits for everything outstanding in front of it, the last block's results included.
+  auto ask = [&](int first) {
+    if constexpr (WHOLE) {
 #pragma unroll
-      for (int i = 0; i + 3 < DPT; i += 4) {
-        const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(kp + i), qv = *reinterpret_cast<const f32x4_t*>(qp + i);
-        f32x4_t av = {one_decay, one_decay, one_decay, one_decay};
-        if (!decay_per_head) av = *reinterpret_cast<const f32x4_t*>(ap + i);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          kk[i + j] = kv[j];
-          qq[i + j] = qv[j];
-          aa[i + j] = av[j];
-        }
+      for (int r = 0; r < FOURS; ++r) {
+        const int e = tid + r * THREADS;
+        const int which = e / (TB * Sh::DP / 4), rest = e - which * (TB * Sh::DP / 4);
+        const int t = rest / (Sh::DP / 4), d = 4 * (rest - t * (Sh::DP / 4));
+        const uint32_t row = row0 + min(first + t, len - 1);
+        const float* src = which == 0 ? k + (int64_t)g * D : which == 1 ? q + (int64_t)g * D : decay + (int64_t)h * D;
+        const uint32_t ld = which == 0 ? (uint32_t)ldk : which == 1 ? (uint32_t)ldq : (uint32_t)ldd;
+        fours[r] = *reinterpret_cast<const scan_f32x4*>(src + (uint64_t)row * ld + d);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < DPT; ++i) {
-        const bool in = d0 + i < D;
-        kk[i] = in ? kp[i] : 0.f;
-        qq[i] = in ? qp[i] : 0.f;
-        aa[i] = in ? ap[i * astep] : 0.f;
+      for (int r = 0; r < Sh::PER_THREAD; ++r) {
+        const int e = tid + r * THREADS;
+        const int which = e / (TB * Sh::DP), rest = e - which * (TB * Sh::DP);
+        const int t = rest / Sh::DP, d = min(rest - t * Sh::DP, D - 1);
+        const int64_t row = row0 + min(first + t, len - 1);
+        wide[r] = which == 0 ? k[row * ldk + (int64_t)g * D + d] : which == 1 ? q[row * ldq + (int64_t)g * D + d]
+                                                                              : decay[row * ldd + (decay_per_head ? (int64_t)h : (int64_t)h * D + d)];
       }
     }
-    if constexpr (RULE == 1) {
-      float p0 = 0.f, p1 = 0.f;
+    const int column = min((int)blockIdx.x * Sh::COLUMNS + tid % Sh::COLUMNS, V - 1);
+    narrow = v[(int64_t)(row0 + min(first + min(tid / Sh::COLUMNS, TB - 1), len - 1)) * ldv + (int64_t)h * V + column];
+    if constexpr (RULE != 0) strength = beta[(int64_t)(row0 + min(first + min(tid, TB - 1), len - 1)) * ldb + h];
+  };
+  auto put = [&](float* buffer) {
+    if constexpr (WHOLE) {
 #pragma unroll
-      for (int i = 0; i < DPT; ++i) {
-        s[i] *= aa[i];
-        if (i & 1) p1 = fmaf(s[i], kk[i], p1); else p0 = fmaf(s[i], kk[i], p0);
+      for (int r = 0; r < FOURS; ++r) {
+        const int e = tid + r * THREADS;
+        const int line = e / (Sh::DP / 4), d = 4 * (e - line * (Sh::DP / 4));      // (lines: k's tokens, q's, a's)
+        *reinterpret_cast<scan_f32x4*>(buffer + line * Sh::DP + Sh::place(d)) = fours[r];
       }
-      u = beta[row * ldb + h] * (u - column_sum(p0 + p1));
+    } else {
+#pragma unroll
+      for (int r = 0; r < Sh::PER_THREAD; ++r) {
+        const int e = tid + r * THREADS;
+        const int line = e / Sh::DP, d = e - line * Sh::DP;
+        buffer[line * Sh::DP + Sh::place(d)] = d < D ? wide[r] : 0.f;
+      }
     }
-    if constexpr (RULE == 2) u *= beta[row * ldb + h];
+    // (said once for all threads: a load that only some of them have waited for counts as outstanding at the loop's top,
+    // and the wait there would be for the results' stores as well)
+    __builtin_amdgcn_s_waitcnt(SCAN_NOTHING_OUTSTANDING);
+    if (tid < TB * Sh::COLUMNS)
+      buffer[Sh::WIDE + tid % Sh::COLUMNS * TB + tid / Sh::COLUMNS] = (int)blockIdx.x * Sh::COLUMNS + tid % Sh::COLUMNS < V ? narrow : 0.f;
+    if (RULE != 0 && tid < TB) buffer[Sh::WIDE + TB * Sh::COLUMNS + tid] = strength;
+  };
+  // What a token does in front of its value (rule 1): the state decays, and the key's part of it is summed up (p0 + p1
+  // is this lane's share).
+  auto decays = [&](const ScanToken<DPT>& x, float& p) {
+    float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < DPT; ++i) {
+      s[i] *= x.a[i];
+      if (i & 1) p1 = fmaf(s[i], x.k[i], p1); else p0 = fmaf(s[i], x.k[i], p0);
+    }
+    p = p0 + p1;
+  };
+  auto writes = [&](const ScanToken<DPT>& x, float u, float& o) {      // ... and behind it; o: this lane's share of the result
     float o0 = 0.f, o1 = 0.f;
 #pragma unroll
     for (int i = 0; i < DPT; ++i) {
-      if constexpr (RULE == 1) s[i] = fmaf(kk[i], u, s[i]);
-      else s[i] = fmaf(s[i], aa[i], kk[i] * u);
-      if (i & 1) o1 = fmaf(s[i], qq[i], o1); else o0 = fmaf(s[i], qq[i], o0);
-        if (mine) S[i * 64] = s[i];
+      if constexpr (RULE == 1) s[i] = fmaf(x.k[i], u, s[i]);
+      else s[i] = fmaf(s[i], x.a[i], x.k[i] * u);
+      if (i & 1) o1 = fmaf(s[i], x.q[i], o1); else o0 = fmaf(s[i], x.q[i], o0);
     }
-    const float o = column_sum(o0 + o1);
-    if (live && part == 0) out[row * ldo + (int64_t)h * V + col] = o;
-    return;
-  }
-
-  float wide[Sh::PER_THREAD], narrow = 0.f, strength = 0.f;
-  auto ask = [&](int first) {          // the block of tokens that begins at `first`, into registers
-#pragma unroll
-    for (int r = 0; r < Sh::PER_THREAD; ++r) {
-      const int e = tid + r * kScanWaves * 64;
-      const int which = e / (Sh::TB * Sh::DP), rest = e - which * (Sh::TB * Sh::DP);
-      const int t = rest / Sh::DP, d = rest - t * Sh::DP;
-      float x = 0.f;
-      if (first + t < len && d < D) {
-        const int64_t row = row0 + first + t;
-        x = which == 0 ? k[row * ldk + (int64_t)g * D + d] : which == 1 ? q[row * ldq + (int64_t)g * D + d]
-                                                                      : decay[row * ldd + (decay_per_head ? (int64_t)h : (int64_t)h * D + d)];
-      }
-      wide[r] = x;
-    }
-    {
-      const int t = tid / (kScanWaves * kScanColumns), cc = tid - t * (kScanWaves * kScanColumns);
-      const int column = blockIdx.x * kScanWaves * kScanColumns + cc;
-      narrow = t < Sh::TB && first + t < len && column < V ? v[(int64_t)(row0 + first + t) * ldv + (int64_t)h * V + column] : 0.f;
-    }
-    if (RULE != 0 && tid < Sh::TB) strength = first + tid < len ? beta[(int64_t)(row0 + first + tid) * ldb + h] : 0.f;
-  };
-  auto put = [&](float* buffer) {
-#pragma unroll
-    for (int r = 0; r < Sh::PER_THREAD; ++r) buffer[tid + r * kScanWaves * 64] = wide[r];
-    if (tid < Sh::TB * kScanWaves * kScanColumns) buffer[Sh::WIDE + tid] = narrow;
-    if (RULE != 0 && tid < Sh::TB) buffer[Sh::WIDE + Sh::TB * kScanWaves * kScanColumns + tid] = strength;
+    o = o0 + o1;
   };
 
   ask(0);
   put(lds);
   __syncthreads();
-  for (int first = 0, turn = 0; first < len; first += Sh::TB, turn ^= 1) {
+  for (int first = 0, turn = 0;; first += TB, turn ^= 1) {
     const float* buffer = lds + turn * Sh::BUFFER;
-    const bool more = first + Sh::TB < len;
-    if (more) ask(first + Sh::TB);
-    const int count = min(Sh::TB, len - first);
-    ScanToken<DPT> now, next;
-    now.read(buffer, 0, d0, wave * kScanColumns + c);
-    for (int t = 0; t < count; ++t) {
-      if (t + 1 < count) next.read(buffer, t + 1, d0, wave * kScanColumns + c);      // (ahead of the sums that wait on one another)
-      float u = now.v;
+    const float* values = buffer + Sh::WIDE + ((tid >> 6) * kScanColumns + w.c) * TB;
+    const float* strengths = buffer + Sh::WIDE + TB * Sh::COLUMNS;
+    ask(first + TB);
+    const int count = min(TB, len - first);
+    float kept = 0.f;                                 // lane `part` keeps the result of the block's token `part`
+    if (count == TB) {
+      // (two tokens ahead: the four waves' reads of one take longer than a token's sums.  The fences keep the reads where
+      // they are written; the compiler puts them in front of their use)
+      constexpr int RING = DPT <= 8 ? 3 : 2;
+      ScanToken<DPT> tokens[RING];
+#pragma unroll
+      for (int t = 0; t + 1 < RING; ++t) tokens[t].read(buffer, t, part);
+      scan_f32x4 v4 = {0.f, 0.f, 0.f, 0.f}, b4 = {0.f, 0.f, 0.f, 0.f};
+      float p = 0.f;
       if constexpr (RULE == 1) {
-        float p0 = 0.f, p1 = 0.f;
+        decays(tokens[0], p);
+        p = column_sum(p);
+      }
 #pragma unroll
-        for (int i = 0; i < DPT; ++i) {
-          s[i] *= now.a[i];
-          if (i & 1) p1 = fmaf(s[i], now.k[i], p1); else p0 = fmaf(s[i], now.k[i], p0);
+      for (int t = 0; t < TB; ++t) {
+        const ScanToken<DPT>& now = tokens[t % RING];
+        const ScanToken<DPT>& next = tokens[(t + 1) % RING];
+        if (t % 4 == 0) {
+          v4 = *reinterpret_cast<const scan_f32x4*>(values + t);
+          if (RULE != 0) b4 = *reinterpret_cast<const scan_f32x4*>(strengths + t);
         }
-        u = now.b * (now.v - column_sum(p0 + p1));
+        if (t + RING - 1 < TB) tokens[(t + RING - 1) % RING].read(buffer, t + RING - 1, part);
+        __builtin_amdgcn_sched_barrier(0);
+        const float u = RULE == 0 ? v4[t % 4] : RULE == 1 ? b4[t % 4] * (v4[t % 4] - p) : b4[t % 4] * v4[t % 4];
+        float o;
+        writes(now, u, o);
+        if (RULE == 1 && t + 1 < TB) {
+          decays(next, p);
+          column_sums(o, p);
+        } else {
+          o = column_sum(o);
+        }
+        kept = part == t ? o : kept;
       }
-      if constexpr (RULE == 2) u = now.b * now.v;
-      float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-      for (int i = 0; i < DPT; ++i) {
-        if constexpr (RULE == 1) s[i] = fmaf(now.k[i], u, s[i]);
-        else s[i] = fmaf(s[i], now.a[i], now.k[i] * u);
-        if (i & 1) o1 = fmaf(s[i], now.q[i], o1); else o0 = fmaf(s[i], now.q[i], o0);
+    } else {
+      for (int t = 0; t < count; ++t) {
+        ScanToken<DPT> now;
+        now.read(buffer, t, part);
+        float u = values[t], o;
+        if constexpr (RULE == 1) {
+          float p;
+          decays(now, p);
+          u = strengths[t] * (u - column_sum(p));
+        }
+        if constexpr (RULE == 2) u = strengths[t] * u;
+        writes(now, u, o);
+        o = column_sum(o);
+        kept = part == t ? o : kept;
       }
-      const float o = column_sum(o0 + o1);
-      if (live && part == 0) out[(int64_t)(row0 + first + t) * ldo + (int64_t)h * V + col] = o;
-      now = next;
     }
-    if (more) put(lds + (turn ^ 1) * Sh::BUFFER);
+    float* mine = out + (int64_t)(row0 + min(first + part, len - 1)) * ldo + (int64_t)h * V + w.col;
+    if (first + TB >= len) {
+      if (w.live && part < count) *mine = kept;
+      break;
+    }
+    // (the results behind the next block's numbers: a wait for loads also waits for every store in front of them)
+    put(lds + (turn ^ 1) * Sh::BUFFER);
+    if (w.live && part < TB) *mine = kept;
     __syncthreads();
   }
-  if (mine) {
+  if (w.mine) {
 #pragma unroll
-    for (int i = 0; i < DPT; ++i) S[i * 64] = s[i];
+    for (int i = 0; i < DPT; ++i) w.S[i * 64] = s[i];
   }
 }
 
@@ -736,12 +887,12 @@ HFEE_API int hfee_scan_gate(float* out, int64_t ldo, const void* z, int64_t ldz,
   return 0;
 }
 
-// skip_from > 0: portions of that many tokens and more are left alone.
+// skip_from > 0: portions of that many tokens and more are left alone.  singles != 0: every segment has one token.
 HFEE_API int hfee_linear_scan(float* out, int64_t ldo, float* state, const float* q, int64_t ldq, const float* k,
                               int64_t ldk, const float* v, int64_t ldv, const float* decay, int64_t ldd,
                               const float* beta, int64_t ldb, const int* segment_rows, const int* segment_lengths,
                               const int* segment_slots, int segments, int heads, int qk_heads, int dim, int vdim,
-                              int rule, int decay_per_head, int skip_from, hipStream_t stream) {
+                              int rule, int decay_per_head, int skip_from, int singles, hipStream_t stream) {
   HFEE_REQUIRE(segments >= 0 && segments <= 65535, "linear_scan: bad segment count");
   if (segments == 0) return 0;
   HFEE_REQUIRE(heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && heads <= 65535,
@@ -754,15 +905,34 @@ HFEE_API int hfee_linear_scan(float* out, int64_t ldo, float* state, const float
   const int columns = kScanWaves * kScanColumns;
   dim3 grid((vdim + columns - 1) / columns, heads, segments);
   const int per = (dim + kScanParts - 1) / kScanParts;
+  const int filled = per <= 1 ? 1 : per <= 2 ? 2 : per <= 4 ? 4 : per <= 8 ? 8 : per <= 16 ? 16 : 32;
+  const bool whole = filled % 4 == 0 && dim == filled * kScanParts && !decay_per_head && ldq % 4 == 0 && ldk % 4 == 0 && ldd % 4 == 0 &&
+                     ldq < INT32_MAX && ldk < INT32_MAX && ldd < INT32_MAX &&
+                     (((uintptr_t)q | (uintptr_t)k | (uintptr_t)decay) & 15) == 0;
+#define GO(DPT, RULE, WHOLE)                                                                                          \
+  linear_scan_kernel<DPT, RULE, WHOLE><<<grid, kScanWaves * 64, 2 * ScanShape<DPT>::BUFFER * sizeof(float), stream>>>(out, ldo, state, q, ldq, k, ldk, v, ldv, \
+      decay, ldd, beta, ldb, segment_rows, segment_lengths, segment_slots, heads, qk_heads, dim, vdim, decay_per_head, skip_from)
 #define LAUNCH(DPT, RULE)                                                                                             \
-  linear_scan_kernel<DPT, RULE><<<grid, kScanWaves * 64, 2 * ScanShape<DPT>::BUFFER * sizeof(float), stream>>>(out, ldo, state, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, \
-      segment_rows, segment_lengths, segment_slots, heads, qk_heads, dim, vdim, decay_per_head, skip_from)
+  do {                                                                                                                \
+    if (singles)                                                                                                      \
+      linear_scan_singles_kernel<DPT, RULE><<<grid, kScanWaves * 64, 0, stream>>>(out, ldo, state, q, ldq, k, ldk, v, ldv, decay, ldd, beta, ldb, \
+          segment_rows, segment_slots, heads, qk_heads, dim, vdim, decay_per_head);                                   \
+    else if (whole) GO(DPT, RULE, DPT % 4 == 0);                                                                      \
+    else GO(DPT, RULE, false);                                                                                        \
+  } while (0)
 #define PICK(RULE)                                                                                                    \
-  if (per <= 1) LAUNCH(1, RULE); else if (per <= 2) LAUNCH(2, RULE); else if (per <= 4) LAUNCH(4, RULE);              \
-  else if (per <= 8) LAUNCH(8, RULE); else if (per <= 16) LAUNCH(16, RULE); else LAUNCH(32, RULE)
+  switch (filled) {                                                                                                   \
+    case 1: LAUNCH(1, RULE); break;                                                                                   \
+    case 2: LAUNCH(2, RULE); break;                                                                                   \
+    case 4: LAUNCH(4, RULE); break;                                                                                   \
+    case 8: LAUNCH(8, RULE); break;                                                                                   \
+    case 16: LAUNCH(16, RULE); break;                                                                                 \
+    default: LAUNCH(32, RULE);                                                                                        \
+  }
   if (rule == 0) { PICK(0); } else if (rule == 1) { PICK(1); } else { PICK(2); }
 #undef PICK
 #undef LAUNCH
+#undef GO
   HFEE_CHECK_LAUNCH("linear_scan");
   return 0;
 }

@@ -1716,7 +1716,7 @@ def delta_inputs(y, decay, beta, x, a, b, state, taps, dt_bias, a_log, token_seg
 
 def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths, segment_slots, heads: int,
                 qk_heads: int, dim: int, vdim: int, rule: str, decay_per_head: bool = False, longest: int = 0,
-                shortest: int = 0, scratch=None):
+                shortest: int = 0, scratch=None, singles: bool = False):
     """Walks each segment's rows in order from state[slot] (float32 [slots, heads, `scan_state_shape`],
     updated in place: a head's matrix in blocks of four columns).  rule "decay_add": S <- diag(decay) S + k v^T; "delta": S <- diag(decay) S,
     S <- S + k (beta (v - S^T k))^T; "scaled_add": S <- diag(decay) S + k (beta v)^T; out = S^T q.
@@ -1725,7 +1725,8 @@ def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths,
     of a head's rows (or [heads]: the same decays for every token); beta [n, heads].
     With rule "decay_add" and the same decays for every token, `scratch` (float32, `linear_chunks_scratch` words) and
     the lengths of the step's longest and shortest portion: long portions go in chunks through the matrix cores,
-    in float32 as well; likewise with rule "delta" and one decay a head and token (`delta_chunks_scratch` words)."""
+    in float32 as well; likewise with rule "delta" and one decay a head and token (`delta_chunks_scratch` words).
+    singles: every segment has exactly one token (a kernel of its own; the lengths are then not read)."""
     _gpu(out, state, q, k, v, decay, beta, segment_rows, segment_lengths, segment_slots)
     n, wq, ldq = _f32rows(q, "linear_scan q")
     nk, wk, ldk = _f32rows(k, "linear_scan k")
@@ -1750,6 +1751,7 @@ def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths,
     _i32(segment_rows, "linear_scan segment_rows")
     _i32(segment_lengths, "linear_scan segment_lengths", segments)
     _i32(segment_slots, "linear_scan segment_slots", segments)
+    _check(not singles or segments == n, "linear_scan: singles are as many rows as segments")
     skip_from = 0
     if scratch is not None:
         _gpu(scratch)
@@ -1775,7 +1777,7 @@ def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths,
     lib.core().call("hfee_linear_scan", _ptr(out), ldo, _ptr(state), _ptr(q), ldq, _ptr(k), ldk, _ptr(v), ldv, _ptr(decay),
                     ldd, _ptr(beta if rule != "decay_add" else None), ldb, _ptr(segment_rows), _ptr(segment_lengths),
                     _ptr(segment_slots), segments, heads, qk_heads, dim, vdim, rules[rule], 1 if decay_per_head else 0, skip_from,
-                    _stream())
+                    1 if singles else 0, _stream())
 
 
 RGLRU_CHUNK = 32        # tokens a chunk of the recurrent unit's kernels for long portions

@@ -77,6 +77,11 @@ class _StateMixer(Mixer):
     def _segments(self, ctx):
         return ctx.segment_rows, ctx.segment_lengths, ctx.segment_slots
 
+    @staticmethod
+    def _singles(ctx) -> bool:
+        """Whether every request of the step brings one token (none brings no token)."""
+        return ctx.n == len(ctx.segments)
+
     def chunk_words(self, longest: int, rows: int) -> int:
         """float32 words with which `ops.linear_scan` walks the long portions of a step (the longest of `longest` tokens,
         `rows` in all) in chunks; 0 where it goes token by token."""
@@ -212,7 +217,7 @@ class GatedDelta(_StateMixer):
         q, k, v = y[:, :self.qk_width], y[:, self.qk_width:2 * self.qk_width], y[:, 2 * self.qk_width:]
         o = ctx.rows("gated_delta.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, decay, beta, rows, lengths, slots, H, G, D, V, "delta",
-                        decay_per_head=self.decay_per_head, **self._chunks(ctx))
+                        decay_per_head=self.decay_per_head, singles=self._singles(ctx), **self._chunks(ctx))
         gate = proj[:, self.g_columns]
         if self.gate_rank is not None:
             gate = ctx.rows("gated_delta.gate", self.v_width)
@@ -303,7 +308,8 @@ class GatedLinearAttention(_StateMixer):
         decay = ctx.rows("gla.decay", self.qk_width, torch.float32)
         ops.scan_gate(decay, z, "root_sigmoid", bias=self.a_bias, number=self.tau)
         o = ctx.rows("gla.read", self.v_width, torch.float32)
-        ops.linear_scan(o, self.state, q, k, v, decay, None, rows, lengths, slots, H, H, D, V, "decay_add")
+        ops.linear_scan(o, self.state, q, k, v, decay, None, rows, lengths, slots, H, H, D, V, "decay_add",
+                        singles=self._singles(ctx))
         gated = ctx.rows("gla.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:self.at_a], self.norm_weight, H, V, self.norm_eps, "silu")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=True)
@@ -380,7 +386,7 @@ class Retention(_StateMixer):
         q, k, v = qkv[:, :self.qk_width], qkv[:, self.qk_width:self.at_v], qkv[:, self.at_v:]
         o = ctx.rows("retention.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, self.decays, None, rows, lengths, slots, H, H, D, V, "decay_add",
-                        decay_per_head=True, **self._chunks(ctx))
+                        decay_per_head=True, singles=self._singles(ctx), **self._chunks(ctx))
         gated = ctx.rows("retention.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:], self.norm_weight, H, V, self.norm_eps, "silu")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)
@@ -448,7 +454,7 @@ class LightningAttention(_StateMixer):
         q, k, v = qkv[:, :self.qk_width], qkv[:, self.qk_width:self.at_v], qkv[:, self.at_v:]
         o = ctx.rows("lightning.read", staggered(self.v_width), torch.float32)[:, :self.v_width]
         ops.linear_scan(o, self.state, q, k, v, self.decays, None, rows, lengths, slots, H, H, D, V, "decay_add",
-                        decay_per_head=True, **self._chunks(ctx))
+                        decay_per_head=True, singles=self._singles(ctx), **self._chunks(ctx))
         gated = ctx.rows("lightning.out", self.v_width)
         ops.head_norm_gate(gated, o, proj[:, self.at_g:], self.norm_weight, 1, self.v_width, self.norm_eps, "sigmoid")
         product(ctx, x, gated, self.w_o, self.w_o_tiles, add=add)
@@ -523,7 +529,8 @@ class StateSpace(_StateMixer):
         ops.scan_gate(dt, dt_raw, "softplus", bias=self.dt_bias)
         ops.scan_gate(decay, dt_raw, "step_decay", bias=self.dt_bias, per_head=self.a_log, head_width=1)
         o = ctx.rows("state_space.read", inner, torch.float32)
-        ops.linear_scan(o, self.state, C, B, xs, decay, dt, rows, lengths, slots, H, G, N, V, "scaled_add", decay_per_head=True)
+        ops.linear_scan(o, self.state, C, B, xs, decay, dt, rows, lengths, slots, H, G, N, V, "scaled_add", decay_per_head=True,
+                        singles=self._singles(ctx))
         gated = ctx.rows("state_space.out", inner)
         ops.gate_group_norm(gated, o, xs, self.skip, z, self.norm_weight, H, self.norm_groups, self.norm_eps)
         product(ctx, out, gated, self.w_o, self.w_o_tiles)

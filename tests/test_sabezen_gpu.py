@@ -329,6 +329,54 @@ def test_linear_scan_in_portions(rule, H, G, D, V):
     assert bool(torch.isnan(state[1]).all()) and float(state[2].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("rule", ["delta", "decay_add", "scaled_add"])
+@pytest.mark.parametrize("D,V,pad", [(64, 20, 0), (128, 17, 4), (128, 32, 1), (256, 16, 0), (512, 8, 4)])
+def test_linear_scan_around_its_blocks(rule, D, V, pad):
+    """Key sizes that fill a lane's rows, whose numbers come in loads of sixteen bytes (rows padded by a multiple of four
+    numbers) or one by one (padded by one), portions that end in front of, on and behind a block of tokens and of
+    blocks, then steps of single tokens, against the recurrence in float64."""
+    from hfee_amd.kernels import ops
+    H, G, block = 2, (2 if rule == "decay_add" else 1), 16 if D <= 128 else 8 if D == 256 else 4
+    T = [1, block - 1, block, block + 1, 2 * block, 3 * block + 1]
+    singles, g = 2, torch.Generator().manual_seed(D + V)
+    slots = [3, 0, 5, 1, 6, 2]
+    state = torch.zeros(7, H, *ops.scan_state_shape(D, V), device="cuda")
+    want_S = torch.zeros(len(T), H, D, V, dtype=torch.float64)
+
+    def step(lengths):
+        n = sum(lengths)
+        q, k = torch.randn(n, G, D, generator=g) * D ** -0.5, torch.randn(n, G, D, generator=g) * D ** -0.5
+        v, a, b = torch.randn(n, H, V, generator=g), torch.rand(n, H, D, generator=g) * 0.3 + 0.7, torch.rand(n, H, generator=g)
+        want = torch.zeros(n, H, V, dtype=torch.float64)
+        rows = np.cumsum([0] + lengths)[:-1]
+        for s, (row, length) in enumerate(zip(rows, lengths)):
+            for h in range(H):
+                S = want_S[s, h]
+                for t in range(row, row + length):
+                    qt, kt, vt = q[t, h * G // H].double(), k[t, h * G // H].double(), v[t, h].double()
+                    S = a[t, h].double()[:, None] * S
+                    u = {"delta": lambda: b[t, h].double() * (vt - S.T @ kt), "decay_add": lambda: vt,
+                         "scaled_add": lambda: b[t, h].double() * vt}[rule]()
+                    S = S + kt[:, None] * u[None, :]
+                    want[t, h] = S.T @ qt
+                want_S[s, h] = S
+
+        def rows_of(x):          # rows that begin `pad` numbers apart from where they end
+            wide = torch.full((n, x[0].numel() + pad), float("nan"), device="cuda")
+            wide[:, :x[0].numel()] = x.reshape(n, -1).cuda()
+            return wide[:, :x[0].numel()]
+        out = torch.full((n, H * V + pad), float("nan"), device="cuda")[:, :H * V]
+        ops.linear_scan(out, state, rows_of(q), rows_of(k), rows_of(v), rows_of(a), b.cuda() if rule != "decay_add" else None,
+                        i32(rows), i32(lengths), i32(slots), H, G, D, V, rule, singles=max(lengths) == 1)
+        assert su.rel(out.cpu(), want.reshape(n, -1)) < 2e-5
+
+    for lengths in [T] + [[1] * len(T)] * singles + [T[::-1]]:
+        step(list(lengths))
+    for s, slot in enumerate(slots):
+        assert su.rel(ops.scan_state_matrix(state[slot], D, V).cpu(), want_S[s]) < 2e-5
+    assert float(state[4].abs().sum()) == 0.0
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("K", [1, 2, 4, 5])
 def test_short_convolution_carries_its_inputs(dtype, K):

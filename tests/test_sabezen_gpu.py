@@ -275,6 +275,49 @@ def test_mixed_attention_on_the_matrix_cores(chunk, H, G, D, half):
             assert su.rel(got[s, t].double().cpu(), want[s][t]) < 3e-2, f"sequence {s} token {t}"
 
 
+@pytest.mark.parametrize("H,G,D", [(8, 2, 64), (16, 4, 128), (32, 8, 128)])
+def test_mixed_attention_in_parts(H, G, D):
+    """Items of unequal lengths in parts of whole pairs of tiles, in the order and number that the plan gives them, and as a
+    step of single tokens has them, against the plain kernel (bfloat16 results of the same inputs: a few rounding steps of
+    2^-9); heads in fours a wave mix on the matrix unit.  The chunk begins inside a tile, the last pair is half a pair."""
+    from hfee_amd.kernels import ops
+    page, chunk, starts, counts = 16, 88, (0, 100, 89, 263), (70, 30, 1, 1)
+    g = torch.Generator().manual_seed(H)
+    pages = [-(-(a + n) // page) for a, n in zip(starts, counts)]
+    tables = torch.zeros(len(starts), max(pages), dtype=torch.int32)
+    order, at = torch.randperm(sum(pages), generator=g), 0
+    for s, n in enumerate(pages):
+        tables[s, :n] = order[at:at + n]
+        at += n
+    tables = tables.cuda()
+    cache = torch.randn(sum(pages), G, page * 2 * D, generator=g).bfloat16().cuda()
+    q = (torch.randn(sum(counts), H * D, generator=g) * 2).bfloat16().cuda()
+    talk = (torch.eye(H) + torch.randn(H, H, generator=g) * 0.2).cuda()
+    items, row = [], 0
+    for s, (start, n) in enumerate(zip(starts, counts)):
+        off = 0
+        while off < n:
+            p = start + off
+            room = min(16, n - off, chunk - p % chunk)
+            items.append((row + off, room, p, s))
+            off += room
+        row += n
+    i32 = lambda a: torch.as_tensor(np.asarray(a), dtype=torch.int32, device="cuda")      # noqa: E731
+    pos = np.concatenate([np.arange(a, a + n) for a, n in zip(starts, counts)])
+    want = torch.zeros_like(q)
+    kw = dict(chunk=chunk, sink="zero")
+    ops.attention_mix(want, q, cache, i32(pos), i32(np.repeat(np.arange(4), counts)), tables, H, G, D, page, D ** -0.5, mix=talk, **kw)
+    for most in (1, 2, 16):
+        splits, part, jobs = ops.attention_mix_parts(items, chunk, most)
+        for order in (i32(jobs), None):
+            partial = torch.full((max(1, ops.attention_mix_partial_words(len(items), H, D, splits)),), float("nan"), device="cuda")
+            got = torch.full_like(q, float("nan"))
+            ops.attention_mix_bf16(got, q, cache, i32(items), tables, H, G, D, page, D ** -0.5, mix_t=talk.t().contiguous(),
+                                   splits=splits, partial=partial if splits > 1 else None, part_tiles=part, jobs=order, **kw)
+            for t in range(len(pos)):
+                assert su.rel(got[t].double().cpu(), want[t].double().cpu()) < 1e-2, f"row {t} in at most {most} parts"
+
+
 @pytest.mark.parametrize("rule", ["delta", "decay_add"])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 8, 16), (3, 3, 20, 12), (2, 1, 33, 70)])
 def test_linear_scan_in_portions(rule, H, G, D, V):

@@ -358,3 +358,33 @@ def test_the_pool_is_sized_from_the_free_memory():
     with pytest.raises(CacheError, match="no page of the cache fits"):
         capacity.choose_pages(None, 100, work + reserve + page - 1, total, work, page)
     assert capacity.choose_pages(None, 100, work + reserve + page, total, work, page) == 1
+
+
+def test_a_chain_of_kept_pages_is_followed_where_it_leads_and_no_further():
+    """Prompts that leave a kept chain at each of its pages, or come back to one that another request has lengthened, take
+    over what a search by digests alone would, and leave the same digests behind."""
+    from hfee_amd.cache.manager import PageDigests
+
+    def digests(tokens, n):
+        d = PageDigests(16)
+        assert d.cover(tokens, n)
+        return list(d.up_to(n))
+
+    base = list(range(100, 100 + 16 * 6 + 5))
+    for change in range(0, 16 * 6, 7):
+        m = CacheManager([FULL], 16, 64, max_requests=4, keep_prefixes=True)
+        for name, tokens in (("a", base), ("b", base[:48] + [7] * 60), ("c", base[:change] + [9] + base[change + 1:])):
+            kept = dict(m._kept)
+            want = 0
+            while want < (len(tokens) - 1) // 16 and digests(tokens, want + 1)[want] in kept:
+                want += 1
+            rc = m.admit(name, tokens)
+            assert rc.length == 16 * want
+            m.reserve(name, len(tokens) - rc.length)
+            m.commit(name, len(tokens) - rc.length)
+            if rc.digests is not None:
+                assert rc.digests.cover(tokens, len(tokens) // 16)
+                assert rc.digests.up_to(len(tokens) // 16) == digests(tokens, len(tokens) // 16)
+            m.release(name, tokens)
+            assert set(digests(tokens, len(tokens) // 16)) <= set(m._kept)
+            m.check()

@@ -4,8 +4,10 @@
 //
 // delta_inputs: everything that enters it from a token's projections in one launch, in float32: the short convolutions
 // with their SiLU, unit vectors a head for queries and keys (x / sqrt(sum x^2 + eps), queries also times a factor),
-// decays exp(-exp(A_h) softplus(a + bias)) and writing strengths sigmoid(b); in a step of single tokens also the
-// convolutions' state.
+// decays exp(-exp(A_h) softplus(a + bias)), one a head or one a key channel, and writing strengths sigmoid(b); in a step of
+// single tokens also the convolutions' state.  (2,048 tokens of 6,144 channels with decays a channel,
+// 16 heads of 128: 36 us, where a launch a mechanism, a value a thread, took 82 for the convolution and 20 for the decays alone;
+// eight single tokens: 5 us for six launches' 29.)
 //
 // delta_chunks: portions of many tokens in chunks of 64 on the float32 matrix instructions (recurrent.hip, rule 1, walks
 // token by token).  With t and j counting from a chunk's first token, S the state that comes into the chunk, L its tokens,
@@ -42,24 +44,26 @@ __device__ __forceinline__ float softplus(float z) { return z > 20.f ? z : log1p
 struct InputArgs {
   float* y;                    // [n, channels]: queries, keys, values
   int64_t ldy;
-  float* decay;                // [n, heads]
+  float* decay;                // [n, heads * decay_width]
   float* beta;                 // [n, heads]
   const void* x;               // [n, channels] projections in T
   int64_t ldx;
-  const void* a;               // [n, heads] in T, ldx apart
-  const void* b;
+  const void* a;               // [n, heads * decay_width] in T, lda apart
+  int64_t lda;
+  const void* b;               // [n, heads], ldx apart
   void* state;                 // [slots][taps - 1][channels] in T, the newest last
   const float* taps;           // [channels][taps], the last column the current token's
-  const float* dt_bias;
-  const float* a_log;
+  const float* dt_bias;        // [heads * decay_width]
+  const float* a_log;          // [heads]
   const int* token_segment;
   const int* segment_rows;
   const int* segment_slots;
-  int n, channels, qk_width, dim, heads, keep;
+  int n, channels, qk_width, dim, heads, keep, decay_width;
   float unit_eps, q_factor;
 };
 
-// grid (groups of TT tokens, blocks of 256 fours of channels and one for decays and strengths).  A thread owns four
+// grid (groups of TT tokens, blocks of 256 fours of channels, with decays a channel blocks of 256 fours of decays, and one for
+// strengths and decays a head).  A thread owns four
 // channels and walks its tokens with the last inputs in registers; the dim / 4 threads of a head are neighbours in a wave
 // (dim / 4 is a power of two up to 64) and meet over the sum of squares.
 template <typename T, int K, int TT>
@@ -68,10 +72,30 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(InputArgs p) {
   if (blockIdx.y == gridDim.y - 1) {
     for (int e = threadIdx.x; e < count * p.heads; e += blockDim.x) {
       const int t = t0 + e / p.heads, h = e % p.heads;
-      const float za = to_float<T>(((const T*)p.a)[(int64_t)t * p.ldx + h]) + p.dt_bias[h];
       const float zb = to_float<T>(((const T*)p.b)[(int64_t)t * p.ldx + h]);
-      p.decay[(int64_t)t * p.heads + h] = expf(-expf(p.a_log[h]) * softplus(za));
+      if (p.decay_width == 1) {
+        const float za = to_float<T>(((const T*)p.a)[(int64_t)t * p.lda + h]) + p.dt_bias[h];
+        p.decay[(int64_t)t * p.heads + h] = expf(-expf(p.a_log[h]) * softplus(za));
+      }
       p.beta[(int64_t)t * p.heads + h] = 1.0f / (1.0f + expf(-zb));
+    }
+    return;
+  }
+  const int conv_blocks = (p.channels / 4 + 255) / 256;
+  if ((int)blockIdx.y >= conv_blocks) {
+    const int width = p.heads * p.decay_width, d = ((blockIdx.y - conv_blocks) * 256 + threadIdx.x) * 4;
+    if (d >= width) return;
+    const float rate = -expf(p.a_log[d / p.decay_width]);          // (the decays of a head are whole fours)
+    float bias[4], z[TT][4];
+    load4<float>(bias, p.dt_bias + d);
+#pragma unroll
+    for (int j = 0; j < TT; ++j) load4<T>(z[j], (const T*)p.a + (int64_t)(t0 + (j < count ? j : 0)) * p.lda + d);
+#pragma unroll
+    for (int j = 0; j < TT; ++j) {
+      if (j >= count) break;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) z[j][i] = expf(rate * softplus(z[j][i] + bias[i]));
+      store4<float>(p.decay + (int64_t)(t0 + j) * width + d, z[j]);
     }
     return;
   }
@@ -470,22 +494,27 @@ HFEE_API int hfee_delta_inputs_fit(int channels, int dim, int taps) {
 }
 
 // x: [n, channels] in dtype (0 float32, 1 bfloat16), the first qk_width columns queries, the next qk_width keys (heads of
-// dim), the rest values; a, b: [n, heads] like x, rows ldx apart; y: float32 [n, channels]; decay, beta: float32
-// [n, heads] contiguous.  keep: every token is its segment's only one, and the state gets its input.
+// dim), the rest values; a: [n, heads * decay_width] like x, rows lda apart, decay_width 1 or dim; b: [n, heads], rows ldx
+// apart; y: float32 [n, channels]; decay: float32 [n, heads * decay_width], beta: float32 [n, heads], both contiguous.  keep: every token is its segment's only one, and the state gets its input.
 HFEE_API int hfee_delta_inputs(float* y, int64_t ldy, float* decay, float* beta, const void* x, int64_t ldx, const void* a,
-                               const void* b, int dtype, void* state, const float* taps, int taps_count, const float* dt_bias,
+                               int64_t lda, const void* b, int dtype, void* state, const float* taps, int taps_count, const float* dt_bias,
                                const float* a_log, const int* token_segment, const int* segment_rows, const int* segment_slots,
-                               int n, int channels, int qk_width, int dim, int heads, float unit_eps, float q_factor, int keep,
+                               int n, int channels, int qk_width, int dim, int heads, int decay_width, float unit_eps,
+                               float q_factor, int keep,
                                hipStream_t stream) {
   HFEE_REQUIRE(n >= 0 && heads > 0 && qk_width > 0 && 2 * qk_width <= channels && dim > 0 && qk_width % dim == 0, "delta_inputs: bad sizes");
   HFEE_REQUIRE(hfee_delta_inputs_fit(channels, dim, taps_count), "delta_inputs: %d channels in heads of %d with %d taps", channels, dim, taps_count);
   HFEE_REQUIRE(dtype == 0 || dtype == 1, "delta_inputs: unknown dtype %d", dtype);
   HFEE_REQUIRE(ldx % 4 == 0 && ldx >= channels && ldy % 4 == 0 && ldy >= channels &&
                (((uintptr_t)y | (uintptr_t)x | (uintptr_t)state) & 15) == 0, "delta_inputs: rows must be aligned");
+  HFEE_REQUIRE(decay_width == 1 || (decay_width > 0 && decay_width % 4 == 0 && lda % 4 == 0 &&
+                                    (((uintptr_t)a | (uintptr_t)decay | (uintptr_t)dt_bias) & 15) == 0),
+               "delta_inputs: decays a channel come in aligned fours");
+  HFEE_REQUIRE(lda >= (int64_t)heads * decay_width, "delta_inputs: the decays' rows are too short");
   if (n == 0) return 0;
-  const InputArgs p{y, ldy, decay, beta, x, ldx, a, b, state, taps, dt_bias, a_log, token_segment, segment_rows, segment_slots,
-                    n, channels, qk_width, dim, heads, keep, unit_eps, q_factor};
-  const int columns = (channels / 4 + 255) / 256 + 1;
+  const InputArgs p{y, ldy, decay, beta, x, ldx, a, lda, b, state, taps, dt_bias, a_log, token_segment, segment_rows, segment_slots,
+                    n, channels, qk_width, dim, heads, keep, decay_width, unit_eps, q_factor};
+  const int columns = (channels / 4 + 255) / 256 + (decay_width > 1 ? (heads * decay_width / 4 + 255) / 256 : 0) + 1;
   HFEE_REQUIRE(columns <= 65535, "delta_inputs: too many channels");
   const bool few = n <= 64;
 #define LAUNCH(T, K)                                                                                                 \

@@ -103,6 +103,16 @@ __global__ __launch_bounds__(256) void unit_heads_kernel(float* __restrict__ x, 
   for (int d = lane; d < D; d += 64) p[d] *= inv;
 }
 
+__device__ __forceinline__ float gate_value(float v, int c, const float* per_head, int head_width, int mode, float number,
+                                            int first_columns) {
+  if (mode == 0) return expf(-expf(per_head[c / head_width]) * softplus(v));
+  if (mode == 1) return expf(log_sigmoid(v) / number);
+  if (mode == 2) return 1.0f / (1.0f + expf(-v));
+  if (mode == 4) return softplus(v);
+  if (mode == 5) return v / (1.0f + expf(-v));
+  return c < first_columns ? v * number : v;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void scan_gate_kernel(float* __restrict__ out, int64_t ldo, const T* __restrict__ z,
                                                         int64_t ldz, const float* __restrict__ bias,
@@ -113,14 +123,26 @@ __global__ __launch_bounds__(256) void scan_gate_kernel(float* __restrict__ out,
   if (c >= width) return;
   float v = to_float<T>(z[t * ldz + c]);
   if (bias != nullptr) v += bias[c];
-  float r;
-  if (mode == 0) r = expf(-expf(per_head[c / head_width]) * softplus(v));
-  else if (mode == 1) r = expf(log_sigmoid(v) / number);
-  else if (mode == 2) r = 1.0f / (1.0f + expf(-v));
-  else if (mode == 4) r = softplus(v);
-  else if (mode == 5) r = v / (1.0f + expf(-v));
-  else r = c < first_columns ? v * number : v;
-  out[t * ldo + c] = r;
+  out[t * ldo + c] = gate_value(v, c, per_head, head_width, mode, number, first_columns);
+}
+
+// The same for rows of whole aligned fours, four values a thread (2,048 rows of 8,192 columns, a cast: 32 -> 22 us).
+template <typename T>
+__global__ __launch_bounds__(256) void scan_gate_fours_kernel(float* __restrict__ out, int64_t ldo, const T* __restrict__ z,
+                                                              int64_t ldz, const float* __restrict__ bias,
+                                                              const float* __restrict__ per_head, int head_width, int mode,
+                                                              float number, int first_columns, int width) {
+  const int64_t t = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (c >= width) return;
+  float v[4];
+  load4<T>(v, z + t * ldz + c);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (bias != nullptr) v[i] += bias[c + i];
+    v[i] = gate_value(v[i], c + i, per_head, head_width, mode, number, first_columns);
+  }
+  store4<float>(out + t * ldo + c, v);
 }
 
 // grid (blocks of 16 columns, heads, segments), four waves; a wave owns four columns of S, lane =
@@ -875,7 +897,16 @@ HFEE_API int hfee_scan_gate(float* out, int64_t ldo, const void* z, int64_t ldz,
   HFEE_REQUIRE(mode != 1 || number > 0.f, "scan_gate: tau must be positive");
   if (n == 0) return 0;
   dim3 grid(n, (width + 255) / 256);
-  if (dtype == 0)
+  const bool fours = width % 4 == 0 && ldo % 4 == 0 && ldz % 4 == 0 && (uintptr_t)out % 16 == 0 &&
+                     (uintptr_t)z % (dtype == 0 ? 16 : 8) == 0;
+  dim3 grid4(n, (width / 4 + 255) / 256);
+  if (dtype == 0 && fours)
+    scan_gate_fours_kernel<float><<<grid4, 256, 0, stream>>>(out, ldo, (const float*)z, ldz, bias, per_head, head_width, mode,
+                                                             number, first_columns, width);
+  else if (dtype == 1 && fours)
+    scan_gate_fours_kernel<bf16_t><<<grid4, 256, 0, stream>>>(out, ldo, (const bf16_t*)z, ldz, bias, per_head, head_width,
+                                                              mode, number, first_columns, width);
+  else if (dtype == 0)
     scan_gate_kernel<float><<<grid, 256, 0, stream>>>(out, ldo, (const float*)z, ldz, bias, per_head, head_width, mode,
                                                       number, first_columns, width);
   else if (dtype == 1)

@@ -79,7 +79,7 @@ _CORE_SIGNATURES = {
     "hfee_token_shift": [P, I, P, P, P, P, P, P, P, I, I, P],
     "hfee_softcap": [P, F, L, P],
     "hfee_delta_inputs_fit": [I, I, I],
-    "hfee_delta_inputs": [P, L, P, P, P, L, P, P, I, P, P, I, P, P, P, P, P, I, I, I, I, I, F, F, I, P],
+    "hfee_delta_inputs": [P, L, P, P, P, L, P, L, P, I, P, P, I, P, P, P, P, P, I, I, I, I, I, I, F, F, I, P],
     "hfee_delta_chunks": [P, L, P, P, L, P, L, P, L, P, L, P, L, P, P, P, I, I, I, I, I, I, I, I, P, L, P],
     "hfee_delta_chunks_least": [],
     "hfee_group_norm": [P, I, P, P, P, F, I, I, I, P],

@@ -1719,10 +1719,10 @@ def delta_inputs_fit(channels: int, dim: int, taps: int) -> bool:
 
 def delta_inputs(y, decay, beta, x, a, b, state, taps, dt_bias, a_log, token_segment, segment_rows, segment_slots,
                  qk_width: int, dim: int, heads: int, unit_eps: float, q_factor: float, keep: bool):
-    """Everything that enters the gated delta rule with one decay a head, from the projections x ([n, channels]: queries,
-    keys, values), a and b ([n, heads], blocks of columns of x's buffer): y (float32 [n, channels]) =
+    """Everything that enters the gated delta rule, from the projections x ([n, channels]: queries, keys, values), b ([n,
+    heads], a block of columns of x's buffer) and a ([n, heads], another, for one decay a head; or [n, heads * dim]): y (float32 [n, channels]) =
     `short_conv_silu` of x, queries and keys then unit vectors over each head of dim (eps unit_eps), queries times
-    q_factor; decay (float32 [n, heads]) = exp(-exp(a_log) * softplus(a + dt_bias)); beta = sigmoid(b).  keep: every row is its
+    q_factor; decay (float32, like a) = exp(-exp(a_log[head]) * softplus(a + dt_bias)); beta = sigmoid(b).  keep: every row is its
     segment's only token, and the state gets its input as by `short_conv_keep`."""
     _gpu(y, decay, beta, x, a, b, state, taps, dt_bias, a_log, token_segment, segment_rows, segment_slots)
     n, C, ldx = _rows2d(x, "delta_inputs x")
@@ -1730,20 +1730,21 @@ def delta_inputs(y, decay, beta, x, a, b, state, taps, dt_bias, a_log, token_seg
     K = taps.shape[1]
     _check(ny == n and wy == C and tuple(taps.shape) == (C, K) and taps.dtype == torch.float32 and taps.is_contiguous(), "delta_inputs: y and taps")
     _check(state.dtype == x.dtype and state.is_contiguous() and tuple(state.shape[1:]) == (K - 1, C), "delta_inputs: state [slots, K - 1, C]")
-    for t in (decay, beta):
-        _check(t.dtype == torch.float32 and t.is_contiguous() and tuple(t.shape) == (n, heads), "delta_inputs: decay and beta float32 [n, heads]")
-    for t in (a, b):
-        na, wa, lda = _rows2d(t, "delta_inputs a, b")
-        _check(na == n and wa == heads and t.dtype == x.dtype and (n == 1 or lda == ldx), "delta_inputs: a and b are columns of x's buffer")
-    for t in (dt_bias, a_log):
-        _check(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == heads, "delta_inputs: dt_bias and a_log float32 [heads]")
+    na, wa, lda = _rows2d(a, "delta_inputs a")
+    nb, wb, ldb = _rows2d(b, "delta_inputs b")
+    _check(na == n and wa in (heads, heads * dim) and a.dtype == x.dtype, "delta_inputs: a [n, heads] or [n, heads * dim]")
+    _check(nb == n and wb == heads and b.dtype == x.dtype and (n == 1 or ldb == ldx), "delta_inputs: b are columns of x's buffer")
+    for t, w in ((decay, wa), (beta, heads)):
+        _check(t.dtype == torch.float32 and t.is_contiguous() and tuple(t.shape) == (n, w), "delta_inputs: decay float32 like a, beta [n, heads]")
+    for t, w in ((dt_bias, wa), (a_log, heads)):
+        _check(t.dtype == torch.float32 and t.is_contiguous() and t.numel() == w, "delta_inputs: dt_bias float32 as wide as a, a_log [heads]")
     _i32(token_segment, "delta_inputs token_segment", n)
     _i32(segment_rows, "delta_inputs segment_rows")
     _i32(segment_slots, "delta_inputs segment_slots")
     _check(not keep or segment_rows.numel() == n, "delta_inputs: keep is for steps of single tokens")
-    lib.core().call("hfee_delta_inputs", _ptr(y), ldy, _ptr(decay), _ptr(beta), _ptr(x), ldx, _ptr(a), _ptr(b), _dt(x), _ptr(state),
+    lib.core().call("hfee_delta_inputs", _ptr(y), ldy, _ptr(decay), _ptr(beta), _ptr(x), ldx, _ptr(a), lda, _ptr(b), _dt(x), _ptr(state),
                     _ptr(taps), K, _ptr(dt_bias), _ptr(a_log), _ptr(token_segment), _ptr(segment_rows), _ptr(segment_slots), n, C,
-                    int(qk_width), int(dim), int(heads), float(unit_eps), float(q_factor), int(keep), _stream())
+                    int(qk_width), int(dim), int(heads), wa // heads, float(unit_eps), float(q_factor), int(keep), _stream())
 
 
 def linear_scan(out, state, q, k, v, decay, beta, segment_rows, segment_lengths, segment_slots, heads: int,

@@ -167,8 +167,7 @@ class GatedDelta(_StateMixer):
         self.g_columns = slice(second, self.at_b) if self.gate_rank is not None else slice(self.channels, second)
         self.conv_taps = torch.cat([f32(n["q_conv"]), f32(n["k_conv"]), f32(n["v_conv"])], dim=0).contiguous()
         # (what enters the recurrence is one launch where its kernel takes the sizes)
-        self.one_launch = (self.decay_per_head and self.w_in.is_cuda
-                           and ops.delta_inputs_fit(self.channels, self.dim, self.taps))
+        self.one_launch = self.w_in.is_cuda and ops.delta_inputs_fit(self.channels, self.dim, self.taps)
         self.a_log, self.dt_bias, self.norm_weight = f32(n["a_log"]), f32(n["dt_bias"]), f32(n["norm"])
         self.w_o = tensors.pop(n["o"]).contiguous()
         self.w_in_tiles, self.w_o_tiles = tiles_of(self.dtype, self.w_in, self.w_o)
@@ -205,9 +204,10 @@ class GatedDelta(_StateMixer):
         y = ctx.rows("gated_delta.conv", staggered(self.channels), torch.float32)[:, :self.channels]
         beta = ctx.rows("gated_delta.beta", H, torch.float32)
         if self.one_launch:
-            decay = ctx.rows("gated_delta.decay", H, torch.float32)
+            step = self._step(ctx, proj)
+            decay = ctx.rows("gated_delta.decay", step.shape[1], torch.float32)
             singles = ctx.n == len(ctx.segments)
-            ops.delta_inputs(y, decay, beta, raw, proj[:, self.a_columns], proj[:, self.at_b:self.at_b + H], self.conv_state,
+            ops.delta_inputs(y, decay, beta, raw, step, proj[:, self.at_b:self.at_b + H], self.conv_state,
                              self.conv_taps, self.dt_bias, self.a_log, ctx.token_segment, rows, slots, self.qk_width, D, H,
                              self.unit_eps, D ** -0.5, keep=singles)
             if not singles:
@@ -229,6 +229,14 @@ class GatedDelta(_StateMixer):
     def chunk_words(self, longest, rows):
         return ops.delta_chunks_scratch(longest, rows, self.heads, self.dim, self.vdim) if self.decay_per_head else 0
 
+    def _step(self, ctx, proj):
+        """What the decays are made of: a number a head, or a key channel through the second half of its product."""
+        if self.decay_per_head:
+            return proj[:, self.a_columns]
+        step = ctx.rows("gated_delta.step", self.heads * self.dim)
+        product(ctx, step, proj[:, self.a_columns], self.w_a_up, self.w_a_up_tiles)
+        return step
+
     def _inputs(self, ctx, y, beta, proj):
         """What enters the recurrence, a launch a mechanism: fills y and beta, returns the decays."""
         H, G, D = self.heads, self.qk_heads, self.dim
@@ -239,10 +247,7 @@ class GatedDelta(_StateMixer):
         ops.unit_heads(y[:, :self.qk_width], G, D, self.unit_eps, D ** -0.5)
         ops.unit_heads(y[:, self.qk_width:2 * self.qk_width], G, D, self.unit_eps, 1.0)
         per_decay = 1 if self.decay_per_head else D
-        step = proj[:, self.a_columns]
-        if not self.decay_per_head:
-            step = ctx.rows("gated_delta.step", H * D)
-            product(ctx, step, proj[:, self.a_columns], self.w_a_up, self.w_a_up_tiles)
+        step = self._step(ctx, proj)
         decay = ctx.rows("gated_delta.decay", H * per_decay, torch.float32)
         ops.scan_gate(decay, step, "step_decay", bias=self.dt_bias, per_head=self.a_log, head_width=per_decay)
         ops.scan_gate(beta, proj[:, self.at_b:self.at_b + H], "sigmoid")

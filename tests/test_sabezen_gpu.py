@@ -318,6 +318,48 @@ def test_mixed_attention_in_parts(H, G, D):
                 assert su.rel(got[t].double().cpu(), want[t].double().cpu()) < 1e-2, f"row {t} in at most {most} parts"
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("lengths", [(1,), (1, 1, 1), (9, 1, 2), (70, 17)])
+def test_inputs_with_decays_a_channel_in_one_launch(dtype, lengths):
+    """Decays a channel beside the convolution, the unit vectors and the strengths, against a launch a mechanism (values by one,
+    as odd widths have them): the sums of squares are added up in another order, everything else is the same arithmetic."""
+    from hfee_amd.kernels import ops
+    dt = getattr(torch, dtype)
+    H, G, D, V, K = 6, 2, 32, 24, 4
+    qk, C, n = G * D, 2 * G * D + H * V, sum(lengths)
+    assert ops.delta_inputs_fit(C, D, K)
+    g = torch.Generator().manual_seed(n)
+    rand = lambda *shape: torch.randn(*shape, generator=g).cuda()      # noqa: E731
+    proj = rand(n, C + 8).to(dt)
+    x, b = proj[:, :C], proj[:, C:C + H]
+    step, taps, state = rand(n, H * D).to(dt), rand(C, K), rand(5, K - 1, C).to(dt)
+    bias, a_log = rand(H * D), rand(H)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")      # noqa: E731
+    rows, lens, slots = i32(np.cumsum((0,) + lengths)[:-1].tolist()), i32(lengths), i32([4, 1, 2][:len(lengths)])
+    seg = i32(np.repeat(np.arange(len(lengths)), lengths).tolist())
+    want, states = torch.zeros(n, C, device="cuda"), [state.clone(), state.clone()]
+    ops.short_conv_silu(want, x, states[0], taps, seg, rows, slots)
+    ops.short_conv_keep(states[0], x, rows, lens, slots)
+    ops.unit_heads(want[:, :qk], G, D, 1e-6, 0.5)
+    ops.unit_heads(want[:, qk:2 * qk], G, D, 1e-6, 1.0)
+    wide = torch.zeros(n, H * D + 1, device="cuda")[:, :H * D]      # (rows that are no aligned fours: a value a thread)
+    beta = torch.zeros(n, H, device="cuda")
+    ops.scan_gate(wide, step, "step_decay", bias=bias, per_head=a_log, head_width=D)
+    ops.scan_gate(beta, b, "sigmoid")
+    got, decay, strength = torch.zeros(n, C, device="cuda"), torch.zeros(n, H * D, device="cuda"), torch.zeros(n, H, device="cuda")
+    singles = max(lengths) == 1
+    ops.delta_inputs(got, decay, strength, x, step, b, states[1], taps, bias, a_log, seg, rows, slots, qk, D, H, 1e-6, 0.5, keep=singles)
+    if not singles:
+        ops.short_conv_keep(states[1], x, rows, lens, slots)
+    assert torch.equal(decay, wide) and torch.equal(strength, beta) and torch.equal(states[0], states[1])
+    assert float((got - want).abs().max()) <= 8 * 2.0 ** -23 * float(want.abs().max())
+    for kind, kw in (("cast", dict(number=0.3, first_columns=D + 1)), ("silu", {}), ("root_sigmoid", dict(number=16.0, bias=bias)), ("softplus", {})):
+        fours = torch.zeros(n, H * D, device="cuda")
+        ops.scan_gate(fours, step, kind, **kw)
+        ops.scan_gate(wide, step, kind, **kw)
+        assert torch.equal(fours, wide), kind
+
+
 @pytest.mark.parametrize("rule", ["delta", "decay_add"])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 8, 16), (3, 3, 20, 12), (2, 1, 33, 70)])
 def test_linear_scan_in_portions(rule, H, G, D, V):

@@ -164,8 +164,14 @@ def load(name: str) -> Library:
         return lib
 
 
+_core = None
+
+
 def core() -> Library:
-    return load("core")
+    global _core
+    if _core is None:
+        _core = load("core")
+    return _core
 
 
 def attention_bf16(head_dim: int) -> Library:

@@ -33,14 +33,16 @@ def _stream():
     global _DEVICE
     if _DEVICE is None:
         _DEVICE = torch.cuda.current_device()
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None:
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    return ctypes.c_void_p(raw(_DEVICE))
+    return _raw_stream(_DEVICE) if _raw_stream is not None else torch.cuda.current_stream().cuda_stream
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+# (Addresses go to the entry points as numbers, and a message is put together where a check has failed: the objects and texts
+# that nobody reads were a third of what a launch takes the host.)
 def _ptr(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _check(cond, msg):
@@ -56,14 +58,18 @@ def _gpu(*tensors):
 
 def _rows2d(t: torch.Tensor, what: str):
     """A 2-D tensor whose rows are contiguous: (rows, cols, leading dimension)."""
-    _check(t.dim() == 2 and t.stride(1) == 1, f"{what}: expected a 2-D tensor with contiguous rows")
-    return t.shape[0], t.shape[1], t.stride(0) if t.shape[0] > 1 else max(t.stride(0), t.shape[1])
+    strides = t.stride()
+    if len(strides) != 2 or strides[1] != 1:
+        raise KernelError(f"{what}: expected a 2-D tensor with contiguous rows")
+    rows, cols = t.shape
+    return rows, cols, strides[0] if rows > 1 else max(strides[0], cols)
 
 
 def _i32(t, what, n=None):
-    _check(t.dtype == torch.int32 and t.is_contiguous(), f"{what}: expected a contiguous int32 tensor")
-    if n is not None:
-        _check(t.numel() >= n, f"{what}: {t.numel()} entries, {n} needed")
+    if t.dtype != torch.int32 or not t.is_contiguous():
+        raise KernelError(f"{what}: expected a contiguous int32 tensor")
+    if n is not None and t.numel() < n:
+        raise KernelError(f"{what}: {t.numel()} entries, {n} needed")
 
 
 # ------------------------------------------------------------------ simple ops
@@ -309,8 +315,8 @@ def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate:
     M, K, lda = _rows2d(x, "linear x")
     N, Kw, ldw = _rows2d(weight, "linear weight")
     Mo, No, ldc = _rows2d(out, "linear out")
-    _check(Kw == K and Mo == M and No == (N // 2 if gate else N),
-           f"linear: shapes x{list(x.shape)} w{list(weight.shape)} out{list(out.shape)}")
+    if not (Kw == K and Mo == M and No == (N // 2 if gate else N)):
+        raise KernelError(f"linear: shapes x{list(x.shape)} w{list(weight.shape)} out{list(out.shape)}")
     if gate:
         _check(x.dtype == weight.dtype == out.dtype == torch.bfloat16 and not accumulate and N % 2 == 0,
                "linear: the gate epilogue takes bfloat16 operands and an even number of weight rows")
@@ -729,7 +735,8 @@ def linear_fused(out, x, weight, epilogue: str, norm_weight=None, eps: float = 0
     Mx, Kx, lda = _rows2d(x, "linear_fused x")
     M = Mx if m is None else m
     _check(Kx == K, "linear_fused: inner sizes differ")
-    _check(M <= SKINNY_MAX_ROWS, f"linear_fused: at most {SKINNY_MAX_ROWS} rows, got {M}")
+    if M > SKINNY_MAX_ROWS:
+        raise KernelError(f"linear_fused: at most {SKINNY_MAX_ROWS} rows, got {M}")
     weight = weight.tiles
     fused_norm = norm_weight is not None
     if fused_norm:
@@ -742,9 +749,9 @@ def linear_fused(out, x, weight, epilogue: str, norm_weight=None, eps: float = 0
     Mo, No, ldc = _rows2d(out, "linear_fused out")
     _check(Mo >= M, "linear_fused: out has too few rows")
     epi = _EPI[epilogue]
-    want = {"bf16": torch.bfloat16, "f32": torch.float32, "add": torch.float32, "swiglu": torch.bfloat16,
-            "qkv": torch.bfloat16}[epilogue]
-    _check(out.dtype == want, f"linear_fused: out must be {want} for {epilogue!r}")
+    want = torch.float32 if epilogue in ("f32", "add") else torch.bfloat16
+    if out.dtype != want:
+        raise KernelError(f"linear_fused: out must be {want} for {epilogue!r}")
     e_args = [None, 0, None, 0, None]
     if emit is not None:
         _gpu(emit["weight"], emit["out"], emit["shares"])

@@ -797,10 +797,18 @@ constexpr int WIDE_MIN_GROUPS_A_CU = 6;
 // waves, a decode step at batch 20 / 24 / 32 / 40 / 48 1.181 / 1.210 / 1.288 / 1.329 / 1.405 -> 1.139 / 1.166 /
 // 1.240 / 1.326 / 1.399 ms; at 64 rows the pair of kernels stays, 1.591 against 1.616)
 constexpr int WIDE_MIN_GROUPS_A_CU_FEW_ROWS = 4;       // of eight: below, the kernels above with their slices of K spread better
+// Fewer row groups a CU, where the pair of kernels would run: from here on this one, with the columns added up in the pair's
+// slices, so that the results are the pair's to the bit (us, the products cold in a captured graph, the pair -> this): at 24
+// rows 8,192 x 3,072 weights 15.2 -> 13.7, 12,288 x 4,096 24.7 -> 21.4, 15,360 x 5,120 (q/k/v of the 13B shape) 36.8 -> 30.6, but
+// 6,144 x 4,096 14.9 -> 16.6; at 43 rows 10,240 x 4,096 24.1 -> 22.8, 15,360 x 5,120 40.6 -> 34.1, but 9,216 x 3,072 17.5 -> 17.9;
+// at 64 rows 15,360 x 5,120 41.7 -> 42.2.
+constexpr float wide_groups_as_pair(int mt) { return mt == 2 ? 2.f : 2.5f; }
 
 constexpr size_t mid_wide_lds_bytes(int mt) { return (size_t)2 * mt * 16 * WIDE_PITCH * sizeof(bf16_t); }
 
-template <int MT, int EPI>
+// CUT > 0: the sums of every CUT slices are made from zero and added up in their order, as the pair of kernels does (a form
+// of its own: as an argument the second set of sums slowed gate/up at 64 rows, a decode step of the 8B shape 5.3 -> 5.9 ms).
+template <int MT, int EPI, int CUT>
 __global__ __launch_bounds__(WAVES * 64) void mid_wide_kernel(Args a, int row_groups, int busy) {
   extern __shared__ __attribute__((aligned(16))) char wide_lds[];
   bf16_t* xs = (bf16_t*)wide_lds;                                    // [2][MT * 16][WIDE_PITCH]
@@ -858,10 +866,23 @@ __global__ __launch_bounds__(WAVES * 64) void mid_wide_kernel(Args a, int row_gr
   for (int first = blockIdx.x * busy; first < row_groups; first += stride) {      // (the same for all waves: barriers inside)
     const int rg = works ? first + wave : row_groups;
     const bf16_t* w_next = row_ptr(rg + stride);                     // past the end: a repeat that nobody uses
-    f32x4 acc[MT];
+    f32x4 acc[MT], total[CUT > 0 ? MT : 1];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (CUT > 0) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) total[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     for (int s = 0; s < slices; ++s) {
+      if constexpr (CUT > 0) {
+        if (s > 0 && s % CUT == 0) {
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            total[t] += acc[t];
+            acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+      }
       ask(fill, s + 1 < slices ? s + 1 : 0);
       const bf16_t* x_lane = xs + (buf * MT * 16 + r16) * WIDE_PITCH + g * 8;
       if (works) {                 // (the same for the whole wave)
@@ -900,6 +921,7 @@ __global__ __launch_bounds__(WAVES * 64) void mid_wide_kernel(Args a, int row_gr
 #pragma unroll
       for (int t = 0; t < MT; ++t) {
         const int m = t * 16 + r16;
+        if constexpr (CUT > 0) acc[t] = total[t] + acc[t];
         float v[4] = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
         if (a.scale_ss != nullptr) {
           const float scale = row_scale[m];
@@ -916,7 +938,7 @@ __global__ __launch_bounds__(WAVES * 64) void mid_wide_kernel(Args a, int row_gr
 
 // Returns true if the kernel for 17 to 64 rows and many weight rows took the product.
 template <int MT>
-bool launch_mid_wide(const Args& a, int epi, int num_cus, hipStream_t stream) {
+bool launch_mid_wide(const Args& a, int epi, int num_cus, bool as_pair, hipStream_t stream) {
   const int row_groups = (a.N + ROWS - 1) / ROWS;
   const int per = (row_groups + num_cus * WAVES - 1) / (num_cus * WAVES);      // rounds of a workgroup, all but equal
   // (gate/up of the 8B shape: seven waves on 256 CUs instead of eight on 224: a decode step at batch 64
@@ -925,17 +947,26 @@ bool launch_mid_wide(const Args& a, int epi, int num_cus, hipStream_t stream) {
   if (busy > WAVES) busy = WAVES;
   const int grid = (row_groups + busy * per - 1) / (busy * per);
   const size_t lds = mid_wide_lds_bytes(MT);
-#define GO(E)                                                                                                  \
+#define GO_CUT(E, CUT)                                                                                                  \
   do {                                                                                                         \
     static bool raised = false;                                                                                \
     if (!raised) {                                                                                             \
-      if (hipFuncSetAttribute((const void*)mid_wide_kernel<MT, E>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+      if (hipFuncSetAttribute((const void*)mid_wide_kernel<MT, E, CUT>, hipFuncAttributeMaxDynamicSharedMemorySize, \
                               (int)lds) != hipSuccess)                                                        \
         return false;                                                                                          \
       raised = true;                                                                                           \
     }                                                                                                          \
-    mid_wide_kernel<MT, E><<<grid, WAVES * 64, lds, stream>>>(a, row_groups, busy);                            \
+    mid_wide_kernel<MT, E, CUT><<<grid, WAVES * 64, lds, stream>>>(a, row_groups, busy);                            \
   } while (0)
+#define GO(E)                                                  \
+  do {                                                         \
+    if constexpr (MT < 4) {                                    \
+      if (as_pair) GO_CUT(E, MID_KS / WIDE_KS); else GO_CUT(E, 0); \
+    } else {                                                   \
+      GO_CUT(E, 0);                                            \
+    }                                                          \
+  } while (0)
+  if (as_pair && MT >= 4) return false;
   switch (epi) {
     case EPI_BF16: GO(EPI_BF16); break;
     case EPI_F32: GO(EPI_F32); break;
@@ -944,6 +975,7 @@ bool launch_mid_wide(const Args& a, int epi, int num_cus, hipStream_t stream) {
     default: GO(EPI_QKV); break;
   }
 #undef GO
+#undef GO_CUT
   return true;
 }
 
@@ -1145,7 +1177,7 @@ bool launch_wide(const Args& a, bool norm, int epi, hipStream_t stream) {
 // ceil(N / 16) * ceil(K / 1024) * ceil(M / 16) * 256 + 64 floats of scratch (none for K <= 1,024);
 // without it, or for other sizes, or where it would not pay, the streaming kernel takes
 // the product (force_mid: 1 takes the pair of kernels with slices of K wherever it applies,
-// 2 the kernel for many weight rows: for tests).
+// 2 the kernel for many weight rows, 3 that one with the pair's sums (up to 48 rows): for tests).
 HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32, int64_t lda, const void* W,
                               int64_t w_stride, int M, int N, int K, int epi,
                               const void* norm_weight, int norm_weight_is_f32, float eps, const int* rows,
@@ -1227,12 +1259,17 @@ HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32,
                prop.multiProcessorCount > 0) ? prop.multiProcessorCount : 256;
   }
   // weight rows enough for most of the CUs to have eight row groups each: nothing is cut along K
-  const bool wide_rows = (N + ROWS - 1) / ROWS >= WIDE_MIN_GROUPS_A_CU * num_cus ||
-                         ((N + ROWS - 1) / ROWS >= WIDE_MIN_GROUPS_A_CU_FEW_ROWS * num_cus && mt <= 3);
-  if (!norm && mt > 1 && K % WIDE_KS == 0 && (force_mid == 2 || (force_mid == 0 && wide_rows))) {
-    const bool took = mt == 2 ? launch_mid_wide<2>(a, epi, num_cus, stream)
-                    : mt == 3 ? launch_mid_wide<3>(a, epi, num_cus, stream)
-                              : launch_mid_wide<4>(a, epi, num_cus, stream);
+  const int row_groups = (N + ROWS - 1) / ROWS;
+  const bool wide_rows = row_groups >= WIDE_MIN_GROUPS_A_CU * num_cus ||
+                         (row_groups >= WIDE_MIN_GROUPS_A_CU_FEW_ROWS * num_cus && mt <= 3);
+  const int64_t pair_floats = (int64_t)row_groups * ((K + MID_KS - 1) / MID_KS) * mt * 256 + SS_STRIDE;
+  const bool wide_as_pair = !wide_rows && mid_pays && K > MID_KS && mt <= 3 && row_groups >= wide_groups_as_pair(mt) * num_cus &&
+                            scratch != nullptr && scratch_floats >= pair_floats;
+  if (!norm && mt > 1 && K % WIDE_KS == 0 && (force_mid >= 2 || (force_mid == 0 && (wide_rows || wide_as_pair)))) {
+    const bool as_pair = force_mid == 3 || (force_mid == 0 && wide_as_pair);
+    const bool took = mt == 2 ? launch_mid_wide<2>(a, epi, num_cus, as_pair, stream)
+                    : mt == 3 ? launch_mid_wide<3>(a, epi, num_cus, as_pair, stream)
+                              : launch_mid_wide<4>(a, epi, num_cus, as_pair, stream);
     if (took) {
       HFEE_CHECK_LAUNCH("gemm_skinny(17 to 64 rows, many weight rows)");
       return 0;

@@ -716,7 +716,7 @@ def linear_fused(out, x, weight, epilogue: str, norm_weight=None, eps: float = 0
     K % 256 == 0 take a kernel that keeps the batch in LDS and cuts K over workgroups, and a
     second one that adds the slices up, where that pays.  Products with weight rows enough to
     fill the chip take a kernel that cuts nothing and needs no scratch.  (force_mid_rows, for
-    tests: 1 takes the first wherever it applies, 2 the second.)
+    tests: 1 takes the first wherever it applies, 2 the second, 3 the second with the first one's sums.)
 
     x: bfloat16 [M, K]; or, with norm_weight, the float32 residual stream (at most 16
     rows; `rows` optionally gathers them, then `m` is their number).

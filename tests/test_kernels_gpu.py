@@ -493,6 +493,28 @@ def test_fused_qkv_through_the_tiled_kernels_with_whole_steps_of_k(H, K, hd, hal
     _check_fused_qkv(H, K, hd, half, M, False, d)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (33, 50, 1536), (40, 4160, 5120), (32, 4112, 3072), (48, 16, 2560)])
+def test_many_weight_rows_with_the_sums_of_the_pair(M, N, K):
+    """The kernel for many weight rows in the pair's slices of K gives the pair's results to the bit, a last slice of half the
+    columns among them, with and without the second half of a norm, through every plain epilogue."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight((torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV))
+    blocks = K // 16
+    row_scale = dict(shares=torch.rand(blocks * 64, generator=g).to(DEV), blocks=blocks, eps=1e-5)
+    c0 = torch.randn(M, N, generator=g).to(DEV)
+    for epilogue in ("bf16", "f32", "add", "swiglu"):
+        for scale in (None, row_scale):
+            got = []
+            for kernel in (1, 3):
+                scratch = torch.full((ops.mid_rows_scratch(M, N, K),), float("nan"), dtype=torch.float32, device=DEV)
+                out = (c0.clone() if epilogue in ("f32", "add") else c0[:, :N // 2 if epilogue == "swiglu" else N].to(torch.bfloat16).contiguous())
+                ops.linear_fused(out, x, w, epilogue, row_scale=scale, scratch=scratch, force_mid_rows=kernel)
+                got.append(out)
+            assert torch.equal(*got), f"{epilogue} {'with' if scale else 'without'} a row scale"
+
+
 @pytest.mark.parametrize("kernel", [1, 2])
 @pytest.mark.parametrize("H,K,hd,half,M,d", [(4, 2, 16, 8, 17, 2048), (5, 1, 64, 32, 64, 1024), (6, 3, 48, 8, 40, 3072)])
 def test_fused_qkv_with_the_batch_in_lds(H, K, hd, half, M, d, kernel):

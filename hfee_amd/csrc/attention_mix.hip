@@ -85,54 +85,6 @@ __global__ __launch_bounds__(256) void mix_prepare_kernel(
   }
 }
 
-// The same with four dims a lane and a row a group of dim / 4 lanes (a power of two up to 64), for aligned rows whose rotated
-// halves are whole fours: 2,048 tokens of 40 heads of 128 44 -> 27 us.
-template <typename T>
-__global__ __launch_bounds__(256) void mix_prepare_fours_kernel(
-    T* __restrict__ q, int64_t ldq, const T* __restrict__ k, int64_t ldk, int num_heads, const int* __restrict__ positions,
-    const int* __restrict__ token_segment, const int* __restrict__ block_tables, int bt_stride,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t, int half, int norm, float eps,
-    T* __restrict__ cache, MixLayout lay) {
-  const int t = blockIdx.x, D = lay.dk, lanes = D / 4, d = 4 * (threadIdx.x & (lanes - 1));
-  const int row = (blockIdx.y * blockDim.x + threadIdx.x) / lanes;
-  const bool is_q = row < num_heads, live = row < num_heads + (k != nullptr ? lay.kv_heads : 0) && (!is_q || q != nullptr);
-  const int pos = positions[t];
-  const T* src = !live ? (q != nullptr ? q : k) : is_q ? q + (int64_t)t * ldq + (int64_t)row * D : k + (int64_t)t * ldk + (int64_t)(row - num_heads) * D;
-  float own[4], turned[4], other[4] = {}, c[4] = {1.f, 1.f, 1.f, 1.f}, s[4] = {};
-  load4<T>(own, src + (live ? d : 0));
-  if (live && d < 2 * half) {
-    const int f = d < half ? d : d - half;
-    load4<T>(other, src + (d < half ? d + half : d - half));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      c[i] = cos_t[(int64_t)pos * half + f + i];
-      s[i] = sin_t[(int64_t)pos * half + f + i];
-    }
-  }
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    turned[i] = d >= 2 * half ? own[i] : d < half ? own[i] * c[i] - other[i] * s[i] : own[i] * c[i] + other[i] * s[i];
-    ss = fmaf(turned[i], turned[i], ss);
-  }
-  for (int off = lanes >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
-  if (!live) return;
-  const float inv = norm ? 1.0f / sqrtf(ss / (float)D + eps) : 1.0f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) turned[i] *= inv;
-  if (is_q) {
-    store4<T>(q + (int64_t)t * ldq + (int64_t)row * D + d, turned);
-    return;
-  }
-  const int page = block_tables[(int64_t)token_segment[t] * bt_stride + (pos >> lay.page_shift)];
-  const int kvh = row - num_heads, slot = pos & (lay.page_size - 1);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    cache[lay.key_offset(page, kvh, slot, d + i)] = finite_for_cache<T>(from_float<T>(turned[i]));
-    cache[lay.value_offset(page, kvh, slot, d + i)] = finite_for_cache<T>(from_float<T>(own[i]));
-  }
-}
-
 constexpr int kKeyTile = 64;
 constexpr int kMaxAcc = 16;     // output elements a thread: num_heads * dim <= 16 * threads
 
@@ -265,21 +217,6 @@ HFEE_API int hfee_attention_mix_prepare(void* q, int64_t ldq, const void* k, int
   const int rows = num_heads + kv_heads;
   int parts = n >= 512 ? 1 : (rows + 3) / 4;
   if (parts > 16) parts = 16;
-  const int size = dtype == 0 ? 4 : 2, lanes = dim / 4;
-  const bool fours = dim % 4 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && half % 4 == 0 &&
-                     (q == nullptr || (ldq % 4 == 0 && (uintptr_t)q % (4 * size) == 0)) &&
-                     (k == nullptr || (ldk % 4 == 0 && (uintptr_t)k % (4 * size) == 0));
-  if (fours && (dtype == 0 || dtype == 1)) {
-    const dim3 grid(n, (rows * lanes + 255) / 256);
-    if (dtype == 0)
-      mix_prepare_fours_kernel<float><<<grid, 256, 0, stream>>>((float*)q, ldq, (const float*)k, ldk, num_heads, positions,
-          token_segment, block_tables, bt_stride, cos_t, sin_t, half, norm, eps, (float*)cache, lay);
-    else
-      mix_prepare_fours_kernel<bf16_t><<<grid, 256, 0, stream>>>((bf16_t*)q, ldq, (const bf16_t*)k, ldk, num_heads, positions,
-          token_segment, block_tables, bt_stride, cos_t, sin_t, half, norm, eps, (bf16_t*)cache, lay);
-    HFEE_CHECK_LAUNCH("attention_mix_prepare");
-    return 0;
-  }
 #define LAUNCH(T)                                                                                                     \
   mix_prepare_kernel<T><<<dim3(n, parts), 256, 0, stream>>>((T*)q, ldq, (const T*)k, ldk, num_heads, positions,       \
       token_segment, block_tables, bt_stride, cos_t, sin_t, half, norm, eps, (T*)cache, lay)

@@ -6,27 +6,29 @@
 // A workgroup of four (or eight) waves takes an item: up to 16 consecutive rows of one sequence that lie in
 // one chunk, and all heads, a wave a quarter (an eighth) of them.  Keys come in tiles of 16 that start at multiples of 16 of
 // the sequence's positions (a tile lies in one page; keys before the chunk are masked), so what is added
-// in which order depends on positions only.  The steps of a tile, or of two at a time:
+// in which order depends on positions only.  A tile's steps:
 //   0. the keys of the wave's key heads (once a key head, whichever of the wave's heads read it) are asked for under
-//      the products of the tiles before, their value columns behind the raw scores.
-//   1. raw scores: v_mfma_f32_16x16x32_bf16, a tile's keys as the first operand, the rows' queries as
+//      the products of the tile before, their value columns behind the raw scores.
+//   1. raw scores: v_mfma_f32_16x16x32_bf16, the tile's keys as the first operand, the rows' queries as
 //      the second; lane l then holds, for row l % 16, the keys 4 (l / 16) .. + 3: sixteen bytes of
 //      raw[head][row][key] in LDS.
 //   2. mixing in float32: the wave's heads h, s_h = sum_g T[h][g] raw_g for the lane's row and four keys.
 //      Where a wave has four heads (or a multiple) v_mfma_f32_4x4x1 does it: its sixteen blocks are the lanes'
 //      own scores, so that a lane gets its four heads' sums of one key from one instruction, in the order of g;
 //      the column of T comes out of one register for sixteen g (the instruction's broadcast of a block).  Else
-//      on the vector units, with T ([g][h]) through scalar loads.
-//   3. the softmax's running maximum and sum for each (head, row), in powers of two (the scale carries log2 e); the
-//      weights of two tiles, rounded to bfloat16, are, as they lie, the second operand of
-//   4. v_mfma_f32_16x16x32_bf16 with four keys of each tile of a value column (8 bytes of a page each) as the
-//      first: out[head][16 dims][row] a register block.
-// A single token is an item of one row.  The key tiles of an item are shared out over several workgroups where a
-// step has few items (`splits` a piece) or items of very different lengths (parts of at most `part_tiles` tiles, an
-// item as many as it needs): each leaves its running maximum, its sum and its unscaled output in float32, and a
-// second kernel joins them in the order of the parts; the sink belongs to the first.
-// What bounds it: a tile is a chain of loads, products, an exchange and exponentials under one workgroup a CU, so the
-// time is the longest workgroup's tiles times a tile's.
+//      on the vector units, with T ([g][h]) through scalar loads.  The same multiply-adds in the same order.
+//   3. the softmax's running maximum and sum for each (head, row), over the lane's four keys and the
+//      four lanes of a row; the weights rounded to bfloat16 are, as they lie, the second operand of
+//   4. v_mfma_f32_16x16x16_bf16 with four keys of a value column (8 bytes of the page) as the first:
+//      out[head][16 dims][row] a register block.
+// A single token is an item of one row.  Where a step has few items, the key tiles of an item are shared
+// out over several workgroups (`splits`): each leaves its running maximum, its sum and its unscaled
+// output in float32, and a second kernel joins them in the order of the splits; the sink belongs to the
+// first split.
+// What bounds it: a tile is a chain of loads, products, an exchange and exponentials under one workgroup a CU.  2,048
+// tokens, 32 heads over 8 of 128, with the join: 244 us with each wave reading the keys of two key heads where it has
+// one, values asked for head by head, queries from the caches and the mixing on the vector units, 180 now; 16 over 4:
+// 172 and 127; eight single tokens at contexts of 150 23 and 17.
 #include "attention_kv.h"
 
 using namespace hfee;
@@ -48,24 +50,22 @@ static_assert(H % WAVES == 0 && D % 32 == 0 && HW * D <= 512, "heads in fours or
 // the most key heads that the consecutive heads of a wave read (a wave's heads begin at a multiple of HW)
 constexpr int NKV_ANY = (HW + PER_KV - 2) / PER_KV + 1 < G ? (HW + PER_KV - 2) / PER_KV + 1 : G;
 constexpr int NKV = PER_KV % HW == 0 ? 1 : HW % PER_KV == 0 ? HW / PER_KV : NKV_ANY;
-// Two tiles at a time where a wave's registers hold them (outputs, both tiles' keys, their scores before and behind the
-// mixing, value columns, a few a head; where the estimate is over the line the compiler spills), else one.
-constexpr int NT = HW * D / 4 + 2 * (NKV * D / 8 + 8 * HW) + NKV * D / 4 + 3 * HW + 24 <= (WAVES == 8 ? 292 : 400) ? 2 : 1;
-// value columns wait in registers behind the raw scores where they fit beside the outputs and the keys of the next tiles (else
+// value columns wait in registers behind the raw scores where they fit beside the outputs and the keys of the next tile (else
 // they are asked for head by head, behind the softmax)
-constexpr bool EARLY_VALUES = HW * D / 4 + NKV * D / 4 + NT * NKV * D / 8 + 4 * HW + 48 <= (WAVES == 8 ? 256 : 384);
-constexpr bool Q_STAYS = WAVES == 4 && NT == 2;          // ... and the queries with them
+constexpr bool EARLY_VALUES = HW * D / 4 + NKV * D / 4 + 8 * HW + 48 <= (WAVES == 8 ? 256 : 384);
+// (keys a tile ahead where they are few: with 64 heads over 64 the registers they wait in were spilled)
+constexpr bool KEYS_AHEAD = WAVES == 4 || NKV * D / 8 <= 32;
+constexpr bool Q_STAYS = WAVES == 4 && HW <= 4;          // the queries in registers for all tiles
 constexpr bool MATRIX_MIX = HW % 4 == 0 && H % 16 == 0;
 // Where the queries do not fit a wave's registers beside the outputs (eight waves) they lie in LDS as operands, each wave
 // its own, if LDS holds them beside the raw scores of one tile: read again from the caches for every tile they were half of
-// what a prompt of 2,048 tokens took from there (32 heads of 128, items in halves: 181 us, 139 from LDS).
+// what a prompt of 2,048 tokens took from there.
 constexpr size_t LDS_MOST = 160 * 1024, RAW_TILE = (size_t)H * ROWS * KEYS * sizeof(float), Q_BYTES = (size_t)H * ROWS * D * sizeof(bf16_t);
 constexpr bool Q_IN_LDS = WAVES == 8 && RAW_TILE + Q_BYTES <= LDS_MOST;
-constexpr int RAW_TILES = NT == 2 && (Q_IN_LDS ? Q_BYTES : 0) + 2 * RAW_TILE <= LDS_MOST ? 2 : 1;      // whose raw scores LDS holds at a time
-constexpr size_t LDS_BYTES = (Q_IN_LDS ? Q_BYTES : 0) + RAW_TILES * RAW_TILE;
-constexpr float LOG2_E = 1.4426950408889634f;
+constexpr size_t LDS_BYTES = RAW_TILE + (Q_IN_LDS ? Q_BYTES : 0);
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -74,18 +74,12 @@ union Operand8 {
   u32x4 u;
   bf16x8 v;
 };
+union Operand4 {
+  u32x2 u;
+  s16x4 v;
+};
 
 __device__ __forceinline__ uint32_t two_bf16(float a, float b) { return (uint32_t)float_to_bf16(a) | ((uint32_t)float_to_bf16(b) << 16); }
-
-// The parts of an item of so many key tiles, and the tiles of each.
-__device__ __forceinline__ int parts_of(int tiles, int splits, int part_tiles) {
-  return part_tiles > 0 ? min(splits, (tiles + part_tiles - 1) / part_tiles) : splits;
-}
-
-__device__ __forceinline__ int tiles_of_item(const int4 item, int chunk) {
-  const int first = chunk > 0 ? item.z / chunk * chunk : 0;
-  return (item.z + item.y - 1) / KEYS - first / KEYS + 1;
-}
 
 // s[four][i][hh] += T[4 four + hh][g] raw[g] of the lane's key i for sixteen g: register t[four] holds T[4 four + hh][g] of the
 // J-th g in the lanes 4 J + hh.
@@ -104,20 +98,18 @@ __device__ __forceinline__ void mix_sixteen(f32x4 (&s)[FOURS][4], const float (&
 
 __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
     bf16_t* __restrict__ out, int64_t ld_out, const bf16_t* __restrict__ q, int64_t ldq, const bf16_t* __restrict__ cache,
-    KvLayout lay, const int* __restrict__ items, const int* __restrict__ jobs, const int* __restrict__ block_tables, int bt_stride, float scale_log2,
-    const float* __restrict__ mix_t, int chunk, int sink_mode, const float* __restrict__ sinks, int splits, int part_tiles,
+    KvLayout lay, const int* __restrict__ items, const int* __restrict__ block_tables, int bt_stride, float scale,
+    const float* __restrict__ mix_t, int chunk, int sink_mode, const float* __restrict__ sinks, int splits,
     float* __restrict__ partial_ml, float* __restrict__ partial_o) {
   extern __shared__ __attribute__((aligned(16))) char mix_lds[];
-  float (*raw)[ROWS][KEYS] = reinterpret_cast<float (*)[ROWS][KEYS]>(mix_lds);                  // [RAW_TILES * H]
-  u32x4* q_lds = reinterpret_cast<u32x4*>(mix_lds + RAW_TILES * RAW_TILE);                      // [wave][head][ks][lane]
-  const int it = jobs != nullptr ? jobs[2 * blockIdx.x] : blockIdx.x, split = jobs != nullptr ? jobs[2 * blockIdx.x + 1] : blockIdx.y;
-  const int4 item = reinterpret_cast<const int4*>(items)[it];
+  float (*raw)[ROWS][KEYS] = reinterpret_cast<float (*)[ROWS][KEYS]>(mix_lds);                  // [H]
+  u32x4* q_lds = reinterpret_cast<u32x4*>(mix_lds + RAW_TILE);                      // [wave][head][ks][lane]
+  const int4 item = reinterpret_cast<const int4*>(items)[blockIdx.x];
   const int row0 = item.x, rows = item.y, p0 = item.z;
-  const int first = chunk > 0 ? p0 / chunk * chunk : 0;
+  const int first = chunk > 0 ? p0 / chunk * chunk : 0, last = p0 + rows - 1;
   // this workgroup's share of the item's key tiles
-  const int tile0 = first / KEYS, tiles = tiles_of_item(item, chunk), parts = parts_of(tiles, splits, part_tiles);
-  if (split >= parts) return;
-  const int share = ((tiles + parts - 1) / parts + 1) & ~1;          // (whole pairs)
+  const int tile0 = first / KEYS, tiles = last / KEYS - tile0 + 1, share = (tiles + splits - 1) / splits;
+  const int split = blockIdx.y;
   const int j_begin = (tile0 + split * share) * KEYS, j_end = min(tile0 + tiles, tile0 + (split + 1) * share) * KEYS;
   const int sinking = split == 0 ? sink_mode : 0;
 
@@ -143,49 +135,27 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
   float m[HW], l[HW];
 #pragma unroll
   for (int hh = 0; hh < HW; ++hh) {
-    m[hh] = sinking == 0 ? -INFINITY : sinking == 1 ? 0.f : sinks[wave * HW + hh] * LOG2_E;
-    l[hh] = sinking == 0 || kq > 0 ? 0.f : 1.f;              // (of the lane's own keys: the sink is counted once)
+    m[hh] = sinking == 0 ? -INFINITY : sinking == 1 ? 0.f : sinks[wave * HW + hh];
+    l[hh] = sinking == 0 ? 0.f : 1.f;
 #pragma unroll
     for (int db = 0; db < DB; ++db) o[hh][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // (the second tile of a pair may lie beyond the part: masked, and its page is that of the part's last tile)
-  struct Pair {
-    int page[NT], slot[NT];
-  };
-  auto pair_at = [&](int j0) {
-    Pair at;
+  // a tile's keys are asked for when the tile before has made its weights
+  Operand8 kop[NKV][KS];
+  auto ask_keys = [&](int page, int j0) {
 #pragma unroll
-    for (int u = 0; u < NT; ++u) {
-      const int j = min(j0 + u * KEYS, j_end - KEYS);
-      at.page[u] = bt[j >> lay.page_shift];
-      at.slot[u] = j & (lay.page_size - 1);
+    for (int kv = 0; kv < NKV; ++kv) {
+      const bf16_t* kr = cache + lay.key_offset(page, min(kv0 + kv, G - 1), (j0 & (lay.page_size - 1)) + r16, kq * 8);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) kop[kv][ks].u = *reinterpret_cast<const u32x4*>(kr + ks * 32);
     }
-    return at;
   };
-  Operand8 kop[NT][NKV][KS];
-  auto ask_keys = [&](const Pair& at) {
+  Operand4 vop[EARLY_VALUES ? NKV : 1][DB];
+  auto ask_values = [&](int page, int slot0, int kvh, Operand4 (&v)[DB]) {
+    const bf16_t* vr = cache + lay.value_offset(page, kvh, slot0 + kq * 4, r16);
 #pragma unroll
-    for (int u = 0; u < NT; ++u)
-#pragma unroll
-      for (int kv = 0; kv < NKV; ++kv) {
-        const bf16_t* kr = cache + lay.key_offset(at.page[u], min(kv0 + kv, G - 1), at.slot[u] + r16, kq * 8);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) kop[u][kv][ks].u = *reinterpret_cast<const u32x4*>(kr + ks * 32);
-      }
-  };
-  // (a value operand: four keys of each of the two tiles of a column)
-  Operand8 vop[EARLY_VALUES ? NKV : 1][DB];
-  auto ask_values = [&](const Pair& at, int kvh, Operand8 (&v)[DB]) {
-    const bf16_t* v0 = cache + lay.value_offset(at.page[0], kvh, at.slot[0] + kq * 4, r16);
-    const bf16_t* v1 = cache + lay.value_offset(at.page[NT - 1], kvh, at.slot[NT - 1] + kq * 4, r16);
-#pragma unroll
-    for (int db = 0; db < DB; ++db) {
-      const u32x2 x = *reinterpret_cast<const u32x2*>(v0 + (int64_t)db * 16 * lay.page_size);
-      u32x2 y = {0u, 0u};                    // (one tile: the product's other half adds nothing)
-      if constexpr (NT == 2) y = *reinterpret_cast<const u32x2*>(v1 + (int64_t)db * 16 * lay.page_size);
-      v[db].u = u32x4{x[0], x[1], y[0], y[1]};
-    }
+    for (int db = 0; db < DB; ++db) v[db].u = *reinterpret_cast<const u32x2*>(vr + (int64_t)db * 16 * lay.page_size);
   };
   u32x4* q_mine = q_lds + (Q_IN_LDS ? wave * HW * KS * 64 + lane : 0);
   if constexpr (Q_IN_LDS) {
@@ -194,25 +164,22 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) q_mine[(hh * KS + ks) * 64] = *reinterpret_cast<const u32x4*>(q_row + hh * D + ks * 32);
   }
-  Pair here, next;
+  int page_next = 0;
   if (j_begin < j_end) {
-    here = pair_at(j_begin);
-    ask_keys(here);
+    page_next = bt[j_begin >> lay.page_shift];
+    if constexpr (KEYS_AHEAD) ask_keys(page_next, j_begin);
   }
-  for (int j0 = j_begin; j0 < j_end; j0 += NT * KEYS) {
-    const bool more = j0 + NT * KEYS < j_end;
+  for (int j0 = j_begin; j0 < j_end; j0 += KEYS) {
+    const int page = page_next, slot0 = j0 & (lay.page_size - 1);
+    const bool more = j0 + KEYS < j_end;
+    if constexpr (!KEYS_AHEAD) ask_keys(page, j0);
     // 1. raw scores of the wave's heads
-    auto put_raw = [&](int u, int hh, const f32x4& x) {
-      *reinterpret_cast<f32x4*>(&raw[u * H + wave * HW + hh][r16][kq * 4]) = x * scale_log2;
-    };
-    f32x4 made[NT][HW];
     const bf16_t* q_now = q_row;
     if constexpr (!Q_STAYS) asm volatile("" : "+v"(q_now));      // (not to be kept for all tiles: they would go to scratch memory)
 #pragma unroll
     for (int hh = 0; hh < HW; ++hh) {
-      const int kv = (wave * HW + hh) / PER_KV - kv0;
-#pragma unroll
-      for (int u = 0; u < NT; ++u) made[u][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int g = wave * HW + hh, kv = g / PER_KV - kv0;
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
         Operand8 qop;
@@ -220,160 +187,117 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
         else qop.u = *reinterpret_cast<const u32x4*>(q_now + hh * D + ks * 32);
 #pragma unroll
         for (int c = 0; c < NKV; ++c)        // (which of the wave's key heads: the same for all lanes)
-          if (NKV == 1 || c == kv) {
-#pragma unroll
-            for (int u = 0; u < NT; ++u) made[u][hh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[u][c][ks].v, qop.v, made[u][hh], 0, 0, 0);
-          }
+          if (NKV == 1 || c == kv) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kop[c][ks].v, qop.v, s, 0, 0, 0);
       }
-      if constexpr (HW > 4) {
-#pragma unroll
-        for (int u = 0; u < RAW_TILES; ++u) put_raw(u, hh, made[u][hh]);
-      }
-    }
-    if constexpr (HW <= 4) {                 // (a few heads: all products in front of the stores)
-#pragma unroll
-      for (int u = 0; u < RAW_TILES; ++u)
-#pragma unroll
-        for (int hh = 0; hh < HW; ++hh) put_raw(u, hh, made[u][hh]);
+      *reinterpret_cast<f32x4*>(&raw[g][r16][kq * 4]) = s * scale;
     }
     if constexpr (EARLY_VALUES) {
 #pragma unroll
-      for (int kv = 0; kv < NKV; ++kv) ask_values(here, min(kv0 + kv, G - 1), vop[kv]);
+      for (int kv = 0; kv < NKV; ++kv) ask_values(page, slot0, min(kv0 + kv, G - 1), vop[kv]);
     }
-    if (more) next = pair_at(j0 + NT * KEYS);
+    if (more) page_next = bt[(j0 + KEYS) >> lay.page_shift];
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     // 2. the scores that enter the softmax
-    f32x4 sc[NT][HW];
+    f32x4 sc[HW];
+    if (mix_t != nullptr) {
+      if constexpr (MATRIX_MIX) {
+        f32x4 s[FOURS][4];                   // [four heads][key of the lane][head]
 #pragma unroll
-    for (int u = 0; u < NT; ++u) {
-      const int at = RAW_TILES == 2 ? u * H : 0;
-      if (RAW_TILES == 1 && u == 1) {
-        __syncthreads();
+        for (int four = 0; four < FOURS; ++four)
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) put_raw(0, hh, made[u][hh]);
-        __syncthreads();
-      }
-      if (mix_t != nullptr) {
-        if constexpr (MATRIX_MIX) {
-          f32x4 s[FOURS][4];                 // [four heads][key of the lane][head]
+          for (int i = 0; i < 4; ++i) s[four][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int four = 0; four < FOURS; ++four)
+        for (int b = 0; b < H / 16; ++b) mix_sixteen<0>(s, mix_w[b], &raw[16 * b][r16][kq * 4]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s[four][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int four = 0; four < FOURS; ++four)
 #pragma unroll
-          for (int b = 0; b < H / 16; ++b) mix_sixteen<0>(s, mix_w[b], &raw[at + 16 * b][r16][kq * 4]);
+          for (int hh = 0; hh < 4; ++hh)
 #pragma unroll
-          for (int four = 0; four < FOURS; ++four)
-#pragma unroll
-            for (int hh = 0; hh < 4; ++hh)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) sc[u][4 * four + hh][i] = s[four][i][hh];
-        } else {
-#pragma unroll
-          for (int hh = 0; hh < HW; ++hh) sc[u][hh] = f32x4{0.f, 0.f, 0.f, 0.f};
-          const float* tw = mix_t + wave * HW;
-#pragma unroll 8
-          for (int g = 0; g < H; ++g) {
-            const f32x4 r = *reinterpret_cast<const f32x4*>(&raw[at + g][r16][kq * 4]);
-#pragma unroll
-            for (int hh = 0; hh < HW; ++hh) {
-              const float w = tw[g * H + hh];
-#pragma unroll
-              for (int i = 0; i < 4; ++i) sc[u][hh][i] = fmaf(w, r[i], sc[u][hh][i]);
-            }
-          }
-        }
+            for (int i = 0; i < 4; ++i) sc[4 * four + hh][i] = s[four][i][hh];
       } else {
 #pragma unroll
-        for (int hh = 0; hh < HW; ++hh) sc[u][hh] = *reinterpret_cast<const f32x4*>(&raw[at + wave * HW + hh][r16][kq * 4]);
+        for (int hh = 0; hh < HW; ++hh) sc[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const float* tw = mix_t + wave * HW;
+#pragma unroll 8
+        for (int g = 0; g < H; ++g) {
+          const f32x4 r = *reinterpret_cast<const f32x4*>(&raw[g][r16][kq * 4]);
+#pragma unroll
+          for (int hh = 0; hh < HW; ++hh) {
+            const float w = tw[g * H + hh];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[hh][i] = fmaf(w, r[i], sc[hh][i]);
+          }
+        }
       }
+    } else {
+#pragma unroll
+      for (int hh = 0; hh < HW; ++hh) sc[hh] = *reinterpret_cast<const f32x4*>(&raw[wave * HW + hh][r16][kq * 4]);
     }
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    // 3. the softmax: m is the running maximum, so that the largest weight is 1 and rounds to itself; the lanes of a row meet
-    // over it, and the outputs are rescaled, only where some row's has moved
-    bool seen[NT][4];
+    // 3. the running softmax of all the wave's heads (their exchanges between lanes side by side)
+    bool seen[4];
 #pragma unroll
-    for (int u = 0; u < NT; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = j0 + u * KEYS + kq * 4 + i;
-        seen[u][i] = j >= first && j <= p0 + r16 && j < j_end && r16 < rows;
-      }
-    float tmax[HW];
-    bool passed = false;
+    for (int i = 0; i < 4; ++i) {
+      const int j = j0 + kq * 4 + i;
+      seen[i] = j >= first && j <= p0 + r16 && r16 < rows;
+    }
+    float tmax[HW], psum[HW], shrink[HW];
+    Operand4 pop[HW];
 #pragma unroll
     for (int hh = 0; hh < HW; ++hh) {
       tmax[hh] = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < NT; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (seen[u][i]) tmax[hh] = fmaxf(tmax[hh], sc[u][hh][i]);
-      passed |= tmax[hh] > m[hh];
+      for (int i = 0; i < 4; ++i)
+        if (seen[i]) tmax[hh] = fmaxf(tmax[hh], sc[hh][i]);
     }
-    if (__builtin_amdgcn_ballot_w64(passed) != 0) {
 #pragma unroll
-      for (int hh = 0; hh < HW; ++hh) tmax[hh] = fmaxf(tmax[hh], __shfl_xor(tmax[hh], 16, kWave));
+    for (int hh = 0; hh < HW; ++hh) tmax[hh] = fmaxf(tmax[hh], __shfl_xor(tmax[hh], 16, kWave));
 #pragma unroll
-      for (int hh = 0; hh < HW; ++hh) {
-        const float m_new = fmaxf(m[hh], fmaxf(tmax[hh], __shfl_xor(tmax[hh], 32, kWave)));
-        const float shrink = m[hh] == -INFINITY ? 0.f : exp2f(m[hh] - m_new);      // (m_new is finite wherever m is)
-        m[hh] = m_new;
-        l[hh] *= shrink;
+    for (int hh = 0; hh < HW; ++hh) tmax[hh] = fmaxf(tmax[hh], __shfl_xor(tmax[hh], 32, kWave));
 #pragma unroll
-        for (int db = 0; db < DB; ++db) o[hh][db] *= shrink;
+    for (int hh = 0; hh < HW; ++hh) {
+      const float m_new = fmaxf(m[hh], tmax[hh]);
+      float p[4];
+      psum[hh] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[i] = seen[i] ? expf(sc[hh][i] - m_new) : 0.f;
+        psum[hh] += p[i];
       }
+      shrink[hh] = m[hh] == -INFINITY ? 0.f : expf(m[hh] - m_new);      // (m_new is finite wherever m is)
+      m[hh] = m_new;
+      pop[hh].u = u32x2{two_bf16(p[0], p[1]), two_bf16(p[2], p[3])};
     }
-    auto weights = [&](int hh) {             // of four keys of each tile
-      float p[2][4] = {};
 #pragma unroll
-      for (int u = 0; u < NT; ++u)
+    for (int hh = 0; hh < HW; ++hh) psum[hh] += __shfl_xor(psum[hh], 16, kWave);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          p[u][i] = seen[u][i] ? __builtin_amdgcn_exp2f(sc[u][hh][i] - m[hh]) : 0.f;
-          l[hh] += p[u][i];
-        }
-      Operand8 w;
-      w.u = u32x4{two_bf16(p[0][0], p[0][1]), two_bf16(p[0][2], p[0][3]), two_bf16(p[1][0], p[1][1]), two_bf16(p[1][2], p[1][3])};
-      return w;
-    };
-    // (all heads' in front of the products where they fit: 67 us a prompt at 16 heads of 128, 77 with each in front of its own)
-    constexpr bool FIRST = HW <= 4;
-    Operand8 pop[FIRST ? HW : 1];
-    if constexpr (FIRST) {
-#pragma unroll
-      for (int hh = 0; hh < HW; ++hh) pop[hh] = weights(hh);
-    }
+    for (int hh = 0; hh < HW; ++hh) psum[hh] += __shfl_xor(psum[hh], 32, kWave);
     __builtin_amdgcn_sched_barrier(0);
-    if (more) ask_keys(next);
+    if (KEYS_AHEAD && more) ask_keys(page_next, j0 + KEYS);
     // 4. the weighted values
 #pragma unroll
     for (int hh = 0; hh < HW; ++hh) {
+      l[hh] = fmaf(l[hh], shrink[hh], psum[hh]);
       const int kv = (wave * HW + hh) / PER_KV - kv0;
-      if constexpr (!EARLY_VALUES) ask_values(here, kv0 + kv, vop[0]);
-      if constexpr (!FIRST) pop[0] = weights(hh);
+      if constexpr (!EARLY_VALUES) ask_values(page, slot0, kv0 + kv, vop[0]);
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+      for (int db = 0; db < DB; ++db) {
+        const f32x4 before = o[hh][db] * shrink[hh];
 #pragma unroll
         for (int c = 0; c < (EARLY_VALUES ? NKV : 1); ++c)
           if (!EARLY_VALUES || NKV == 1 || c == kv)
-            o[hh][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop[c][db].v, pop[FIRST ? hh : 0].v, o[hh][db], 0, 0, 0);
+            o[hh][db] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vop[c][db].v, pop[hh].v, before, 0, 0, 0);
+      }
     }
-    here = next;
   }
-  // (a lane has added up its own keys' weights)
-#pragma unroll
-  for (int hh = 0; hh < HW; ++hh) l[hh] += __shfl_xor(l[hh], 16, kWave);
-#pragma unroll
-  for (int hh = 0; hh < HW; ++hh) l[hh] += __shfl_xor(l[hh], 32, kWave);
   // register i of lane l: dim 16 db + 4 (l / 16) + i of row l % 16
-  if (parts > 1) {
+  if (splits > 1) {
     if (r16 < rows) {
 #pragma unroll
       for (int hh = 0; hh < HW; ++hh) {
-        const int64_t at = (((int64_t)it * splits + split) * H + wave * HW + hh) * ROWS + r16;
+        const int64_t at = (((int64_t)blockIdx.x * splits + split) * H + wave * HW + hh) * ROWS + r16;
         if (kq == 0) {
           partial_ml[2 * at] = m[hh];
           partial_ml[2 * at + 1] = l[hh];
@@ -398,41 +322,33 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
   }
 }
 
-// grid (items, heads): out[row][head] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), the parts in their order; a thread
+// grid (items, heads): out[row][head] = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M), the splits in their order; a thread
 // has four dims of a row, and a round's parts are asked for together.
 __global__ __launch_bounds__(256) void mix_join_kernel(bf16_t* __restrict__ out, int64_t ld_out, const int* __restrict__ items,
-                                                       int chunk, int splits, int part_tiles,
-                                                       const float* __restrict__ partial_ml, const float* __restrict__ partial_o) {
+                                                       int splits, const float* __restrict__ partial_ml, const float* __restrict__ partial_o) {
   constexpr int TOGETHER = 8;
   const int4 item = reinterpret_cast<const int4*>(items)[blockIdx.x];
   const int row0 = item.x, rows = item.y, h = blockIdx.y;
-  const int parts = parts_of(tiles_of_item(item, chunk), splits, part_tiles);
-  if (parts == 1) return;                                   // (written by its only part)
   for (int e = threadIdx.x; e < rows * (D / 4); e += blockDim.x) {
     const int r = e / (D / 4), d = 4 * (e - r * (D / 4));
     const int64_t at0 = ((int64_t)blockIdx.x * splits * H + h) * ROWS + r, step = (int64_t)H * ROWS;
     float top = -INFINITY, sum = 0.f;
+    for (int s = 0; s < splits; ++s) top = fmaxf(top, partial_ml[2 * (at0 + s * step)]);
     f32x4 value = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < parts; s0 += TOGETHER) {
+    for (int s0 = 0; s0 < splits; s0 += TOGETHER) {
       f32x4 o[TOGETHER];
-      float ms[TOGETHER], ls[TOGETHER], most = top;
+      float ms[TOGETHER], ls[TOGETHER];
 #pragma unroll
-      for (int j = 0; j < TOGETHER; ++j) {                  // past the end: the last part again, which is not added
-        const int64_t at = at0 + min(s0 + j, parts - 1) * step;
+      for (int j = 0; j < TOGETHER; ++j) {                  // past the end: the last split again, which is not added
+        const int64_t at = at0 + min(s0 + j, splits - 1) * step;
         ms[j] = partial_ml[2 * at];
         ls[j] = partial_ml[2 * at + 1];
         o[j] = *reinterpret_cast<const f32x4*>(partial_o + at * D + d);
       }
 #pragma unroll
-      for (int j = 0; j < TOGETHER; ++j) most = fmaxf(most, ms[j]);
-      const float shrink = top == -INFINITY ? 0.f : exp2f(top - most);
-      sum *= shrink;
-      value *= shrink;
-      top = most;
-#pragma unroll
       for (int j = 0; j < TOGETHER; ++j) {
-        if (s0 + j >= parts || ms[j] == -INFINITY) continue;          // (a share in which the row saw nothing)
-        const float w = exp2f(ms[j] - most);
+        if (s0 + j >= splits || ms[j] == -INFINITY) continue;         // (a share in which the row saw nothing)
+        const float w = expf(ms[j] - top);
         sum = fmaf(ls[j], w, sum);
 #pragma unroll
         for (int i = 0; i < 4; ++i) value[i] = fmaf(o[j][i], w, value[i]);
@@ -454,15 +370,12 @@ HFEE_API int hfee_attention_mix_bf16_dim() { return D; }
 // items: int32 [count][4] on the device: first row, rows (1..16), first position, block-table row; the rows
 // of an item are consecutive positions of one sequence within one chunk.  mix_t: float32 [H][H], the
 // mixing matrix transposed (mix_t[g][h] multiplies head g's raw score into head h's), or null.
-// splits > 1: every item's key tiles over so many workgroups, or, with part_tiles > 0, over so many as parts of part_tiles
-// tiles take (`splits` at most, the parts then longer; each a whole number of pairs of tiles).  jobs: null, or int32
-// [job_count][2] on the device, every (item, part) that there is, in the order in which the workgroups are to start.  partial: count * splits * H * 16 * (D + 2) float32.
+// splits > 1: every item's key tiles over so many workgroups; partial: count * splits * H * 16 * (D + 2) float32.
 HFEE_API int hfee_attention_mix_bf16(void* out, int64_t ld_out, const void* q, int64_t ldq, const void* cache,
-                                     const int* items, int count, const int* jobs, int job_count,
-                                     const int* block_tables, int bt_stride, int kv_heads, int page_size, float scale,
-                                     const float* mix_t, int chunk, int sink_mode,
-                                     const float* sinks, int splits, int part_tiles, float* partial,
-                                     int64_t partial_floats, hipStream_t stream) {
+                                     const int* items, int count, const int* block_tables, int bt_stride, int kv_heads,
+                                     int page_size, float scale, const float* mix_t, int chunk, int sink_mode,
+                                     const float* sinks, int splits, float* partial, int64_t partial_floats,
+                                     hipStream_t stream) {
   HFEE_REQUIRE(count >= 0, "attention_mix_bf16: bad item count");
   if (count == 0) return 0;
   HFEE_REQUIRE(kv_heads == G, "attention_mix_bf16: compiled for %d key heads, called with %d", G, kv_heads);
@@ -471,11 +384,10 @@ HFEE_API int hfee_attention_mix_bf16(void* out, int64_t ld_out, const void* q, i
   HFEE_REQUIRE(ldq >= (int64_t)H * D && ld_out >= (int64_t)H * D && ldq % 8 == 0 && ld_out % 4 == 0 &&
                (uintptr_t)q % 16 == 0 && (uintptr_t)out % 8 == 0 && (uintptr_t)cache % 16 == 0,
                "attention_mix_bf16: q and out rows too short or not aligned");
-  HFEE_REQUIRE(splits >= 1 && splits <= 65535 && part_tiles >= 0, "attention_mix_bf16: 1 to 65535 splits");
+  HFEE_REQUIRE(splits >= 1 && splits <= 65535, "attention_mix_bf16: 1 to 65535 splits");
   const int64_t places = (int64_t)count * splits * H * ROWS;
   HFEE_REQUIRE(splits == 1 || (partial != nullptr && partial_floats >= places * (D + 2) && (uintptr_t)partial % 16 == 0),
                "attention_mix_bf16: the splits need %lld float32 of scratch", (long long)(places * (D + 2)));
-  HFEE_REQUIRE(jobs == nullptr || (part_tiles > 0 && job_count >= count), "attention_mix_bf16: jobs are the parts of every item");
   KvLayout lay;
   if (make_kv_layout(&lay, kv_heads, D, D, page_size)) return 1;
   float* partial_o = partial;                               // [places][D], then [places][2]
@@ -486,13 +398,12 @@ HFEE_API int hfee_attention_mix_bf16(void* out, int64_t ld_out, const void* q, i
     HFEE_REQUIRE(e == hipSuccess, "attention_mix_bf16: cannot raise the LDS limit: %s", hipGetErrorString(e));
     raised = true;
   }
-  mix_attend_bf16_kernel<<<jobs != nullptr ? dim3(job_count) : dim3(count, splits), WAVES * 64, LDS_BYTES, stream>>>(
-      (bf16_t*)out, ld_out, (const bf16_t*)q, ldq, (const bf16_t*)cache, lay, items, jobs, block_tables, bt_stride, scale * LOG2_E, mix_t,
-      chunk, sink_mode, sinks, splits, part_tiles, partial_ml, partial_o);
+  mix_attend_bf16_kernel<<<dim3(count, splits), WAVES * 64, LDS_BYTES, stream>>>(
+      (bf16_t*)out, ld_out, (const bf16_t*)q, ldq, (const bf16_t*)cache, lay, items, block_tables, bt_stride, scale, mix_t, chunk,
+      sink_mode, sinks, splits, partial_ml, partial_o);
   HFEE_CHECK_LAUNCH("attention_mix_bf16");
   if (splits > 1) {
-    mix_join_kernel<<<dim3(count, H), 256, 0, stream>>>((bf16_t*)out, ld_out, items, chunk, splits, part_tiles,
-                                                           partial_ml, partial_o);
+    mix_join_kernel<<<dim3(count, H), 256, 0, stream>>>((bf16_t*)out, ld_out, items, splits, partial_ml, partial_o);
     HFEE_CHECK_LAUNCH("attention_mix_join");
   }
   return 0;

@@ -204,6 +204,26 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+// The sum of squares of a head that lies in fours in `group` neighbouring lanes, in the order of a wave whose lane l has the
+// head's values l, l + 64, ... and adds its lanes up with wave_sum: the same bits.
+__device__ __forceinline__ float head_squares(const float (&y)[4], int group) {
+  const int lane = threadIdx.x & 63, base = lane & ~(group - 1), place = lane & (group - 1) & 15;
+  float part[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    part[i] = 0.f;
+    for (int k = 0; k < group; k += 16) {
+      const float v = __shfl(y[i], base + k + (group < 16 ? lane & (group - 1) : place), kWave);
+      part[i] = fmaf(v, v, part[i]);
+    }
+  }
+  for (int off = (group < 16 ? group : 16) >> 1; off > 0; off >>= 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part[i] += __shfl_xor(part[i], off, kWave);
+  }
+  return (part[0] + part[2]) + (part[1] + part[3]);
+}
+
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));

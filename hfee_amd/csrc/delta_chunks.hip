@@ -139,7 +139,11 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(InputArgs p) {
       y[i] = mine ? sum / (1.0f + expf(-sum)) : 0.f;
       ss = fmaf(y[i], y[i], ss);
     }
-    for (int off = group >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+    if (p.decay_width == 1) {
+      for (int off = group >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+    } else {
+      ss = head_squares(y, group);
+    }
     if (unit) {
       const float inv = factor / sqrtf(ss + p.unit_eps);
 #pragma unroll

@@ -7,7 +7,6 @@ from __future__ import annotations
 
 import ctypes
 
-import numpy as np
 import torch
 
 from . import lib
@@ -1503,45 +1502,15 @@ def attention_mix_partial_words(num_items: int, num_heads: int, dim: int, splits
     return num_items * splits * num_heads * ATTENTION_MIX_ROWS * (dim + 2) if splits > 1 else 0
 
 
-def attention_mix_parts(items, chunk: int, most_splits: int, cus: int | None = None) -> tuple:
-    """How the key tiles of `attention_mix_bf16`'s items (as it takes them, on the host) are shared out: (splits, part_tiles,
-    jobs int32 [number, 2]).  A workgroup has a CU to itself and a tile takes it about 3.4 us
-    (32 heads of 128), so a launch is as long as the longest part, or as the CUs' share of all tiles and half a part where there
-    are more parts than CUs; a part of an item of several costs the 0.1 us that its float32 outputs take to memory and
-    back.  Parts are whole pairs of tiles; the longest start first."""
-    items = np.asarray(items, dtype=np.int64).reshape(-1, 4)
-    first = items[:, 2] // chunk * chunk if chunk else np.zeros(len(items), dtype=np.int64)
-    tiles = (items[:, 2] + items[:, 1] - 1) // 16 - first // 16 + 1          # (as the kernel counts them)
-    longest = int(tiles.max())
-    part = np.arange(2, longest + 2, 2)
-    part = part[-(-longest // part) <= max(1, most_splits)]
-    parts = -(-tiles[:, None] // part[None, :])
-    number = parts.sum(axis=0)
-    cus = cus or compute_units()
-    cost = 3.4 * np.maximum(np.minimum(part, longest), tiles.sum() / cus + np.where(number > cus, part / 2, 0)) \
-        + 0.1 * np.where(parts > 1, parts, 0).sum(axis=0)
-    best = int(cost.argmin())
-    counts = parts[:, best]
-    owner = np.repeat(np.arange(len(tiles)), counts)
-    jobs = np.stack([owner, np.arange(len(owner)) - np.repeat(np.cumsum(counts) - counts, counts)], axis=1)
-    order = np.argsort(-(tiles / counts)[owner], kind="stable")
-    return int(counts.max()), int(part[best]), jobs[order].astype(np.int32)
-
-
 def attention_mix_bf16(out, q, cache_layer, items, block_tables, num_heads: int, kv_heads: int, dim: int, page_size: int,
-                       scale: float, mix_t=None, chunk: int = 0, sink=None, splits: int = 1, partial=None, part_tiles: int = 0,
-                       jobs=None):
+                       scale: float, mix_t=None, chunk: int = 0, sink=None, splits: int = 1, partial=None):
     """`attention_mix` on the matrix cores, bfloat16.  items: int32 [count, 4] on the device (first row,
     rows (1 to 16), first position, block-table row), the rows of an item consecutive positions of one
     sequence within one chunk; mix_t: the mixing matrix transposed, float32 [heads, heads]
     (score_h = sum_g mix_t[g, h] score_g), or None.  splits > 1: the key tiles of every item are shared out
     over so many workgroups, which leave their parts in `partial` (float32, `attention_mix_partial_words`)
-    for a joining kernel; with part_tiles > 0 over as many as parts of so many tiles of 16 keys take, `splits` at
-    most.  jobs: `attention_mix_parts`' for the items, int32 on the device: the parts in the order in which they start."""
-    _gpu(out, q, cache_layer, items, block_tables, mix_t, partial, jobs)
-    if jobs is not None:
-        _check(jobs.dtype == torch.int32 and jobs.dim() == 2 and jobs.shape[1] == 2 and jobs.is_contiguous() and part_tiles > 0,
-               "attention_mix: jobs must be [number, 2] int32, with part_tiles")
+    for a joining kernel."""
+    _gpu(out, q, cache_layer, items, block_tables, mix_t, partial)
     if partial is not None:
         _check(partial.dtype == torch.float32 and partial.is_contiguous(), "attention_mix: float32 partial buffer expected")
     n, w, ldq = _rows2d(q, "attention_mix q")
@@ -1566,9 +1535,8 @@ def attention_mix_bf16(out, q, cache_layer, items, block_tables, num_heads: int,
         sinks, mode = sink, 2
     lib.attention_mix_bf16(num_heads, kv_heads, dim).call(
         "hfee_attention_mix_bf16", _ptr(out), ldo, _ptr(q), ldq, _ptr(cache_layer), _ptr(items), items.shape[0],
-        _ptr(jobs), 0 if jobs is None else jobs.shape[0], _ptr(block_tables), block_tables.stride(0), kv_heads, page_size,
-        float(scale), _ptr(mix_t), int(chunk), mode,
-        _ptr(sinks), int(splits), int(part_tiles), _ptr(partial), 0 if partial is None else partial.numel(), _stream())
+        _ptr(block_tables), block_tables.stride(0), kv_heads, page_size, float(scale), _ptr(mix_t), int(chunk), mode,
+        _ptr(sinks), int(splits), _ptr(partial), 0 if partial is None else partial.numel(), _stream())
 
 
 # ------------------------------------------------ mixers with a state of fixed size a request

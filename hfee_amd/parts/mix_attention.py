@@ -29,7 +29,7 @@ from .base import LazyNorm, Mixer, lookup, register_mixer
 from .kv_attention import product, tiles_of
 
 _WORKGROUPS_WANTED = 256        # items split their keys until about this many workgroups run (one a CU)
-_MOST_SPLITS = 16
+_MOST_SPLITS = 8
 _PARTIAL_LIMIT = 64 << 20       # float32 words of the splits' parts
 _LAYOUT = "by key head: the keys as scored by slot, then the keys as projected by dimension"
 
@@ -116,12 +116,6 @@ class MixedAttention(Mixer):
                 items.append((seg.row0 + off, room, p, s))
                 off += room
         plan.add(self.items_key, np.asarray(items, dtype=np.int32).reshape(-1, 4))
-        # (steps of single tokens are recorded: how their keys are shared out must not follow positions)
-        if any(seg.length > 1 for seg in plan.segments):
-            most = 2 * _PARTIAL_LIMIT // ops.attention_mix_partial_words(len(items), self.num_heads, self.dim, 2)
-            splits, part, jobs = ops.attention_mix_parts(items, self.chunk, min(_MOST_SPLITS, most))
-            plan.host[self.items_key] = (splits, part)
-            plan.add(self.items_key + ".jobs", jobs)
 
     def forward_add(self, ctx, x, h, cache_layer: int, writes_cache: bool):
         hn = h.tensor() if isinstance(h, LazyNorm) else h
@@ -148,18 +142,15 @@ class MixedAttention(Mixer):
             # table's whole width, so that a replay runs what was recorded)
             span = self.chunk or ctx.host.get("graph.max_context", ctx.max_position + 1)
             count = items.shape[0]
-            if self.items_key in ctx.host:
-                (splits, part), jobs = ctx.host[self.items_key], ctx.extra[self.items_key + ".jobs"]
-            else:
-                splits, part, jobs = max(1, min(-(-span // 16) // 2, _WORKGROUPS_WANTED // count, _MOST_SPLITS)), 2, None
-                while splits > 1 and ops.attention_mix_partial_words(count, H, D, splits) > _PARTIAL_LIMIT:
-                    splits -= 1
+            splits = max(1, min(-(-span // 16) // 4, _WORKGROUPS_WANTED // count, _MOST_SPLITS))
+            while splits > 1 and ops.attention_mix_partial_words(count, H, D, splits) > _PARTIAL_LIMIT:
+                splits -= 1
             partial = None
             if splits > 1:
                 partial = ctx.workspace.flat("mixed_attention.partial", ops.attention_mix_partial_words(count, H, D, splits),
                                              torch.float32)
             ops.attention_mix_bf16(att, q, cache, items, tables, H, G, D, ctx.page_size, self.scale, mix_t=self.mix_t,
-                                   chunk=self.chunk, sink=sink, splits=splits, partial=partial, part_tiles=part, jobs=jobs)
+                                   chunk=self.chunk, sink=sink, splits=splits, partial=partial)
         else:
             ops.attention_mix(att, q, cache, ctx.positions, ctx.token_segment, tables, H, G, D, ctx.page_size, self.scale,
                               mix=self.mix, chunk=self.chunk, sink=sink)

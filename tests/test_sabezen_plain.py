@@ -102,24 +102,3 @@ def test_the_sink_takes_its_share():
     # the first token sees its own key only: its weight is e^s / (1 + e^s)
     assert float(far_away[0].abs().max()) < float(away[0].abs().max()) < float(towards[0].abs().max())
     assert float(far_away[0].abs().max()) < 1e-9 and float(towards[0].abs().max()) > 0.9 * float(k[0].abs().max())
-
-
-def test_parts_of_mixed_attention_cover_every_tile():
-    """Every part of every item is a job once, no item has more than its share of the splits, and a part of the size that was
-    chosen holds the item's tiles as the kernel counts them."""
-    from hfee_amd.kernels import ops
-    rng = np.random.default_rng(0)
-    for chunk in (0, 16, 88, 1024):
-        for count, most in ((1, 16), (7, 1), (64, 3), (400, 16)):
-            items = []
-            for i in range(count):
-                p = int(rng.integers(0, 3000))
-                items.append((0, min(int(rng.integers(1, 17)), (chunk - p % chunk) if chunk else 16), p, i))
-            splits, part, jobs = ops.attention_mix_parts(items, chunk, most, cus=256)
-            assert part % 2 == 0 and 1 <= splits <= most
-            want = set()
-            for i, (_, rows, p, _) in enumerate(items):
-                tiles = (p + rows - 1) // 16 - (p // chunk * chunk if chunk else 0) // 16 + 1
-                want |= {(i, s) for s in range(min(splits, -(-tiles // part)))}
-                assert -(-tiles // part) <= splits
-            assert sorted(map(tuple, jobs.tolist())) == sorted(want)

@@ -87,7 +87,8 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(InputArgs p) {
     if (d >= width) return;
     const float rate = -expf(p.a_log[d / p.decay_width]);          // (the decays of a head are whole fours)
     float bias[4], z[TT][4];
-    load4<float>(bias, p.dt_bias + d);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bias[i] = p.dt_bias[d + i];          // (a model's own tensor: it may begin at any number)
 #pragma unroll
     for (int j = 0; j < TT; ++j) load4<T>(z[j], (const T*)p.a + (int64_t)(t0 + (j < count ? j : 0)) * p.lda + d);
 #pragma unroll
@@ -512,7 +513,7 @@ HFEE_API int hfee_delta_inputs(float* y, int64_t ldy, float* decay, float* beta,
   HFEE_REQUIRE(ldx % 4 == 0 && ldx >= channels && ldy % 4 == 0 && ldy >= channels &&
                (((uintptr_t)y | (uintptr_t)x | (uintptr_t)state) & 15) == 0, "delta_inputs: rows must be aligned");
   HFEE_REQUIRE(decay_width == 1 || (decay_width > 0 && decay_width % 4 == 0 && lda % 4 == 0 &&
-                                    (((uintptr_t)a | (uintptr_t)decay | (uintptr_t)dt_bias) & 15) == 0),
+                                    (((uintptr_t)a | (uintptr_t)decay) & 15) == 0),
                "delta_inputs: decays a channel come in aligned fours");
   HFEE_REQUIRE(lda >= (int64_t)heads * decay_width, "delta_inputs: the decays' rows are too short");
   if (n == 0) return 0;

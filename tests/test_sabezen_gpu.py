@@ -359,6 +359,26 @@ def test_inputs_with_decays_a_channel_in_one_launch(dtype, lengths, D):
         assert torch.equal(fours, wide), kind
 
 
+@pytest.mark.parametrize("per_channel", [True, False])
+@pytest.mark.parametrize("at", [0, 1, 2, 7])
+def test_inputs_whose_bias_begins_at_any_number(at, per_channel):
+    """The decays' bias is a model's own tensor, which may be a view of a larger one: where it begins moves no bit."""
+    from hfee_amd.kernels import ops
+    H, D, n, K = 6, 16, 5, 4
+    C, W, g = 3 * H * D, H * D if per_channel else H, torch.Generator().manual_seed(at)
+    rand = lambda *shape: torch.randn(*shape, generator=g).cuda()      # noqa: E731
+    proj, step, taps, a_log = rand(n, C + 8), rand(n, W), rand(C, K), rand(H)
+    bias, held = rand(W), torch.full((W + 8,), float("nan"), device="cuda")
+    held[at:at + W] = bias
+    decays = []
+    for b in (bias, held[at:at + W]):
+        y, decay, beta = (torch.full((n, w), float("nan"), device="cuda") for w in (C, W, H))
+        ops.delta_inputs(y, decay, beta, proj[:, :C], step, proj[:, C:C + H], torch.zeros(2, K - 1, C, device="cuda"), taps, b, a_log,
+                         i32([0] * n), i32([0]), i32([1]), H * D, D, H, 1e-6, 0.5, keep=False)
+        decays.append(decay)
+    assert torch.equal(*decays) and bool(torch.isfinite(decays[0]).all())
+
+
 @pytest.mark.parametrize("rule", ["delta", "decay_add"])
 @pytest.mark.parametrize("H,G,D,V", [(4, 2, 8, 16), (3, 3, 20, 12), (2, 1, 33, 70)])
 def test_linear_scan_in_portions(rule, H, G, D, V):

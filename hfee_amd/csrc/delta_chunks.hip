@@ -7,7 +7,7 @@
 // decays exp(-exp(A_h) softplus(a + bias)), one a head or one a key channel, and writing strengths sigmoid(b); in a step of
 // single tokens also the convolutions' state.  (2,048 tokens of 6,144 channels with decays a channel,
 // 16 heads of 128: 36 us, where a launch a mechanism, a value a thread, took 82 for the convolution and 20 for the decays alone;
-// eight single tokens: 5 us for six launches' 29.)
+// eight single tokens: 4 us for six launches' 29.)
 //
 // delta_chunks: portions of many tokens in chunks of 64 on the float32 matrix instructions (recurrent.hip, rule 1, walks
 // token by token).  With t and j counting from a chunk's first token, S the state that comes into the chunk, L its tokens,
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void delta_inputs_kernel(InputArgs p) {
     }
     if (p.decay_width == 1) {
       for (int off = group >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
-    } else {
+    } else if (__any(unit)) {                  // (heads do not reach over waves)
       ss = head_squares(y, group);
     }
     if (unit) {
@@ -521,7 +521,11 @@ HFEE_API int hfee_delta_inputs(float* y, int64_t ldy, float* decay, float* beta,
                     n, channels, qk_width, dim, heads, keep, decay_width, unit_eps, q_factor};
   const int columns = (channels / 4 + 255) / 256 + (decay_width > 1 ? (heads * decay_width / 4 + 255) / 256 : 0) + 1;
   HFEE_REQUIRE(columns <= 65535, "delta_inputs: too many channels");
-  const bool few = n <= 64;
+  // A token a workgroup, or eight, which share what came before them but are walked one after the other.  With decays a channel
+  // (whose sums of squares are the longer way, head_squares) eight win from where one fills the chip some times over: 4 heads of
+  // 256 at 100 tokens 20.5 us by eight, 7.6 by one, at 2,048 27.5 and 26.5; 16 of 128 with values of 256 at 600 tokens 22.6 and 22.0,
+  // at 2,048 48 and 53 (the state's launch included).
+  const bool few = n <= 64 || (decay_width > 1 && (int64_t)n * columns <= 8192);
 #define LAUNCH(T, K)                                                                                                 \
   do {                                                                                                               \
     if (few) delta_inputs_kernel<T, K, 1><<<dim3(n, columns), 256, 0, stream>>>(p);                                  \

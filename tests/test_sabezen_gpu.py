@@ -317,11 +317,11 @@ def test_mixed_attention_over_several_workgroups(H, G, D):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("lengths", [(1,), (1, 1, 1), (9, 1, 2), (70, 17)])
+@pytest.mark.parametrize("lengths", [(1,), (1, 1, 1), (9, 1, 2), (70, 17), (2755, 17, 3)])
 @pytest.mark.parametrize("D", [4, 32, 128, 256])
 def test_inputs_with_decays_a_channel_in_one_launch(dtype, lengths, D):
     """Decays a channel beside the convolution, the unit vectors and the strengths, to the bit what a launch a mechanism gives
-    (values by one, as odd widths have them)."""
+    (values by one, as odd widths have them); a token a workgroup, and of the many tokens eight."""
     from hfee_amd.kernels import ops
     dt = getattr(torch, dtype)
     H, G, V, K = 6, 2, 24, 4

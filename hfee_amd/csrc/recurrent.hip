@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void scan_gate_kernel(float* __restrict__ out,
   out[t * ldo + c] = gate_value(v, c, per_head, head_width, mode, number, first_columns);
 }
 
-// The same for rows of whole aligned fours, four values a thread (2,048 rows of 8,192 columns, a cast: 32 -> 22 us).
+// The same for rows of whole aligned fours, four values a thread, where there are many (see kGateFours).
 template <typename T>
 __global__ __launch_bounds__(256) void scan_gate_fours_kernel(float* __restrict__ out, int64_t ldo, const T* __restrict__ z,
                                                               int64_t ldz, const float* __restrict__ bias,
@@ -897,7 +897,11 @@ HFEE_API int hfee_scan_gate(float* out, int64_t ldo, const void* z, int64_t ldz,
   HFEE_REQUIRE(mode != 1 || number > 0.f, "scan_gate: tau must be positive");
   if (n == 0) return 0;
   dim3 grid(n, (width + 255) / 256);
-  const bool fours = width % 4 == 0 && ldo % 4 == 0 && ldz % 4 == 0 && (uintptr_t)out % 16 == 0 &&
+  // Four values a thread cost four of the functions one after the other, which pays where what counts is the bytes: a cast of 2,048
+  // rows of 8,192 29.1 -> 16.8 us, of 1,024 5.3 -> 4.3, softplus of these 9.1 -> 8.9; but 600 rows of 1,024 3.4 -> 3.6 (SiLU) and
+  // 4.4 -> 5.0 (softplus), 8 rows 3.0 -> 3.8.
+  constexpr int64_t kGateFours = 1 << 21;
+  const bool fours = (int64_t)n * width >= kGateFours && width % 4 == 0 && ldo % 4 == 0 && ldz % 4 == 0 && (uintptr_t)out % 16 == 0 &&
                      (uintptr_t)z % (dtype == 0 ? 16 : 8) == 0;
   dim3 grid4(n, (width / 4 + 255) / 256);
   if (dtype == 0 && fours)

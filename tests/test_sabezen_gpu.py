@@ -359,6 +359,22 @@ def test_inputs_with_decays_a_channel_in_one_launch(dtype, lengths, D):
         assert torch.equal(fours, wide), kind
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("n,width", [(512, 4096), (2049, 1028)])
+def test_gates_of_many_values_in_fours(dtype, n, width):
+    """Four values a thread give what one gives (rows that are no aligned fours go one by one), through every function."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device="cuda").manual_seed(n)
+    z = (torch.randn(n, width, device="cuda", generator=g) * 4).to(getattr(torch, dtype))
+    bias, a_log = torch.randn(width, device="cuda", generator=g), torch.randn(width // 4, device="cuda", generator=g)
+    for kind, kw in (("cast", dict(number=0.3, first_columns=width // 2 + 1)), ("silu", {}), ("sigmoid", {}), ("softplus", dict(bias=bias)),
+                     ("root_sigmoid", dict(number=16.0, bias=bias)), ("step_decay", dict(bias=bias, per_head=a_log, head_width=4))):
+        fours, ones = torch.zeros(n, width, device="cuda"), torch.zeros(n, width + 1, device="cuda")[:, :width]
+        ops.scan_gate(fours, z, kind, **kw)
+        ops.scan_gate(ones, z, kind, **kw)
+        assert torch.equal(fours, ones) and int((fours != 0).sum()) > n * width // 2, kind
+
+
 @pytest.mark.parametrize("per_channel", [True, False])
 @pytest.mark.parametrize("at", [0, 1, 2, 7])
 def test_inputs_whose_bias_begins_at_any_number(at, per_channel):

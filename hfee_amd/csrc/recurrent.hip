@@ -10,9 +10,9 @@
 //                                     (b_t the step size a head; with `decay_per_head` a_t is one number a head)
 //
 // `linear_scan` walks the tokens that a step brings for a request one after the other, from the
-// state that the steps before left in the request's slot, and leaves the new state there: a
-// portion of a prompt and a single token are the same kernel, and a token's result does not
-// depend on where its prompt was cut.  A wave owns four columns of S, a lane a sixteenth of the rows of
+// state that the steps before left in the request's slot, and leaves the new state there: single
+// tokens (a kernel of their own where a step has no other) add in the order of a portion's, so that a token's
+// result does not depend on where its prompt was cut.  A wave owns four columns of S, a lane a sixteenth of the rows of
 // one of them; the sixteen lanes of a column add their parts up in a fixed order.  In memory the state of a
 // head lies in blocks of four columns, each in the order in which a wave's lanes hold it.
 //
@@ -160,8 +160,11 @@ __global__ __launch_bounds__(256) void scan_gate_fours_kernel(float* __restrict_
 // of 16 bytes a lane is 256 bytes in a row; with a lane's eight rows in a row every second bank stood idle); a block's
 // tokens are one straight piece of code, in which the sum that a token's value waits for runs beside the sum of the
 // token before; a block's results leave in one store a wave instead of one a token, and its numbers come in loads of
-// sixteen bytes where the rows allow.  One request, 16 heads of 128 x 256, 2,048 tokens: rule 1 704 -> 309 us, rule 0 633 ->
-// 248; eight requests of 100 tokens 152 -> 92 and 137 -> 77 (81 ns a token and workgroup, what the LDS reads take alone).
+// sixteen bytes where the rows allow.  One request, 16 heads of 128 x 256, 2,048 tokens: rule 1 705 -> 287 us, rule 0 634 ->
+// 236; eight requests of 100 tokens 134 -> 85 and 120 -> 75.  Portions of less than a block are one, and what a thread has to
+// know of its loads is kept to a few registers (one decay a head, rows that are no fours: 24 addresses a lane took the third
+// workgroup a CU): eight requests of 5 tokens, 64 heads of 128 x 64 with rule 2 and a decay a head, 16.7 -> 15.3 (22.5 with
+// both), 32 of 9 68 -> 54 (85), 600 tokens of one 198 -> 95.
 constexpr int kScanParts = 16, kScanColumns = 4, kScanWaves = 4;
 
 typedef float scan_f32x4 __attribute__((ext_vector_type(4)));
@@ -371,6 +374,9 @@ __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
   constexpr int FOURS = Sh::PER_THREAD / 4;                          // WHOLE: loads of sixteen bytes a thread and block
   scan_f32x4 fours[WHOLE ? FOURS : 1];
   float wide[WHOLE ? 1 : Sh::PER_THREAD], narrow = 0.f, strength = 0.f;
+  // (a token's row is one or more waves' where it fills them: then its address is the same for a wave)
+  const int64_t decay_column = decay_per_head ? (int64_t)h : (int64_t)h * D;
+  const int line = Sh::DP >= THREADS ? 0 : Sh::DP % 64 == 0 ? __builtin_amdgcn_readfirstlane(tid / Sh::DP) : tid / Sh::DP;
   // The block of tokens that begins at `first`, into registers.  No load stands under a condition (past the portion's end
   // it brings the last token again, past a row's end its last number), and what must not be used is left out by `put`:
   // under a branch the compiler waits for everything outstanding in front of it, the last block's results included.
@@ -389,12 +395,11 @@ __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
     } else {
 #pragma unroll
       for (int r = 0; r < Sh::PER_THREAD; ++r) {
-        const int e = tid + r * THREADS;
-        const int which = e / (TB * Sh::DP), rest = e - which * (TB * Sh::DP);
-        const int t = rest / Sh::DP, d = min(rest - t * Sh::DP, D - 1);
+        constexpr int ROUNDS = TB * Sh::DP / THREADS, LINES = THREADS > Sh::DP ? THREADS / Sh::DP : 1, PIECES = Sh::DP > THREADS ? Sh::DP / THREADS : 1;
+        const int which = r / ROUNDS, t = r % ROUNDS / PIECES * LINES + line, d = min(r % PIECES * THREADS + tid % Sh::DP, D - 1);
         const int64_t row = row0 + min(first + t, len - 1);
         wide[r] = which == 0 ? k[row * ldk + (int64_t)g * D + d] : which == 1 ? q[row * ldq + (int64_t)g * D + d]
-                                                                              : decay[row * ldd + (decay_per_head ? (int64_t)h : (int64_t)h * D + d)];
+                                                                              : decay[row * ldd + decay_column + (decay_per_head ? 0 : d)];
       }
     }
     const int column = min((int)blockIdx.x * Sh::COLUMNS + tid % Sh::COLUMNS, V - 1);
@@ -446,10 +451,38 @@ __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
     o = o0 + o1;
   };
 
+  // A block that is not full.  Lane `part` gets the result of the block's token `part`.
+  auto part_block = [&](const float* buffer, int count) {
+    const float* values = buffer + Sh::WIDE + ((tid >> 6) * kScanColumns + w.c) * TB;
+    const float* strengths = buffer + Sh::WIDE + TB * Sh::COLUMNS;
+    float kept = 0.f;
+    for (int t = 0; t < count; ++t) {
+      ScanToken<DPT> now;
+      now.read(buffer, t, part);
+      float u = values[t], o;
+      if constexpr (RULE == 1) {
+        float p;
+        decays(now, p);
+        u = strengths[t] * (u - column_sum(p));
+      }
+      if constexpr (RULE == 2) u = strengths[t] * u;
+      writes(now, u, o);
+      o = column_sum(o);
+      kept = part == t ? o : kept;
+    }
+    return kept;
+  };
+
   ask(0);
   put(lds);
   __syncthreads();
-  for (int first = 0, turn = 0;; first += TB, turn ^= 1) {
+  // (a portion of one block asks for none behind it)
+  const bool one_block = len < TB;
+  if (one_block) {
+    const float kept = part_block(lds, len);
+    if (w.live && part < len) out[(int64_t)(row0 + part) * ldo + (int64_t)h * V + w.col] = kept;
+  }
+  for (int first = 0, turn = 0; !one_block; first += TB, turn ^= 1) {
     const float* buffer = lds + turn * Sh::BUFFER;
     const float* values = buffer + Sh::WIDE + ((tid >> 6) * kScanColumns + w.c) * TB;
     const float* strengths = buffer + Sh::WIDE + TB * Sh::COLUMNS;
@@ -491,20 +524,7 @@ __global__ __launch_bounds__(kScanWaves * 64) void linear_scan_kernel(
         kept = part == t ? o : kept;
       }
     } else {
-      for (int t = 0; t < count; ++t) {
-        ScanToken<DPT> now;
-        now.read(buffer, t, part);
-        float u = values[t], o;
-        if constexpr (RULE == 1) {
-          float p;
-          decays(now, p);
-          u = strengths[t] * (u - column_sum(p));
-        }
-        if constexpr (RULE == 2) u = strengths[t] * u;
-        writes(now, u, o);
-        o = column_sum(o);
-        kept = part == t ? o : kept;
-      }
+      kept = part_block(buffer, count);
     }
     float* mine = out + (int64_t)(row0 + min(first + part, len - 1)) * ldo + (int64_t)h * V + w.col;
     if (first + TB >= len) {

@@ -497,6 +497,30 @@ def test_linear_scan_around_its_blocks(rule, D, V, pad):
     assert float(state[4].abs().sum()) == 0.0
 
 
+@pytest.mark.parametrize("rule", ["delta", "decay_add", "scaled_add"])
+@pytest.mark.parametrize("D", [12, 20, 64, 96, 128, 256, 400, 512])
+def test_linear_scan_with_a_decay_a_head(rule, D):
+    """One decay a head, of each token or the same for all, gives to the bit what it gives spelled out a channel: portions of a
+    few tokens, which are one block and ask for none behind it, and around the blocks of every key size."""
+    from hfee_amd.kernels import ops
+    H, V, block = 2, 20, 16 if D <= 128 else 8 if D <= 256 else 4
+    lengths = [2, 3, block - 1, block, block + 1, 2 * block + 3, 1]
+    G, n, g = (H if rule == "decay_add" else 1), sum(lengths), torch.Generator().manual_seed(D)
+    rand = lambda *shape: torch.randn(*shape, generator=g).cuda()      # noqa: E731
+    q, k, v, b = rand(n, G * D) * D ** -0.5, rand(n, G * D) * D ** -0.5, rand(n, H * V), rand(n, H).sigmoid()
+    start = rand(len(lengths) + 1, H, *ops.scan_state_shape(D, V))
+    rows, lens, slots = i32(np.cumsum([0] + lengths)[:-1]), i32(lengths), i32([3, 0, 5, 1, 6, 2, 7])
+    for a in (rand(n, H).sigmoid(), rand(H).sigmoid()):
+        got = []
+        for decay, per_head in ((a, True), (a.expand(n, H).repeat_interleave(D, 1).contiguous(), False)):
+            state, out = start.clone(), torch.full((n, H * V), float("nan"), device="cuda")
+            ops.linear_scan(out, state, q, k, v, decay, None if rule == "decay_add" else b, rows, lens, slots, H, G, D, V, rule,
+                            decay_per_head=per_head)
+            got.append((out, state))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+        assert bool(torch.isfinite(got[0][0]).all()) and torch.equal(got[0][1][4], start[4])
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("K", [1, 2, 4, 5])
 def test_short_convolution_carries_its_inputs(dtype, K):

@@ -8,7 +8,8 @@
 // the sequence's positions (a tile lies in one page; keys before the chunk are masked), so what is added
 // in which order depends on positions only.  A tile's steps:
 //   0. the keys of the wave's key heads (once a key head, whichever of the wave's heads read it) are asked for under
-//      the products of the tile before, their value columns behind the raw scores.
+//      the products of the tile before where registers hold them (KEYS_AHEAD, else at the tile's start), their value columns
+//      in front of or behind the raw scores (VALUES_FIRST; without EARLY_VALUES head by head, behind the softmax).
 //   1. raw scores: v_mfma_f32_16x16x32_bf16, the tile's keys as the first operand, the rows' queries as
 //      the second; lane l then holds, for row l % 16, the keys 4 (l / 16) .. + 3: sixteen bytes of
 //      raw[head][row][key] in LDS.
@@ -41,28 +42,41 @@ namespace {
 
 constexpr int H = HFEE_MIX_HEADS, G = HFEE_MIX_KV_HEADS, D = HFEE_MIX_DIM, PER_KV = H / G;
 static_assert(H % G == 0, "heads are a multiple of key heads");
-// (what a wave keeps in registers for all tiles, its heads' queries and outputs, is 3/8 of a register a
-// head and dim: four waves where that fits their 512 registers, eight waves of half as many heads and
-// 256 registers beyond)
+// (a wave's outputs, a quarter of a register a head and dim, stay in registers for all tiles, beside keys, values, scores and, where
+// they fit, queries: four waves of 512 registers up to 128 of outputs, eight waves of half as many heads and 256
+// registers beyond)
 constexpr int WAVES = H / 4 * D > 512 ? 8 : 4;
 constexpr int HW = H / WAVES, KS = D / 32, DB = D / 16, ROWS = 16, KEYS = 16;
 static_assert(H % WAVES == 0 && D % 32 == 0 && HW * D <= 512, "heads in fours or eights, head sizes in multiples of 32");
 // the most key heads that the consecutive heads of a wave read (a wave's heads begin at a multiple of HW)
 constexpr int NKV_ANY = (HW + PER_KV - 2) / PER_KV + 1 < G ? (HW + PER_KV - 2) / PER_KV + 1 : G;
 constexpr int NKV = PER_KV % HW == 0 ? 1 : HW % PER_KV == 0 ? HW / PER_KV : NKV_ANY;
-// value columns wait in registers behind the raw scores where they fit beside the outputs and the keys of the next tile (else
-// they are asked for head by head, behind the softmax)
+// value columns wait in registers where they fit beside the outputs and the keys of the next tile (else they are asked for head by
+// head, behind the softmax)
 constexpr bool EARLY_VALUES = HW * D / 4 + NKV * D / 4 + 8 * HW + 48 <= (WAVES == 8 ? 256 : 384);
-// (keys a tile ahead where they are few: with 64 heads over 64 the registers they wait in were spilled)
-constexpr bool KEYS_AHEAD = WAVES == 4 || NKV * D / 8 <= 32;
-constexpr bool Q_STAYS = WAVES == 4 && HW <= 4;          // the queries in registers for all tiles
-constexpr bool MATRIX_MIX = HW % 4 == 0 && H % 16 == 0;
+#ifdef HFEE_MIX_ON_VECTORS
+constexpr bool MATRIX_MIX = false;                       // (a library to compare the two ways with: they give the same bits)
+#else
+constexpr bool MATRIX_MIX = HW % 4 == 0;
+#endif
+// ... in front of the raw scores where the mixing on the vector units has to hide them or a wave has few heads, and there is much
+// to bring (64 single tokens at contexts around 500, 8 heads over 8 of 256: 81 us behind the scores, 71 in front; 16 over 16 of 128
+// 101 and 93; the other way round 32 over 8 of 64, 85 and 87, and 8 over 8 of 32, 25.3 and 26.8)
+constexpr bool VALUES_FIRST = (HW <= 4 || HW % 4 != 0) && D > 32;
+// (keys a tile ahead where they are few, if a wave has 256 registers: with 64 heads over 64 of 64 those that they wait in were spilled)
+constexpr bool KEYS_AHEAD = WAVES == 4 || NKV * D / 8 <= 40;
+// the queries in registers for all tiles (read again for every tile, 24 heads over 24 of 32 took 72 us for such 64 tokens instead
+// of 64; with eight and more heads a wave and the matrix unit's operands beside them they would be spilled)
+constexpr bool Q_STAYS = WAVES == 4 && (HW <= 4 || HW % 4 != 0);
 // Where the queries do not fit a wave's registers beside the outputs (eight waves) they lie in LDS as operands, each wave
 // its own, if LDS holds them beside the raw scores of one tile: read again from the caches for every tile they were half of
 // what a prompt of 2,048 tokens took from there.
 constexpr size_t LDS_MOST = 160 * 1024, RAW_TILE = (size_t)H * ROWS * KEYS * sizeof(float), Q_BYTES = (size_t)H * ROWS * D * sizeof(bf16_t);
 constexpr bool Q_IN_LDS = WAVES == 8 && RAW_TILE + Q_BYTES <= LDS_MOST;
-constexpr size_t LDS_BYTES = RAW_TILE + (Q_IN_LDS ? Q_BYTES : 0);
+// Heads whose raw scores the mixing on the vector units asks for together, with their HW numbers of T each in scalar registers: left to
+// the compiler it asks for one, waits, and asks for the next (eight single tokens at contexts around 1,000, 40 heads over 40 of 64:
+// 92 us, 82 so; by four instead of eight 24 over 6 of 32 takes 3 % longer).
+constexpr int BATCH = H % 8 == 0 && HW <= 6 ? 8 : 4;
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -101,9 +115,8 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
     KvLayout lay, const int* __restrict__ items, const int* __restrict__ block_tables, int bt_stride, float scale,
     const float* __restrict__ mix_t, int chunk, int sink_mode, const float* __restrict__ sinks, int splits,
     float* __restrict__ partial_ml, float* __restrict__ partial_o) {
-  extern __shared__ __attribute__((aligned(16))) char mix_lds[];
-  float (*raw)[ROWS][KEYS] = reinterpret_cast<float (*)[ROWS][KEYS]>(mix_lds);                  // [H]
-  u32x4* q_lds = reinterpret_cast<u32x4*>(mix_lds + RAW_TILE);                      // [wave][head][ks][lane]
+  __shared__ float raw[H][ROWS][KEYS];                        // (its size known to the compiler: it plans registers by it)
+  extern __shared__ u32x4 q_lds[];                            // [wave][head][ks][lane], where the queries lie there
   const int4 item = reinterpret_cast<const int4*>(items)[blockIdx.x];
   const int row0 = item.x, rows = item.y, p0 = item.z;
   const int first = chunk > 0 ? p0 / chunk * chunk : 0, last = p0 + rows - 1;
@@ -173,6 +186,10 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
     const int page = page_next, slot0 = j0 & (lay.page_size - 1);
     const bool more = j0 + KEYS < j_end;
     if constexpr (!KEYS_AHEAD) ask_keys(page, j0);
+    if constexpr (EARLY_VALUES && VALUES_FIRST) {
+#pragma unroll
+      for (int kv = 0; kv < NKV; ++kv) ask_values(page, slot0, min(kv0 + kv, G - 1), vop[kv]);
+    }
     // 1. raw scores of the wave's heads
     const bf16_t* q_now = q_row;
     if constexpr (!Q_STAYS) asm volatile("" : "+v"(q_now));      // (not to be kept for all tiles: they would go to scratch memory)
@@ -191,7 +208,7 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
       }
       *reinterpret_cast<f32x4*>(&raw[g][r16][kq * 4]) = s * scale;
     }
-    if constexpr (EARLY_VALUES) {
+    if constexpr (EARLY_VALUES && !VALUES_FIRST) {
 #pragma unroll
       for (int kv = 0; kv < NKV; ++kv) ask_values(page, slot0, min(kv0 + kv, G - 1), vop[kv]);
     }
@@ -219,15 +236,23 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
 #pragma unroll
         for (int hh = 0; hh < HW; ++hh) sc[hh] = f32x4{0.f, 0.f, 0.f, 0.f};
         const float* tw = mix_t + wave * HW;
-#pragma unroll 8
-        for (int g = 0; g < H; ++g) {
-          const f32x4 r = *reinterpret_cast<const f32x4*>(&raw[g][r16][kq * 4]);
+#pragma unroll 1
+        for (int g0 = 0; g0 < H; g0 += BATCH) {
+          f32x4 r[BATCH];
+          float t[BATCH][HW];
 #pragma unroll
-          for (int hh = 0; hh < HW; ++hh) {
-            const float w = tw[g * H + hh];
+          for (int j = 0; j < BATCH; ++j) {
+            r[j] = *reinterpret_cast<const f32x4*>(&raw[g0 + j][r16][kq * 4]);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sc[hh][i] = fmaf(w, r[i], sc[hh][i]);
+            for (int hh = 0; hh < HW; ++hh) t[j][hh] = tw[(g0 + j) * H + hh];
           }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < BATCH; ++j)
+#pragma unroll
+            for (int hh = 0; hh < HW; ++hh)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sc[hh][i] = fmaf(t[j][hh], r[j][i], sc[hh][i]);
         }
       }
     } else {
@@ -323,10 +348,10 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
 }
 
 // grid (items, heads): out[row][head] = sum_s o_s exp(m_s - M) / sum_s l_s exp(m_s - M), the splits in their order; a thread
-// has four dims of a row, and a round's parts are asked for together.
+// has four dims of a row, and a round's TOGETHER parts are asked for together.
+template <int TOGETHER>
 __global__ __launch_bounds__(256) void mix_join_kernel(bf16_t* __restrict__ out, int64_t ld_out, const int* __restrict__ items,
                                                        int splits, const float* __restrict__ partial_ml, const float* __restrict__ partial_o) {
-  constexpr int TOGETHER = 8;
   const int4 item = reinterpret_cast<const int4*>(items)[blockIdx.x];
   const int row0 = item.x, rows = item.y, h = blockIdx.y;
   for (int e = threadIdx.x; e < rows * (D / 4); e += blockDim.x) {
@@ -393,17 +418,18 @@ HFEE_API int hfee_attention_mix_bf16(void* out, int64_t ld_out, const void* q, i
   float* partial_o = partial;                               // [places][D], then [places][2]
   float* partial_ml = partial != nullptr ? partial + places * D : nullptr;
   static bool raised = false;
-  if (LDS_BYTES > 48 * 1024 && !raised) {
-    const hipError_t e = hipFuncSetAttribute((const void*)mix_attend_bf16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES);
+  if (Q_IN_LDS && !raised) {
+    const hipError_t e = hipFuncSetAttribute((const void*)mix_attend_bf16_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Q_BYTES);
     HFEE_REQUIRE(e == hipSuccess, "attention_mix_bf16: cannot raise the LDS limit: %s", hipGetErrorString(e));
     raised = true;
   }
-  mix_attend_bf16_kernel<<<dim3(count, splits), WAVES * 64, LDS_BYTES, stream>>>(
+  mix_attend_bf16_kernel<<<dim3(count, splits), WAVES * 64, Q_IN_LDS ? Q_BYTES : 0, stream>>>(
       (bf16_t*)out, ld_out, (const bf16_t*)q, ldq, (const bf16_t*)cache, lay, items, block_tables, bt_stride, scale, mix_t, chunk,
       sink_mode, sinks, splits, partial_ml, partial_o);
   HFEE_CHECK_LAUNCH("attention_mix_bf16");
   if (splits > 1) {
-    mix_join_kernel<<<dim3(count, H), 256, 0, stream>>>((bf16_t*)out, ld_out, items, splits, partial_ml, partial_o);
+    if (splits <= 4) mix_join_kernel<4><<<dim3(count, H), 256, 0, stream>>>((bf16_t*)out, ld_out, items, splits, partial_ml, partial_o);
+    else mix_join_kernel<8><<<dim3(count, H), 256, 0, stream>>>((bf16_t*)out, ld_out, items, splits, partial_ml, partial_o);
     HFEE_CHECK_LAUNCH("attention_mix_join");
   }
   return 0;

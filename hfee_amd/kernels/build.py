@@ -8,7 +8,8 @@ Two kinds of library:
     different sizes, compiled per pair of sizes, on demand; with `_sigmoid` behind the name
     the same kernels without a softmax (a key weighs sigmoid(score + a number a head));
   * `attention_mix_bf16_h<H>_g<G>_d<D>`: the matrix-core attention whose heads' scores are mixed,
-    compiled per number of heads, of key heads and head size, on demand.
+    compiled per number of heads, of key heads and head size, on demand; with `_vectors` behind the name the
+    mixing itself is on the vector units whatever the sizes (to compare the two: the bits are the same).
 Libraries are built in-tree (hfee_amd/_lib); if that folder cannot be written, in a
 per-user folder under the system's temporary directory; $HFEE_BUILD_DIR, if set, comes
 before both.  A library is rebuilt when its sources or flags no longer match the stamp
@@ -45,7 +46,10 @@ ATTENTION_KV_SOURCE = "attention_kv_bf16.hip"      # compiled per (key size, val
 ATTENTION_KV_MOST = (1024, 512)
 ATTENTION_MIX_SOURCE = "attention_mix_bf16.hip"    # compiled per (heads, key heads, head size)
 # the sizes that `build_all` compiles: those of the tests and of bench.py's comparison
-ATTENTION_MIX_SIZES = ((4, 2, 32), (4, 4, 32), (8, 2, 32), (8, 8, 32), (8, 2, 64), (16, 4, 128), (32, 8, 128))
+ATTENTION_MIX_SIZES = ((4, 2, 32), (4, 4, 32), (8, 2, 32), (8, 8, 32), (8, 2, 64), (16, 4, 128), (32, 8, 128), (8, 8, 64),
+                       (12, 3, 32), (24, 6, 64), (40, 10, 32), (40, 40, 64), (32, 8, 64), (32, 32, 128), (64, 16, 64), (64, 64, 64))
+# the same with the mixing on the vector units, for the tests to compare
+ATTENTION_MIX_VECTORS_SIZES = ((16, 4, 128), (32, 8, 64), (64, 16, 64))
 
 
 def attention_mix_fits(heads: int, dim: int) -> bool:
@@ -140,14 +144,16 @@ def library_spec(name: str):
         return [ATTENTION_KV_SOURCE], [f"-DHFEE_DK={dk}", f"-DHFEE_DV={dv}"] + (["-DHFEE_KV_WEIGHTS=1"] if weights else [])
     if name.startswith("attention_mix_bf16_h"):
         try:
-            heads, rest = name[len("attention_mix_bf16_h"):].split("_g")
+            sizes, vectors = name[len("attention_mix_bf16_h"):], name.endswith("_vectors")
+            heads, rest = sizes.removesuffix("_vectors").split("_g")
             kv_heads, dim = rest.split("_d")
             heads, kv_heads, dim = int(heads), int(kv_heads), int(dim)
         except ValueError:
             raise BuildError(f"unknown kernel library {name!r}") from None
         if not attention_mix_fits(heads, dim) or kv_heads < 1 or heads % kv_heads:
             raise BuildError(f"the matrix-core attention with mixed heads does not take {heads} heads on {kv_heads} of {dim}")
-        return [ATTENTION_MIX_SOURCE], [f"-DHFEE_MIX_HEADS={heads}", f"-DHFEE_MIX_KV_HEADS={kv_heads}", f"-DHFEE_MIX_DIM={dim}"]
+        return [ATTENTION_MIX_SOURCE], [f"-DHFEE_MIX_HEADS={heads}", f"-DHFEE_MIX_KV_HEADS={kv_heads}", f"-DHFEE_MIX_DIM={dim}"] + \
+            (["-DHFEE_MIX_ON_VECTORS=1"] if vectors else [])
     raise BuildError(f"unknown kernel library {name!r}")
 
 
@@ -222,13 +228,14 @@ def build_library(name: str, force: bool = False) -> str:
 
 
 def build_all(head_dims=HEAD_DIMS, force: bool = True, kv_sizes=ATTENTION_KV_SIZES, mix_sizes=ATTENTION_MIX_SIZES,
-              kv_sigmoid_sizes=ATTENTION_KV_SIGMOID_SIZES) -> list:
+              kv_sigmoid_sizes=ATTENTION_KV_SIGMOID_SIZES, mix_vectors_sizes=ATTENTION_MIX_VECTORS_SIZES) -> list:
     """Compiles the core library, the attention library of every head size, and the attention
     libraries for keys and values of different sizes of the listed pairs."""
     out = [build_library("core", force=force)]
     # the attention libraries are independent: build them side by side
     names = [f"attention_bf16_hd{hd}" for hd in head_dims] + [f"attention_kv_bf16_k{dk}_v{dv}" for dk, dv in kv_sizes]
     names += [f"attention_mix_bf16_h{h}_g{g}_d{d}" for h, g, d in mix_sizes]
+    names += [f"attention_mix_bf16_h{h}_g{g}_d{d}_vectors" for h, g, d in mix_vectors_sizes]
     names += [f"attention_kv_bf16_k{dk}_v{dv}_sigmoid" for dk, dv in kv_sigmoid_sizes]
     errors = []
 

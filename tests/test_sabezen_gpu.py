@@ -275,11 +275,13 @@ def test_mixed_attention_on_the_matrix_cores(chunk, H, G, D, half):
             assert su.rel(got[s, t].double().cpu(), want[s][t]) < 3e-2, f"sequence {s} token {t}"
 
 
-@pytest.mark.parametrize("H,G,D", [(8, 2, 64), (16, 4, 128), (32, 8, 128)])
+@pytest.mark.parametrize("H,G,D", [(8, 2, 64), (16, 4, 128), (32, 8, 128), (8, 8, 64), (12, 3, 32), (24, 6, 64), (40, 10, 32),
+                                   (40, 40, 64), (32, 8, 64), (32, 32, 128), (64, 16, 64), (64, 64, 64)])
 def test_mixed_attention_over_several_workgroups(H, G, D):
     """Items of unequal lengths whole and over several workgroups, some without a tile, against the plain kernel (bfloat16
-    results of the same inputs: a few rounding steps of 2^-9); heads in fours a wave mix on the matrix unit, in registers or LDS
-    the queries.  The chunk begins inside a tile."""
+    results of the same inputs: a few rounding steps of 2^-9); four, eight and other numbers of heads a wave, mixed on the matrix
+    unit or the vector units, queries in registers, in LDS or read again, keys and values early or late.  The chunk begins inside a
+    tile.  (64 heads are mixed within each half of them: the plain kernel takes the halves one by one.)"""
     from hfee_amd.kernels import ops
     page, chunk, starts, counts = 16, 88, (0, 100, 89, 263), (70, 30, 1, 1)
     g = torch.Generator().manual_seed(H)
@@ -292,7 +294,9 @@ def test_mixed_attention_over_several_workgroups(H, G, D):
     tables = tables.cuda()
     cache = torch.randn(sum(pages), G, page * 2 * D, generator=g).bfloat16().cuda()
     q = (torch.randn(sum(counts), H * D, generator=g) * 2).bfloat16().cuda()
-    talk = (torch.eye(H) + torch.randn(H, H, generator=g) * 0.2).cuda()
+    halves = 2 if H == 64 else 1
+    h, k = H // halves, G // halves
+    talk = torch.block_diag(*(torch.eye(h) + torch.randn(h, h, generator=g) * 0.2 for _ in range(halves))).cuda()
     items, row = [], 0
     for s, (start, n) in enumerate(zip(starts, counts)):
         off = 0
@@ -306,7 +310,11 @@ def test_mixed_attention_over_several_workgroups(H, G, D):
     pos = np.concatenate([np.arange(a, a + n) for a, n in zip(starts, counts)])
     want = torch.zeros_like(q)
     kw = dict(chunk=chunk, sink="zero")
-    ops.attention_mix(want, q, cache, i32(pos), i32(np.repeat(np.arange(4), counts)), tables, H, G, D, page, D ** -0.5, mix=talk, **kw)
+    for i in range(halves):
+        mine, heads = torch.zeros_like(q[:, :h * D]).contiguous(), slice(i * h, (i + 1) * h)
+        ops.attention_mix(mine, q[:, i * h * D:(i + 1) * h * D].contiguous(), cache[:, i * k:(i + 1) * k].contiguous(), i32(pos),
+                          i32(np.repeat(np.arange(4), counts)), tables, h, k, D, page, D ** -0.5, mix=talk[heads, heads].contiguous(), **kw)
+        want[:, i * h * D:(i + 1) * h * D] = mine
     for splits in (1, 2, 3, 16):
         partial = torch.full((max(1, ops.attention_mix_partial_words(len(items), H, D, splits)),), float("nan"), device="cuda")
         got = torch.full_like(q, float("nan"))
@@ -314,6 +322,26 @@ def test_mixed_attention_over_several_workgroups(H, G, D):
                                splits=splits, partial=partial if splits > 1 else None, **kw)
         for t in range(len(pos)):
             assert su.rel(got[t].double().cpu(), want[t].double().cpu()) < 1e-2, f"row {t} over {splits} workgroups"
+
+
+@pytest.mark.parametrize("H,G,D", [(16, 4, 128), (32, 8, 64), (64, 16, 64)])
+def test_mixing_on_the_matrix_unit_adds_as_the_vector_units_do(H, G, D, monkeypatch):
+    """Four and eight heads of a wave mixed by the matrix unit give to the bit what the vector units give: the same
+    multiply-adds in the order of the heads."""
+    from hfee_amd.kernels import lib, ops
+    page, n, g = 16, 75, torch.Generator().manual_seed(H)
+    table = torch.randperm(-(-n // page), generator=g).to(torch.int32).cuda()[None]
+    cache = torch.randn(table.numel(), G, page * 2 * D, generator=g).bfloat16().cuda()
+    q = (torch.randn(n, H * D, generator=g) * 3).bfloat16().cuda()
+    talk = torch.randn(H, H, generator=g).cuda()
+    items = i32([[p, min(16, n - p), p, 0] for p in range(0, n, 16)])
+    results = []
+    for kernels in (lib.attention_mix_bf16, lambda h, k, d: lib.load(f"attention_mix_bf16_h{h}_g{k}_d{d}_vectors")):
+        monkeypatch.setattr(lib, "attention_mix_bf16", kernels)
+        out = torch.full_like(q, float("nan"))
+        ops.attention_mix_bf16(out, q, cache, items, table, H, G, D, page, D ** -0.5, mix_t=talk, sink="zero")
+        results.append(out)
+    assert torch.equal(*results) and bool(torch.isfinite(results[0]).all())
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -798,11 +798,19 @@ constexpr int WIDE_MIN_GROUPS_A_CU = 6;
 // 1.240 / 1.326 / 1.399 ms; at 64 rows the pair of kernels stays, 1.591 against 1.616)
 constexpr int WIDE_MIN_GROUPS_A_CU_FEW_ROWS = 4;       // of eight: below, the kernels above with their slices of K spread better
 // Fewer row groups a CU, where the pair of kernels would run: from here on this one, with the columns added up in the pair's
-// slices, so that the results are the pair's to the bit (us, the products cold in a captured graph, the pair -> this): at 24
-// rows 8,192 x 3,072 weights 15.2 -> 13.7, 12,288 x 4,096 24.7 -> 21.4, 15,360 x 5,120 (q/k/v of the 13B shape) 36.8 -> 30.6, but
-// 6,144 x 4,096 14.9 -> 16.6; at 43 rows 10,240 x 4,096 24.1 -> 22.8, 15,360 x 5,120 40.6 -> 34.1, but 9,216 x 3,072 17.5 -> 17.9;
-// at 64 rows 15,360 x 5,120 41.7 -> 42.2.
-constexpr float wide_groups_as_pair(int mt) { return mt == 2 ? 2.f : 2.5f; }
+// slices, so that the results are the pair's to the bit.  What it costs is a workgroup's few busy waves (two of eight at two row
+// groups a CU), which grows with K, while the pair's second launch and its shares do not: so the line lies higher for long rows.
+// Measured over 8,192 to 16,368 weight rows, K from 1,536 to 28,672 and 17 to 48 rows, cold in a captured graph (us, the pair ->
+// this).  24 rows: 8,192 x 3,072 15.2 -> 13.9, 8,192 x 5,120 22.7 -> 21.0, but 8,192 x 8,192 30.4 -> 31.1 and x 28,672 98 -> 103;
+// 10,240 x 8,192 37.6 -> 34.4, x 28,672 118 -> 110; 15,360 x 5,120 (q/k/v of the 13B shape) 36.8 -> 30.4; 6,144 x 4,096 14.9 -> 16.6.
+// 48 rows: 10,240 x 4,096 24.0 -> 23.4, x 5,120 28.0 -> 28.1, but x 8,192 40.5 -> 41.4 and x 28,672 124 -> 136; 12,288 x 8,192
+// 48.2 -> 44.1, x 28,672 150 -> 145; 15,360 x 5,120 40.9 -> 34.3.  At 64 rows 15,360 x 5,120 41.7 -> 42.2.
+constexpr int WIDE_AS_PAIR_SHORT_K = 5120, WIDE_AS_PAIR_MOST_K = 28672;
+inline bool wide_as_pair_pays(int mt, int K, int row_groups, int cus) {
+  if (mt > 3 || K > WIDE_AS_PAIR_MOST_K) return false;
+  const float least = K <= WIDE_AS_PAIR_SHORT_K ? (mt == 2 ? 2.f : 2.5f) : mt == 2 ? 2.5f : 3.f;      // row groups a CU
+  return row_groups >= least * cus;
+}
 
 constexpr size_t mid_wide_lds_bytes(int mt) { return (size_t)2 * mt * 16 * WIDE_PITCH * sizeof(bf16_t); }
 
@@ -1263,13 +1271,16 @@ HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32,
   const bool wide_rows = row_groups >= WIDE_MIN_GROUPS_A_CU * num_cus ||
                          (row_groups >= WIDE_MIN_GROUPS_A_CU_FEW_ROWS * num_cus && mt <= 3);
   const int64_t pair_floats = (int64_t)row_groups * ((K + MID_KS - 1) / MID_KS) * mt * 256 + SS_STRIDE;
-  const bool wide_as_pair = !wide_rows && mid_pays && K > MID_KS && mt <= 3 && row_groups >= wide_groups_as_pair(mt) * num_cus &&
+  const bool wide_as_pair = !wide_rows && mid_pays && K > MID_KS && wide_as_pair_pays(mt, K, row_groups, num_cus) &&
                             scratch != nullptr && scratch_floats >= pair_floats;
+  HFEE_REQUIRE(force_mid != 3 || (!norm && (mt == 2 || mt == 3) && K % WIDE_KS == 0),
+               "gemm_skinny: the kernel for many weight rows with the pair's sums takes 17 to 48 rows and K in multiples of %d", WIDE_KS);
   if (!norm && mt > 1 && K % WIDE_KS == 0 && (force_mid >= 2 || (force_mid == 0 && (wide_rows || wide_as_pair)))) {
     const bool as_pair = force_mid == 3 || (force_mid == 0 && wide_as_pair);
     const bool took = mt == 2 ? launch_mid_wide<2>(a, epi, num_cus, as_pair, stream)
                     : mt == 3 ? launch_mid_wide<3>(a, epi, num_cus, as_pair, stream)
                               : launch_mid_wide<4>(a, epi, num_cus, as_pair, stream);
+    HFEE_REQUIRE(took || force_mid != 3, "gemm_skinny: the kernel for many weight rows could not be launched");
     if (took) {
       HFEE_CHECK_LAUNCH("gemm_skinny(17 to 64 rows, many weight rows)");
       return 0;

@@ -515,6 +515,58 @@ def test_many_weight_rows_with_the_sums_of_the_pair(M, N, K):
             assert torch.equal(*got), f"{epilogue} {'with' if scale else 'without'} a row scale"
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (48, 50, 1536), (33, 4112, 2560)])
+def test_a_following_norm_with_the_sums_of_the_pair(M, N, K):
+    """... and through the accumulating product that emits the norm behind it: stream, emitted rows and shares of the squares."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight((torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV))
+    c0, nw = torch.randn(M, N, generator=g).to(DEV), torch.rand(N, generator=g).to(DEV)
+    got = []
+    for kernel in (1, 3):
+        scratch = torch.full((ops.mid_rows_scratch(M, N, K),), float("nan"), device=DEV)
+        out, emitted = c0.clone(), torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+        shares = torch.zeros((N + 15) // 16 * 64, device=DEV)
+        ops.linear_fused(out, x, w, "add", emit=dict(weight=nw, out=emitted, shares=shares), scratch=scratch, force_mid_rows=kernel)
+        got.append((out, emitted, shares))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("H,K,hd,half,M,d", [(4, 2, 16, 8, 17, 2048), (6, 3, 48, 8, 40, 3072), (5, 1, 64, 32, 33, 2560), (2, 2, 128, 64, 48, 1536)])
+def test_fused_qkv_with_the_sums_of_the_pair(H, K, hd, half, M, d):
+    """... and through q/k/v: the rotated queries and the cache, against the plain form and to the bit."""
+    from hfee_amd.kernels import ops
+    scratch = torch.full((ops.mid_rows_scratch(M, (H + 2 * K) * hd, d),), float("nan"), device=DEV)
+    got = [_check_fused_qkv(H, K, hd, half, M, False, d, scratch=scratch.clone(), force_mid_rows=kernel) for kernel in (1, 3)]
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("M,N,K,whole", [(17, 8192, 3072, True), (20, 15360, 1536, True), (48, 10240, 2048, True), (32, 10240, 8192, True),
+                                         (17, 8176, 3072, False), (17, 8192, 8192, False), (48, 9216, 2048, False), (33, 10240, 8192, False)])
+def test_which_products_run_whole_with_the_sums_of_the_pair(M, N, K, whole):
+    """Where the line lies between the pair of kernels (which leaves its shares in the scratch) and the one that cuts nothing, which
+    leaves the scratch alone; both give the same bits.  (With the row groups a CU of 256 CUs.)  The one is refused, not replaced,
+    where it was asked for and does not apply."""
+    from hfee_amd.kernels import ops
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are on the two sides of the line for 256 CUs")
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x = torch.randn(M, K, device=DEV, generator=g).to(torch.bfloat16)
+    w = ops.tile_weight((torch.randn(N, K, device=DEV, generator=g) / math.sqrt(K)).to(torch.bfloat16))
+    got = []
+    for kernel in (0, 1):
+        scratch = torch.full((ops.mid_rows_scratch(M, N, K),), float("nan"), device=DEV)
+        out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+        ops.linear_fused(out, x, w, "bf16", scratch=scratch, force_mid_rows=kernel)
+        got.append((out, bool(torch.isnan(scratch).all())))
+    assert torch.equal(got[0][0], got[1][0]) and got[0][1] == whole and not got[1][1]
+    few = torch.zeros(16, N, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(ops.KernelError, match="17 to 48 rows"):
+        ops.linear_fused(few, x[:16], w, "bf16", scratch=scratch, force_mid_rows=3)
+
+
 @pytest.mark.parametrize("kernel", [1, 2])
 @pytest.mark.parametrize("H,K,hd,half,M,d", [(4, 2, 16, 8, 17, 2048), (5, 1, 64, 32, 64, 1024), (6, 3, 48, 8, 40, 3072)])
 def test_fused_qkv_with_the_batch_in_lds(H, K, hd, half, M, d, kernel):
@@ -567,6 +619,7 @@ def _check_fused_qkv(H, K, hd, half, M, norm, d, **kw):
             close(kslot(lay[page, 0, kh], ps, hd, slot).reshape(hd), k_ref[m, kh], 2e-2)
             close(lay[page, 1, kh].view(hd, ps)[:, vslot(slot)], v_ref[m, kh], 2e-2)
     assert int((lay != 0).sum()) <= M * 2 * K * hd, "nothing but the tokens' own slots is written"
+    return q_out, layer
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

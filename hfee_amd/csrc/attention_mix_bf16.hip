@@ -27,9 +27,9 @@
 // output in float32, and a second kernel joins them in the order of the splits; the sink belongs to the
 // first split.
 // What bounds it: a tile is a chain of loads, products, an exchange and exponentials under one workgroup a CU.  2,048
-// tokens, 32 heads over 8 of 128, with the join: 244 us with each wave reading the keys of two key heads where it has
-// one, values asked for head by head, queries from the caches and the mixing on the vector units, 180 now; 16 over 4:
-// 172 and 127; eight single tokens at contexts of 150 23 and 17.
+// tokens, 32 heads over 8 of 128, with the join: 245 us with each wave reading the keys of two key heads where it has
+// one, values asked for head by head, queries from the caches and the mixing on the vector units, 177 now; 16 over 4:
+// 172 and 128; eight single tokens at contexts of 150 23 and 17.5.
 #include "attention_kv.h"
 
 using namespace hfee;
@@ -299,7 +299,6 @@ __global__ __launch_bounds__(WAVES * 64) void mix_attend_bf16_kernel(
     for (int hh = 0; hh < HW; ++hh) psum[hh] += __shfl_xor(psum[hh], 16, kWave);
 #pragma unroll
     for (int hh = 0; hh < HW; ++hh) psum[hh] += __shfl_xor(psum[hh], 32, kWave);
-    __builtin_amdgcn_sched_barrier(0);
     if (KEYS_AHEAD && more) ask_keys(page_next, j0 + KEYS);
     // 4. the weighted values
 #pragma unroll

@@ -77,3 +77,11 @@ def model_folders(tmp_path_factory):
                                                    dtype=dtype, std=0.1,
                                                    norm_init="one_plus_normal" if name != "B" else "normal")
     return out
+
+
+# The 2-norm of a float32 product's error over the result's, against 64 bits, at K columns: one and a half times what the
+# matrix product of the 32-bit path measures (5.0e-8, 1.0e-7, 1.4e-7 and 2.6e-7 for normal operands, 8.6e-8, 1.6e-7, 2.2e-7 and
+# 3.9e-7 where one column is a thousand times the others; a chain of float32 additions in eight segments 1.07e-7, 2.9e-7,
+# 4.1e-7, 7.6e-7 and 1.45e-7, 4.1e-7, 5.7e-7, 1.06e-6).
+GEMM_F32_ERROR = {64: 7.5e-8, 2048: 1.5e-7, 4096: 2.1e-7, 14336: 3.9e-7}
+GEMM_F32_ERROR_OF_ONE_COLUMN = {64: 1.3e-7, 2048: 2.4e-7, 4096: 3.3e-7, 14336: 5.9e-7}

@@ -147,6 +147,33 @@ def test_gemm_f32_in_cuts_and_turns_gives_one_row_the_same_bits(M, N, K, accumul
     assert ((full.double() - ref).abs() <= (K / 8 + 48) * 2.0 ** -24 * mag).all()
 
 
+@pytest.mark.parametrize("M,N,cut", [(3, 1024, False), (16, 1024, False), (3, 12288, False), (24, 1024, False), (200, 1024, False),
+                                     (200, 1024, True)])
+@pytest.mark.parametrize("K", [64, 2048, 4096, 14336])
+@pytest.mark.parametrize("kind", ["normal", "small", "denormal", "one column"])
+def test_gemm_f32_errors_against_64_bits(M, N, cut, K, kind):
+    """Every kernel's error at a model's K, which operands that are small (x of 2^-118, or denormal, of 2^-129, beside large
+    weights) or a sum that one column dominates do not make larger than a chain of float32 additions has; and what is the
+    same in every element stays far below the error."""
+    from conftest import GEMM_F32_ERROR, GEMM_F32_ERROR_OF_ONE_COLUMN
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    if kind == "one column":
+        x[:, 0] *= 1000
+    elif kind != "normal":
+        x, w = x * 2.0 ** (-118 if kind == "small" else -129), w * 2.0 ** 96
+    words = ops.linear_scratch(M, N, K, torch.float32) if cut else 0
+    out = torch.empty(M, N, device=DEV)
+    ops.linear(out, x, w, scratch=torch.empty(words, device=DEV) if words else None)
+    ref = x.double() @ w.double().t()
+    err = out.double() - ref
+    bound = (GEMM_F32_ERROR_OF_ONE_COLUMN if kind == "one column" else GEMM_F32_ERROR)[K] * float(ref.norm())
+    assert float(err.norm()) <= bound, float(err.norm() / ref.norm())
+    # (rows of a batch share the roundings of their own operands, so a mean over few of them is a noisy one)
+    assert abs(float(err.mean())) * err.numel() ** 0.5 <= (0.05 if M >= 16 else 0.12) * bound, float(err.mean() * err.numel() ** 0.5 / bound)
+
+
 @pytest.mark.parametrize("M", [3, 16, 24, 70, 300])
 @pytest.mark.parametrize("N,K", [(96, 320), (80, 1027), (4160, 2048)])
 def test_gemm_f32_of_infinities_and_large_numbers(M, N, K):

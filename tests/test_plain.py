@@ -236,3 +236,39 @@ def test_product_frequencies_and_random_stream_match_their_plain_twins():
     us = [uniform(12345, i) for i in range(2000)]
     assert all(0 <= u < 1 for u in us) and abs(sum(us) / 2000 - 0.5) < 0.03 and len(set(us)) == 2000
     assert uniform(1, 0) != uniform(2, 0)
+
+
+def test_a_float32_product_in_bfloat16_pieces():
+    """Three bfloat16 pieces are a float32 value to the bit; the products of pieces that are left out are 2^-24 of the whole at
+    worst; and without the low pieces, or without their scaling where operands are small, the error exceeds what the product
+    of the 32-bit path is held to."""
+    from conftest import GEMM_F32_ERROR
+
+    def pieces(v):
+        out = []
+        for _ in range(3):
+            out.append(v.to(torch.bfloat16).float())
+            v = v - out[-1]
+        assert not v.any()
+        return [p.double() for p in out]
+
+    g = torch.Generator().manual_seed(1)
+    x, w = (torch.randn(200000, generator=g) for _ in range(2))
+    x[0] = w[0] = 1 + 2.0 ** -8 - 2.0 ** -17
+    (xh, xm, xl), (wh, wm, wl) = pieces(x), pieces(w)
+    kept = wl * xh + wm * xh + wh * xh + wh * xm + wm * xm + wh * xl
+    left_out = ((x.double() * w.double() - kept) / (x.double() * w.double())).abs()
+    assert 2.0 ** -24.1 < float(left_out.max()) <= 2.0 ** -24 and float(left_out.pow(2).mean().sqrt()) < 2.0 ** -27
+    for K, bound in GEMM_F32_ERROR.items():
+        x, w = torch.randn(8, K, generator=g), torch.randn(64, K, generator=g)
+        ref = x.double() @ w.double().t()
+        (xh, xm, xl), (wh, wm, wl) = pieces(x), pieces(w)
+        whole = wh @ (xh + xm + xl).t() + wm @ (xh + xm).t() + wl @ xh.t()
+        assert float((whole.t() - ref).norm()) < 0.1 * bound * float(ref.norm())
+        no_low = (wh + wm) @ (xh + xm).t()
+        assert float((no_low.t() - ref).norm()) > 5 * bound * float(ref.norm())
+        small = x * 2.0 ** -118
+        rest = small - small.to(torch.bfloat16).float()            # its low piece would be denormal
+        normal = [small.to(torch.bfloat16).double(), rest.to(torch.bfloat16).double()]
+        of_two = w.double() @ (normal[0] + normal[1]).t() * 2.0 ** 118
+        assert float((of_two.t() - ref).norm()) > 5 * bound * float(ref.norm())

@@ -109,8 +109,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
     }
     const bool mine = valid && token >= from && token < to;
     const int* bt = p.block_tables + (int64_t)segment * p.bt_stride;
-    // lane i keeps the page of block first_block + i, of those that hold a key of the run
-    const int last_block = last >> lay.page_shift;
+    // lane i keeps the page of block first_block + i, of those that hold a key of the run (without one, where every position is
+    // below zero, the table's first entry is read and no tile)
+    const int last_block = max(last, 0) >> lay.page_shift;
     int first_block = first >> lay.page_shift;
     int page_of_lane = bt[min(first_block + lane, last_block)];
 
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(Args p, Cache
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) o[c] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, sum = 0.f;
-    const int tile0 = first / TILE, tile1 = last / TILE;
+    const int tile0 = first / TILE, tile1 = last < 0 ? -1 : last / TILE;
     for (int t = tile0 + ((wave - tile0) & (WAVES - 1)); t <= tile1; t += WAVES) {
       bool there[2];
       int slot[2];

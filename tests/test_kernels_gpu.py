@@ -1025,6 +1025,28 @@ def test_attention_f32_of_many_pages_and_of_rows_off_sixteen_bytes(H, K, hd, win
     assert torch.equal(*outs)
 
 
+def test_attention_f32_of_rows_without_a_key():
+    """A row at a position below zero has no key: nothing in front of its table or its cache is read (one such row is alone in
+    its workgroup, with a table that begins where its memory does), and the rows beside it are what they are without it."""
+    from hfee_amd.kernels import ops
+    H, K, hd, ps, n = 4, 2, 64, 16, 40
+    g = torch.Generator().manual_seed(3)
+    cache = torch.randn(4, 2, K, ps * hd, generator=g).to(DEV)
+    q = torch.randn(n, H * hd, generator=g).to(DEV)
+    table = torch.tensor([[1, 3, 0]], dtype=torch.int32, device=DEV)
+    segment = torch.zeros(n, dtype=torch.int32, device=DEV)
+    positions = torch.arange(n, dtype=torch.int32, device=DEV) % 41
+    whole, some = torch.zeros_like(q), torch.zeros_like(q)
+    ops.attention_plain(whole, q, cache, positions, segment, table, H, K, hd, ps, hd ** -0.5)
+    without = positions.clone()
+    without[[0, 5, 39]] = -1
+    for singles in (False, True):
+        ops.attention_plain(some, q, cache, without, segment, table, H, K, hd, ps, hd ** -0.5, 0, singles)
+        keep = without >= 0
+        assert torch.equal(some[keep], whole[keep])
+        assert not torch.isfinite(some[~keep]).any()
+
+
 @pytest.mark.parametrize("H,K,hd,T,window,ps", [(4, 1, 128, 130, 0, 32), (8, 2, 64, 150, 40, 64), (4, 1, 48, 300, 0, 128),
                                                 (16, 2, 32, 97, 50, 32)])
 def test_attention_kernels_with_larger_pages(H, K, hd, T, window, ps):

@@ -228,6 +228,14 @@ def linear_scratch(m: int, n: int, k: int, dtype=torch.bfloat16) -> int:
     return int(lib.core().raw(fn)(int(m), int(n), int(k)))
 
 
+def linear_f32_plan(m: int, n: int, k: int, cut: bool):
+    """How a float32 product of more than 32 rows, whole steps of K and rows on 16 bytes is done: ("rows", the
+    number of the blocks) or (the pairs of K's segments that a workgroup does, 0 for all, the number of the tile).
+    cut: with scratch at hand.  (For tests.)"""
+    plan = int(lib.core().raw("hfee_gemm_f32_plan")(int(m), int(n), int(k), int(cut)))
+    return ("rows", plan - 256) if plan >= 256 else (plan // 16, plan % 16)
+
+
 def linear_cuts(x: torch.Tensor, weight: torch.Tensor, scratch) -> int:
     """x @ weight.T (bfloat16) cut along K over workgroups, the partial products left in scratch
     as that many float32 matrices [M, N] one after the other, for a kernel that adds them up on
@@ -301,7 +309,8 @@ def linear_add_norm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, no
 def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate: bool = False, kernel: int = 0,
            gate: bool = False, scratch=None, activation: str = "silu", numbers=None):
     """out (+)= x @ weight.T, weight stored [out_features, in_features].
-    scratch: float32, `linear_scratch(M, N, K, x.dtype)` words, or None.
+    scratch: float32, `linear_scratch(M, N, K, x.dtype)` words, or None (float32 operands: the call then
+    takes what it has a use for from torch's pool; with an empty tensor K is not cut).
 
     float32 x and weight: the true 32-bit product, out float32.
     bfloat16 x and weight: matrix cores with float32 accumulation; out bfloat16, or
@@ -326,7 +335,10 @@ def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate:
     _check(x.dtype == weight.dtype, "linear: x and weight dtypes differ")
     if x.dtype == torch.float32:
         _check(out.dtype == torch.float32, "linear: float32 product needs a float32 out")
-        if scratch is not None:
+        if scratch is None:
+            words = linear_scratch(M, N, K, torch.float32)
+            scratch = torch.empty(words, dtype=torch.float32, device=out.device) if words else None
+        else:
             _gpu(scratch)
             _check(scratch.dtype == torch.float32 and scratch.is_contiguous(), "linear: float32 scratch expected")
         lib.core().call("hfee_gemm_f32", _ptr(out), ldc, _ptr(x), lda, _ptr(weight), ldw, M, N, K,

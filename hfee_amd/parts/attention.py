@@ -209,7 +209,8 @@ class Attention(Mixer):
                     k = qkv[:, self.q_width:self.q_width + self.kv_width]
                     v = qkv[:, self.q_width + self.kv_width:]
                 else:   # this run of the layer reads keys and values that another run wrote
-                    ops.linear(q, hn, self.w_qkv[:self.q_width])
+                    w_q = self.w_qkv[:self.q_width]
+                    ops.linear(q, hn, w_q, **ctx.workspace.split_scratch_f32(n, w_q))
                     k = v = None
                 if self.after_projection is not None:
                     self.after_projection.forward(ctx, q, k, v)

@@ -309,6 +309,10 @@ class Workspace:
         words = ops.linear_scratch(n_rows, weight.shape[0], weight.shape[1], weight.dtype)
         return dict(scratch=self.flat("product.partial", words, torch.float32)) if words else {}
 
+    def split_scratch_f32(self, n_rows: int, weight: torch.Tensor) -> dict:
+        """The same for products whose K is cut with float32 operands only."""
+        return self.split_scratch(n_rows, weight) if weight.dtype == torch.float32 else {}
+
     def counters(self, name: str, count: int) -> torch.Tensor:
         """`count` int32 that are zero, for kernels whose workgroups count themselves
         (the one that finishes last does a final piece of work and sets the counter

@@ -116,4 +116,4 @@ class Head(Part):
             return
         normed = ctx.rows("head.normed", self.hidden, n=w)
         self.norm.forward(ctx, normed, x, rows)
-        ops.linear(logits, normed, self.weight)
+        ops.linear(logits, normed, self.weight, **ctx.workspace.split_scratch_f32(w, self.weight))

@@ -293,7 +293,8 @@ class KvAttention(_KvMixer):
             k = qkv[:, self.q_width:self.q_width + self.k_width]
             v = qkv[:, self.q_width + self.k_width:]
         else:       # this run of the layer reads keys and values that another run wrote
-            ops.linear(q, hn, self.w_qkv[:self.q_width])
+            w_q = self.w_qkv[:self.q_width]
+            ops.linear(q, hn, w_q, **ctx.workspace.split_scratch_f32(ctx.n, w_q))
             k = v = None
         if self.prepares or (self.blend is None and self.pairing):
             made = ctx.rows("kv_attention.q", self.q_width)
@@ -379,7 +380,8 @@ class SigmoidAttention(_KvMixer):
             k = qkv[:, self.q_width:self.q_width + self.k_width]
             v = qkv[:, self.q_width + self.k_width:]
         else:       # this run of the layer reads keys and values that another run wrote
-            ops.linear(q, hn, self.w_qkv[:self.q_width])
+            w_q = self.w_qkv[:self.q_width]
+            ops.linear(q, hn, w_q, **ctx.workspace.split_scratch_f32(ctx.n, w_q))
         ops.qk_norm_write(q, k, v, ctx.positions, ctx.token_segment, tables, cache, self.q_norm, self.k_norm, self.norm_eps,
                           H, G, dk, dv, ctx.page_size, temperature=self.temperature)
         att = ctx.rows("kv_attention.out", self.out_width)
@@ -478,7 +480,8 @@ class LatentAttention(_KvMixer):
         if writes_cache or not self.own_keys:
             product(ctx, down, hn, self.w_down, self.w_down_tiles)
         else:
-            ops.linear(down[:, :self.q_rank], hn, self.w_down[:self.q_rank])
+            w_q = self.w_down[:self.q_rank]
+            ops.linear(down[:, :self.q_rank], hn, w_q, **ctx.workspace.split_scratch_f32(n, w_q))
         cq = ctx.rows("latent.q_latent", self.q_rank)
         ops.rmsnorm_cols(cq, down[:, :self.q_rank], self.q_norm, self.eps)
         q = ctx.rows("latent.q", H * (Dn + Dr))

@@ -130,7 +130,8 @@ class MixedAttention(Mixer):
             product(ctx, qk, hn, self.w_qk, self.w_qk_tiles)
             k = qk[:, self.q_width:]
         else:       # this run of the layer reads the keys that another run wrote
-            ops.linear(q, hn, self.w_qk[:self.q_width])
+            w_q = self.w_qk[:self.q_width]
+            ops.linear(q, hn, w_q, **ctx.workspace.split_scratch_f32(ctx.n, w_q))
             k = None
         ops.attention_mix_prepare(q, k, ctx.positions, ctx.token_segment, tables, cos, sin, cache, H, G, D, ctx.page_size,
                                   ctx.max_position, norm=self.qk_norm is not None, eps=self.norm_eps)

@@ -106,8 +106,7 @@ class GatedMLP(FeedForward):
             ops.linear(act, hn, self.w_gate_up, gate=True, activation=self.activation, numbers=self.numbers)
         else:
             gate_up = ctx.rows("mlp.gate_up", 2 * F)
-            cut = ctx.workspace.split_scratch(n, self.w_gate_up) if self.dtype == torch.float32 else {}
-            ops.linear(gate_up, hn, self.w_gate_up, **cut)
+            ops.linear(gate_up, hn, self.w_gate_up, **ctx.workspace.split_scratch_f32(n, self.w_gate_up))
             ops.swiglu(act, gate_up[:, 0::2], gate_up[:, 1::2], activation=self.activation, numbers=self.numbers)
         # the down projection adds into x and, if asked, goes on with the norm that follows
         # (where its K is cut over workgroups: the kernel that adds the cuts up has the row at hand)

@@ -206,7 +206,7 @@ class RoutedMoE(FeedForward):
         """(chosen, weights, the shared expert's gate before its sigmoid or None)."""
         n, top = ctx.n, self.top
         made = ctx.rows("routed_moe.logits", self.w_router.shape[0], torch.float32)
-        ops.linear(made, hn, self.w_router)
+        ops.linear(made, hn, self.w_router, **ctx.workspace.split_scratch_f32(n, self.w_router))
         logits = made[:, :self.outputs]
         ws = ctx.workspace
         chosen = ws.flat("routed_moe.chosen", ws.capacity * top, torch.int32)[:n * top].view(n, top)

@@ -147,6 +147,47 @@ def test_gemm_f32_in_cuts_and_turns_gives_one_row_the_same_bits(M, N, K, accumul
     assert ((full.double() - ref).abs() <= (K / 8 + 48) * 2.0 ** -24 * mag).all()
 
 
+@pytest.mark.parametrize("M,N,K,plan", [(200, 64, 4096, ("rows", 0)), (33, 65, 4096, ("rows", 0)), (100, 1000, 320, ("rows", 1)),
+                                        (64, 2048, 2048, ("rows", 1)), (33, 4096, 512, ("rows", 2)), (100, 4096, 512, ("rows", 4)),
+                                        (100, 1600, 1600, (1, 2)), (300, 1601, 1600, (1, 0)), (257, 2050, 1088, (1, 1)),
+                                        (64, 4096, 14336, (1, 2)), (100, 2050, 2048, (1, 1)), (40, 28672, 4096, (2, 1)),
+                                        (400, 4096, 4096, (2, 0)), (500, 4096, 2720, (2, 0))])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_f32_that_would_leave_the_chip_idle_goes_by_blocks_of_rows_or_cuts(M, N, K, plan, accumulate):
+    """Products of few tiles: narrow ones in blocks of rows whose waves share K, others cut along K whatever their number of
+    columns and of K's segments, with scratch of the caller's, of torch's pool and without: the bits of a row alone, within
+    the bound of the test above, an infinity and a NaN where they belong, and nothing behind the scratch is written."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    x[1, 7], w[3, 9] = float("nan"), float("inf")
+    c0 = torch.randn(M, N, generator=g, device=DEV)
+    assert ops.linear_f32_plan(M, N, K, True) == plan
+    words = ops.linear_scratch(M, N, K, torch.float32)
+    pairs = -(-K // (2 * (-(-K // 512) * 64)))
+    assert words == (0 if plan[0] == "rows" else pairs * M * -(-N // 4) * 4)
+    scratch = torch.full((words + 64,), 7.0, device=DEV)
+    outs = []
+    for kw in (dict(scratch=scratch[:words]), dict(), dict(scratch=scratch[:0])):
+        out = c0.clone()
+        ops.linear(out, x, w, accumulate=accumulate, **kw)
+        outs.append(out)
+    assert bool((scratch[words:] == 7.0).all())
+    full = outs[0]
+    for other in outs[1:]:
+        assert torch.equal(full.view(torch.int32), other.view(torch.int32))
+    for r in (0, 1, M // 2, M - 1):
+        one = c0[r:r + 1].clone()
+        ops.linear(one, x[r:r + 1], w, accumulate=accumulate)
+        assert torch.equal(one[0].view(torch.int32), full[r].view(torch.int32))
+    ref = x.double() @ w.double().t() + (c0.double() if accumulate else 0)
+    mag = x.abs().double() @ w.abs().double().t() + c0.abs().double()
+    assert torch.equal(torch.isnan(full), torch.isnan(ref)) and torch.equal(torch.isinf(full), torch.isinf(ref))
+    finite = torch.isfinite(ref)
+    assert int(finite.sum()) == (M - 1) * (N - 1)
+    assert ((full.double() - ref).abs()[finite] <= ((K / 8 + 48) * 2.0 ** -24 * mag)[finite]).all()
+
+
 @pytest.mark.parametrize("M,N,cut", [(3, 1024, False), (16, 1024, False), (3, 12288, False), (24, 1024, False), (200, 1024, False),
                                      (200, 1024, True)])
 @pytest.mark.parametrize("K", [64, 2048, 4096, 14336])

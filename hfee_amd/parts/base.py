@@ -272,7 +272,9 @@ class Workspace:
         self.capacity = capacity
         self.device = device
         self._buffers: dict = {}
-        self._retired: list = []     # outgrown buffers stay alive: captured graphs may still point at them
+        # outgrown buffers stay alive: captured graphs may still point at them (a new one is at least twice as large, so
+        # that those of one name never hold more than it does, however slowly the steps grow)
+        self._retired: list = []
 
     def rows(self, name: str, n: int, width: int, dtype: torch.dtype) -> torch.Tensor:
         """A [n, width] view of the buffer `name` ([capacity, width])."""
@@ -288,9 +290,11 @@ class Workspace:
         key = (name, "flat", dtype)
         buf = self._buffers.get(key)
         if buf is None or buf.numel() < count:
+            words = count
             if buf is not None:
                 self._retired.append(buf)
-            buf = self._buffers[key] = torch.empty((count,), dtype=dtype, device=self.device)
+                words = max(count, 2 * buf.numel())
+            buf = self._buffers[key] = torch.empty((words,), dtype=dtype, device=self.device)
         return buf[:count]
 
     def product_scratch(self, n_rows: int, weight: torch.Tensor) -> dict:
@@ -320,9 +324,11 @@ class Workspace:
         key = (name, "counters", torch.int32)
         buf = self._buffers.get(key)
         if buf is None or buf.numel() < count:
+            words = max(count, 256)
             if buf is not None:
                 self._retired.append(buf)
-            buf = self._buffers[key] = torch.zeros((max(count, 256),), dtype=torch.int32, device=self.device)
+                words = max(count, 2 * buf.numel())
+            buf = self._buffers[key] = torch.zeros((words,), dtype=torch.int32, device=self.device)
         return buf[:count]
 
 

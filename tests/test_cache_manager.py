@@ -388,3 +388,20 @@ def test_a_chain_of_kept_pages_is_followed_where_it_leads_and_no_further():
             m.release(name, tokens)
             assert set(digests(tokens, len(tokens) // 16)) <= set(m._kept)
             m.check()
+
+
+def test_outgrown_buffers_of_a_workspace_hold_no_more_than_the_one_in_use():
+    """A buffer that grows a little with every step (prompts of ever more rows) leaves those behind that recorded graphs may
+    point at: together they stay below it, and it below twice what was asked for."""
+    import torch
+    from hfee_amd.parts.base import Workspace
+    ws = Workspace(8, "cpu")
+    kept = []
+    for count in range(300, 3000, 7):
+        for buf in (ws.flat("product.partial", count, torch.float32), ws.counters("counts", count)):
+            assert buf.numel() == count
+        kept.append(ws.flat("product.partial", 100, torch.float32).data_ptr())
+    for dtype in (torch.float32, torch.int32):
+        current, retired = ([b.numel() for b in bufs if b.dtype == dtype] for bufs in (ws._buffers.values(), ws._retired))
+        assert len(current) == 1 and current[0] < 2 * 3000 and sum(retired) < current[0]
+    assert set(kept) <= {b.data_ptr() for b in [*ws._buffers.values(), *ws._retired]}

@@ -1229,6 +1229,18 @@ bool launch_wide(const Args& a, bool norm, int epi, hipStream_t stream) {
 #undef GO
 }
 
+// Whether four neighbouring results of a row (a lane's weight rows n .. n + 3; n is a multiple of 4) lie as one load or store
+// takes them, and what is added to them and the next norm's weights as well.
+bool in_fours(const Args& a, int epi) {
+  const auto on = [](const void* p, int bytes) { return (uintptr_t)p % bytes == 0; };
+  if (a.N % 4 != 0) return false;
+  if (epi == EPI_BF16) return a.ldc % 4 == 0 && on(a.C, 8);
+  if (epi == EPI_SWIGLU) return a.ldc % 2 == 0 && on(a.C, 4);
+  if (epi != EPI_ADD && epi != EPI_F32) return false;
+  return a.ldc % 4 == 0 && on(a.C, 16) &&
+         (a.emit_out == nullptr || (a.ld_emit % 4 == 0 && on(a.emit_out, 8) && on(a.emit_weight, a.emit_weight_is_f32 ? 16 : 8)));
+}
+
 }  // namespace
 
 // One entry point for every variant.  a_is_f32 != 0 selects the fused RMSNorm (M <= 16).
@@ -1242,18 +1254,6 @@ bool launch_wide(const Args& a, bool norm, int epi, hipStream_t stream) {
 // without it, or for other sizes, or where it would not pay, the streaming kernel takes
 // the product (force_mid: 1 takes the pair of kernels with slices of K wherever it applies,
 // 2 the kernel for many weight rows, 3 that one with the pair's sums (up to 48 rows): for tests).
-// Whether four neighbouring results of a row (a lane's weight rows n .. n + 3; n is a multiple of 4) lie as one load or store
-// takes them, and what is added to them and the next norm's weights as well.
-static bool in_fours(const Args& a, int epi) {
-  const auto on = [](const void* p, int bytes) { return (uintptr_t)p % bytes == 0; };
-  if (a.N % 4 != 0) return false;
-  if (epi == EPI_BF16) return a.ldc % 4 == 0 && on(a.C, 8);
-  if (epi == EPI_SWIGLU) return a.ldc % 2 == 0 && on(a.C, 4);
-  if (epi != EPI_ADD && epi != EPI_F32) return false;
-  return a.ldc % 4 == 0 && on(a.C, 16) &&
-         (a.emit_out == nullptr || (a.ld_emit % 4 == 0 && on(a.emit_out, 8) && on(a.emit_weight, a.emit_weight_is_f32 ? 16 : 8)));
-}
-
 HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32, int64_t lda, const void* W,
                               int64_t w_stride, int M, int N, int K, int epi,
                               const void* norm_weight, int norm_weight_is_f32, float eps, const int* rows,

@@ -1253,7 +1253,7 @@ bool in_fours(const Args& a, int epi) {
 // ceil(N / 16) * ceil(K / 1024) * ceil(M / 16) * 256 + 64 floats of scratch (none for K <= 1,024);
 // without it, or for other sizes, or where it would not pay, the streaming kernel takes
 // the product (force_mid: 1 takes the pair of kernels with slices of K wherever it applies,
-// 2 the kernel for many weight rows, 3 that one with the pair's sums (up to 48 rows): for tests).
+// 2 the kernel for many weight rows, 3 that one with the pair's sums: for tests).
 HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32, int64_t lda, const void* W,
                               int64_t w_stride, int M, int N, int K, int epi,
                               const void* norm_weight, int norm_weight_is_f32, float eps, const int* rows,
@@ -1342,8 +1342,8 @@ HFEE_API int hfee_gemm_skinny(void* C, int64_t ldc, const void* A, int a_is_f32,
   const int64_t pair_floats = (int64_t)row_groups * ((K + MID_KS - 1) / MID_KS) * mt * 256 + SS_STRIDE;
   const bool wide_as_pair = !wide_rows && mid_pays && K > MID_KS && wide_as_pair_pays(mt, K, row_groups, num_cus) &&
                             scratch != nullptr && scratch_floats >= pair_floats;
-  HFEE_REQUIRE(force_mid != 3 || (!norm && (mt == 2 || mt == 3) && K % WIDE_KS == 0),
-               "gemm_skinny: the kernel for many weight rows with the pair's sums is asked for by number at 17 to 48 rows and K in multiples of %d", WIDE_KS);
+  HFEE_REQUIRE(force_mid != 3 || (!norm && mt > 1 && K % WIDE_KS == 0),
+               "gemm_skinny: the kernel for many weight rows with the pair's sums is asked for by number at 17 to 64 rows and K in multiples of %d", WIDE_KS);
   if (!norm && mt > 1 && K % WIDE_KS == 0 && (force_mid >= 2 || (force_mid == 0 && (wide_rows || wide_as_pair)))) {
     const bool as_pair = force_mid == 3 || (force_mid == 0 && wide_as_pair);
     const bool took = mt == 2 ? launch_mid_wide<2>(a, epi, num_cus, as_pair, stream)

@@ -649,7 +649,8 @@ def test_fused_qkv_through_the_tiled_kernels_with_whole_steps_of_k(H, K, hd, hal
     _check_fused_qkv(H, K, hd, half, M, False, d)
 
 
-@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (33, 50, 1536), (40, 4160, 5120), (32, 4112, 3072), (48, 16, 2560)])
+@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (33, 50, 1536), (40, 4160, 5120), (32, 4112, 3072), (48, 16, 2560),
+                                   (49, 50, 1536), (60, 4160, 5120), (64, 96, 2048)])
 def test_many_weight_rows_with_the_sums_of_the_pair(M, N, K):
     """The kernel for many weight rows in the pair's slices of K gives the pair's results to the bit, a last slice of half the
     columns among them, with and without the second half of a norm, through every plain epilogue."""
@@ -671,7 +672,7 @@ def test_many_weight_rows_with_the_sums_of_the_pair(M, N, K):
             assert torch.equal(*got), f"{epilogue} {'with' if scale else 'without'} a row scale"
 
 
-@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (48, 50, 1536), (33, 4112, 2560)])
+@pytest.mark.parametrize("M,N,K", [(17, 96, 2048), (48, 50, 1536), (33, 4112, 2560), (49, 50, 1536), (64, 4112, 2560)])
 def test_a_following_norm_with_the_sums_of_the_pair(M, N, K):
     """... and through the accumulating product that emits the norm behind it: stream, emitted rows and shares of the squares."""
     from hfee_amd.kernels import ops
@@ -690,7 +691,8 @@ def test_a_following_norm_with_the_sums_of_the_pair(M, N, K):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("H,K,hd,half,M,d", [(4, 2, 16, 8, 17, 2048), (6, 3, 48, 8, 40, 3072), (5, 1, 64, 32, 33, 2560), (2, 2, 128, 64, 48, 1536)])
+@pytest.mark.parametrize("H,K,hd,half,M,d", [(4, 2, 16, 8, 17, 2048), (6, 3, 48, 8, 40, 3072), (5, 1, 64, 32, 33, 2560), (2, 2, 128, 64, 48, 1536),
+                                             (6, 3, 48, 8, 49, 3072), (5, 1, 64, 32, 64, 2560)])
 def test_fused_qkv_with_the_sums_of_the_pair(H, K, hd, half, M, d):
     """... and through q/k/v: the rotated queries and the cache, against the plain form and to the bit."""
     from hfee_amd.kernels import ops
@@ -719,7 +721,7 @@ def test_which_products_run_whole_with_the_sums_of_the_pair(M, N, K, whole):
         got.append((out, bool(torch.isnan(scratch).all())))
     assert torch.equal(got[0][0], got[1][0]) and got[0][1] == whole and not got[1][1]
     few = torch.zeros(16, N, dtype=torch.bfloat16, device=DEV)
-    with pytest.raises(ops.KernelError, match="17 to 48 rows"):
+    with pytest.raises(ops.KernelError, match="17 to 64 rows"):
         ops.linear_fused(few, x[:16], w, "bf16", scratch=scratch, force_mid_rows=3)
 
 

@@ -99,10 +99,11 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch():
                                        (6144, 96, 0), (6150, 260, 0)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_gemm_f32_kernels_give_one_row_the_same_bits(N, K, shift, accumulate):
-    """Every number of rows at which the kernel changes (8 / 9, 16 / 17, 32 / 33 rows, tiles of 32 and 64), output widths and
-    K that fill no tile, K that 16-byte loads do not take, rows that do not start on 16 bytes (`shift`): within the bound of
-    the sums' order (a chain of at most K / 8 + 32 roundings of half an ulp a segment, eight segments, the addition), and
-    the same bits for every number of rows."""
+    """The numbers of rows between which the kernel or its blocks change (5 / 6, 8 / 9, 16 / 17, 24 / 25, 32 / 33 and above by
+    the cost model), output widths and K that fill no tile, K that 16-byte loads do not take, rows that do not start on 16
+    bytes (`shift`): every element within what a chain of float32 additions may be off (K / 8 + 32 roundings of half an
+    ulp a segment, eight segments, the addition; the errors as they are: `test_gemm_f32_errors_against_64_bits`), and the same
+    bits for every number of rows."""
     from hfee_amd.kernels import ops
     g = torch.Generator().manual_seed(N + K)
     most = 200
@@ -124,8 +125,8 @@ def test_gemm_f32_kernels_give_one_row_the_same_bits(N, K, shift, accumulate):
                                    (500, 2048, 2080), (18, 8196, 512), (9, 24580, 288)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_gemm_f32_in_cuts_and_turns_gives_one_row_the_same_bits(M, N, K, accumulate):
-    """Products whose K is cut over workgroups (scratch at hand) and those of few rows whose workgroups go from weight rows to
-    weight rows: the bits of the same rows alone, and nothing behind the scratch that was asked for is written."""
+    """Products in blocks of rows whose waves share K, and one whose K is cut over workgroups (scratch at hand; the numbers of cuts
+    are those of the test below): the bits of the same rows alone, and nothing behind the scratch that was asked for is written."""
     from hfee_amd.kernels import ops
     g = torch.Generator().manual_seed(M + N + K)
     x, w = torch.randn(M, K, generator=g).to(DEV), torch.randn(N, K, generator=g).to(DEV)
@@ -136,7 +137,7 @@ def test_gemm_f32_in_cuts_and_turns_gives_one_row_the_same_bits(M, N, K, accumul
     ops.linear(full, x, w, accumulate=accumulate, scratch=scratch[:words] if words else None)
     assert bool((scratch[words:] == 7.0).all())
     plain = c0.clone()
-    ops.linear(plain, x, w, accumulate=accumulate)
+    ops.linear(plain, x, w, accumulate=accumulate, scratch=scratch[:0])        # (uncut)
     assert torch.equal(plain, full)
     for r in (0, M // 2, M - 1):
         one = c0[r:r + 1].clone()
@@ -189,7 +190,7 @@ def test_gemm_f32_that_would_leave_the_chip_idle_goes_by_blocks_of_rows_or_cuts(
 
 
 @pytest.mark.parametrize("M,N,cut", [(3, 1024, False), (16, 1024, False), (3, 12288, False), (24, 1024, False), (200, 1024, False),
-                                     (200, 1024, True)])
+                                     (200, 1024, True), (500, 4096, False), (500, 4096, True)])
 @pytest.mark.parametrize("K", [64, 2048, 4096, 14336])
 @pytest.mark.parametrize("kind", ["normal", "small", "denormal", "one column"])
 def test_gemm_f32_errors_against_64_bits(M, N, cut, K, kind):
@@ -205,8 +206,9 @@ def test_gemm_f32_errors_against_64_bits(M, N, cut, K, kind):
     elif kind != "normal":
         x, w = x * 2.0 ** (-118 if kind == "small" else -129), w * 2.0 ** 96
     words = ops.linear_scratch(M, N, K, torch.float32) if cut else 0
+    assert not cut or K == 64 or words
     out = torch.empty(M, N, device=DEV)
-    ops.linear(out, x, w, scratch=torch.empty(words, device=DEV) if words else None)
+    ops.linear(out, x, w, scratch=torch.empty(words, device=DEV))       # (without a word K is not cut)
     ref = x.double() @ w.double().t()
     err = out.double() - ref
     bound = (GEMM_F32_ERROR_OF_ONE_COLUMN if kind == "one column" else GEMM_F32_ERROR)[K] * float(ref.norm())

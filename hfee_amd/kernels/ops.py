@@ -220,19 +220,23 @@ def mfma_loop(iterations: int, workgroups: int) -> float:
 
 # ---------------------------------------------------------------- matrix product
 
-def linear_scratch(m: int, n: int, k: int, dtype=torch.bfloat16) -> int:
+def linear_scratch(m: int, n: int, k: int, dtype=torch.bfloat16, pieces: bool = False) -> int:
     """float32 words of scratch that `linear` can use for a product of m rows with an [n, k] weight
     (0: none): with too few tiles for the chip, K is cut over more workgroups, which leave their
-    partial products there for a second kernel to add up.  dtype: bfloat16 or float32, the operands'."""
-    fn = "hfee_gemm_f32_scratch" if dtype == torch.float32 else "hfee_gemm_bf16_scratch"
+    partial products there for a second kernel to add up.  dtype: bfloat16 or float32, the operands'.
+    pieces: with room for x as the bfloat16 pieces that large float32 products multiply."""
+    fn = "hfee_gemm_bf16_scratch" if dtype != torch.float32 else "hfee_gemm_f32_pieces_scratch" if pieces else "hfee_gemm_f32_scratch"
     return int(lib.core().raw(fn)(int(m), int(n), int(k)))
 
 
-def linear_f32_plan(m: int, n: int, k: int, cut: bool):
+def linear_f32_plan(m: int, n: int, k: int, cut: bool, pieces: bool = False):
     """How a float32 product of more than 32 rows, whole steps of K and rows on 16 bytes is done: ("rows", the
-    number of the blocks) or (the pairs of K's segments that a workgroup does, 0 for all, the number of the tile).
-    cut: with scratch at hand.  (For tests.)"""
-    plan = int(lib.core().raw("hfee_gemm_f32_plan")(int(m), int(n), int(k), int(cut)))
+    number of the blocks) or (the pairs of K's segments that a workgroup does, 0 for all, the number of the tile),
+    ("pieces", pairs, tile) with x cut into pieces by a launch of its own.
+    cut: with scratch at hand; pieces: with scratch for pieces too.  (For tests.)"""
+    plan = int(lib.core().raw("hfee_gemm_f32_plan")(int(m), int(n), int(k), 2 if pieces else int(cut)))
+    if plan >= 1024:
+        return ("pieces", (plan - 1024) // 16, plan % 16)
     return ("rows", plan - 256) if plan >= 256 else (plan // 16, plan % 16)
 
 
@@ -309,8 +313,9 @@ def linear_add_norm(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, no
 def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate: bool = False, kernel: int = 0,
            gate: bool = False, scratch=None, activation: str = "silu", numbers=None):
     """out (+)= x @ weight.T, weight stored [out_features, in_features].
-    scratch: float32, `linear_scratch(M, N, K, x.dtype)` words, or None (float32 operands: the call then
-    takes what it has a use for from torch's pool; with an empty tensor K is not cut).
+    scratch: float32, `linear_scratch(M, N, K, x.dtype)` words (float32 operands: with as many as `pieces` asks for there,
+    x may lie in it as pieces too), or None (float32 operands: the call then takes what it has a use for from torch's
+    pool; with an empty tensor K is not cut).
 
     float32 x and weight: the true 32-bit product, out float32.
     bfloat16 x and weight: matrix cores with float32 accumulation; out bfloat16, or
@@ -336,7 +341,7 @@ def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate:
     if x.dtype == torch.float32:
         _check(out.dtype == torch.float32, "linear: float32 product needs a float32 out")
         if scratch is None:
-            words = linear_scratch(M, N, K, torch.float32)
+            words = linear_scratch(M, N, K, torch.float32, pieces=True)
             scratch = torch.empty(words, dtype=torch.float32, device=out.device) if words else None
         else:
             _gpu(scratch)

@@ -310,11 +310,11 @@ class Workspace:
         """The `scratch` argument of `ops.linear` for a product of n_rows rows with this weight
         (empty where it has no use for it)."""
         from ..kernels import ops
-        words = ops.linear_scratch(n_rows, weight.shape[0], weight.shape[1], weight.dtype)
+        words = ops.linear_scratch(n_rows, weight.shape[0], weight.shape[1], weight.dtype, pieces=True)
         return dict(scratch=self.flat("product.partial", words, torch.float32)) if words else {}
 
     def split_scratch_f32(self, n_rows: int, weight: torch.Tensor) -> dict:
-        """The same for products whose K is cut with float32 operands only."""
+        """The same for products that use scratch with float32 operands only."""
         return self.split_scratch(n_rows, weight) if weight.dtype == torch.float32 else {}
 
     def counters(self, name: str, count: int) -> torch.Tensor:

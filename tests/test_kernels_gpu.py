@@ -189,6 +189,39 @@ def test_gemm_f32_that_would_leave_the_chip_idle_goes_by_blocks_of_rows_or_cuts(
     assert ((full.double() - ref).abs()[finite] <= ((K / 8 + 48) * 2.0 ** -24 * mag)[finite]).all()
 
 
+@pytest.mark.parametrize("M,N,K,pairs", [(500, 16384, 512, 0), (385, 10497, 2080, 0), (640, 7000, 4128, 0), (1300, 4100, 16384, 0),
+                                         (999, 2050, 4096, 1), (300, 8190, 4096, 1)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_f32_of_rows_cut_into_pieces_first(M, N, K, pairs, accumulate):
+    """Large products whose rows are laid down as pieces by a launch of their own (last tiles of one row and of few, widths that fill no tile,
+    K of few steps, of an odd number and in one segment's remainder, more rows than are done at a time, K cut over workgroups): the
+    bits of the product that cuts the rows itself, an infinity and a NaN where they belong, and nothing behind the scratch is written."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K + 4, generator=g, device=DEV)[:, :K]
+    w = torch.randn(N, K, generator=g, device=DEV)
+    x[1, 7], w[3, 9] = float("nan"), float("inf")
+    c0 = torch.randn(M, N, generator=g, device=DEV)
+    rows = min(M, (3 << 23) // (K // 32 * 768 * 8) * 128)
+    assert ops.linear_f32_plan(rows, N, K, True, pieces=True) == ("pieces", pairs, 0)
+    words = ops.linear_scratch(M, N, K, torch.float32, pieces=True)
+    assert words >= -(-rows // 16) * (K // 32) * 768
+    scratch = torch.full((words + 64,), 7.0, device=DEV)
+    outs = []
+    for kw in (dict(scratch=scratch[:words]), dict(), dict(scratch=scratch[:0])):
+        out = c0.clone()
+        ops.linear(out, x, w, accumulate=accumulate, **kw)
+        outs.append(out)
+    assert bool((scratch[words:] == 7.0).all()) and not bool((scratch[:words] == 7.0).all())
+    for other in outs[1:]:
+        assert torch.equal(outs[0].view(torch.int32), other.view(torch.int32))
+    ref = x.double() @ w.double().t() + (c0.double() if accumulate else 0)
+    mag = x.abs().double() @ w.abs().double().t() + c0.abs().double()
+    finite = torch.isfinite(ref)
+    assert torch.equal(torch.isnan(outs[0]), torch.isnan(ref)) and int(finite.sum()) == (M - 1) * (N - 1)
+    assert ((outs[0].double() - ref).abs()[finite] <= ((K / 8 + 48) * 2.0 ** -24 * mag)[finite]).all()
+
+
 @pytest.mark.parametrize("M,N,cut", [(3, 1024, False), (16, 1024, False), (3, 12288, False), (24, 1024, False), (200, 1024, False),
                                      (200, 1024, True), (500, 4096, False), (500, 4096, True)])
 @pytest.mark.parametrize("K", [64, 2048, 4096, 14336])

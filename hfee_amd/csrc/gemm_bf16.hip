@@ -735,8 +735,6 @@ inline int large_tile_cuts(int M, int N, int K) {
   return (K + k_split - 1) / k_split;
 }
 
-inline bool cuts_by_large_tiles(int M, int N, int K, int splits) { return splits > 1 && large_tile_cuts(M, N, K) == splits; }
-
 // One round of at most 256 tiles of 128 x 128 by the kernel that loads straight into LDS is faster
 // whole than in cuts once the tiles are many for the length of K: the cuts' partial products and the kernel
 // that adds them cost more than the idle CUs (us, whole against cut, the cut ones with the norm that their
@@ -753,12 +751,12 @@ inline bool whole_in_one_round(int M, int N, int K, int64_t tiles) {
          (int64_t)M * K < (1ll << 30) && (int64_t)N * K < (1ll << 30);
 }
 
-// How many ways K is cut for M x N x K (1: not at all): the large tiles' cuts where they apply;
+// How many ways K is cut for M x N x K (1: not at all) by tiles of 256 or 128 rows: the large tiles' cuts where they apply;
 // else through 128 x 128 tiles: with fewer than 256 of them (384 where K is long) a part of the
 // chip stands idle while a few workgroups walk the whole of K (the output and down products of a
 // prompt of 128 tokens: 32 tiles); the cut makes up to 512 workgroups of them, each with at least
 // 512 columns.
-inline int pipelined_splits(int M, int N, int K) {
+inline int even_splits(int M, int N, int K) {
   const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
   if (whole_in_one_round(M, N, K, tiles)) return 1;
   if (const int cuts = large_tile_cuts(M, N, K); cuts > 1 && K >= 2048) return cuts;
@@ -781,11 +779,69 @@ inline int pipelined_splits(int M, int N, int K) {
   return (K + k_split - 1) / k_split;
 }
 
+// How K is cut, and by which tiles of the kernel that loads straight into LDS: 64 tm rows x 64 tn columns.
+struct Cuts {
+  int cuts, tm, tn;
+};
+
+// Its workgroups: every XCD has as many tiles, and every cut as many workgroups.
+inline int64_t cut_workgroups(const Cuts& c, int M, int N) {
+  const int64_t tiles = (int64_t)((M + 64 * c.tm - 1) / (64 * c.tm)) * ((N + 64 * c.tn - 1) / (64 * c.tn));
+  return (tiles + XCDS - 1) / XCDS * XCDS * c.cuts;
+}
+
+// What a product in cuts takes, in us, while its workgroups are one round: a start and an end, a time a step of 64 columns (both
+// less where CUs stand idle: the others' clock is higher), and the cuts' partial products there and back.  Measured inside
+// 0.9 to 1.15 of it at 96 to 1,024 rows of the 8B and 13B shapes' narrow products.
+inline double cuts_us(const Cuts& c, int M, int N, int K) {
+  struct { double ends, step; } t = c.tm == 4 ? decltype(t){18.5, 0.67} : c.tm == 3 ? decltype(t){15, 0.59}
+                                  : decltype(t){6.5, 0.535};
+  const int64_t workgroups = cut_workgroups(c, M, N);
+  const int steps = ((K + c.cuts - 1) / c.cuts + 63) / 64;
+  const double rounds = (double)((workgroups + 255) / 256), filled = workgroups >= 256 ? 1.0 : workgroups / 256.0;
+  return rounds * (t.ends + steps * t.step) * (0.65 + 0.35 * filled) + c.cuts * (double)M * N * 4 / 5e6;
+}
+
+// The tiles of 256 rows pad many numbers of rows by up to a half, and the matrix cores spend their power on the padding as on the
+// rest; and their number may leave CUs idle.  The same cuts (so the same bits) go through tiles of 192 x 128 where those are
+// expected to be faster.
+// us, tiles of 256 x 128 or 128 x 128 against them, with the kernel that adds the cuts: N 4,096, K 14,336 at 181 / 320 / 520 / 602 /
+// 700 rows 45 / 62 / 90 / 96 / 100 against 38.5 / 55 / 86 / 85 / 90; N 4,096, K 4,096 at 320 / 602 rows 31.5 / 40 against 28 / 36; N 5,120,
+// K 13,824 at 181 / 300 / 520 rows 47 / 72 / 99 against 44 / 62.5 / 88; N 2,048, K 8,192 at 320 rows 31 against 26; the product alone, N 6,144,
+// K 4,096 at 181 / 320 rows 23 / 31 against 21 / 28; N 15,360, K 5,120 at 181 rows 46 against 42.5.
+inline Cuts cuts_of(int M, int N, int K) {
+  const int cuts = even_splits(M, N, K);
+  const Cuts best{cuts, large_tile_cuts(M, N, K) == cuts ? 4 : 2, 2};
+  if (cuts < 2 || M <= 128 || K % 64 != 0) return best;
+  const Cuts rows192{cuts, 3, 2};
+  return cuts_us(rows192, M, N, K) < 0.97 * cuts_us(best, M, N, K) ? rows192 : best;
+}
+
 template <int MODE, int TM, int TN, int NBUF>
 int launch_direct64(void* C, int64_t ldc, const bf16_t* A, int64_t lda, const bf16_t* W, int64_t ldw,
                     int M, int N, int K, const QkvArgs& qkv, hipStream_t stream, int k_split = 0, int splits = 1,
                     int64_t split_stride = 0);
 inline bool large_fits(int64_t lda, int64_t ldw, int M, int N, int K);
+
+// The partial products of a product in cuts, `M * N` words apart from `at` on.  (Two to four us less a product than the kernel of
+// two workgroups a CU, for every cut product of 65 to 512 rows of the 8B, 13B, 3B and 1B shapes, 20 to 50 us each; that one
+// takes what the others do not.)
+inline int launch_cuts(const Cuts& c, float* at, const bf16_t* A, int64_t lda, const bf16_t* W, int64_t ldw, int M, int N, int K,
+                       const QkvArgs& qkv, hipStream_t stream) {
+  const int k_split = ((K + c.cuts - 1) / c.cuts + 63) / 64 * 64;
+  const int64_t stride = (int64_t)M * N;
+  if (large_fits(lda, ldw, M, N, K)) {
+    if (c.tm == 4) return launch_direct64<OUT_F32, 4, 2, 3>(at, N, A, lda, W, ldw, M, N, K, qkv, stream, k_split, c.cuts, stride);
+    if (c.tm == 3) return launch_direct64<OUT_F32, 3, 2, 3>(at, N, A, lda, W, ldw, M, N, K, qkv, stream, k_split, c.cuts, stride);
+    return launch_direct64<OUT_F32, 2, 2, 3>(at, N, A, lda, W, ldw, M, N, K, qkv, stream, k_split, c.cuts, stride);
+  }
+  const size_t lds = (size_t)2 * 256 * PPITCH * sizeof(bf16_t);
+  if (raise_pipelined_lds<OUT_F32>(lds)) return 1;
+  const int64_t tiles = (int64_t)((N + 127) / 128) * ((M + 127) / 128);
+  dim3 grid((unsigned)((tiles + XCDS - 1) / XCDS * XCDS), c.cuts);
+  gemm_bf16_pipelined_kernel<OUT_F32, 2, 2, 3><<<grid, 256, lds, stream>>>(at, N, A, lda, W, ldw, M, N, K, qkv, k_split, stride);
+  return 0;
+}
 
 template <int MODE>
 int launch_pipelined(void* C, int64_t ldc, const bf16_t* A, int64_t lda, const bf16_t* W, int64_t ldw,
@@ -804,27 +860,12 @@ int launch_pipelined(void* C, int64_t ldc, const bf16_t* A, int64_t lda, const b
   if (tiles > (1 << 30)) return fail("gemm_bf16: too many tiles");
   dim3 grid((unsigned)((tiles + XCDS - 1) / XCDS * XCDS));
   if constexpr (MODE == OUT_BF16 || MODE == OUT_F32 || MODE == OUT_ADD_F32) {
-    const int splits = pipelined_splits(M, N, K);
+    const Cuts cut = cuts_of(M, N, K);
+    const int splits = cut.cuts;
     const bool rows_fit = MODE == OUT_BF16 ? (ldc % 4 == 0 && (uintptr_t)C % 8 == 0) : (ldc % 4 == 0 && (uintptr_t)C % 16 == 0);
     if (splits > 1 && rows_fit && partial.at != nullptr && (uintptr_t)partial.at % 16 == 0 &&
         partial.floats >= (int64_t)splits * M * N) {
-      if (raise_pipelined_lds<OUT_F32>(lds)) return 1;
-      const int k_split = ((K + splits - 1) / splits + 63) / 64 * 64;
-      if (cuts_by_large_tiles(M, N, K, splits) && large_fits(lda, ldw, M, N, K)) {
-        if (launch_direct64<OUT_F32, 4, 2, 3>(partial.at, N, A, lda, W, ldw, M, N, K, qkv, stream, k_split, splits,
-                                              (int64_t)M * N))
-          return 1;
-      } else if (large_fits(lda, ldw, M, N, K)) {
-        // (the kernel that loads straight into LDS, with 128 x 128 tiles: 2 to 4 us less than the one below
-        // for every cut product of 65 to 512 rows of the 8B, 13B, 3B and 1B shapes, 20 to 50 us each)
-        if (launch_direct64<OUT_F32, 2, 2, 3>(partial.at, N, A, lda, W, ldw, M, N, K, qkv, stream, k_split, splits,
-                                              (int64_t)M * N))
-          return 1;
-      } else {
-        grid.y = splits;
-        gemm_bf16_pipelined_kernel<OUT_F32, TM, TN, STAGES><<<grid, 256, lds, stream>>>(
-            partial.at, N, A, lda, W, ldw, M, N, K, qkv, k_split, (int64_t)M * N);
-      }
+      if (launch_cuts(cut, partial.at, A, lda, W, ldw, M, N, K, qkv, stream)) return 1;
       if constexpr (MODE == OUT_ADD_F32) {
         if (norm.normed != nullptr && launch_finish_norm((float*)C, ldc, partial.at, splits, M, N, norm, stream)) {
           *normed = true;
@@ -1356,7 +1397,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_bf16_skinny_kernel(
 
 // Which tiled kernel takes an aligned product: force_kernel 2 the 128 x 128 tiles, 4 the
 // 256 x 256 tiles, 5 the 256 x 128 tiles, 6 the 256 x 192 tiles, 7 and 8 the 128 x 128 and 128 x 192 tiles
-// of the kernel that loads straight into LDS, anything else the one expected to be fastest:
+// of the kernel that loads straight into LDS, anything else the one expected to be fastest (9 and 10, its tiles of 192 x 128 and
+// 192 x 192, among them):
 // rounds of tiles over the chip times the time of a tile, with the share of the matrix
 // peak that each kernel was measured to reach on a busy CU (128 x 128: two workgroups a
 // CU; the large tiles reach more the longer K is, and a tile of empty rows costs as
@@ -1380,13 +1422,15 @@ inline TiledPlan plan_tiled(int M, int N, int K, bool large_ok, bool may_split) 
   auto rounds = [&](double t, int slots) { return (double)(int64_t)((t + slots - 1) / slots); };
   // time of kernel k on n columns, in tile elements over the share of the peak
   auto cost = [&](int k, int n) {
-    const int bm = k == 2 || k == 8 ? 128 : 256, bn = k == 2 ? 128 : k == 4 ? 256 : k == 5 ? 128 : 192;
+    const int bm = k == 2 || k == 8 ? 128 : k == 9 || k == 10 ? 192 : 256, bn = k == 2 || k == 5 || k == 9 ? 128 : k == 4 ? 256 : 192;
     const double t = (double)((M + bm - 1) / bm) * ((n + bn - 1) / bn);
     // (128 x 192 tiles, the 256 x 128 kernel compiled for them: where they are at most one a CU.  2,048 rows of
     // 3,072 columns are 256 of them and 96 of 256 x 128: N 3,072 at K 2,048 / 3,072 / 8,192 33.2 / 48.9 / 97.0 us against
     // 35.6 / 53.3 / 101.9; 1,024 rows of N 6,144, K 4,096 52.2 against 56.6, of N 5,120, K 5,120 60.6 against 66.8;
-    // in a second round they lose to every other tile)
-    if (k == 8) return t <= cus ? 128.0 * 192 / (0.335 * fill) : 1e30;
+    // in more rounds they are as good as what they pad and leave idle)
+    if (k == 8) return rounds(t, cus) * 128 * 192 / (0.34 * fill);
+    if (k == 9) return rounds(t, cus) * 192 * 128 / (0.335 * fill);
+    if (k == 10) return rounds(t, cus) * 192 * 192 / (0.42 * fill);
     // (up to a tile a CU: the 128 x 128 tiles go to the kernel that loads straight into LDS)
     if (k == 2) return t <= cus ? 128.0 * 128 / (t <= 256 ? 0.30 : 0.22) : rounds(t, 2 * cus) * 2 * 128 * 128 / 0.31;
     return rounds(t, cus) * bm * bn / ((k == 4 ? 0.46 : k == 5 ? 0.42 : 0.44) * fill);
@@ -1394,7 +1438,8 @@ inline TiledPlan plan_tiled(int M, int N, int K, bool large_ok, bool may_split) 
   TiledPlan best{2, N, 0};
   double best_cost = cost(2, N);
   for (int k : {5, 6, 4, 8})
-    if (cost(k, N) < best_cost || (k == 4 && cost(k, N) <= best_cost)) {
+    if (k == 8 && (int64_t)((M + 127) / 128) * ((N + 191) / 192) > cus) continue;      // (more rounds: below)
+    else if (cost(k, N) < best_cost || (k == 4 && cost(k, N) <= best_cost)) {
       best = TiledPlan{k, N, 0};
       best_cost = cost(k, N);
     }
@@ -1421,6 +1466,17 @@ inline TiledPlan plan_tiled(int M, int N, int K, bool large_ok, bool may_split) 
       }
     }
   }
+  // Tiles of 192 rows where those of 256 pad more, and rounds of 128 x 192: us, 256 x 128 or 256 x 192 tiles or two launches against
+  // them: N 28,672, K 4,096 at 130 / 192 / 520 / 602 rows 61.7 / 64.0 / 151 / 156 against 56.9 / 59.9 / 125 / 147; N 16,384, K 2,048 at 260 / 384
+  // rows 33.7 / 33.6 against 28.3 / 29.6; N 15,360, K 5,120 at 520 / 1,100 rows 98 / 171 against 80 / 152; N 6,144, K 4,096 at 1,400
+  // rows 74.8 against 61.4; N 4,096, K 14,336 at 1,479 rows 179 against 160.  The sums have these kernels' one order; products that go to the
+  // kernel of two workgroups a CU, or are cut, stay there.
+  const bool another_order = best.first == 2 || (best.second == 2 && (int64_t)((M + 127) / 128) * ((N - best.n1 + 127) / 128) > 256);
+  for (int k : {8, 9, 10})
+    if (!another_order && cost(k, N) < best_cost) {
+      best = TiledPlan{k, N, 0};
+      best_cost = cost(k, N);
+    }
   return best;
 }
 
@@ -1433,6 +1489,8 @@ int launch_tiled_kernel(int choice, void* C, int64_t ldc, const bf16_t* A, int64
   if (choice == 5) return launch_direct64<MODE, 4, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream);
   if (choice == 7) return launch_direct64<MODE, 2, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream);
   if (choice == 8) return launch_direct64<MODE, 2, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream);
+  if (choice == 9) return launch_direct64<MODE, 3, 2, 3>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream);
+  if (choice == 10) return launch_direct64<MODE, 3, 3, 3>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream);
   return launch_pipelined<MODE>(C, ldc, A, lda, W, ldw, M, N, K, qkv, stream, partial, NormAfter{}, nullptr, forced);
 }
 
@@ -1507,12 +1565,22 @@ HFEE_API int hfee_gemm_bf16_plan(int M, int N, int K, int* first, int* n1, int* 
   return 0;
 }
 
+// How such a product is cut along K where it is (1 cut: it is not), and the rows and columns of the tiles: for tests.
+HFEE_API int hfee_gemm_bf16_cut_plan(int M, int N, int K, int* cuts, int* rows, int* columns) {
+  HFEE_REQUIRE(M > 0 && N > 0 && K > 0 && cuts && rows && columns, "gemm_bf16_cut_plan: bad arguments");
+  const Cuts c = cuts_of(M, N, K);
+  *cuts = c.cuts;
+  *rows = 64 * c.tm;
+  *columns = 64 * c.tn;
+  return 0;
+}
+
 // float32 words of scratch that hfee_gemm_bf16 can use for M x N x K (0: none): products with
 // too few tiles for the chip are cut along K over more workgroups, which leave their partial
 // products there for a second kernel to add up.
 HFEE_API int hfee_gemm_bf16_scratch(int M, int N, int K) {
   if (skinny_pays(M, N, K)) return 0;                    // (the streaming kernel cuts nothing)
-  const int splits = pipelined_splits(M, N, K);          // (fewer than 256 tiles of 128 x 128, at most 8 cuts: it fits an int)
+  const int splits = cuts_of(M, N, K).cuts;              // (fewer than 256 tiles of 128 x 128, at most 8 cuts: it fits an int)
   return splits > 1 ? splits * M * N : 0;
 }
 
@@ -1616,28 +1684,11 @@ HFEE_API int hfee_gemm_bf16_cuts(const void* A, int64_t lda, const void* W, int6
   const bool vec = (K % 8 == 0) && (lda % 8 == 0) && (ldw % 8 == 0) && ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);
   if (!vec || skinny_pays(M, N, K) || scratch == nullptr || (uintptr_t)scratch % 16 != 0 || N % 4 != 0) return 0;
   const TiledPlan plan = plan_tiled(M, N, K, large_fits(lda, ldw, M, N, K), true);
-  const int splits = pipelined_splits(M, N, K);
-  if (plan.first != 2 || plan.second != 0 || splits < 2 || scratch_floats < (int64_t)splits * M * N) return 0;
-  constexpr int TM = 2, TN = 2, STAGES = 3;
-  const int k_split = ((K + splits - 1) / splits + 63) / 64 * 64;
-  if (cuts_by_large_tiles(M, N, K, splits) && large_fits(lda, ldw, M, N, K)) {
-    if (launch_direct64<OUT_F32, 4, 2, 3>(scratch, N, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, QkvArgs{}, stream,
-                                          k_split, splits, (int64_t)M * N))
-      return 1;
-  } else if (large_fits(lda, ldw, M, N, K)) {
-    if (launch_direct64<OUT_F32, 2, 2, 3>(scratch, N, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, QkvArgs{}, stream,
-                                          k_split, splits, (int64_t)M * N))
-      return 1;
-  } else {
-    const size_t lds = (size_t)2 * (64 * TM + 64 * TN) * PPITCH * sizeof(bf16_t);
-    if (raise_pipelined_lds<OUT_F32>(lds)) return 1;
-    const int64_t tiles = (int64_t)((N + 64 * TN - 1) / (64 * TN)) * ((M + 64 * TM - 1) / (64 * TM));
-    dim3 grid((unsigned)((tiles + XCDS - 1) / XCDS * XCDS), splits);
-    gemm_bf16_pipelined_kernel<OUT_F32, TM, TN, STAGES><<<grid, 256, lds, stream>>>(
-        scratch, N, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, QkvArgs{}, k_split, (int64_t)M * N);
-  }
+  const Cuts cut = cuts_of(M, N, K);
+  if (plan.first != 2 || plan.second != 0 || cut.cuts < 2 || scratch_floats < (int64_t)cut.cuts * M * N) return 0;
+  if (launch_cuts(cut, scratch, (const bf16_t*)A, lda, (const bf16_t*)W, ldw, M, N, K, QkvArgs{}, stream)) return 1;
   HFEE_CHECK_LAUNCH("gemm_bf16_cuts");
-  *cuts = splits;
+  *cuts = cut.cuts;
   return 0;
 }
 

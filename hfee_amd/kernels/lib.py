@@ -32,6 +32,7 @@ _CORE_SIGNATURES = {
     "hfee_rope_cache_write": [P, L, P, L, P, L, I, P, P, P, I, P, P, I, I, I, I, P, I, I, I, I, I, I, P],
     "hfee_gemm_f32": [P, L, P, L, P, L, I, I, I, I, P, L, P],
     "hfee_gemm_f32_scratch": [I, I, I],
+    "hfee_gemm_f32_pieces_scratch": [I, I, I],
     "hfee_gemm_f32_plan": [I, I, I, I],
     "hfee_attention_f32": [P, L, P, L, P, P, P, P, I, I, I, I, I, F, I, P, I, I, I, P],
     "hfee_attention_ref": [P, L, P, L, P, I, P, P, P, I, I, I, I, I, F, I, I, P],
@@ -41,6 +42,7 @@ _CORE_SIGNATURES = {
     "hfee_rope_cache_write_cuts": [P, L, P, I, P, P, P, I, P, P, I, I, I, P, I, I, I, I, I, I, P],
     "hfee_gemm_bf16_scratch": [I, I, I],
     "hfee_gemm_bf16_plan": [I, I, I, P, P, P],
+    "hfee_gemm_bf16_cut_plan": [I, I, I, P, P, P],
     "hfee_gemm_skinny": [P, L, P, I, L, P, L, I, I, I, I, P, I, F, P, P, P, P, I, P, P, I, I, P, I, I, I, I,
                          P, I, P, L, P, P, I, F, P, L, I, P],
     "hfee_gemm_qkv_rows": [P, L, P, L, P, L, I, I, I, P, P, P, I, P, P, I, I, P, I, I, I, I, P],

@@ -373,6 +373,13 @@ def tiled_plan(m: int, n: int, k: int) -> tuple:
     return first.value, n1.value, second.value
 
 
+def cut_plan(m: int, n: int, k: int) -> tuple:
+    """(cuts, tile rows, tile columns) of an aligned bfloat16 product whose K is cut over workgroups (1 cut: it is not)."""
+    cuts, rows, columns = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    lib.core().call("hfee_gemm_bf16_cut_plan", m, n, k, ctypes.byref(cuts), ctypes.byref(rows), ctypes.byref(columns))
+    return cuts.value, rows.value, columns.value
+
+
 # --------------------------------------------------------- rotation and the cache
 
 def rope_cache_write(q, k, v, positions, token_segment, block_tables, cos, sin, pairing: int,

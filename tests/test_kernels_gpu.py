@@ -447,6 +447,62 @@ def test_gemm_bf16_tiled_large(M, N, K, kernel):
         assert (err <= 2e-2 * (1 + mag[:, 0::2]) * (1 + mag[:, 1::2])).all()
 
 
+# (the tile that the rule takes for these: 9 is 192 x 128, 10 is 192 x 192, 8 128 x 192 in three rounds)
+@pytest.mark.parametrize("M,N,K,tile", [(129, 28672, 512, 9), (192, 28570, 576, 9), (191, 27648, 1088, 9), (513, 28672, 512, 10),
+                                        (576, 28674, 704, 10), (1281, 6144, 1024, 10), (602, 28672, 512, 8)])
+def test_gemm_bf16_in_tiles_of_192_rows(M, N, K, tile):
+    """Whole products whose tiles of 192 rows pad less than those of 256 (first, last and full numbers of rows, weight rows that
+    are no multiple of a tile, K of an odd number of steps), and rounds of 128 x 192: every epilogue, the bits of 256 x 128 tiles."""
+    from hfee_amd.kernels import ops
+    assert ops.tiled_plan(M, N, K) == (tile, N, 0)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    c0 = torch.randn(M, N, generator=g, device=DEV)
+    for mode in ("bf16", "f32", "add", "gate"):
+        outs = []
+        for kernel in (0, 5):
+            if mode == "gate":
+                out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+                ops.linear(out, x, w, gate=True, kernel=kernel)
+            elif mode == "add":
+                out = c0.clone()
+                ops.linear(out, x, w, accumulate=True, kernel=kernel)
+            else:
+                out = torch.full((M, N), float("nan"), dtype=torch.bfloat16 if mode == "bf16" else torch.float32, device=DEV)
+                ops.linear(out, x, w, kernel=kernel)
+            outs.append(out)
+        assert torch.equal(*outs), mode
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    assert ((outs[0].double() - torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]).abs() <=
+            2e-2 * (1 + mag[:, 0::2]) * (1 + mag[:, 1::2])).all()
+
+
+@pytest.mark.parametrize("M,N,K,cuts", [(129, 4096, 14336, 8), (192, 15360, 4160, 2), (257, 6144, 4096, 2), (384, 4100, 8256, 3),
+                                        (300, 5120, 13824, 3), (602, 4092, 14400, 2)])
+def test_gemm_bf16_cut_for_tiles_that_pad_less(M, N, K, cuts):
+    """K cut over workgroups whose tiles are 192 x 128 (a last cut that is shorter, rows and columns that fill no tile): the partial products are the same columns' whole products to the bit, and their sum is added as ever."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g, device=DEV) / math.sqrt(K)).to(torch.bfloat16)
+    assert ops.linear_scratch(M, N, K) == cuts * M * N and ops.cut_plan(M, N, K) == (cuts, 192, 128)
+    scratch = torch.full((cuts * M * N + 64,), 7.0, dtype=torch.float32, device=DEV)
+    assert ops.linear_cuts(x, w, scratch) == cuts
+    assert bool((scratch[cuts * M * N:] == 7.0).all())
+    parts, split = scratch[:cuts * M * N].view(cuts, M, N), ((K + cuts - 1) // cuts + 63) // 64 * 64
+    total = None
+    for i in range(cuts):
+        part = torch.empty(M, N, dtype=torch.float32, device=DEV)
+        ops.linear(part, x[:, i * split:(i + 1) * split], w[:, i * split:(i + 1) * split], kernel=5)
+        assert torch.equal(parts[i], part), i
+        total = part if total is None else total + part
+    c0 = torch.randn(M, N, generator=g, device=DEV)
+    out = c0.clone()
+    ops.linear(out, x, w, accumulate=True, scratch=scratch[:cuts * M * N])
+    assert torch.equal(out, total + c0)
+
+
 def test_gemm_bf16_over_two_launches():
     """A product whose last round of large tiles would fill a part of the chip only goes
     to two kernels, split along the weight rows: every epilogue, the seam included."""

@@ -30,12 +30,13 @@
 // (moe_up_by_expert, moe_down_by_expert), an expert's rows once for up to four of its pairs, with the same sums.
 //
 // Grouped (moe_group, moe_group_tiled, moe_combine; bfloat16): the (token, expert) pairs of a step are put
-// in the order of their experts on the device, cut into tiles of up to 128 pairs of one expert, and a workgroup
+// in the order of their experts on the device, cut into tiles of up to 192 pairs of one expert, and a workgroup
 // multiplies a tile by 256 rows of that expert's matrix on the matrix cores, both operands straight into LDS
 // (moe_direct; sizes that are no multiples of 64 and many pairs of a width of 64: tiles of 64 pairs by way of registers):
 // an expert's matrices are read once for its pairs and not once a pair.  A pair's numbers do not depend on which pairs share its tile.
 #include "common.h"
 
+#include <cmath>
 #include <type_traits>
 
 using namespace hfee;
@@ -403,7 +404,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kTilePairs = 64, kTileRows = 256;
 
 // One workgroup.  order: the pairs (t * top + j) by expert; tiles: (expert, first place in order, pairs)
-// for every tile, tiles[3 * most_tiles] holds their number.  Which of an expert's pairs comes first is
+// for every tile, tiles[3 * most_tiles] holds their number.  An expert's pairs make as few tiles of up to tile_pairs as they
+// can, of whole 32s but the last one and alike to within one 32.  Which of an expert's pairs comes first is
 // left to chance; nothing that is computed depends on it.
 __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order, int* __restrict__ tiles, int most_tiles,
                                                          const int* __restrict__ chosen, const int* __restrict__ table,
@@ -437,13 +439,17 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
     const int e = expert_of(chosen, table, token_ids, p / top, p % top, top);
     if (e >= 0 && e < experts) order[starts[e] + atomicAdd(&cursor[e], 1)] = p;
   }
-  for (int e = threadIdx.x; e < experts; e += blockDim.x)
-    for (int i = 0; i * tile_pairs < counts[e]; ++i) {
+  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
+    const int n_tiles = (counts[e] + tile_pairs - 1) / tile_pairs, groups = (counts[e] + 31) / 32;
+    for (int i = 0, at = 0; i < n_tiles; ++i) {
+      const int mine = 32 * (groups / n_tiles + (i < groups % n_tiles ? 1 : 0));
       int* tl = tiles + 3 * (first_tile[e] + i);
       tl[0] = e;
-      tl[1] = starts[e] + i * tile_pairs;
-      tl[2] = min(tile_pairs, counts[e] - i * tile_pairs);
+      tl[1] = starts[e] + at;
+      tl[2] = min(mine, counts[e] - at);
+      at += mine;
     }
+  }
 }
 
 // The grouped products through LDS.  A workgroup takes a tile of up to 64 pairs of one expert and 256 rows of
@@ -613,22 +619,30 @@ __device__ __forceinline__ void store_pair_rows(void* dst, int64_t ldo, int pair
   }
 }
 
-// The same products for K in multiples of 64: tiles of up to 128 pairs and 256 rows of weights, four waves with all the
+// The same products for K in multiples of 64: tiles of up to 192 pairs and 256 rows of weights, four waves with all the
 // pairs and 64 rows each (KIND 0: 32 of each matrix).  The instruction and the order of a sum over K are those of
-// moe_group_tiled, so a pair has the same bits in both.  A step of 64 columns is 128 bytes a row; rows go from memory
-// straight into one of three buffers in LDS, asked for two steps before they are read, and a row's eight 16-byte chunks lie
-// at chunk ^ (row % 8), so that the rows that a read asks the same chunk of spread over the banks.  A tile of at most 64
-// pairs brings and multiplies only those, and has room for a fourth buffer.
+// moe_group_tiled, so a pair has the same bits in both.  Rows go from memory straight into one of three or four buffers in LDS,
+// asked for as many steps before they are read less one.  A tile brings and multiplies its pairs in groups of 32.  Up to 128
+// pairs a step is 64 columns, 128 bytes a row, whose eight 16-byte chunks lie at chunk ^ (row % 8), so that the rows that a
+// read asks the same chunk of spread over the banks (up to 64 pairs leave room for a fourth buffer); with more pairs a step is
+// 32 columns, 64 bytes a row, its four chunks at chunk ^ (bit 3 of the row | bit 2 << 1), and there are four buffers.
 //
-// Why 128 pairs: with 64 pairs a step's 20 KB fed 256 cycles of the matrix cores, more than the 64 bytes a cycle that a CU
-// gets from L2, and the loads came by way of registers one step ahead.  The whole feed-forward, 9 / 128 / 800 / 2,048 tokens
+// Why so many pairs: with 64 pairs a step's 20 KB fed 256 cycles of the matrix cores, more than the 64 bytes a cycle that a CU
+// gets from L2, and an expert's rows came once for every tile of its pairs.  The whole feed-forward, 9 / 128 / 800 / 2,048 tokens
 // on two of 16 experts of 2,048, width 4,096 (206 GFLOP at 2,048; 805 MB of weights): moe_group_tiled 225 / 252 / 428 / 804
-// us, this 128 / 178 / 213 / 374 (with three buffers at 64 pairs too 160 / 208 / 246 / 388).  What bounds it now is the wait
-// for weight rows from memory: LDS holds two or three steps ahead.  (Blocks of rows that begin their walk over K at places of
-// their own spread their lines over more of the memory's channels, 123 / 168 / 200 / 400 us with instructions of 16 x 16 and
-// three buffers, but then a pair's sums have another order of additions, and bits, than in moe_group_tiled.)
-constexpr int kWidePairs = 128, kDirectLds = 4 * (kWidePairs / 2 + kTileRows) * 128;      // (three buffers with all the pairs are less)
-static_assert(kDirectLds >= 3 * (kWidePairs + kTileRows) * 128 && kDirectLds <= 160 * 1024);
+// us, tiles of 128 pairs 128 / 178 / 213 / 374 (380 with weights that are in no cache), this 356 for 2,048; 1,200 276 -> 266;
+// 16 of 1,024, width 2,048, 2,048 tokens 155 -> 115 (an expert's 256 pairs, and a few more, are two tiles instead of three).
+// What bounds it now is memory: all workgroups walk the same columns of rows that lie 8 KB apart, and such a walk alone, 128
+// bytes of 65,536 rows a step without any product, gets 4.4 TB/s whatever is in flight (121 us of the up product's 537 MB).
+// (Blocks of rows that begin their walk over K at places of their own get 6.0 TB/s, but then a pair's sums have another order
+// of additions, and bits, than in moe_group_tiled; so would 512 bytes a row, 5.1, for which LDS has no room.)
+constexpr int kMostGroups = 6;                                        // of 32 pairs a tile
+constexpr int direct_row(int groups) { return groups <= 4 ? 128 : 64; }                       // bytes of a row in a buffer
+constexpr int direct_buffers(int groups) { return groups == 3 || groups == 4 ? 3 : 4; }
+constexpr int direct_pair_rows(int groups) { return groups <= 4 ? 32 * groups : (groups + 1) / 2 * 64; }      // (a request of 64-byte rows is 16 of them a wave)
+constexpr int direct_lds(int groups) { return direct_buffers(groups) * (direct_pair_rows(groups) + kTileRows) * direct_row(groups); }
+constexpr int kDirectLds = direct_lds(2);                             // the most of all
+static_assert(kDirectLds >= direct_lds(4) && kDirectLds >= direct_lds(kMostGroups) && kDirectLds <= 160 * 1024);
 
 template <int KIND>
 __global__ __launch_bounds__(256) void moe_direct_kernel(
@@ -637,7 +651,6 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
     int n_rows, int K, int add, const float* __restrict__ pair_weights, float weight, int gate_act, GateNumbers numbers,
     uint32_t src_bytes) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the host pass has no buffer resources; it only needs the stub
-  constexpr int ROW = 128;
   constexpr int kRowsOut = KIND == 0 ? kTileRows / 2 : kTileRows;      // rows of the result a workgroup makes
   extern __shared__ __attribute__((aligned(1024))) char lds_bytes[];
   const int n_tiles = tiles[3 * most_tiles], row_blocks = (n_rows + kRowsOut - 1) / kRowsOut, items = n_tiles * row_blocks;
@@ -663,47 +676,52 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
   const int* tl = tiles + 3 * (tile0 + within % (tile1 - tile0));
   const int first = tl[1], count = tl[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 31, g = lane >> 5;
-  const int steps = K / 64;
 
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  const int lrow = 8 * wave + (lane >> 3), chunk = (lane & 7) ^ (lrow & 7);      // of the rows that a wave's request t brings: + 32 t
   const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, (int)src_bytes, 0x00020000);
   const int64_t expert = (int64_t)e * n_rows * K;
   const int matrix_bytes = (int)((uint32_t)n_rows * (uint32_t)K * 2u);
   const __amdgpu_buffer_rsrc_t w0_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)(w0 + expert), 0, matrix_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t w1_rsrc =
       __builtin_amdgcn_make_buffer_rsrc((void*)((KIND == 0 ? w1 : w0) + expert), 0, matrix_bytes, 0x00020000);
-  uint32_t a_off[kWidePairs / 32], w_off[kTileRows / 32];
-#pragma unroll
-  for (int t = 0; t < kWidePairs / 32; ++t) {
-    const int pair = order[first + min(lrow + 32 * t, count - 1)];
-    a_off[t] = (uint32_t)((KIND == 2 ? pair : pair / top) * ld_src + 8 * chunk) * 2;
-  }
-#pragma unroll
-  for (int t = 0; t < kTileRows / 32; ++t) {
-    const int s = lrow + 32 * t;                                     // the row's place in the staged tile
-    w_off[t] = ((uint32_t)min(row0 + (KIND == 0 && s >= kRowsOut ? s - kRowsOut : s), n_rows - 1) * (uint32_t)K + 8 * chunk) * 2;
-  }
-
   const auto work = [&](auto subtiles) {
     constexpr int PT = decltype(subtiles)::value;                    // groups of 32 pairs
-    // (a request a 32 rows; what a wave reads and multiplies of 32 columns, which are two instructions' 16 each)
-    constexpr int BUFFERS = PT == 4 ? 3 : 4, BUFFER = (32 * PT + kTileRows) * ROW;       // (kDirectLds bytes in all)
-    constexpr int A_LOADS = PT, LOADS = A_LOADS + kTileRows / 32, READS = 2 * (2 + PT), PRODUCTS = 2 * 2 * PT;
+    constexpr int ROW = direct_row(PT), BUFFERS = direct_buffers(PT), A_ROWS = direct_pair_rows(PT), BUFFER = (A_ROWS + kTileRows) * ROW;
+    constexpr int CHUNKS = ROW / 16;                                  // of a row
+    // (a request a wave is a kilobyte, REQUEST rows of the four waves; what a wave reads and multiplies of half a step's
+    // columns, which are SIXTEENS instructions' 16 each)
+    constexpr int REQUEST = 4096 / ROW, SIXTEENS = ROW / 64;
+    constexpr int A_LOADS = A_ROWS / REQUEST, LOADS = A_LOADS + kTileRows / REQUEST, READS = SIXTEENS * (2 + PT), PRODUCTS = SIXTEENS * 2 * PT;
+    constexpr int EARLY = LOADS / 2;                                  // of a step's requests that go out in a step's second half
+    const int steps = K * 2 / ROW;
+    // where a row's chunk lies in it
+    const auto turned = [](int row, int chunk) { return CHUNKS == 8 ? chunk ^ (row & 7) : chunk ^ (((row >> 3) & 1) | ((row >> 1) & 2)); };
+    const int lrow = (64 / CHUNKS) * wave + lane / CHUNKS, chunk = turned(lrow, lane % CHUNKS);      // of the rows that a wave's request t brings: + REQUEST t
+    uint32_t a_off[A_LOADS], w_off[kTileRows / REQUEST];
+#pragma unroll
+    for (int t = 0; t < A_LOADS; ++t) {
+      const int pair = order[first + min(lrow + REQUEST * t, count - 1)];
+      a_off[t] = (uint32_t)((KIND == 2 ? pair : pair / top) * ld_src + 8 * chunk) * 2;
+    }
+#pragma unroll
+    for (int t = 0; t < kTileRows / REQUEST; ++t) {
+      const int s = lrow + REQUEST * t;                                // the row's place in the staged tile
+      w_off[t] = ((uint32_t)min(row0 + (KIND == 0 && s >= kRowsOut ? s - kRowsOut : s), n_rows - 1) * (uint32_t)K + 8 * chunk) * 2;
+    }
     const auto load_one = [&](int step, int buffer, int t) {
       const int at = min(step, steps - 1) * ROW;                     // (past the end: a repeat that nobody uses)
       char* to = lds_bytes + buffer * BUFFER + wave * 1024;
       if (t < A_LOADS) __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (lds_ptr)(to + t * 4096), 16, a_off[t], at, 0, 0);
-      else __builtin_amdgcn_raw_ptr_buffer_load_lds(t - A_LOADS < kTileRows / 64 ? w0_rsrc : w1_rsrc,
+      else __builtin_amdgcn_raw_ptr_buffer_load_lds(t - A_LOADS < kTileRows / REQUEST / 2 ? w0_rsrc : w1_rsrc,
                                                     (lds_ptr)(to + t * 4096), 16, w_off[t - A_LOADS], at, 0, 0);
     };
     struct Operands {
-      bf16x8 w[2][2], a[2][PT];
+      bf16x8 w[SIXTEENS][2], a[SIXTEENS][PT];
     };
     const auto read_one = [&](int buffer, int half, Operands& o, int i) {      // in the order in which the products need them
       const int sixteen = i / (2 + PT), t = i % (2 + PT);
-      const char* tile = lds_bytes + buffer * BUFFER + r * ROW + (((4 * half + 2 * sixteen + g) ^ (r & 7)) << 4);
-      if (t < 2) o.w[sixteen][t] = *reinterpret_cast<const bf16x8*>(tile + (32 * PT + (KIND == 0 ? t * kRowsOut + wave * 32 : wave * 64 + t * 32)) * ROW);
+      const char* tile = lds_bytes + buffer * BUFFER + r * ROW + (turned(r, 2 * SIXTEENS * half + 2 * sixteen + g) << 4);
+      if (t < 2) o.w[sixteen][t] = *reinterpret_cast<const bf16x8*>(tile + (A_ROWS + (KIND == 0 ? t * kRowsOut + wave * 32 : wave * 64 + t * 32)) * ROW);
       else o.a[sixteen][t - 2] = *reinterpret_cast<const bf16x8*>(tile + (t - 2) * 32 * ROW);
     };
     f32x16 acc[2][PT];
@@ -732,25 +750,31 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
         for (int p = 0; p < PRODUCTS; ++p) multiply_one(o, p);
       }
     } else {
+      // A step's buffer is free from the middle of its step on (its reads end before the barrier there): the first EARLY
+      // requests of step s + BUFFERS go out in the second half of step s, the others in the first half of step s + 1, so
+      // that they stand between matrix instructions one by one.
 #pragma unroll
       for (int s = 0; s < BUFFERS; ++s)
 #pragma unroll
-        for (int t = 0; t < LOADS; ++t) load_one(s, s, t);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFFERS - 1) * LOADS) : "memory");
+        for (int t = 0; t < (s < BUFFERS - 1 ? LOADS : EARLY); ++t) load_one(s, s, t);
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFFERS - 2) * LOADS + EARLY) : "memory");
       barrier_no_fence();
       Operands o[2];
 #pragma unroll
       for (int i = 0; i < READS; ++i) read_one(0, 0, o[0], i);
-      int now = 0;                                                     // the step's buffer
+      int now = 0, before = BUFFERS - 1;                               // the step's buffer, and that of the step before
       for (int s = 0; s < steps; ++s) {
         const int next = now == BUFFERS - 1 ? 0 : now + 1;
-        // the first 32 columns, with the reads of the others
+        // the first half of the columns, with the reads of the others
 #pragma unroll
         for (int p = 0; p < PRODUCTS; ++p) {
           multiply_one(o[0], p);
 #pragma unroll
           for (int i = 0; i < READS; ++i)
             if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(now, 1, o[1], i);
+#pragma unroll
+          for (int l = 0; l < LOADS - EARLY; ++l)
+            if (l >= (LOADS - EARLY) * p / PRODUCTS && l < (LOADS - EARLY) * (p + 1) / PRODUCTS) load_one(s + BUFFERS - 1, before, EARLY + l);
           __builtin_amdgcn_sched_barrier(0);
         }
         // this wave's part of step s + 1 has landed and its reads of step s are done; behind the barrier everybody's
@@ -763,10 +787,11 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
           for (int i = 0; i < READS; ++i)
             if (i >= 2 * READS * p / PRODUCTS && i < 2 * READS * (p + 1) / PRODUCTS) read_one(next, 0, o[0], i);
 #pragma unroll
-          for (int l = 0; l < LOADS; ++l)
-            if (l >= LOADS * p / PRODUCTS && l < LOADS * (p + 1) / PRODUCTS) load_one(s + BUFFERS, now, l);
+          for (int l = 0; l < EARLY; ++l)
+            if (l >= EARLY * p / PRODUCTS && l < EARLY * (p + 1) / PRODUCTS) load_one(s + BUFFERS, now, l);
           __builtin_amdgcn_sched_barrier(0);
         }
+        before = now;
         now = next;
       }
       // the repeats asked for past the end still write into this workgroup's LDS: they land before the wave ends
@@ -791,8 +816,13 @@ __global__ __launch_bounds__(256) void moe_direct_kernel(
         }
     }
   };
-  if (count > 64) work(std::integral_constant<int, 4>{});
-  else work(std::integral_constant<int, 2>{});
+  switch ((count + 31) / 32) {
+    case 0: case 1: case 2: return work(std::integral_constant<int, 2>{});
+    case 3: return work(std::integral_constant<int, 3>{});
+    case 4: return work(std::integral_constant<int, 4>{});
+    case 5: return work(std::integral_constant<int, 5>{});
+    default: return work(std::integral_constant<int, kMostGroups>{});
+  }
 #endif
 }
 
@@ -811,6 +841,20 @@ int launch_direct(int most, void* dst, int64_t ldo, const bf16_t* src, int64_t l
                                                               (uint32_t)(((src_rows - 1) * ld_src + K) * 2));
   HFEE_CHECK_LAUNCH("moe_grouped");
   return 0;
+}
+
+// The most pairs of a tile for moe_direct.  Tiles of up to 192 read an expert's rows fewer times; where those of 128 leave CUs without
+// one all the same (a CU has one workgroup at a time), more of them work side by side.  The feed-forward with weights that are in no
+// cache, us with tiles of 128 / 160 / 192 / 256 pairs: 16 experts of 2,048, width 4,096, 800 tokens on two 230 / 229 / 230 / 229, 1,200
+// 273 / 349 / 266 / 266, 2,048 381 / 356 / 356 / 441; 16 of 1,024, width 2,048, 2,048 on two 155 / 115 / 115 / 141; 128 of 768, width
+// 2,048, 2,048 on eight 458 / 432 / 430 / 430; 64 of 1,408, 2,048 on six 455 / 469 / 462 / 440; 8 of 4,096, width 4,096, 2,048 on two 555
+// / 589 / 538 / 619, of 14,336 1,759 / 1,913 / 1,777 / 1,922.  (Tiles of more than 256 pairs do not fit the accumulation registers.)
+int direct_tile_pairs(int64_t pairs, int experts, int ff, int width, bool gated) {
+  constexpr int CUS = 256;
+  const int rows_up = gated ? kTileRows / 2 : kTileRows;
+  const int64_t up = (ff + rows_up - 1) / rows_up, down = (width + kTileRows - 1) / kTileRows;
+  const int64_t tiles = (pairs / experts / 128 + 1) * experts;
+  return tiles * (up < down ? up : down) > CUS ? 32 * kMostGroups : 128;
 }
 
 // x[t] += sum_j weight_tj y[t * top + j], j ascending.
@@ -1041,7 +1085,7 @@ HFEE_API int hfee_moe_grouped(float* x, int64_t ldx, const void* h, int64_t ldh,
   const int64_t limit32 = (int64_t)1 << 31;
   const bool direct = width % 64 == 0 && ff % 64 == 0 && (width > 64 || (int64_t)n * top < 960) && ((int64_t)n * ldh) * 2 < limit32 && (int64_t)n * top * ff * 2 < limit32 &&
                       (int64_t)ff * width * 2 < limit32;
-  const int tile_pairs = direct ? kWidePairs : kTilePairs, most = (int)(((int64_t)n * top + tile_pairs - 1) / tile_pairs) + experts;
+  const int tile_pairs = direct ? direct_tile_pairs((int64_t)n * top, experts, ff, width, w_gate != nullptr) : kTilePairs, most = (int)(((int64_t)n * top + tile_pairs - 1) / tile_pairs) + experts;
   moe_group_kernel<<<1, 1024, 4 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts, tile_pairs);
   HFEE_CHECK_LAUNCH("moe_group");
   const bool straight = top == 1 && x != nullptr;

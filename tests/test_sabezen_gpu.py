@@ -708,6 +708,47 @@ def test_grouped_experts_at_the_edges_of_their_tiles(counts, width, ff, gated):
     assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
 
 
+@pytest.mark.parametrize("E,width,ff,gated", [(24, 1344, 1472, True), (24, 1344, 2944, False), (330, 128, 64, True), (330, 192, 192, False)])
+def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
+    """Enough tiles to fill the GPU with up to 192 pairs each, at every number of 32s of them and at the edges between, of which
+    one and two tiles and more are made; two, four, six and many steps of K.  Every value against the sums in float64 (a float32 sum
+    of K products is off by at most K roundings of its terms' sizes, an activation by half a bfloat16 ulp more); a pair's numbers
+    stay the same, bit for bit, where few others have its expert."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    edges = (129, 160, 161, 192, 193, 224, 225, 256, 257, 383, 384, 385, 96, 97, 128, 65, 64, 33, 32, 1, 0, 150, 180, 190)
+    counts = [edges[e % len(edges)] for e in range(E)]
+    n = sum(counts)
+    assert (n // E // 128 + 1) * E * min(-(-ff // (128 if gated else 256)), -(-width // 256)) > 256
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(n, generator=g)].to(torch.int32).view(n, 1).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(ff)
+    rand = lambda *shape: (torch.randn(*shape, generator=gen, device="cuda") * shape[-1] ** -0.5).to(torch.bfloat16)      # noqa: E731
+    h, wg, wu, wd = (rand(n, width).float() * width ** 0.5).to(torch.bfloat16), rand(E, ff, width), rand(E, ff, width), rand(E, width, ff)
+
+    def run(rows):
+        m = len(rows)
+        order = torch.zeros(m, dtype=torch.int32, device="cuda")
+        tiles = torch.zeros(3 * ops.moe_group_tiles(m, 1, E) + 1, dtype=torch.int32, device="cuda")
+        act = torch.zeros(m, ff, dtype=torch.bfloat16, device="cuda")
+        y = torch.full((m, width), 7.0, dtype=torch.float32, device="cuda")
+        ops.moe_grouped(None, h[rows].contiguous(), wg if gated else None, wu, wd, 1, order, tiles, act, y, chosen=chosen[rows].contiguous())
+        return act, y
+    everything = torch.arange(n, device="cuda")
+    act, y = run(everything)
+    for e in range(min(E, len(edges))):
+        at = (chosen.view(-1) == e).nonzero().squeeze(1)
+        up = h[at].double() @ wu[e].double().t().contiguous()
+        gate = h[at].double() @ wg[e].double().t().contiguous()
+        want = gate / (1 + torch.exp(-gate)) * up if gated else torch.relu(up) ** 2
+        assert ((act[at].double() - want).abs() <= 2.0 ** -8 * want.abs() + width * 2.0 ** -24 * 30).all()
+        down = act[at].double() @ wd[e].double().t().contiguous()
+        size = act[at].double().abs() @ wd[e].double().abs().t().contiguous()
+        assert ((y[at].double() - down).abs() <= (ff + 2) * 2.0 ** -24 * size).all()
+    some = everything[::5]
+    act2, y2 = run(some)
+    assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
+
+
 @pytest.mark.parametrize("form", ["gated", "clipped", "not gated"])
 @pytest.mark.parametrize("top", [1, 2])
 def test_grouped_experts_have_one_order_of_additions(form, top):

@@ -9,7 +9,8 @@ Two kinds of library:
     the same kernels without a softmax (a key weighs sigmoid(score + a number a head));
   * `attention_mix_bf16_h<H>_g<G>_d<D>`: the matrix-core attention whose heads' scores are mixed,
     compiled per number of heads, of key heads and head size, on demand; with `_vectors` behind the name the
-    mixing itself is on the vector units whatever the sizes (to compare the two: the bits are the same).
+    mixing itself is on the vector units whatever the sizes (to compare the two: the bits are the same);
+  * `pages`: no kernels, the cache manager's loops over pages, for the running Python.
 Libraries are built in-tree (hfee_amd/_lib); if that folder cannot be written, in a
 per-user folder under the system's temporary directory; $HFEE_BUILD_DIR, if set, comes
 before both.  A library is rebuilt when its sources or flags no longer match the stamp
@@ -24,6 +25,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -40,6 +42,7 @@ CORE_SOURCES = ["elementwise.hip", "gemm_f32.hip", "attention_ref.hip", "attenti
                 "sampling.hip", "random_fill.hip", "yardstick.hip", "attention_kv.hip", "rowwise.hip", "attention_mix.hip",
                 "recurrent.hip", "moe.hip", "gated_rows.hip", "post_norm.hip", "linear_chunks.hip",
                 "grouped_rows.hip", "delta_chunks.hip"]
+PAGES_SOURCE = "pages.cpp"
 ATTENTION_SOURCE = "attention_bf16.hip"
 HEAD_DIMS = tuple(range(16, 257, 16))
 ATTENTION_KV_SOURCE = "attention_kv_bf16.hip"      # compiled per (key size, value size)
@@ -124,6 +127,8 @@ def _stamp(sources, defines) -> str:
 def library_spec(name: str):
     if name == "core":
         return CORE_SOURCES, []
+    if name == "pages":
+        return [PAGES_SOURCE], [f"-DHFEE_PYTHON=\"{sys.implementation.cache_tag}\""]
     if name.startswith("attention_bf16_hd"):
         hd = int(name[len("attention_bf16_hd"):])
         if hd not in HEAD_DIMS:
@@ -212,9 +217,12 @@ def build_library(name: str, force: bool = False) -> str:
     t0 = time.time()
     cmds, objs = [], []
     for src in sources:
-        obj = os.path.join(obj_dir, src.replace(".hip", ".o"))
+        obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
         objs.append(obj)
-        cmds.append((src, [cc, *FLAGS, *extra_flags(), *defines, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]))
+        flags = [*FLAGS, *extra_flags()]
+        if src.endswith(".cpp"):                # host code on Python's own objects
+            flags = ["-x", "c++", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-I", sysconfig.get_paths()["include"]]
+        cmds.append((src, [cc, *flags, *defines, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]))
     _run_with_heartbeat(cmds, name)
     so = os.path.join(out_dir, f"libhfee_{name}.so")
     tmp = so + f".{os.getpid()}.tmp"
@@ -229,9 +237,9 @@ def build_library(name: str, force: bool = False) -> str:
 
 def build_all(head_dims=HEAD_DIMS, force: bool = True, kv_sizes=ATTENTION_KV_SIZES, mix_sizes=ATTENTION_MIX_SIZES,
               kv_sigmoid_sizes=ATTENTION_KV_SIGMOID_SIZES, mix_vectors_sizes=ATTENTION_MIX_VECTORS_SIZES) -> list:
-    """Compiles the core library, the attention library of every head size, and the attention
-    libraries for keys and values of different sizes of the listed pairs."""
-    out = [build_library("core", force=force)]
+    """Compiles the core library, that of the cache manager's loops, the attention library of every head size, and
+    the attention libraries for keys and values of different sizes of the listed pairs."""
+    out = [build_library("core", force=force), build_library("pages", force=force)]
     # the attention libraries are independent: build them side by side
     names = [f"attention_bf16_hd{hd}" for hd in head_dims] + [f"attention_kv_bf16_k{dk}_v{dv}" for dk, dv in kv_sizes]
     names += [f"attention_mix_bf16_h{h}_g{g}_d{d}" for h, g, d in mix_sizes]

@@ -178,6 +178,31 @@ def core() -> Library:
     return _core
 
 
+_PAGES_SIGNATURES = {
+    "hfee_token_bytes": [ctypes.py_object],
+    "hfee_follow_chain": [ctypes.py_object, ctypes.py_object, ctypes.c_ssize_t, ctypes.c_ssize_t] + [ctypes.py_object] * 3,
+    "hfee_keep_pages": [ctypes.py_object] * 4 + [ctypes.c_ssize_t] * 2,
+    "hfee_hand_over": [ctypes.py_object] * 4,
+}
+_pages = None
+
+
+def pages():
+    """The cache manager's loops over pages: functions on Python's own objects, called with the interpreter's lock held."""
+    global _pages
+    if _pages is None:
+        with _lock:
+            try:
+                dll = ctypes.PyDLL(build.build_library("pages"))
+                for fn, argtypes in _PAGES_SIGNATURES.items():
+                    f = getattr(dll, fn)
+                    f.argtypes, f.restype = argtypes, ctypes.py_object
+            except (build.BuildError, OSError, AttributeError) as e:
+                raise KernelLibraryError(f"the library 'pages' is not available: {e}") from None
+            _pages = dll
+    return _pages
+
+
 def attention_bf16(head_dim: int) -> Library:
     if head_dim % 16 != 0 or not 16 <= head_dim <= 256:
         raise KernelError(f"the bfloat16 attention kernels take head sizes 16..256 in steps of 16, "

@@ -405,3 +405,82 @@ def test_outgrown_buffers_of_a_workspace_hold_no_more_than_the_one_in_use():
         current, retired = ([b.numel() for b in bufs if b.dtype == dtype] for bufs in (ws._buffers.values(), ws._retired))
         assert len(current) == 1 and current[0] < 2 * 3000 and sum(retired) < current[0]
     assert set(kept) <= {b.data_ptr() for b in [*ws._buffers.values(), *ws._retired]}
+
+
+@pytest.mark.parametrize("pages,groups,stop", [(1, 1, 1), (5, 1, 0), (5, 2, 3), (40, 3, 40), (40, 1, 39)])
+def test_the_native_walks_over_pages(pages, groups, stop):
+    """The walks on the manager's own objects against the same in Python: what is left behind, in which order and under what,
+    where a chain is left (at its end, at another page's tokens, before its first page), who owns what, and that nothing
+    holds on to an object that it has let go."""
+    import sys
+    from collections import OrderedDict
+
+    from hfee_amd.cache.manager import KEPT, PageDigests
+    from hfee_amd.kernels import lib
+    native, size, rng = lib.pages(), 128, random.Random(pages + stop)
+    tokens = [rng.randrange(1 << 40) for _ in range(16 * pages)]
+    own = PageDigests(16)
+    assert own.cover(tokens, pages)
+    digests, tables = list(own.up_to(pages)), [[1000 * g + 700 + b for b in range(pages)] for g in range(groups)]
+    there = digests[pages // 2] if pages > 1 else None
+    kept, want = (OrderedDict({there: "kept before"} if there else {}) for _ in range(2))
+    behind, stays, twice = None, [], []
+    for b in range(pages - 1, -1, -1):
+        if digests[b] in want:
+            twice.append(b)
+        else:
+            want[digests[b]] = (tuple(t[b] for t in tables), own.data[b * size:(b + 1) * size], behind)
+            stays.append(b)
+        behind = digests[b]
+    assert native.hfee_keep_pages(kept, digests, tables, own.data, size, pages) == (
+        [[t[b] for b in stays] for t in tables], [[t[b] for b in twice] for t in tables])
+    assert list(kept.items()) == list(want.items())
+    for short in (dict(digests=digests[1:]), dict(data=own.data[1:]), dict(tables=[t[1:] for t in tables])):
+        args = dict(dict(digests=digests, tables=tables, data=own.data), **short)
+        with pytest.raises(ValueError):
+            native.hfee_keep_pages(OrderedDict(), args["digests"], args["tables"], args["data"], size, pages)
+
+    chain = OrderedDict((d, (tuple(t[b] for t in tables), own.data[b * size:(b + 1) * size], digests[b + 1] if b + 1 < pages else None))
+                        for b, d in enumerate(digests))
+    if stop < pages:                                  # (another page's tokens)
+        chain[digests[stop]] = (chain[digests[stop]][0], b"\0" * size, chain[digests[stop]][2])
+    refs = [sys.getrefcount(d) for d in digests]
+    followed, taken = [], []
+    at, after = native.hfee_follow_chain(chain, own.data, size, 0, digests[0], followed, taken)
+    assert (at, after) == (stop * size, digests[stop] if stop < pages else None)
+    assert followed == digests[:stop] and taken == [tuple(t[b] for t in tables) for b in range(stop)]
+    assert list(chain) == digests[stop:]
+    del followed, taken, chain, at, after
+    assert all(sys.getrefcount(d) <= r for d, r in zip(digests, refs))
+
+    owners = [None] * 4000
+    for page in tables[0]:
+        owners[page] = "a"
+    assert native.hfee_hand_over(owners, tables[0], "a", KEPT) is None and [owners[p] for p in tables[0]] == [KEPT] * pages
+    assert native.hfee_hand_over(owners, tables[0], ("kept prefix",), "b") is None           # (equal, not the same)
+    owners[tables[0][-1]] = "c"
+    assert native.hfee_hand_over(owners, tables[0], "b", "d") == tables[0][-1]
+    assert [owners[p] for p in tables[0]] == ["d"] * (pages - 1) + ["c"]
+    assert native.hfee_hand_over([None], [0], None, "a") == 0 and native.hfee_hand_over(["a"], [0], "a", None) == 0
+    with pytest.raises(IndexError):
+        native.hfee_hand_over(owners, [4000], "a", "b")
+    with pytest.raises(TypeError):
+        native.hfee_hand_over(owners, ["x"], "a", "b")
+
+
+def test_tokens_as_bytes():
+    """Whole numbers of a list as int64; what is no plain one (or no list) is left to the array that takes it; what does not fit is refused."""
+    import numpy as np
+
+    from hfee_amd.cache.manager import PageDigests
+    from hfee_amd.kernels import lib
+    numbers = [0, 1, -1, 128255, 2 ** 63 - 1, -2 ** 63]
+    to_bytes = lib.pages().hfee_token_bytes
+    assert to_bytes(numbers) == np.asarray(numbers, dtype=np.int64).tobytes() and to_bytes([]) == b""
+    assert to_bytes([1, True]) is None and to_bytes([np.int64(3)]) is None and to_bytes((1, 2)) is None
+    for wrong in (2 ** 63, -2 ** 63 - 1):
+        with pytest.raises(OverflowError):
+            to_bytes([1, wrong])
+    for tokens in (list(range(16)), np.arange(16), [np.int64(i) for i in range(16)], [True] * 16):
+        d = PageDigests(16)
+        assert d.cover(tokens, 1) and d.data == np.asarray(tokens, dtype=np.int64).tobytes()

@@ -364,6 +364,24 @@ def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate:
         raise KernelError(f"linear: unsupported dtype {x.dtype}")
 
 
+def linear_gated_f32(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, scratch=None):
+    """out[m, j] = silu(row 2j) * row 2j+1 of the float32 product x @ weight.T, the rows of weight alternating gate / up: `linear`
+    and `swiglu` in one, to the bit.  out [M, N/2]; scratch as in `linear`."""
+    _gpu(out, x, weight, scratch)
+    M, K, lda = _rows2d(x, "linear_gated_f32 x")
+    N, Kw, ldw = _rows2d(weight, "linear_gated_f32 weight")
+    Mo, No, ldc = _rows2d(out, "linear_gated_f32 out")
+    _check(Kw == K and Mo == M and N % 2 == 0 and No == N // 2, "linear_gated_f32: shapes")
+    _check(x.dtype == weight.dtype == out.dtype == torch.float32, "linear_gated_f32: float32 operands expected")
+    if scratch is None:
+        words = linear_scratch(M, N, K, torch.float32, pieces=True)
+        scratch = torch.empty(words, dtype=torch.float32, device=out.device) if words else None
+    else:
+        _check(scratch.dtype == torch.float32 and scratch.is_contiguous(), "linear_gated_f32: float32 scratch expected")
+    lib.core().call("hfee_gemm_f32", _ptr(out), ldc, _ptr(x), lda, _ptr(weight), ldw, M, N, K, 3, _ptr(scratch),
+                    0 if scratch is None else scratch.numel(), _stream())
+
+
 def tiled_plan(m: int, n: int, k: int) -> tuple:
     """(kernel of the first n1 weight rows, n1, kernel of the rest or 0): how `linear`
     lays an aligned bfloat16 product of more than 64 rows over the tiled kernels."""

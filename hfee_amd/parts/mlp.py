@@ -104,6 +104,8 @@ class GatedMLP(FeedForward):
         hn = h.tensor() if lazy else h
         if aligned:   # the gate in the product's epilogue
             ops.linear(act, hn, self.w_gate_up, gate=True, activation=self.activation, numbers=self.numbers)
+        elif self.dtype == torch.float32 and self.activation == "silu":
+            ops.linear_gated_f32(act, hn, self.w_gate_up, **ctx.workspace.split_scratch_f32(n, self.w_gate_up))
         else:
             gate_up = ctx.rows("mlp.gate_up", 2 * F)
             ops.linear(gate_up, hn, self.w_gate_up, **ctx.workspace.split_scratch_f32(n, self.w_gate_up))

@@ -1856,3 +1856,36 @@ def test_a_cache_layer_of_more_than_four_gigabytes():
         close(out, ref_last, 2e-2)
     del layer
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("scratch", ["whole", "cut", "pieces"])
+@pytest.mark.parametrize("M,N,K", [(1, 6, 64), (3, 4096, 512), (3, 6144, 256), (2, 24576, 4096), (16, 4096, 256), (13, 8194, 512), (20, 5002, 320),
+                                   (30, 2048, 64), (40, 2048, 2048), (64, 64, 4096), (127, 4094, 2048), (300, 16384, 256),
+                                   (500, 2048, 2048), (640, 8192, 2048), (5, 1002, 1003), (64, 1002, 1003), (200, 1000, 1028), (400, 2002, 1003)])
+def test_the_gated_float32_product_is_the_product_and_the_gate(M, N, K, scratch):
+    """Every kernel of the float32 product with the gate at its end (few rows at once and by turns, tiles, cuts of K, A in pieces,
+    rows that start anywhere, columns that are no fours) against the product and the gate one after the other: the same
+    bits, with infinities and NaN among the operands too; into rows on 16 bytes and into others."""
+    from hfee_amd.kernels import ops
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 2 / K ** 0.5
+    if M > 1:
+        x[M // 2, K // 3] = float("inf")
+    w[N // 2, K // 2] = float("nan")
+    words = ops.linear_scratch(M, N, K, torch.float32, pieces=scratch == "pieces") if scratch != "whole" else 0
+    room = torch.empty(words, device="cuda")
+    both = torch.empty(M, N, device="cuda")
+    ops.linear(both, x, w, scratch=room)
+    want = torch.empty(M, N // 2, device="cuda")
+    ops.swiglu(want, both[:, 0::2], both[:, 1::2])
+    assert float(want.nan_to_num(0, 0, 0).std()) > 0
+    for pad, at in ((0, 0), (3, 1)):
+        buf = torch.full((M, N // 2 + pad), 7.0, device="cuda")
+        out = buf[:, at:at + N // 2]
+        ops.linear_gated_f32(out, x, w, scratch=room)
+        assert ((out == want) | (out.isnan() & want.isnan())).all()
+        assert (buf[:, :at] == 7.0).all() and (buf[:, at + N // 2:] == 7.0).all()
+    with pytest.raises(ops.KernelError):
+        ops.linear_gated_f32(want, x.double(), w)
+    with pytest.raises(ops.KernelError):
+        ops.linear_gated_f32(both, x, w)

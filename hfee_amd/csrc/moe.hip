@@ -870,6 +870,33 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* __restrict__ x,
   }
 }
 
+// The same for rows on 16 bytes, four values a thread, the pairs' rows asked for two at a time: bound by its bytes.  2,048 tokens of
+// 4,096 on two experts each (134 MB) 37 us by single values, 22 so (6.1 TB/s).
+__global__ __launch_bounds__(256) void moe_combine_fours_kernel(float* __restrict__ x, int64_t ldx, const float* __restrict__ y,
+                                                                const float* __restrict__ pair_weights, float weight, int top,
+                                                                int width) {
+  const int64_t t = blockIdx.x;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  if (c >= width) return;
+  f32x4* to = reinterpret_cast<f32x4*>(x + t * ldx + c);
+  const f32x4 before = *to;
+  const float* from = y + t * top * width + c;
+  f32x4 total = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < top; j += 2) {
+    const bool two = j + 1 < top;
+    const f32x4 one = *reinterpret_cast<const f32x4*>(from + (int64_t)j * width);
+    const f32x4 other = *reinterpret_cast<const f32x4*>(from + (int64_t)(two ? j + 1 : j) * width);
+    const float w1 = pair_weights != nullptr ? pair_weights[t * top + j] : weight;
+    const float w2 = pair_weights != nullptr ? pair_weights[t * top + (two ? j + 1 : j)] : weight;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      total[i] = fmaf(one[i], w1, total[i]);
+      if (two) total[i] = fmaf(other[i], w2, total[i]);
+    }
+  }
+  *to = before + total;
+}
+
 // One wave a token.  A lane looks through its share of the experts (lane, lane + 64, ...) for the largest
 // logit that is not chosen yet (a bit a share in the lane's own registers says which are); the wave's lanes
 // meet over (logit, number), the larger logit and of two equal ones the lower number, and every lane ends
@@ -1117,9 +1144,14 @@ HFEE_API int hfee_moe_grouped(float* x, int64_t ldx, const void* h, int64_t ldh,
     HFEE_CHECK_LAUNCH("moe_group_down");
   }
   if (top > 1 && x != nullptr) {
-    int parts = (width + 255) / 256;
-    if (parts > 64) parts = 64;
-    moe_combine_kernel<<<dim3(n, parts), 256, 0, stream>>>(x, ldx, y, pair_weights, weight, top, width);
+    // (the width is a multiple of 32)
+    if (ldx % 4 == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0 && width <= 65535 * 1024) {
+      moe_combine_fours_kernel<<<dim3(n, (width / 4 + 255) / 256), 256, 0, stream>>>(x, ldx, y, pair_weights, weight, top, width);
+    } else {
+      int parts = (width + 255) / 256;
+      if (parts > 64) parts = 64;
+      moe_combine_kernel<<<dim3(n, parts), 256, 0, stream>>>(x, ldx, y, pair_weights, weight, top, width);
+    }
     HFEE_CHECK_LAUNCH("moe_combine");
   }
   return 0;

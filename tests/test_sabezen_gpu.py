@@ -749,6 +749,37 @@ def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
     assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
 
 
+@pytest.mark.parametrize("n,top,width", [(70, 2, 32), (33, 3, 1024), (300, 5, 1056), (17, 4, 4128)])
+@pytest.mark.parametrize("weighted", [True, False])
+def test_experts_outputs_add_up_to_the_same_bits_in_any_rows(n, top, width, weighted):
+    """The kernel that adds up a token's experts, by fours into rows on 16 bytes and by single values into others: the weighted sums in
+    the order of the experts, rounded where a float32 multiply-add rounds, then added to the stream."""
+    from hfee_amd.kernels import ops
+    E, ff = 7, 32
+    g = torch.Generator().manual_seed(n)
+    rand = lambda *shape: (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).to(torch.bfloat16).cuda()      # noqa: E731
+    h, wg, wu, wd = rand(n, width) * 16, rand(E, ff, width), rand(E, ff, width), rand(E, width, ff)
+    chosen = torch.rand(n, E, generator=g).topk(top).indices.to(torch.int32).cuda()
+    weights = torch.rand(n, top, generator=g).cuda() if weighted else None
+    results = []
+    for pad, at in ((0, 0), (4, 0), (3, 0), (4, 1)):
+        x = torch.ones(n, width + pad, device="cuda")[:, at:at + width]
+        order = torch.zeros(n * top, dtype=torch.int32, device="cuda")
+        tiles = torch.zeros(3 * ops.moe_group_tiles(n, top, E) + 1, dtype=torch.int32, device="cuda")
+        act = torch.zeros(n * top, ff, dtype=torch.bfloat16, device="cuda")
+        y = torch.zeros(n * top, width, device="cuda")
+        ops.moe_grouped(x, h, wg, wu, wd, top, order, tiles, act, y, weight=1.0 / top, chosen=chosen, pair_weights=weights)
+        results.append(x.clone())
+    assert all(torch.equal(results[0], r) for r in results[1:])
+    total = torch.zeros(n, width, dtype=torch.float64, device="cuda")
+    for j in range(top):
+        w = weights[:, j:j + 1].double() if weighted else torch.tensor(1.0 / top, dtype=torch.float32).double().item()
+        total = (total + y.view(n, top, width)[:, j].double() * w).float().double()
+    # (a float64 sum that is then rounded may round twice: one ulp of the sum's largest part)
+    assert ((results[0].double() - (1.0 + total)).abs() <= 2.0 ** -22 * (1 + y.view(n, top, width).double().abs().sum(1))).all()
+    assert float((results[0] - 1).std()) > 0
+
+
 @pytest.mark.parametrize("form", ["gated", "clipped", "not gated"])
 @pytest.mark.parametrize("top", [1, 2])
 def test_grouped_experts_have_one_order_of_additions(form, top):

@@ -265,3 +265,13 @@ def test_where_a_product_of_a_prompt_is_cut_along_k():
     assert cuts(17, 4096, 14336) == 8 and cuts(64, 4096, 4096) == 8 and cuts(64, 6144, 4096) == 5
     # products that fill the chip
     assert cuts(2048, 4096, 4096) == 0 and cuts(2048, 28672, 4096) == 0 and cuts(512, 28672, 4096) == 0
+
+
+def test_no_float32_product_gets_pieces_where_smaller_tiles_are_faster():
+    """Shapes timed both ways: the rule that lays rows down as pieces knows that a product's last round of tiles may be nearly
+    empty and that a segment of K has an end of its own."""
+    from hfee_amd.kernels import ops
+    for M, N, K in [(1025, 8192, 512), (300, 16384, 2048), (257, 16384, 2048), (129, 28672, 4096), (129, 12288, 1536), (4096, 2560, 1024)]:
+        assert ops.linear_f32_plan(M, N, K, True, pieces=True) == ops.linear_f32_plan(M, N, K, True), (M, N, K)
+    for M, N, K in [(1000, 28672, 4096), (500, 16384, 2048), (1200, 8192, 8192), (800, 4096, 4096), (127, 28672, 4096)]:
+        assert ops.linear_f32_plan(M, N, K, True, pieces=True)[0] == "pieces", (M, N, K)

@@ -34,6 +34,7 @@ _CORE_SIGNATURES = {
     "hfee_gemm_f32_scratch": [I, I, I],
     "hfee_gemm_f32_pieces_scratch": [I, I, I],
     "hfee_gemm_f32_plan": [I, I, I, I],
+    "hfee_gemm_f32_rows_at_a_time": [I, I, I],
     "hfee_attention_f32": [P, L, P, L, P, P, P, P, I, I, I, I, I, F, I, P, I, I, I, P],
     "hfee_attention_ref": [P, L, P, L, P, I, P, P, P, I, I, I, I, I, F, I, I, P],
     "hfee_gemm_bf16": [P, I, L, P, L, P, L, I, I, I, I, P, L, I, F, F, P],

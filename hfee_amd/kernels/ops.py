@@ -240,6 +240,11 @@ def linear_f32_plan(m: int, n: int, k: int, cut: bool, pieces: bool = False):
     return ("rows", plan - 256) if plan >= 256 else (plan // 16, plan % 16)
 
 
+def linear_f32_rows_at_a_time(m: int, n: int, k: int) -> int:
+    """How many of m rows a float32 product does at a time where it has all scratch that it can use.  (For tests.)"""
+    return int(lib.core().raw("hfee_gemm_f32_rows_at_a_time")(int(m), int(n), int(k)))
+
+
 def linear_cuts(x: torch.Tensor, weight: torch.Tensor, scratch) -> int:
     """x @ weight.T (bfloat16) cut along K over workgroups, the partial products left in scratch
     as that many float32 matrices [M, N] one after the other, for a kernel that adds them up on

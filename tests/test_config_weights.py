@@ -267,11 +267,39 @@ def test_where_a_product_of_a_prompt_is_cut_along_k():
     assert cuts(2048, 4096, 4096) == 0 and cuts(2048, 28672, 4096) == 0 and cuts(512, 28672, 4096) == 0
 
 
+def test_how_many_rows_a_float32_product_does_at_a_time():
+    """The host's rule for float32 products whose rows may be laid down as pieces first: at once where the pieces are at most 384 MB,
+    else at once without them or in parts that are in pieces; scratch that is asked for is what the way that is taken uses, so a
+    product that is not in pieces is still cut along K."""
+    import torch
+
+    from hfee_amd.kernels import ops
+    assert ops.linear_scratch(1200, 64, 16384, torch.float32, pieces=True) == ops.linear_scratch(1200, 64, 16384, torch.float32) > 0
+    for M, N, K in [(2048, 4096, 14336), (1500, 4096, 14336), (1153, 5120, 13824), (1665, 512, 14336), (2048, 256, 28672), (2304, 256, 28672)]:
+        assert ops.linear_f32_rows_at_a_time(M, N, K) == M
+    most, in_parts = 3 << 25, 0
+    for K in (512, 4096, 14336, 28672, 65536):
+        for N in (64, 256, 2050, 4096, 28672):
+            for M in (17, 40, 129, 512, 1200, 2048, 2305, 5000, 9000):
+                rows = ops.linear_f32_rows_at_a_time(M, N, K)
+                pieces, cut = (ops.linear_scratch(M, N, K, torch.float32, pieces=p) for p in (True, False))
+                plan = ops.linear_f32_plan(rows, N, K, True, pieces=True) if rows > 32 else (0, 0)
+                too_many = -(-M // 128) * 128 * K * 3 // 2 > most          # (in whole tiles)
+                if rows < M:
+                    in_parts += 1
+                    assert too_many and most >= rows * K * 3 // 2 and rows % 128 == 0 and plan[0] == "pieces" and pieces >= rows * K * 3 // 2
+                elif plan[0] != "pieces" or too_many:
+                    assert pieces == cut, (M, N, K)
+                else:
+                    assert pieces >= M * K * 3 // 2
+    assert in_parts > 0
+
+
 def test_no_float32_product_gets_pieces_where_smaller_tiles_are_faster():
     """Shapes timed both ways: the rule that lays rows down as pieces knows that a product's last round of tiles may be nearly
     empty and that a segment of K has an end of its own."""
     from hfee_amd.kernels import ops
     for M, N, K in [(1025, 8192, 512), (300, 16384, 2048), (257, 16384, 2048), (129, 28672, 4096), (129, 12288, 1536), (4096, 2560, 1024)]:
         assert ops.linear_f32_plan(M, N, K, True, pieces=True) == ops.linear_f32_plan(M, N, K, True), (M, N, K)
-    for M, N, K in [(1000, 28672, 4096), (500, 16384, 2048), (1200, 8192, 8192), (800, 4096, 4096), (127, 28672, 4096)]:
+    for M, N, K in [(1000, 28672, 4096), (500, 16384, 2048), (1200, 8192, 8192), (800, 4096, 4096), (127, 28672, 4096), (2048, 4096, 14336)]:
         assert ops.linear_f32_plan(M, N, K, True, pieces=True)[0] == "pieces", (M, N, K)

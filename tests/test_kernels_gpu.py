@@ -190,11 +190,11 @@ def test_gemm_f32_that_would_leave_the_chip_idle_goes_by_blocks_of_rows_or_cuts(
 
 
 @pytest.mark.parametrize("M,N,K,pairs", [(500, 16384, 512, 0), (385, 7937, 2080, 0), (640, 6440, 4128, 0), (1300, 4100, 16384, 0),
-                                         (999, 2050, 4096, 1), (300, 8190, 4096, 1)])
+                                         (2400, 2100, 28672, 1), (999, 2050, 4096, 1), (300, 8190, 4096, 1)])
 @pytest.mark.parametrize("accumulate", [False, True])
 def test_gemm_f32_of_rows_cut_into_pieces_first(M, N, K, pairs, accumulate):
     """Large products whose rows are laid down as pieces by a launch of their own (last tiles of one row and of few, widths that fill no tile,
-    K of few steps, of an odd number and in one segment's remainder, more rows than are done at a time, K cut over workgroups): the
+    K of few steps, of an odd number and in one segment's remainder, rows in two parts, K cut over workgroups): the
     bits of the product that cuts the rows itself, an infinity and a NaN where they belong, and nothing behind the scratch is written."""
     from hfee_amd.kernels import ops
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
@@ -202,8 +202,8 @@ def test_gemm_f32_of_rows_cut_into_pieces_first(M, N, K, pairs, accumulate):
     w = torch.randn(N, K, generator=g, device=DEV)
     x[1, 7], w[3, 9] = float("nan"), float("inf")
     c0 = torch.randn(M, N, generator=g, device=DEV)
-    rows = min(M, (3 << 23) // (K // 32 * 768 * 8) * 128)
-    assert ops.linear_f32_plan(rows, N, K, True, pieces=True) == ("pieces", pairs, 0)
+    rows = ops.linear_f32_rows_at_a_time(M, N, K)
+    assert ops.linear_f32_plan(rows, N, K, True, pieces=True) == ("pieces", pairs, 0) and rows == (1280 if M == 2400 else M)
     words = ops.linear_scratch(M, N, K, torch.float32, pieces=True)
     assert words >= -(-rows // 16) * (K // 32) * 768
     scratch = torch.full((words + 64,), 7.0, device=DEV)

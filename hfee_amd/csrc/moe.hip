@@ -403,19 +403,33 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTilePairs = 64, kTileRows = 256;
 
+// How many pairs of one expert a tile holds at most: `pairs`, or `more` (0: never) where the step's pairs lie so that larger tiles are
+// faster, by the blocks of rows and the columns of the two products.
+struct TileSizes {
+  int pairs, more, up_blocks, up_columns, down_blocks, down_columns;
+};
+
+// What the two products take in tiles of which the largest has `groups` groups of 32 pairs, in a unit of its own: rounds of a workgroup a
+// CU, each as long as that tile.
+__device__ __forceinline__ float tiles_cost(const TileSizes& s, int tiles, int groups) {
+  constexpr int CUS = 256;
+  const float rounds = (float)((tiles * s.up_blocks + CUS - 1) / CUS) * s.up_columns + (float)((tiles * s.down_blocks + CUS - 1) / CUS) * s.down_columns;
+  return rounds * ((float)max(groups, 2) + 0.5f);
+}
+
 // One workgroup.  order: the pairs (t * top + j) by expert; tiles: (expert, first place in order, pairs)
-// for every tile, tiles[3 * most_tiles] holds their number.  An expert's pairs make as few tiles of up to tile_pairs as they
+// for every tile, tiles[3 * most_tiles] holds their number.  An expert's pairs make as few tiles of up to the step's tile size as they
 // can, of whole 32s but the last one and alike to within one 32.  Which of an expert's pairs comes first is
-// left to chance; nothing that is computed depends on it.
+// left to chance; nothing that is computed depends on it.  The first wave goes over the experts, 64 at a time.  (One thread took 128 of
+// them one by one, 6 us of the feed-forward: 512 tokens on eight 281 us -> 275 with the choice of a size.)
 __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order, int* __restrict__ tiles, int most_tiles,
                                                          const int* __restrict__ chosen, const int* __restrict__ table,
                                                          const int* __restrict__ token_ids, int n, int top, int experts,
-                                                         int tile_pairs) {
+                                                         TileSizes sizes) {
   extern __shared__ int lds[];
   int* counts = lds;                  // [experts]
   int* starts = lds + experts;        // [experts]
   int* cursor = lds + 2 * experts;    // [experts]
-  int* first_tile = lds + 3 * experts;
   const int pairs = n * top;
   for (int e = threadIdx.x; e < experts; e += blockDim.x) counts[e] = cursor[e] = 0;
   __syncthreads();
@@ -424,31 +438,58 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(int* __restrict__ order
     if (e >= 0 && e < experts) atomicAdd(&counts[e], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, tile = 0;
-    for (int e = 0; e < experts; ++e) {
-      starts[e] = at;
-      first_tile[e] = tile;
-      at += counts[e];
-      tile += (counts[e] + tile_pairs - 1) / tile_pairs;
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x;
+    int tile_pairs = sizes.pairs;
+    if (sizes.more > 0) {
+      int number[2] = {0, 0}, largest[2] = {0, 0};      // of tiles, and groups of 32 pairs in one, by either size
+      for (int e = lane; e < experts; e += 64)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int count = counts[e], size = i == 0 ? sizes.pairs : sizes.more, mine = (count + size - 1) / size;
+          number[i] += mine;
+          if (mine > 0) largest[i] = max(largest[i], ((count + 31) / 32 + mine - 1) / mine);
+        }
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          number[i] += __shfl_xor(number[i], off, kWave);
+          largest[i] = max(largest[i], __shfl_xor(largest[i], off, kWave));
+        }
+      if (tiles_cost(sizes, number[1], largest[1]) < 0.93f * tiles_cost(sizes, number[0], largest[0])) tile_pairs = sizes.more;
     }
-    tiles[3 * most_tiles] = tile;
+    int at = 0, tile = 0;             // of the experts behind
+    for (int e0 = 0; e0 < experts; e0 += 64) {
+      const int e = e0 + lane, count = e < experts ? counts[e] : 0, n_tiles = (count + tile_pairs - 1) / tile_pairs;
+      int pairs_to = count, tiles_to = n_tiles;      // of the lanes up to this one
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int p = __shfl_up(pairs_to, off, kWave), t = __shfl_up(tiles_to, off, kWave);
+        if (lane >= off) {
+          pairs_to += p;
+          tiles_to += t;
+        }
+      }
+      const int start = at + pairs_to - count, first_tile = tile + tiles_to - n_tiles, groups = (count + 31) / 32;
+      if (e < experts) starts[e] = start;
+      for (int i = 0, to = 0; i < n_tiles; ++i) {
+        const int mine = 32 * (groups / n_tiles + (i < groups % n_tiles ? 1 : 0));
+        int* tl = tiles + 3 * (first_tile + i);
+        tl[0] = e;
+        tl[1] = start + to;
+        tl[2] = min(mine, count - to);
+        to += mine;
+      }
+      at += __shfl(pairs_to, 63, kWave);
+      tile += __shfl(tiles_to, 63, kWave);
+    }
+    if (lane == 0) tiles[3 * most_tiles] = tile;
   }
   __syncthreads();
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = expert_of(chosen, table, token_ids, p / top, p % top, top);
     if (e >= 0 && e < experts) order[starts[e] + atomicAdd(&cursor[e], 1)] = p;
-  }
-  for (int e = threadIdx.x; e < experts; e += blockDim.x) {
-    const int n_tiles = (counts[e] + tile_pairs - 1) / tile_pairs, groups = (counts[e] + 31) / 32;
-    for (int i = 0, at = 0; i < n_tiles; ++i) {
-      const int mine = 32 * (groups / n_tiles + (i < groups % n_tiles ? 1 : 0));
-      int* tl = tiles + 3 * (first_tile[e] + i);
-      tl[0] = e;
-      tl[1] = starts[e] + at;
-      tl[2] = min(mine, counts[e] - at);
-      at += mine;
-    }
   }
 }
 
@@ -843,18 +884,21 @@ int launch_direct(int most, void* dst, int64_t ldo, const bf16_t* src, int64_t l
   return 0;
 }
 
-// The most pairs of a tile for moe_direct.  Tiles of up to 192 read an expert's rows fewer times; where those of 128 leave CUs without
-// one all the same (a CU has one workgroup at a time), more of them work side by side.  The feed-forward with weights that are in no
-// cache, us with tiles of 128 / 160 / 192 / 256 pairs: 16 experts of 2,048, width 4,096, 800 tokens on two 230 / 229 / 230 / 229, 1,200
-// 273 / 349 / 266 / 266, 2,048 381 / 356 / 356 / 441; 16 of 1,024, width 2,048, 2,048 on two 155 / 115 / 115 / 141; 128 of 768, width
-// 2,048, 2,048 on eight 458 / 432 / 430 / 430; 64 of 1,408, 2,048 on six 455 / 469 / 462 / 440; 8 of 4,096, width 4,096, 2,048 on two 555
-// / 589 / 538 / 619, of 14,336 1,759 / 1,913 / 1,777 / 1,922.  (Tiles of more than 256 pairs do not fit the accumulation registers.)
-int direct_tile_pairs(int64_t pairs, int experts, int ff, int width, bool gated) {
-  constexpr int CUS = 256;
+// The tiles of moe_direct.  Tiles of up to 192 pairs read an expert's rows fewer times, and are fewer: a gain where the workgroups (one
+// a CU) then are fewer rounds and the last one's CUs are not idle for as long as the tiles are larger.  How many tiles there are
+// depends on how the pairs lie, which only the device knows, and so does the largest tile, for which an XCD with few pairs of many
+// experts waits for another one: rounds times the largest tile is what a step is expected to take, and the larger tiles are taken where that
+// is 7 % less.  Fitted to 160 steps (8 to 128 experts, 512 to 2,048 tokens; pairs spread evenly, over half or a quarter of the
+// experts, by a power law, all on as few as a token uses): of the better of 128 and 192 it misses 0.05 %, and none is more than 1.5 % slower than
+// with 128.  (By the mean number of pairs instead, which is known on the host, steps whose pairs are not spread evenly lost up to a third.)
+// The feed-forward with weights that are in no cache, us with 128 / 192: 16 experts of 2,048, width 4,096, 2,048 tokens on two, evenly
+// 359 / 342, on two experts 248 / 320, by a power law 350 / 366; on one expert each, evenly 289 / 246, by a power law 271 / 355; 1,200 on two 255 / 249 and 262 /
+// 328; 16 of 1,024, width 2,048, 2,048 on two 152 / 109; 64 of 1,408, 2,048 on six 437 / 451; 128 of 768, 2,048 on eight 422 / 398 and 432 / 490; 8 of 4,096,
+// width 4,096, 2,048 on two 541 / 525 and 543 / 622.  (Tiles of more than 192: 256 pairs leave CUs idle, 440 us in the first case; more do not fit the
+// accumulation registers.)
+TileSizes direct_tiles(int ff, int width, bool gated) {
   const int rows_up = gated ? kTileRows / 2 : kTileRows;
-  const int64_t up = (ff + rows_up - 1) / rows_up, down = (width + kTileRows - 1) / kTileRows;
-  const int64_t tiles = (pairs / experts / 128 + 1) * experts;
-  return tiles * (up < down ? up : down) > CUS ? 32 * kMostGroups : 128;
+  return TileSizes{128, 32 * kMostGroups, (ff + rows_up - 1) / rows_up, width, (width + kTileRows - 1) / kTileRows, ff};
 }
 
 // x[t] += sum_j weight_tj y[t * top + j], j ascending.
@@ -1112,8 +1156,9 @@ HFEE_API int hfee_moe_grouped(float* x, int64_t ldx, const void* h, int64_t ldh,
   const int64_t limit32 = (int64_t)1 << 31;
   const bool direct = width % 64 == 0 && ff % 64 == 0 && (width > 64 || (int64_t)n * top < 960) && ((int64_t)n * ldh) * 2 < limit32 && (int64_t)n * top * ff * 2 < limit32 &&
                       (int64_t)ff * width * 2 < limit32;
-  const int tile_pairs = direct ? direct_tile_pairs((int64_t)n * top, experts, ff, width, w_gate != nullptr) : kTilePairs, most = (int)(((int64_t)n * top + tile_pairs - 1) / tile_pairs) + experts;
-  moe_group_kernel<<<1, 1024, 4 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts, tile_pairs);
+  const TileSizes sizes = direct ? direct_tiles(ff, width, w_gate != nullptr) : TileSizes{kTilePairs, 0, 0, 0, 0, 0};
+  const int most = (int)(((int64_t)n * top + sizes.pairs - 1) / sizes.pairs) + experts;      // (larger tiles are not more)
+  moe_group_kernel<<<1, 1024, 3 * experts * sizeof(int), stream>>>(order, tiles, most, chosen, table, token_ids, n, top, experts, sizes);
   HFEE_CHECK_LAUNCH("moe_group");
   const bool straight = top == 1 && x != nullptr;
   void* down = straight ? (void*)x : (void*)y;

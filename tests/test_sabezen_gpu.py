@@ -708,10 +708,11 @@ def test_grouped_experts_at_the_edges_of_their_tiles(counts, width, ff, gated):
     assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
 
 
-@pytest.mark.parametrize("E,width,ff,gated", [(24, 1344, 1472, True), (24, 1344, 2944, False), (330, 128, 64, True), (330, 192, 192, False)])
+@pytest.mark.parametrize("E,width,ff,gated", [(24, 1344, 1472, True), (24, 1344, 2944, False), (186, 128, 64, True), (186, 192, 192, False),
+                                              (330, 128, 64, True), (330, 192, 192, False)])
 def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
-    """Enough tiles to fill the GPU with up to 192 pairs each, at every number of 32s of them and at the edges between, of which
-    one and two tiles and more are made; two, four, six and many steps of K.  Every value against the sums in float64 (a float32 sum
+    """Enough tiles to fill the GPU with up to 192 pairs each (the last two: 128), at every number of 32s of them and at the edges
+    between, of which one and two tiles and more are made; two, four, six and many steps of K.  Every value against the sums in float64 (a float32 sum
     of K products is off by at most K roundings of its terms' sizes, an activation by half a bfloat16 ulp more); a pair's numbers
     stay the same, bit for bit, where few others have its expert."""
     from hfee_amd.kernels import ops
@@ -719,7 +720,6 @@ def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
     edges = (129, 160, 161, 192, 193, 224, 225, 256, 257, 383, 384, 385, 96, 97, 128, 65, 64, 33, 32, 1, 0, 150, 180, 190)
     counts = [edges[e % len(edges)] for e in range(E)]
     n = sum(counts)
-    assert (n // E // 128 + 1) * E * min(-(-ff // (128 if gated else 256)), -(-width // 256)) > 256
     chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(n, generator=g)].to(torch.int32).view(n, 1).cuda()
     gen = torch.Generator(device="cuda").manual_seed(ff)
     rand = lambda *shape: (torch.randn(*shape, generator=gen, device="cuda") * shape[-1] ** -0.5).to(torch.bfloat16)      # noqa: E731
@@ -732,9 +732,11 @@ def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
         act = torch.zeros(m, ff, dtype=torch.bfloat16, device="cuda")
         y = torch.full((m, width), 7.0, dtype=torch.float32, device="cuda")
         ops.moe_grouped(None, h[rows].contiguous(), wg if gated else None, wu, wd, 1, order, tiles, act, y, chosen=chosen[rows].contiguous())
-        return act, y
+        return act, y, tiles
     everything = torch.arange(n, device="cuda")
-    act, y = run(everything)
+    act, y, tiles = run(everything)
+    most = 3 * ((n + 127) // 128 + E)
+    assert int(tiles[:most].view(-1, 3)[:int(tiles[most]), 2].max()) == (128 if E == 330 else 192)
     for e in range(min(E, len(edges))):
         at = (chosen.view(-1) == e).nonzero().squeeze(1)
         up = h[at].double() @ wu[e].double().t().contiguous()
@@ -745,8 +747,54 @@ def test_grouped_experts_with_many_pairs_each(E, width, ff, gated):
         size = act[at].double().abs() @ wd[e].double().abs().t().contiguous()
         assert ((y[at].double() - down).abs() <= (ff + 2) * 2.0 ** -24 * size).all()
     some = everything[::5]
-    act2, y2 = run(some)
+    act2, y2, _ = run(some)
     assert torch.equal(act2, act[some]) and torch.equal(y2, y[some])
+
+
+@pytest.mark.parametrize("size,experts,counts", [
+    (1024, 16, (192, [300] * 16)), (1024, 16, (128, [4800] + [0] * 15)), (1024, 16, (192, [0, 600] * 8)), (1024, 18, (192, [0] + [300] * 16)),
+    (1024, 16, (128, [1600, 800, 530, 400, 320, 265, 228, 200, 178, 160, 145, 133, 123, 114, 106, 100])), (1024, 1, (128, [300])),
+    (512, 64, (192, [300] * 64)), (512, 65, (128, [128] * 65)), (512, 65, (128, [0] * 64 + [7200])), (256, 129, (192, [0] + [300] * 128)),
+    (256, 200, (192, list(range(200)))), (256, 200, (192, [3000 // (e + 1) for e in range(200)]))])
+@pytest.mark.parametrize("top", [1, 3])
+def test_tiles_of_grouped_experts_go_by_how_the_pairs_lie(size, experts, counts, top):
+    """What the device makes of a step's pairs: every pair in the order once, among its expert's; an expert's tiles as few as their size
+    allows, of whole 32s and alike; and the larger size where the rule expects it to be faster: rounds of 256 workgroups times the
+    largest tile, 7 % less.  The same number of pairs spread evenly and on one expert go two ways."""
+    from hfee_amd.kernels import ops
+    E, width, ff, (most_pairs, counts) = experts, size, size, counts
+    counts = list(counts) + [0] * (E - len(counts))
+    none = -sum(counts) % top                              # (pairs of no expert)
+    g = torch.Generator().manual_seed(E + top)
+    flat = torch.cat([torch.full((c,), e) for e, c in enumerate(counts + [none])])
+    chosen = flat[torch.randperm(len(flat), generator=g)].to(torch.int32).view(-1, top)
+    n = chosen.shape[0]
+
+    def cost(pairs):
+        made = [(-(-c // pairs), -(-c // 32)) for c in counts if c]
+        tiles, largest = sum(t for t, _ in made), max(2, *(-(-groups // t) for t, groups in made), 2)
+        return (-(-tiles * (ff // 128) // 256) * width + -(-tiles * (width // 256) // 256) * ff) * (largest + 0.5)
+    assert most_pairs == (192 if cost(192) < 0.93 * cost(128) else 128)
+    h = torch.zeros(n, width, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(E, ff, width, dtype=torch.bfloat16, device="cuda")
+    order = torch.full((n * top,), -1, dtype=torch.int32, device="cuda")
+    tiles = torch.zeros(3 * ops.moe_group_tiles(n, top, E) + 1, dtype=torch.int32, device="cuda")
+    act, y = torch.zeros(n * top, ff, dtype=torch.bfloat16, device="cuda"), torch.zeros(n * top, width, device="cuda")
+    ops.moe_grouped(None, h, w, w, w, top, order, tiles, act, y, chosen=chosen.cuda())
+    lie, most = tiles.tolist(), 3 * ((n * top + 127) // 128 + E)
+    want, start = [], 0
+    for e, count in enumerate(counts):
+        n_tiles, groups, at = -(-count // most_pairs), -(-count // 32), 0
+        for i in range(n_tiles):
+            mine = min(32 * (groups // n_tiles + (i < groups % n_tiles)), count - at)
+            want.append((e, start + at, mine))
+            at += mine
+        assert at == count
+        start += count
+    assert [tuple(lie[3 * i:3 * i + 3]) for i in range(lie[most])] == want
+    order, of = order.tolist(), chosen.view(-1).tolist()
+    assert sorted(order[:start]) == [p for p, e in enumerate(of) if e < E] and set(order[start:]) <= {-1}
+    assert all(of[p] == e for e, first, count in want for p in order[first:first + count])
 
 
 @pytest.mark.parametrize("n,top,width", [(70, 2, 32), (33, 3, 1024), (300, 5, 1056), (17, 4, 4128)])

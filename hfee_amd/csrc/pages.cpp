@@ -140,7 +140,7 @@ HFEE_API PyObject* hfee_hand_over(PyObject* owners, PyObject* pages, PyObject* o
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(pages); ++i) {
     PyObject* number = PyList_GET_ITEM(pages, i);
     Py_INCREF(number);
-    Py_ssize_t page = PyLong_AsSsize_t(number);
+    Py_ssize_t page = PyNumber_AsSsize_t(number, PyExc_IndexError);      // (whatever a list takes for an index)
     if (page < 0 && !PyErr_Occurred()) page += PyList_GET_SIZE(owners);      // (as a list's own index does)
     PyObject* other = nullptr;                      // whether somebody else has it
     if (!PyErr_Occurred()) {

@@ -468,6 +468,23 @@ def test_the_native_walks_over_pages(pages, groups, stop):
         native.hfee_hand_over(owners, ["x"], "a", "b")
 
 
+def test_pages_are_handed_over_by_any_number_that_is_an_index():
+    """Page numbers that come out of an array, from a generator, negative ones: as a list's own index takes them; what it refuses is
+    refused, and nothing behind it is handed over."""
+    import numpy as np
+    pool = PagePool(8)
+    for _ in range(5):
+        pool.take("a")
+    pool.hand_over(np.array([0, 1], dtype=np.int32), "a", "b")
+    pool.hand_over((p for p in [np.int64(2), -5]), "a", "c")
+    pool.hand_over([True], "b", "d")
+    assert [pool.owner_of(p) for p in range(6)] == ["b", "d", "c", "c", "a", None]
+    for wrong, error in (("x", TypeError), (1.0, TypeError), (8, IndexError), (2 ** 70, IndexError), (5, CacheError)):
+        with pytest.raises(error):
+            pool.hand_over([wrong, 4], "a", "b")
+        assert pool.owner_of(4) == "a"
+
+
 def test_tokens_as_bytes():
     """Whole numbers of a list as int64; what is no plain one (or no list) is left to the array that takes it; what does not fit is refused."""
     import numpy as np

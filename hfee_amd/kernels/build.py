@@ -10,7 +10,8 @@ Two kinds of library:
   * `attention_mix_bf16_h<H>_g<G>_d<D>`: the matrix-core attention whose heads' scores are mixed,
     compiled per number of heads, of key heads and head size, on demand; with `_vectors` behind the name the
     mixing itself is on the vector units whatever the sizes (to compare the two: the bits are the same);
-  * `pages`: no kernels, the cache manager's loops over pages, for the running Python.
+  * `pages`: no kernels, the cache manager's loops over pages, for the running Python, by the host's compiler ($CXX first) and
+    without the HIP runtime.
 Libraries are built in-tree (hfee_amd/_lib); if that folder cannot be written, in a
 per-user folder under the system's temporary directory; $HFEE_BUILD_DIR, if set, comes
 before both.  A library is rebuilt when its sources or flags no longer match the stamp
@@ -37,6 +38,9 @@ ARCH = "gfx950"
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument"]
+
+# host code, on Python's own objects: its library is for one interpreter's layout of them
+HOST_FLAGS = ["-x", "c++", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden"]
 
 CORE_SOURCES = ["elementwise.hip", "gemm_f32.hip", "attention_ref.hip", "attention_f32.hip", "gemm_bf16.hip", "gemm_skinny.hip",
                 "sampling.hip", "random_fill.hip", "yardstick.hip", "attention_kv.hip", "rowwise.hip", "attention_mix.hip",
@@ -87,6 +91,18 @@ def hipcc() -> str:
                      "the HIP kernels cannot be built")
 
 
+def host_compiler() -> str:
+    for cand in (os.environ.get("CXX"), "g++", "c++", "clang++", "/opt/rocm/llvm/bin/clang++"):
+        found = shutil.which(cand) if cand else None
+        if found:
+            return found
+    raise BuildError("no C++ compiler was found (looked at $CXX, g++, c++ and clang++)")
+
+
+def _is_host(sources) -> bool:
+    return all(src.endswith(".cpp") for src in sources)
+
+
 def _writable(path: str) -> bool:
     try:
         os.makedirs(path, exist_ok=True)
@@ -117,7 +133,7 @@ def build_dirs() -> list:
 
 def _stamp(sources, defines) -> str:
     h = hashlib.sha256()
-    h.update(" ".join(FLAGS + extra_flags() + sorted(defines)).encode())
+    h.update(" ".join((HOST_FLAGS if _is_host(sources) else FLAGS) + extra_flags() + sorted(defines)).encode())
     for name in sorted(set(sources) | {"common.h"} | {f for f in os.listdir(CSRC) if f.endswith(".h")}):
         with open(os.path.join(CSRC, name), "rb") as f:
             h.update(name.encode() + b"\0" + f.read())
@@ -128,7 +144,7 @@ def library_spec(name: str):
     if name == "core":
         return CORE_SOURCES, []
     if name == "pages":
-        return [PAGES_SOURCE], [f"-DHFEE_PYTHON=\"{sys.implementation.cache_tag}\""]
+        return [PAGES_SOURCE], [f"-DHFEE_PYTHON=\"{sysconfig.get_config_var('SOABI') or sys.implementation.cache_tag}\""]
     if name.startswith("attention_bf16_hd"):
         hd = int(name[len("attention_bf16_hd"):])
         if hd not in HEAD_DIMS:
@@ -197,7 +213,7 @@ def _run_with_heartbeat(cmds, what: str):
             _say(f"still compiling {what} ({int(last - start)} s; {len(procs) + len(pending)} file(s) to go)")
         time.sleep(0.05)
     if failed:
-        raise BuildError("hipcc failed:\n" + "\n".join(f"--- {l} ---\n{o}" for l, o in failed))
+        raise BuildError("the compiler failed:\n" + "\n".join(f"--- {l} ---\n{o}" for l, o in failed))
 
 
 def build_library(name: str, force: bool = False) -> str:
@@ -210,23 +226,23 @@ def build_library(name: str, force: bool = False) -> str:
     out_dir = next((d for d in build_dirs() if _writable(d)), None)
     if out_dir is None:
         raise BuildError("no writable folder for the kernel library (set HFEE_BUILD_DIR)")
-    cc = hipcc()
+    host = _is_host(sources)
+    cc = host_compiler() if host else hipcc()
     obj_dir = os.path.join(out_dir, "obj", name)
     os.makedirs(obj_dir, exist_ok=True)
-    _say(f"compiling kernel library '{name}' for {ARCH} ({len(sources)} source file(s)) into {out_dir}")
+    _say(f"compiling {'host' if host else 'kernel'} library '{name}' for {'this Python' if host else ARCH} ({len(sources)} source file(s)) into {out_dir}")
     t0 = time.time()
     cmds, objs = [], []
     for src in sources:
         obj = os.path.join(obj_dir, os.path.splitext(src)[0] + ".o")
         objs.append(obj)
-        flags = [*FLAGS, *extra_flags()]
-        if src.endswith(".cpp"):                # host code on Python's own objects
-            flags = ["-x", "c++", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-I", sysconfig.get_paths()["include"]]
-        cmds.append((src, [cc, *flags, *defines, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]))
+        flags = [*HOST_FLAGS, "-I", sysconfig.get_paths()["include"]] if host else FLAGS
+        cmds.append((src, [cc, *flags, *extra_flags(), *defines, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]))
     _run_with_heartbeat(cmds, name)
     so = os.path.join(out_dir, f"libhfee_{name}.so")
     tmp = so + f".{os.getpid()}.tmp"
-    _run_with_heartbeat([("link", [cc, "--offload-arch=" + ARCH, "-shared", "-fPIC", *objs, "-o", tmp])], name)
+    link = [cc, *extra_flags()] if host else [cc, "--offload-arch=" + ARCH]
+    _run_with_heartbeat([("link", [*link, "-shared", "-fPIC", *objs, "-o", tmp])], name)
     os.replace(tmp, so)
     with open(so + ".stamp", "w") as f:
         f.write(_stamp(sources, defines))

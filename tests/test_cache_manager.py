@@ -501,3 +501,29 @@ def test_tokens_as_bytes():
     for tokens in (list(range(16)), np.arange(16), [np.int64(i) for i in range(16)], [True] * 16):
         d = PageDigests(16)
         assert d.cover(tokens, 1) and d.data == np.asarray(tokens, dtype=np.int64).tobytes()
+
+
+def test_the_walks_library_is_the_hosts_own(tmp_path, monkeypatch):
+    """It is compiled and linked without hipcc and needs no HIP runtime; flags that are given are applied, to it too, and make another
+    library; and a library is for one layout of Python's objects."""
+    import ctypes
+
+    from hfee_amd.kernels import build
+
+    def no_hipcc():
+        raise build.BuildError("no hipcc here")
+    monkeypatch.setattr(build, "hipcc", no_hipcc)
+    monkeypatch.setenv("HFEE_BUILD_DIR", str(tmp_path / "plain"))
+    with open(build.build_library("pages"), "rb") as f:
+        assert b"libamdhip64" not in f.read()
+    plain = build._stamp(*build.library_spec("pages"))
+    (tmp_path / "mark.h").write_text('extern "C" __attribute__((visibility("default"))) int hfee_mark() { return 7; }\n')
+    monkeypatch.setenv("HFEE_EXTRA_FLAGS", f"-include {tmp_path / 'mark.h'}")
+    monkeypatch.setenv("HFEE_BUILD_DIR", str(tmp_path / "marked"))
+    assert ctypes.CDLL(build.build_library("pages")).hfee_mark() == 7 and build._stamp(*build.library_spec("pages")) != plain
+    monkeypatch.delenv("HFEE_EXTRA_FLAGS")
+    monkeypatch.setattr(build, "HOST_FLAGS", [*build.HOST_FLAGS, "-O1"])
+    assert build._stamp(*build.library_spec("pages")) != plain
+    monkeypatch.undo()
+    monkeypatch.setattr(build.sysconfig, "get_config_var", lambda name: "another-abi")
+    assert build._stamp(*build.library_spec("pages")) != plain

@@ -27,7 +27,7 @@ chain before the pages in front of it.  Only models whose groups all keep every 
 do this (a window group has given pages back; fixed-size state cannot be cut back).
 
 This file is bookkeeping only (no tensors); storage.py holds the device memory.  The walks over the pages of a kept
-prefix, of which the GPU waits for every one at an admission and a release, are native (csrc/pages.cpp).
+prefix, of which the GPU waits for every one at an admission and a release, are native where they can be (walks.py).
 """
 from __future__ import annotations
 
@@ -37,7 +37,7 @@ from dataclasses import dataclass, field
 
 import numpy as np
 
-from ..kernels import lib
+from .walks import walks
 
 
 class OutOfPages(RuntimeError):
@@ -126,7 +126,7 @@ class PagePool:
         return self._owner[page]
 
     def hand_over(self, pages, owner, new_owner) -> None:
-        wrong = lib.pages().hfee_hand_over(self._owner, list(pages), owner, new_owner)
+        wrong = walks().hfee_hand_over(self._owner, list(pages), owner, new_owner)
         if wrong is not None:
             raise CacheError(f"page {wrong} belongs to {self._owner[wrong]!r}, not {owner!r}")
 
@@ -156,7 +156,7 @@ class PageDigests:
             return False
         if end > have:
             more = list(tokens[have:end])
-            data = lib.pages().hfee_token_bytes(more)      # (raises before anything is taken in)
+            data = walks().hfee_token_bytes(more)      # (raises before anything is taken in)
             self.data += np.asarray(more, dtype=np.int64).tobytes() if data is None else data
             self.tokens += more
         return True
@@ -178,7 +178,7 @@ class PageDigests:
         """From the first page on, the pages that `kept` has under these digests with these tokens: they leave it.  A kept
         page says which digest the page behind it had when it was kept: the page that lies under it, if it holds these
         tokens, is the one that a digest made here would find, so that a chain is followed without making its digests."""
-        taken, size, data, follow = [], self.page_bytes, self.data, lib.pages().hfee_follow_chain
+        taken, size, data, follow = [], self.page_bytes, self.data, walks().hfee_follow_chain
         at, following = 0, None
         while True:
             at, following = follow(kept, data, size, at, following, self._digests, taken)
@@ -242,7 +242,7 @@ class CacheManager:
         self._kept: OrderedDict = OrderedDict()
         self.prefix_hits = 0          # tokens taken over from kept prefixes so far
         if self.keep_prefixes:
-            lib.pages()               # (loaded here, not by the first admission)
+            walks()               # (settled here, not by the first admission)
         for pool in self.pools:
             pool.reclaimable = lambda: len(self._kept)
             pool.reclaim = self._drop_oldest_kept
@@ -295,7 +295,7 @@ class CacheManager:
                 own = PageDigests(self.page_size)
                 own.cover(tokens, keep)
             # (the deepest page first: it is the first to go; a prefix that is kept already needs no copy)
-            stays, twice = lib.pages().hfee_keep_pages(self._kept, own.up_to(keep), rc.tables, own.data, own.page_bytes, keep)
+            stays, twice = walks().hfee_keep_pages(self._kept, own.up_to(keep), rc.tables, own.data, own.page_bytes, keep)
             for pool, staying, copies in zip(self.pools, stays, twice):
                 pool.hand_over(staying, request_id, KEPT)
                 for page in copies:

@@ -255,7 +255,11 @@ def build_all(head_dims=HEAD_DIMS, force: bool = True, kv_sizes=ATTENTION_KV_SIZ
               kv_sigmoid_sizes=ATTENTION_KV_SIGMOID_SIZES, mix_vectors_sizes=ATTENTION_MIX_VECTORS_SIZES) -> list:
     """Compiles the core library, that of the cache manager's loops, the attention library of every head size, and
     the attention libraries for keys and values of different sizes of the listed pairs."""
-    out = [build_library("core", force=force), build_library("pages", force=force)]
+    out = [build_library("core", force=force)]
+    try:
+        out.append(build_library("pages", force=force))
+    except BuildError as e:            # (the manager's loops are there in Python too)
+        _say(f"the library 'pages' was left out: {e}")
     # the attention libraries are independent: build them side by side
     names = [f"attention_bf16_hd{hd}" for hd in head_dims] + [f"attention_kv_bf16_k{dk}_v{dv}" for dk, dv in kv_sizes]
     names += [f"attention_mix_bf16_h{h}_g{g}_d{d}" for h, g, d in mix_sizes]

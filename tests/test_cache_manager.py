@@ -527,3 +527,72 @@ def test_the_walks_library_is_the_hosts_own(tmp_path, monkeypatch):
     monkeypatch.undo()
     monkeypatch.setattr(build.sysconfig, "get_config_var", lambda name: "another-abi")
     assert build._stamp(*build.library_spec("pages")) != plain
+
+
+def test_kept_prefixes_without_the_native_walks(monkeypatch):
+    """Where the library cannot be had the manager warns once and does the same in Python: two managers, one each way, through the same
+    admissions, steps, releases and pages that run out, agree in everything that they hold; what is refused is refused in both."""
+    import warnings
+
+    from hfee_amd.cache import manager, walks
+    from hfee_amd.kernels import build, lib
+
+    def unavailable():
+        raise lib.KernelLibraryError("no Python.h here")
+    with monkeypatch.context() as m:
+        m.setattr(lib, "pages", unavailable)
+        m.setattr(walks, "_walks", None)
+        with pytest.warns(RuntimeWarning, match="no Python.h here"):
+            CacheManager([CacheGroupSpec("full", (2, 1, 16), (0,))], 16, 8, 2, keep_prefixes=True)
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            assert walks.walks() is walks.PythonWalks
+            CacheManager([CacheGroupSpec("full", (2, 1, 16), (0,))], 16, 8, 2, keep_prefixes=True)
+    groups = [CacheGroupSpec("full", (2, 1, 16), (0,)), CacheGroupSpec("full", (2, 2, 16), (1,))]
+    both = [CacheManager(groups, 16, 40, 6, keep_prefixes=True) for _ in range(2)]
+    sides = (lib.pages(), walks.PythonWalks)
+    rng, live, prefix = random.Random(4), {}, [5] * 70
+    for step in range(400):
+        name, tokens = f"r{step}", None
+        if live and (len(live) == 6 or rng.random() < 0.45):
+            name = rng.choice(sorted(live))
+            tokens, act = live.pop(name), "release"
+        else:
+            tokens, act = prefix[:rng.randrange(71)] + [rng.randrange(9) for _ in range(rng.randrange(1, 60))], "admit"
+            live[name] = tokens
+        results = []
+        for side, mgr in zip(sides, both):
+            with monkeypatch.context() as m:
+                m.setattr(manager, "walks", lambda side=side: side)
+                if act == "release":
+                    mgr.release(name, tokens)
+                    results.append(None)
+                else:
+                    rc = mgr.admit(name, tokens)
+                    try:
+                        mgr.reserve(name, len(tokens) - rc.length)
+                        mgr.commit(name, len(tokens) - rc.length)
+                        results.append((rc.length, rc.reused, rc.tables))
+                    except OutOfPages:
+                        mgr.release(name)
+                        results.append("none free")
+                mgr.check()
+        assert results[0] == results[1]
+        if results[0] == "none free":
+            del live[name]
+        a, b = both
+        assert list(a._kept.items()) == list(b._kept.items()) and a.prefix_hits == b.prefix_hits
+        assert [(p._free, p._owner) for p in a.pools] == [(p._free, p._owner) for p in b.pools]
+    assert both[0].prefix_hits > 1000
+    for side in sides:
+        with pytest.raises(ValueError):
+            side.hfee_keep_pages({}, [b"d"], [[1, 2]], b"\0" * 256, 128, 2)
+        with pytest.raises(IndexError):
+            side.hfee_hand_over(["a"], [1], "a", "b")
+        assert side.hfee_hand_over([None], [0], None, "a") == 0
+
+    monkeypatch.setattr(build, "build_library", lambda name, force=False: unavailable_library() if name == "pages" else name)
+
+    def unavailable_library():
+        raise build.BuildError("no Python.h here")
+    assert "core" in build.build_all(head_dims=(), kv_sizes=(), mix_sizes=(), kv_sigmoid_sizes=(), mix_vectors_sizes=())

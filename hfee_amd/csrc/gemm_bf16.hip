@@ -1396,9 +1396,8 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_bf16_skinny_kernel(
 }
 
 // Which tiled kernel takes an aligned product: force_kernel 2 the 128 x 128 tiles, 4 the
-// 256 x 256 tiles, 5 the 256 x 128 tiles, 6 the 256 x 192 tiles, 7 and 8 the 128 x 128 and 128 x 192 tiles
-// of the kernel that loads straight into LDS, anything else the one expected to be fastest (9 and 10, its tiles of 192 x 128 and
-// 192 x 192, among them):
+// 256 x 256 tiles, 5 the 256 x 128 tiles, 6 the 256 x 192 tiles, 7 to 10 the 128 x 128, 128 x 192, 192 x 128 and 192 x 192 tiles
+// of the kernel that loads straight into LDS, anything else the one expected to be fastest:
 // rounds of tiles over the chip times the time of a tile, with the share of the matrix
 // peak that each kernel was measured to reach on a busy CU (128 x 128: two workgroups a
 // CU; the large tiles reach more the longer K is, and a tile of empty rows costs as
@@ -1499,7 +1498,7 @@ int launch_aligned(void* C, int64_t ldc, const bf16_t* A, int64_t lda, const bf1
                    int M, int N, int K, int force_kernel, hipStream_t stream, const QkvArgs& qkv = QkvArgs{},
                    const Partial& partial = Partial{}) {
   const bool large_ok = large_fits(lda, ldw, M, N, K);
-  if (force_kernel == 2 || (force_kernel >= 4 && force_kernel <= 8))
+  if (force_kernel == 2 || (force_kernel >= 4 && force_kernel <= 10))
     return launch_tiled_kernel<MODE>(force_kernel >= 4 && !large_ok ? 2 : force_kernel, C, ldc, A, lda, W, ldw, M, N, K,
                                      stream, qkv, partial, true);
   // (the q/k/v epilogue finds a column's head by its number: those products stay whole)
@@ -1554,11 +1553,11 @@ int launch(void* C, int64_t ldc, const bf16_t* A, int64_t lda, const bf16_t* W, 
 }  // namespace
 
 // How an aligned product of more than 64 rows is laid over the tiled kernels when nothing
-// is forced: kernel of the first n1 columns, n1, kernel of the rest (0: none).  For
-// tests and for reading a profile.
-HFEE_API int hfee_gemm_bf16_plan(int M, int N, int K, int* first, int* n1, int* second) {
+// is forced: kernel of the first n1 columns, n1, kernel of the rest (0: none; the q/k/v product
+// is one launch always).  For tests and for reading a profile.
+HFEE_API int hfee_gemm_bf16_plan(int M, int N, int K, int qkv, int* first, int* n1, int* second) {
   HFEE_REQUIRE(M > 0 && N > 0 && K > 0 && first && n1 && second, "gemm_bf16_plan: bad arguments");
-  const TiledPlan p = plan_tiled(M, N, K, large_fits(K, K, M, N, K), true);
+  const TiledPlan p = plan_tiled(M, N, K, large_fits(K, K, M, N, K), qkv == 0);
   *first = p.first;
   *n1 = p.n1;
   *second = p.second;
@@ -1589,8 +1588,8 @@ HFEE_API int hfee_gemm_bf16_scratch(int M, int N, int K) {
 // rows of W alternate gate/up; C is [M, N/2] bfloat16 = activation(gate) * up, the
 // activation being gate_act: GATE_SILU ..., with its two numbers where it has any; aligned operands only).
 // force_kernel: 0 choose by the sizes, 1 skinny, 2 tiled 128 x 128, 3 the simple tiled
-// kernel, 4 tiled 256 x 256, 5 tiled 256 x 128, 6 tiled 256 x 192, 7 tiled 128 x 128 and 8 tiled 128 x 192 loaded
-// straight into LDS (for tests of each kernel alone; 4 to 8 fall back to 2 where they do not apply).
+// kernel, 4 tiled 256 x 256, 5 tiled 256 x 128, 6 tiled 256 x 192, 7 to 10 tiled 128 x 128, 128 x 192, 192 x 128 and
+// 192 x 192 loaded straight into LDS (for tests of each kernel alone; 4 to 10 fall back to 2 where they do not apply).
 // scratch: null, or hfee_gemm_bf16_scratch(M, N, K) float32 words, 16-byte aligned.
 HFEE_API int hfee_gemm_bf16(void* C, int out_mode, int64_t ldc, const void* A, int64_t lda, const void* W,
                             int64_t ldw, int M, int N, int K, int force_kernel, float* scratch,
@@ -1603,7 +1602,7 @@ HFEE_API int hfee_gemm_bf16(void* C, int out_mode, int64_t ldc, const void* A, i
   HFEE_REQUIRE(lda >= K && ldw >= K, "gemm_bf16: a leading dimension is shorter than its row");
   HFEE_REQUIRE(out_mode >= 0 && out_mode <= 3, "gemm_bf16: unknown output mode %d", out_mode);
   HFEE_REQUIRE(ldc >= (out_mode == 3 ? N / 2 : N), "gemm_bf16: ldc is shorter than a row of the result");
-  HFEE_REQUIRE(force_kernel >= 0 && force_kernel <= 8, "gemm_bf16: unknown kernel choice %d", force_kernel);
+  HFEE_REQUIRE(force_kernel >= 0 && force_kernel <= 10, "gemm_bf16: unknown kernel choice %d", force_kernel);
   if (M == 0) return 0;
   const bool vec = (K % 8 == 0) && (lda % 8 == 0) && (ldw % 8 == 0) &&
                    ((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0);

@@ -328,8 +328,8 @@ def linear(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, accumulate:
     gate (bfloat16, aligned shapes): the rows of weight alternate gate/up and
     out[m, j] = activation(row 2j) * row 2j+1, out [M, N/2] ("clipped" with its `numbers`, see GATE_ACTIVATIONS).
     kernel (bfloat16 only): 0 automatic, 1 skinny, 2 tiled 128x128, 3 the simple tiled
-    kernel, 4 tiled 256x256, 5 tiled 256x128, 6 tiled 256x192, 7 and 8 tiled 128x128 and 128x192
-    loaded straight into LDS."""
+    kernel, 4 tiled 256x256, 5 tiled 256x128, 6 tiled 256x192, 7 to 10 tiled 128x128, 128x192,
+    192x128 and 192x192 loaded straight into LDS."""
     _gpu(out, x, weight)
     M, K, lda = _rows2d(x, "linear x")
     N, Kw, ldw = _rows2d(weight, "linear weight")
@@ -387,12 +387,12 @@ def linear_gated_f32(out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, s
                     0 if scratch is None else scratch.numel(), _stream())
 
 
-def tiled_plan(m: int, n: int, k: int) -> tuple:
+def tiled_plan(m: int, n: int, k: int, qkv: bool = False) -> tuple:
     """(kernel of the first n1 weight rows, n1, kernel of the rest or 0): how `linear`
-    lays an aligned bfloat16 product of more than 64 rows over the tiled kernels."""
+    lays an aligned bfloat16 product of more than 64 rows over the tiled kernels, or, with `qkv`, `linear_fused` the q/k/v product."""
     import ctypes
     first, n1, second = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
-    lib.core().call("hfee_gemm_bf16_plan", m, n, k, ctypes.byref(first), ctypes.byref(n1), ctypes.byref(second))
+    lib.core().call("hfee_gemm_bf16_plan", m, n, k, int(qkv), ctypes.byref(first), ctypes.byref(n1), ctypes.byref(second))
     return first.value, n1.value, second.value
 
 

@@ -452,7 +452,8 @@ def test_gemm_bf16_tiled_large(M, N, K, kernel):
                                         (576, 28674, 704, 10), (1281, 6144, 1024, 10), (602, 28672, 512, 8)])
 def test_gemm_bf16_in_tiles_of_192_rows(M, N, K, tile):
     """Whole products whose tiles of 192 rows pad less than those of 256 (first, last and full numbers of rows, weight rows that
-    are no multiple of a tile, K of an odd number of steps), and rounds of 128 x 192: every epilogue, the bits of 256 x 128 tiles."""
+    are no multiple of a tile, K of an odd number of steps), and rounds of 128 x 192: every epilogue but that of q/k/v, the bits of
+    256 x 128 tiles; the same where the tile is asked for by its number."""
     from hfee_amd.kernels import ops
     assert ops.tiled_plan(M, N, K) == (tile, N, 0)
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
@@ -461,7 +462,7 @@ def test_gemm_bf16_in_tiles_of_192_rows(M, N, K, tile):
     c0 = torch.randn(M, N, generator=g, device=DEV)
     for mode in ("bf16", "f32", "add", "gate"):
         outs = []
-        for kernel in (0, 5):
+        for kernel in (0, 5, tile):
             if mode == "gate":
                 out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
                 ops.linear(out, x, w, gate=True, kernel=kernel)
@@ -472,7 +473,7 @@ def test_gemm_bf16_in_tiles_of_192_rows(M, N, K, tile):
                 out = torch.full((M, N), float("nan"), dtype=torch.bfloat16 if mode == "bf16" else torch.float32, device=DEV)
                 ops.linear(out, x, w, kernel=kernel)
             outs.append(out)
-        assert torch.equal(*outs), mode
+        assert torch.equal(*outs[:2]) and torch.equal(*outs[1:]), mode
     ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
     assert ((outs[0].double() - torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]).abs() <=
             2e-2 * (1 + mag[:, 0::2]) * (1 + mag[:, 1::2])).all()
@@ -737,6 +738,18 @@ def test_fused_qkv_rotation_and_cache_write(H, K, hd, half, M, norm):
 def test_fused_qkv_through_the_tiled_kernels_with_whole_steps_of_k(H, K, hd, half, M, d):
     """The same epilogue behind the tiled kernels that take a K of whole steps of 64: one round of
     128 x 128 tiles loaded straight into LDS (the first three), the large tiles (the last)."""
+    _check_fused_qkv(H, K, hd, half, M, False, d)
+
+
+@pytest.mark.parametrize("H,K,hd,half,M,d,tile", [(30, 1, 128, 64, 1415, 640, 9), (46, 1, 128, 64, 1290, 512, 10), (75, 1, 80, 16, 1301, 576, 10),
+                                                  (152, 1, 128, 64, 790, 512, 8)])
+def test_fused_qkv_through_tiles_of_192_rows(H, K, hd, half, M, d, tile):
+    """The same epilogue behind the tiles of 192 x 128 and 192 x 192 and in rounds of 128 x 192, whose columns begin within heads of 128 and
+    of 80, with a last tile of few rows."""
+    from hfee_amd.kernels import ops
+    N = (H + 2 * K) * hd
+    assert ops.tiled_plan(M, N, d, qkv=True) == (tile, N, 0)
+    assert tile != 8 or -(-M // 128) * -(-N // 192) > 256
     _check_fused_qkv(H, K, hd, half, M, False, d)
 
 

@@ -793,27 +793,37 @@ inline int64_t cut_workgroups(const Cuts& c, int M, int N) {
 // What a product in cuts takes, in us, while its workgroups are one round: a start and an end, a time a step of 64 columns (both
 // less where CUs stand idle: the others' clock is higher), and the cuts' partial products there and back.  Measured inside
 // 0.9 to 1.15 of it at 96 to 1,024 rows of the 8B and 13B shapes' narrow products.
+struct CutCost {
+  double ends, step;
+};
+
+inline int cut_steps(const Cuts& c, int K) { return ((K + c.cuts - 1) / c.cuts + 63) / 64; }
+
 inline double cuts_us(const Cuts& c, int M, int N, int K) {
-  struct { double ends, step; } t = c.tm == 4 ? decltype(t){18.5, 0.67} : c.tm == 3 ? decltype(t){15, 0.59}
-                                  : decltype(t){6.5, 0.535};
+  const CutCost t = c.tm == 4 ? CutCost{18.5, 0.67} : c.tm == 3 ? CutCost{15, 0.59} : CutCost{6.5, 0.535};
   const int64_t workgroups = cut_workgroups(c, M, N);
-  const int steps = ((K + c.cuts - 1) / c.cuts + 63) / 64;
   const double rounds = (double)((workgroups + 255) / 256), filled = workgroups >= 256 ? 1.0 : workgroups / 256.0;
-  return rounds * (t.ends + steps * t.step) * (0.65 + 0.35 * filled) + c.cuts * (double)M * N * 4 / 5e6;
+  return rounds * (t.ends + cut_steps(c, K) * t.step) * (0.65 + 0.35 * filled) + c.cuts * (double)M * N * 4 / 5e6;
 }
 
 // The tiles of 256 rows pad many numbers of rows by up to a half, and the matrix cores spend their power on the padding as on the
 // rest; and their number may leave CUs idle.  The same cuts (so the same bits) go through tiles of 192 x 128 where those are
 // expected to be faster.
-// us, tiles of 256 x 128 or 128 x 128 against them, with the kernel that adds the cuts: N 4,096, K 14,336 at 181 / 320 / 520 / 602 /
-// 700 rows 45 / 62 / 90 / 96 / 100 against 38.5 / 55 / 86 / 85 / 90; N 4,096, K 4,096 at 320 / 602 rows 31.5 / 40 against 28 / 36; N 5,120,
+// us, tiles of 256 x 128 or 128 x 128 against them, with the kernel that adds the cuts: N 4,096, K 14,336 at 181 / 320 / 602 /
+// 700 rows 45 / 62 / 96 / 100 against 38.5 / 55 / 85 / 90; N 4,096, K 4,096 at 320 / 602 rows 31.5 / 40 against 28 / 36; N 5,120,
 // K 13,824 at 181 / 300 / 520 rows 47 / 72 / 99 against 44 / 62.5 / 88; N 2,048, K 8,192 at 320 rows 31 against 26; the product alone, N 6,144,
 // K 4,096 at 181 / 320 rows 23 / 31 against 21 / 28; N 15,360, K 5,120 at 181 rows 46 against 42.5.
+// The formula does not know what bounds a long cut whose tiles are nearly full and leave an eighth of the CUs idle: not power.  There
+// the larger tiles stay: N 4,096, K 14,336 at 538 / 561 rows 83.6 / 84.2 against 86.5 / 87.5, K 11,008 68.3 / 68.4 against 70.0 / 71.0; N 2,048, K 8,192
+// at 1,297 rows 55.2 against 57.2; N 6,144, K 24,576 at 372 rows 144.7 against 148.2 (but at 300 rows, a fifth of a tile padding, 157
+// against 135).  Elsewhere tiles of 192 rows gain 7 % over 331 products in cuts, and none is more than 1.6 % slower.
 inline Cuts cuts_of(int M, int N, int K) {
   const int cuts = even_splits(M, N, K);
   const Cuts best{cuts, large_tile_cuts(M, N, K) == cuts ? 4 : 2, 2};
   if (cuts < 2 || M <= 128 || K % 64 != 0) return best;
   const Cuts rows192{cuts, 3, 2};
+  const int padded = (M + 191) / 192 * 192;
+  if (cut_workgroups(rows192, M, N) <= 224 && cut_steps(rows192, K) >= 64 && M * 10ll >= padded * 9ll) return best;
   return cuts_us(rows192, M, N, K) < 0.97 * cuts_us(best, M, N, K) ? rows192 : best;
 }
 
@@ -1426,7 +1436,8 @@ inline TiledPlan plan_tiled(int M, int N, int K, bool large_ok, bool may_split) 
     // (128 x 192 tiles, the 256 x 128 kernel compiled for them: where they are at most one a CU.  2,048 rows of
     // 3,072 columns are 256 of them and 96 of 256 x 128: N 3,072 at K 2,048 / 3,072 / 8,192 33.2 / 48.9 / 97.0 us against
     // 35.6 / 53.3 / 101.9; 1,024 rows of N 6,144, K 4,096 52.2 against 56.6, of N 5,120, K 5,120 60.6 against 66.8;
-    // in more rounds they are as good as what they pad and leave idle)
+    // in more rounds they are as good as what they pad and leave idle; N 28,672, K 4,096 at 577 / 602 / 640 rows 148 / 144 / 151 where two
+    // launches, which a share of 0.335 would prefer there and nowhere else among the shapes of this repository, take 159 / 151 / 155)
     if (k == 8) return rounds(t, cus) * 128 * 192 / (0.34 * fill);
     if (k == 9) return rounds(t, cus) * 192 * 128 / (0.335 * fill);
     if (k == 10) return rounds(t, cus) * 192 * 192 / (0.42 * fill);

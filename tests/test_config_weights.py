@@ -303,3 +303,14 @@ def test_no_float32_product_gets_pieces_where_smaller_tiles_are_faster():
         assert ops.linear_f32_plan(M, N, K, True, pieces=True) == ops.linear_f32_plan(M, N, K, True), (M, N, K)
     for M, N, K in [(1000, 28672, 4096), (500, 16384, 2048), (1200, 8192, 8192), (800, 4096, 4096), (127, 28672, 4096), (2048, 4096, 14336)]:
         assert ops.linear_f32_plan(M, N, K, True, pieces=True)[0] == "pieces", (M, N, K)
+
+
+def test_which_products_in_cuts_take_tiles_of_192_rows():
+    """Shapes timed both ways: cuts of 64 steps and more whose tiles of 192 rows are nearly full and leave CUs idle stay with the larger
+    ones; what the cuts are does not depend on it (nor do the bits)."""
+    from hfee_amd.kernels import ops
+    for M, N, K, cuts in [(538, 4096, 14336, 2), (576, 4096, 14336, 2), (561, 4096, 11008, 2), (1297, 2048, 8192, 2), (372, 6144, 24576, 2)]:
+        assert ops.cut_plan(M, N, K) == (cuts, 256, 128)
+    for M, N, K, cuts in [(300, 6144, 24576, 2), (577, 4096, 14336, 2), (320, 4096, 14336, 4), (520, 5120, 13824, 2), (181, 4096, 14336, 8),
+                          (520, 4096, 4096, 2), (300, 5120, 13824, 3)]:
+        assert ops.cut_plan(M, N, K) == (cuts, 192, 128)
